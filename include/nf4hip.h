@@ -90,6 +90,18 @@ int nf4hip_dq_compress(const float* absmax, int64_t nblocks, int nested_blocksiz
 int nf4hip_dq_reconstruct(const uint8_t* absmax_q, const float* absmax2, const float* map256, float offset,
                           int64_t nblocks, int nested_blocksize, float* absmax, void* stream);
 
+/*
+ * nf4hip_quantize followed by the nested quantisation of its absmax, what bitsandbytes' quantize_4bit(...,
+ * compress_statistics=True) does: offset = the mean of absmax (float64 sum, rounded to fp32 once), written to the device
+ * (one fp32) so that nothing waits for the host, then nf4hip_dq_compress with it.  map_out / code_out (NULL: not wanted)
+ * receive copies of map256 and of the 16-entry NF4 code book.  `workspace`: nf4hip_quantize_dq_workspace_bytes(n,
+ * blocksize) bytes, 16-byte aligned, in any state.
+ */
+size_t nf4hip_quantize_dq_workspace_bytes(int64_t n, int blocksize);
+int nf4hip_quantize_dq(const void* w, int w_dtype, int64_t n, int blocksize, int nested_blocksize, const float* map256,
+                       uint8_t* packed, uint8_t* absmax_q, float* absmax2, float* offset, float* map_out_or_null,
+                       float* code_out_or_null, void* workspace, size_t workspace_bytes, void* stream);
+
 /* Same as nf4hip_dequantize with absmax given in nested form. */
 int nf4hip_dequantize_dq(const uint8_t* packed, const uint8_t* absmax_q, const float* absmax2, const float* map256,
                          float offset, int nested_blocksize, const float* lut16, int64_t n, int blocksize, void* out,

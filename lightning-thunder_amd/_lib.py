@@ -50,6 +50,8 @@ SYMBOLS = {
     "nf4hip_abi_version": (_i32, []),
     "nf4hip_last_error": (ctypes.c_char_p, []),
     "nf4hip_quantize": (_i32, [_vp, _i32, _i64, _i32, _vp, _vp, _vp]),
+    "nf4hip_quantize_dq_workspace_bytes": (_sz, [_i64, _i32]),
+    "nf4hip_quantize_dq": (_i32, [_vp, _i32, _i64, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
     "nf4hip_dequantize": (_i32, [_vp, _vp, _vp, _i64, _i32, _vp, _i32, _vp]),
     "nf4hip_dq_compress": (_i32, [_vp, _i64, _i32, _vp, _f32, _vp, _vp, _vp]),
     "nf4hip_dq_reconstruct": (_i32, [_vp, _vp, _vp, _f32, _i64, _i32, _vp, _vp]),

@@ -211,6 +211,35 @@ int nf4hip_quantize(const void* w, int w_dtype, int64_t n, int blocksize, uint8_
     return NF4HIP_OK;
 }
 
+size_t nf4hip_quantize_dq_workspace_bytes(int64_t n, int blocksize) {
+    const int bl = block_log2(blocksize);
+    if (n <= 0 || bl < 0) return 0;
+    return nf4::DQ_SUMS * sizeof(double) + (size_t)((n + blocksize - 1) / blocksize) * sizeof(float);
+}
+
+int nf4hip_quantize_dq(const void* w, int w_dtype, int64_t n, int blocksize, int nested_blocksize, const float* map256,
+                       uint8_t* packed, uint8_t* absmax_q, float* absmax2, float* offset, float* map_out_or_null,
+                       float* code_out_or_null, void* workspace, size_t workspace_bytes, void* stream) {
+    const char* name = "nf4hip_quantize_dq";
+    if (n <= 0) return fail(NF4HIP_E_SHAPE, "%s: n = %lld is not positive", name, (long long)n);
+    if (!valid_dtype(w_dtype)) return fail(NF4HIP_E_DTYPE, "%s: unknown dtype code %d", name, w_dtype);
+    const int bl = block_log2(blocksize), nl = block_log2(nested_blocksize);
+    if (bl < 0 || nl < 0) return fail(NF4HIP_E_BLOCKSIZE, "%s: blocksize %d / %d unsupported", name, blocksize, nested_blocksize);
+    if (!w || !map256 || !packed || !absmax_q || !absmax2 || !offset) return fail(NF4HIP_E_NULL, "%s: null pointer", name);
+    if (!aligned16(w) || !aligned16(packed) || !aligned16(absmax_q) || !aligned16(absmax2) || !aligned4(map256) ||
+        !aligned4(offset) || !aligned4(map_out_or_null) || !aligned4(code_out_or_null))
+        return fail(NF4HIP_E_ALIGN, "%s: w / packed / absmax_q / absmax2 not 16-byte aligned or a table not 4-byte aligned", name);
+    const size_t need = nf4hip_quantize_dq_workspace_bytes(n, blocksize);
+    if (!workspace || workspace_bytes < need)
+        return fail(NF4HIP_E_WORKSPACE, "%s: workspace of %zu bytes required, got %zu", name, need, workspace ? workspace_bytes : (size_t)0);
+    if (!aligned16(workspace)) return fail(NF4HIP_E_ALIGN, "%s: workspace not 16-byte aligned", name);
+    float* absmax = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + nf4::DQ_SUMS * sizeof(double));
+    const hipError_t e = nf4::launch_quantize_dq(w, w_dtype, n, bl, nl, map256, packed, absmax, static_cast<double*>(workspace), offset,
+                                                 absmax_q, absmax2, map_out_or_null, code_out_or_null, static_cast<hipStream_t>(stream));
+    if (e != hipSuccess) return hip_fail(name, e);
+    return NF4HIP_OK;
+}
+
 int nf4hip_dequantize(const uint8_t* packed, const float* absmax, const float* lut16, int64_t n, int blocksize,
                       void* out, int out_dtype, void* stream) {
     if (n < 0) return fail(NF4HIP_E_SHAPE, "nf4hip_dequantize: n = %lld is negative", (long long)n);
@@ -238,7 +267,7 @@ int nf4hip_dq_compress(const float* absmax, int64_t nblocks, int nested_blocksiz
     if (!aligned16(absmax) || !aligned16(absmax_q) || !aligned16(absmax2) || !aligned4(map256))
         return fail(NF4HIP_E_ALIGN, "nf4hip_dq_compress: absmax / absmax_q / absmax2 not 16-byte aligned or map256 not 4-byte aligned");
     const hipError_t e =
-        nf4::launch_dq_compress(absmax, nblocks, nl, map256, offset, absmax_q, absmax2, static_cast<hipStream_t>(stream));
+        nf4::launch_dq_compress(absmax, nblocks, nl, map256, offset, nullptr, absmax_q, absmax2, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail("nf4hip_dq_compress", e);
     return NF4HIP_OK;
 }

@@ -67,9 +67,10 @@ def nf4_code(device=None, dtype: torch.dtype = torch.float32) -> torch.Tensor:
     return master.clone()
 
 
-def dynamic_map(device=None) -> torch.Tensor:
-    """The 256-entry signed "dynamic" 8-bit code bitsandbytes uses for nested absmax quantisation
-    (``create_dynamic_map(signed=True, max_exponent_bits=7, total_bits=8)``)."""
+_map_masters: dict[str, torch.Tensor] = {}
+
+
+def _dynamic_map_values() -> torch.Tensor:
     data: list[float] = []
     for i in range(7):
         boundaries = torch.linspace(0.1, 1, 2**i + 1)
@@ -80,7 +81,25 @@ def dynamic_map(device=None) -> torch.Tensor:
     data += [0.0, 1.0]
     assert len(data) == 256
     data.sort()
-    return torch.tensor(data, dtype=torch.float32, device=device)
+    return torch.tensor(data, dtype=torch.float32, device="cpu")
+
+
+def _dynamic_map_master(device=None) -> torch.Tensor:
+    """The map as this package's own tensor, one per device: read it, never hand it out (``dynamic_map`` gives copies)."""
+    dev = torch.device(device) if device is not None else torch.device("cpu")
+    if dev.type == "cuda" and dev.index is None:
+        dev = torch.device("cuda", torch.cuda.current_device())
+    master = _map_masters.get(str(dev))
+    if master is None:
+        master = _map_masters[str(dev)] = _dynamic_map_values().to(dev)
+    return master
+
+
+def dynamic_map(device=None) -> torch.Tensor:
+    """The 256-entry signed "dynamic" 8-bit code bitsandbytes uses for nested absmax quantisation
+    (``create_dynamic_map(signed=True, max_exponent_bits=7, total_bits=8)``), as a new tensor.  One master copy per
+    device is kept and cloned: building it on the host and copying it over took 0.1 ms of every nested quantisation."""
+    return _dynamic_map_master(device).clone()
 
 
 @dataclass
@@ -274,11 +293,30 @@ def quantize_nf4_dq(w: torch.Tensor, blocksize: int = 64, nested_blocksize: int 
     """NF4 quantisation with double-quantised statistics (bitsandbytes' ``compress_statistics=True``).  Returns
     ``(qweight, absmax_q, nested_absmax, nested_quant_map, nested_offset, code)``; ``nested_offset`` is a one-element
     fp32 tensor so that it can live in a state dict."""
-    qw, absmax, code = quantize_nf4(w, blocksize)
-    nq = compress_absmax(absmax, nested_blocksize)
-    offset = torch.tensor([nq.offset], dtype=torch.float32, device=qw.device)
-    _remember_offset(offset, float(nq.offset))
-    return qw, nq.q, nq.absmax2, nq.map256, offset, code
+    if not w.is_cuda or w.numel() == 0 or w.dtype not in _DTYPE_CODE:
+        qw, absmax, code = quantize_nf4(w, blocksize)
+        nq = compress_absmax(absmax, nested_blocksize)
+        offset = torch.tensor([nq.offset], dtype=torch.float32, device=qw.device)
+        _remember_offset(offset, float(nq.offset))
+        return qw, nq.q, nq.absmax2, nq.map256, offset, code
+    _check_blocksize(blocksize)
+    _check_blocksize(nested_blocksize)
+    lib = _lib.load()
+    w = _aligned(w.detach())
+    dev, n = w.device, w.numel()
+    nblocks = (n + blocksize - 1) // blocksize
+    with _on_device(dev):
+        qw = torch.empty(((n + 1) // 2, 1), dtype=torch.uint8, device=dev)
+        q = torch.empty(nblocks, dtype=torch.uint8, device=dev)
+        absmax2 = torch.empty(((nblocks + nested_blocksize - 1) // nested_blocksize,), dtype=torch.float32, device=dev)
+        map256, code, offset = (torch.empty(k, dtype=torch.float32, device=dev) for k in (256, 16, 1))
+        need = lib.nf4hip_quantize_dq_workspace_bytes(n, blocksize)
+        scratch = torch.empty(need, dtype=torch.uint8, device=dev)  # absmax in fp32, which nobody keeps
+        _lib.check(lib.nf4hip_quantize_dq(w.data_ptr(), _DTYPE_CODE[w.dtype], n, blocksize, nested_blocksize, _dynamic_map_master(dev).data_ptr(),
+                                          qw.data_ptr(), q.data_ptr(), absmax2.data_ptr(), offset.data_ptr(), map256.data_ptr(),
+                                          code.data_ptr(), scratch.data_ptr(), need, _stream()))
+        _offset_value(offset)  # one read back, behind all three kernels: the matmuls' C ABI takes the offset by value
+    return qw, q, absmax2, map256, offset, code
 
 
 def dequantize_nf4_dq(qweight, absmax_q, nested_absmax, nested_quant_map, nested_offset, quant_map, blocksize, nested_blocksize,

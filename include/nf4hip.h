@@ -232,14 +232,29 @@ size_t nf4hip_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K);
 /*
  * The launch plan nf4hip_gemm would use for a shape (no GPU needed): plan[0] rows of x per tile (64, 128 or 256),
  * plan[1] tiles (tiles of x rows x tiles of 256 weight rows), plan[2] pieces a tile is cut into along K (they meet in
- * the workspace), plan[3] workgroups launched.  For host code that chooses between this kernel and dequantize +
- * dense GEMM (the choice bitsandbytes.matmul_4bit makes at thunder/transforms/quantization.py:39) without keeping
+ * the workspace), plan[3] workgroups launched.  Up to 128 rows of x this is what the workspace is sized by; the
+ * kernel (nf4hip_stream's) lays its own tiles out inside it, cut into no more pieces.  For host code that chooses
+ * between this kernel and dequantize + dense GEMM (the choice bitsandbytes.matmul_4bit makes at thunder/transforms/quantization.py:39) without keeping
  * a copy of the launcher's rules.  K must be a multiple of 64.
  */
 int nf4hip_gemm_plan(int64_t M, int64_t N, int64_t K, int32_t plan[4]);
 int nf4hip_gemm(const void* x, int x_dtype, int64_t M, const uint8_t* packed, const float* absmax, const float* lut16,
                 const void* bias_or_null, int64_t N, int64_t K, int blocksize, void* out, void* workspace,
                 size_t workspace_bytes, void* stream);
+/*
+ * The same product for 1..128 rows of bf16 or fp16 x (then bias and out are fp16 too), every weight rounded to x's type as
+ * nf4hip_dequantize rounds it: the kernel between the decode step and the prompt, and for fp16 also at decode shapes.
+ * K % 64 == 0, blocksize dividing K.  With nf4hip_stream_workspace_bytes(M, N, K) bytes of workspace (rules of nf4hip_gemv's;
+ * the kernels may share one) K may be split over workgroups; with less, or NULL, it is not.  Deterministic either way.
+ */
+size_t nf4hip_stream_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int nf4hip_stream(const void* x, int x_dtype, int64_t M, const uint8_t* packed, const float* absmax, const float* lut16,
+                  const void* bias_or_null, int64_t N, int64_t K, int blocksize, void* out, void* workspace,
+                  size_t workspace_bytes, void* stream);
+int nf4hip_stream_dq(const void* x, int x_dtype, int64_t M, const uint8_t* packed, const uint8_t* absmax_q,
+                     const float* absmax2, const float* map256, float offset, int nested_blocksize, const float* lut16,
+                     const void* bias_or_null, int64_t N, int64_t K, int blocksize, void* out, void* workspace,
+                     size_t workspace_bytes, void* stream);
 /*
  * Dense linear on a dequantized weight: out[M, N] = x[M, K] . w[N, K]^T (+ bias), bf16 operands, fp32 accumulation,
  * bf16 output.  The GEMM of the dequantize_4bit + torch.nn.functional.linear route of bitsandbytes.matmul_4bit

@@ -69,6 +69,9 @@ SYMBOLS = {
     "nf4hip_gemm_plan": (_i32, [_i64, _i64, _i64, ctypes.POINTER(_i32 * 4)]),
     "nf4hip_gemm": (_i32, _MATMUL),
     "nf4hip_gemm_dq": (_i32, _MATMUL_DQ),
+    "nf4hip_stream_workspace_bytes": (_sz, [_i64, _i64, _i64]),
+    "nf4hip_stream": (_i32, _MATMUL),
+    "nf4hip_stream_dq": (_i32, _MATMUL_DQ),
     "nf4hip_linear_workspace_bytes": (_sz, [_i64, _i64, _i64]),
     "nf4hip_linear_plan": (_i32, [_i64, _i64, _i64, ctypes.POINTER(_i32 * 4)]),
     "nf4hip_linear": (_i32, [_vp, _i32, _i64, _vp, _vp, _i64, _i64, _vp, _vp, _sz, _vp]),

@@ -59,6 +59,13 @@ class WorkspacePool:
         self._live[key] = new
         return new
 
+    def get_or_none(self, device: torch.device, nbytes: int, stream: int | None = None) -> torch.Tensor | None:
+        """``get``, or None where that would have to allocate while the stream is capturing."""
+        ws = self._live.get(self._key(device, stream))
+        if ws is not None and ws.numel() >= nbytes:
+            return ws
+        return None if torch.cuda.is_current_stream_capturing() else self.get(device, nbytes, stream)
+
     def reserve(self, device: torch.device, nbytes: int | None = None, stream: int | None = None) -> int:
         """Make sure (device, stream) owns a buffer of ``nbytes`` (default: the floor) before a capture."""
         return self.get(device, self.floor_bytes if nbytes is None else nbytes, stream).numel()

@@ -95,19 +95,19 @@ int check_nested(const uint8_t* absmax_q, const float* absmax2, const float* map
     return NF4HIP_OK;
 }
 
-enum MatmulKind { GEMV, GEMM };
+enum MatmulKind { GEMV, GEMM, STREAM };
 
 // use_static: the workspace is the library's own `scratch` array (nf4hip_gemv_static)
 int matmul_common(MatmulKind kind, const void* x, int x_dtype, int64_t M, const uint8_t* packed, const float* absmax,
                   const nf4::NestedAbsmax* nested, const float* lut16, const void* bias, int64_t N, int64_t K,
                   int blocksize, void* out, void* workspace, size_t workspace_bytes, void* stream,
                   bool use_static = false, const nf4hip_epilogue* epi = nullptr) {
-    const char* name = epi ? "nf4hip_gemv_epilogue" : use_static ? "nf4hip_gemv_static" : kind == GEMV ? "nf4hip_gemv" : "nf4hip_gemm";
+    const char* name = epi ? "nf4hip_gemv_epilogue" : use_static ? "nf4hip_gemv_static" : kind == GEMV ? "nf4hip_gemv" : kind == GEMM ? "nf4hip_gemm" : "nf4hip_stream";
     if (!x || !packed || !lut16 || !out) return fail(NF4HIP_E_NULL, "%s: null pointer", name);
     if (!nested && !absmax) return fail(NF4HIP_E_NULL, "%s: absmax is null", name);
-    if (x_dtype != NF4HIP_BF16)
-        return fail(valid_dtype(x_dtype) ? NF4HIP_E_DTYPE : NF4HIP_E_DTYPE, "%s: only bf16 x is fused (got dtype %d)",
-                    name, x_dtype);
+    if (x_dtype != NF4HIP_BF16 && !(kind == STREAM && x_dtype == NF4HIP_F16))
+        return fail(valid_dtype(x_dtype) ? NF4HIP_E_DTYPE : NF4HIP_E_DTYPE, "%s: only bf16 x %sis fused (got dtype %d)",
+                    name, kind == STREAM ? "or fp16 x " : "", x_dtype);
     const int bl = block_log2(blocksize);
     if (bl < 0) return fail(NF4HIP_E_BLOCKSIZE, "%s: blocksize %d unsupported", name, blocksize);
     if (M <= 0 || N <= 0 || K <= 0) return fail(NF4HIP_E_SHAPE, "%s: M, N, K must be positive", name);
@@ -120,7 +120,10 @@ int matmul_common(MatmulKind kind, const void* x, int x_dtype, int64_t M, const 
         if (M > 4 && K > (1 << 24))
             return fail(NF4HIP_E_SHAPE, "nf4hip_gemv: K = %lld > 2^24 with M > 4 (use nf4hip_gemm)", (long long)K);
     } else {
-        if (K % 64) return fail(NF4HIP_E_SHAPE, "nf4hip_gemm: K = %lld is not a multiple of 64", (long long)K);
+        if (K % 64) return fail(NF4HIP_E_SHAPE, "%s: K = %lld is not a multiple of 64", name, (long long)K);
+        if (kind == STREAM && !nf4::stream_possible(M, N, K))
+            return fail(NF4HIP_E_SHAPE, "%s: M = %lld, N = %lld, K = %lld: more than 128 rows, or a weight too large for 32-bit offsets", name,
+                        (long long)M, (long long)N, (long long)K);
     }
     if (!(kind == GEMV && M <= 4) && K % blocksize)
         return fail(NF4HIP_E_SHAPE, "%s: blocksize %d does not divide K = %lld", name, blocksize, (long long)K);
@@ -128,7 +131,8 @@ int matmul_common(MatmulKind kind, const void* x, int x_dtype, int64_t M, const 
         (bias && (reinterpret_cast<uintptr_t>(bias) & 1u)) || !aligned4(lut16))
         return fail(NF4HIP_E_ALIGN, "%s: x / packed / absmax / out not 16-byte aligned, lut16 not 4-byte or bias not 2-byte aligned",
                     name);
-    const size_t need = kind == GEMV ? nf4::gemv_workspace_bytes(M, N, K) : nf4::gemm_workspace_bytes(M, N, K);
+    // (nf4hip_stream uses what workspace it is given)
+    const size_t need = kind == GEMV ? nf4::gemv_workspace_bytes(M, N, K) : kind == GEMM ? nf4::gemm_workspace_bytes(M, N, K) : 0;
     if (use_static) {
         if (need > (size_t)NF4HIP_STATIC_SCRATCH_BYTES)
             return fail(NF4HIP_E_WORKSPACE,
@@ -140,6 +144,8 @@ int matmul_common(MatmulKind kind, const void* x, int x_dtype, int64_t M, const 
             return fail(NF4HIP_E_WORKSPACE, "%s: workspace of %zu bytes required, got %zu", name, need,
                         workspace ? workspace_bytes : (size_t)0);
         if (!aligned16(workspace)) return fail(NF4HIP_E_ALIGN, "%s: workspace not 16-byte aligned", name);
+    } else if (kind == STREAM && !aligned16(workspace)) {
+        return fail(NF4HIP_E_ALIGN, "%s: workspace not 16-byte aligned", name);
     }
 
     nf4::MatmulArgs a;
@@ -155,7 +161,7 @@ int matmul_common(MatmulKind kind, const void* x, int x_dtype, int64_t M, const 
     a.K = (int)K;
     a.block_log2 = bl;
     a.workspace = workspace;
-    a.workspace_bytes = workspace_bytes;
+    a.workspace_bytes = workspace ? workspace_bytes : 0;
     a.epi = nf4::Epilogue{nf4::EPI_NONE, 0.0f, nullptr, 0, nullptr, nullptr, nullptr, nullptr, nullptr};
     if (epi && epi->flags) {
         const int f = epi->flags;
@@ -182,8 +188,9 @@ int matmul_common(MatmulKind kind, const void* x, int x_dtype, int64_t M, const 
         if (es != hipSuccess) return hip_fail(name, es);
         a.workspace_bytes = NF4HIP_STATIC_SCRATCH_BYTES;
     }
-    const hipError_t e = kind == GEMV ? nf4::launch_gemv(a, static_cast<hipStream_t>(stream))
-                                      : nf4::launch_gemm(a, static_cast<hipStream_t>(stream));
+    const hipError_t e = kind == GEMV   ? nf4::launch_gemv(a, static_cast<hipStream_t>(stream))
+                         : kind == GEMM ? nf4::launch_gemm(a, static_cast<hipStream_t>(stream))
+                                        : nf4::launch_stream(a, x_dtype == NF4HIP_F16, 8, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(name, e);
     return NF4HIP_OK;
 }
@@ -404,6 +411,27 @@ int nf4hip_gemm(const void* x, int x_dtype, int64_t M, const uint8_t* packed, co
                 const void* bias_or_null, int64_t N, int64_t K, int blocksize, void* out, void* workspace,
                 size_t workspace_bytes, void* stream) {
     return matmul_common(GEMM, x, x_dtype, M, packed, absmax, nullptr, lut16, bias_or_null, N, K, blocksize, out,
+                         workspace, workspace_bytes, stream);
+}
+
+size_t nf4hip_stream_workspace_bytes(int64_t M, int64_t N, int64_t K) { return nf4::stream_workspace_bytes(M, N, K); }
+
+int nf4hip_stream(const void* x, int x_dtype, int64_t M, const uint8_t* packed, const float* absmax, const float* lut16,
+                  const void* bias_or_null, int64_t N, int64_t K, int blocksize, void* out, void* workspace,
+                  size_t workspace_bytes, void* stream) {
+    return matmul_common(STREAM, x, x_dtype, M, packed, absmax, nullptr, lut16, bias_or_null, N, K, blocksize, out,
+                         workspace, workspace_bytes, stream);
+}
+
+int nf4hip_stream_dq(const void* x, int x_dtype, int64_t M, const uint8_t* packed, const uint8_t* absmax_q,
+                     const float* absmax2, const float* map256, float offset, int nested_blocksize, const float* lut16,
+                     const void* bias_or_null, int64_t N, int64_t K, int blocksize, void* out, void* workspace,
+                     size_t workspace_bytes, void* stream) {
+    int nl = 0;
+    const int rc = check_nested(absmax_q, absmax2, map256, nested_blocksize, &nl);
+    if (rc) return rc;
+    const nf4::NestedAbsmax nq{absmax_q, absmax2, map256, offset, nl};
+    return matmul_common(STREAM, x, x_dtype, M, packed, nullptr, &nq, lut16, bias_or_null, N, K, blocksize, out,
                          workspace, workspace_bytes, stream);
 }
 

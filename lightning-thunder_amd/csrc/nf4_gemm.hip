@@ -1,4 +1,4 @@
-// Prefill-shape fused NF4 dequant-matmul for gfx950, M > 16 rows of x.
+// Entry of the fused NF4 matmul with exact weights, and its general kernel.
 //
 // Replaces the dequantize_4bit + F.linear route of bitsandbytes.matmul_4bit
 // (MatMul4Bit.forward), reached from thunder/transforms/quantization.py:39: instead of writing
@@ -6,20 +6,19 @@
 // bf16 in registers -- bf16_rne(lut16[code] * absmax), the same value nf4hip_dequantize produces --
 // and contracts them with bf16 MFMA, fp32 accumulation, bf16 output.
 //
-// Tile: BM (64, 128 or 256 rows of x) x 256 (n) x 64 (k) per workgroup of 512 threads.  Wave w of 8
-// owns weight rows 32 w .. + 31 of the tile against all BM rows of x: BM / 32 accumulators of
+// Up to 128 rows of x: nf4_gemm_stream.hip.  More: nf4_gemm_wide.hip.  The kernel here takes what their 32-bit offsets
+// do not reach, x of 4 GB and more or a weight of 2^31 blocks: 64-bit addresses, one workgroup per tile.
+//
+// Tile: 256 rows of x x 256 (n) x 64 (k) per workgroup of 512 threads.  Wave w of 8
+// owns weight rows 32 w .. + 31 of the tile against all rows of x: eight accumulators of
 // v_mfma_f32_32x32x16_bf16 with A = x (from LDS) and B = W (from this wave's registers).  A lane
 // loads 16 bytes = 32 codes of one weight row per k step; each of its four dwords becomes the B
 // fragment of one 16-k slice, so the weights never pass through LDS.  The k order inside a step
 // follows the codes (lane half h, slice s: k = 32 h + 8 s .. + 7) and the x fragments are read from
-// LDS in the same order.  LDS holds two stages of BM rows of x padded to 144 bytes (128-bit
+// LDS in the same order.  LDS holds two stages of 256 rows of x padded to 144 bytes (128-bit
 // fragment reads without bank conflicts) and the code book as a table of pairs: for every byte
 // value the two fp32 entries of its codes, in 32 copies laid out so that the 32 lanes the LDS serves
 // together never share a bank -- one ds_read_b64 per byte of codes.
-//
-// Up to 128 rows of x (one tile of x rows) K is split over up to 8 workgroups per weight tile when the
-// weight has too few tiles for the chip; their fp32 partial tiles meet in the workspace and the last
-// one to arrive adds them in split order.
 //
 // Pipeline per k step kt: x rows of step kt + 1 go from registers to the other LDS stage at the
 // top of the step and the registers are refilled with step kt + 2; codes and absmax run two steps
@@ -44,7 +43,7 @@ constexpr int THREADS = 512;
 constexpr int ROW_BYTES = BK * 2 + 16;  // padded LDS row
 constexpr int LUT_BYTES = 256 * 256;    // byte -> (fp32, fp32) of its two codes, 32 copies: 256 B per byte value
 
-template <int BM>
+constexpr int BM = 256;
 struct Tile {
     static constexpr int XA = BM / 64;  // 16-byte x loads per thread and k step
     static constexpr int STAGE_BYTES = BM * ROW_BYTES;
@@ -117,10 +116,9 @@ __device__ __forceinline__ bf16x8 scale_round(const float (&v)[8], float scale) 
 // 8 waves, wave w: all BM rows of x by weight rows n0 + 32 w .. + 31.  Lane l holds weight row l % 32,
 // codes 32 (l / 32) .. + 31 of the k step; its dword s is the B fragment of slice s, covering
 // k = 32 (l / 32) + 8 s .. + 7, and the x fragments are read from LDS in the same k order.
-template <bool NESTED, int BM>
-__global__ __launch_bounds__(THREADS) void gemm_kernel(MatmulArgs a, int m_tiles, int n_tiles, int splits,
-                                                           uint32_t* counters, float* partials) {
-    using T = Tile<BM>;
+template <bool NESTED>
+__global__ __launch_bounds__(THREADS) void gemm_kernel(MatmulArgs a, int m_tiles, int n_tiles) {
+    using T = Tile;
     extern __shared__ __attribute__((aligned(4096))) uint8_t smem[];
     uint8_t* stages = smem + LUT_BYTES;
     const int tid = threadIdx.x;
@@ -146,9 +144,7 @@ __global__ __launch_bounds__(THREADS) void gemm_kernel(MatmulArgs a, int m_tiles
     const int nt = id / m_tiles;
     const int mt = id - nt * m_tiles;
     const int m0 = mt * BM, n0 = nt * BN;
-    // K split over blockIdx.y: this workgroup's steps start at k_base
-    const int ksteps = a.K / BK / splits;
-    const int k_base = blockIdx.y * ksteps * BK;
+    const int ksteps = a.K / BK;
 
     f32x16 acc[T::TI];
 #pragma unroll
@@ -159,9 +155,9 @@ __global__ __launch_bounds__(THREADS) void gemm_kernel(MatmulArgs a, int m_tiles
     const uint16_t* xrow[T::XA];
 #pragma unroll
     for (int u = 0; u < T::XA; ++u)
-        xrow[u] = a.x + (int64_t)min(m0 + (tid >> 3) + 64 * u, a.M - 1) * a.K + k_base + (tid & 7) * 8;
+        xrow[u] = a.x + (int64_t)min(m0 + (tid >> 3) + 64 * u, a.M - 1) * a.K + (tid & 7) * 8;
     const int a_st = (tid >> 3) * ROW_BYTES + (tid & 7) * 16;  // + 64 u rows
-    const int64_t e0 = (int64_t)min(n0 + wave * 32 + (lane & 31), a.N - 1) * a.K + k_base + (lane >> 5) * 32;
+    const int64_t e0 = (int64_t)min(n0 + wave * 32 + (lane & 31), a.N - 1) * a.K + (lane >> 5) * 32;
     const int a_off = (lane & 31) * ROW_BYTES + (lane >> 5) * 64;  // + 32 i rows, + 16 bytes per slice
 
     uint4 xa[T::XA];
@@ -267,57 +263,6 @@ __global__ __launch_bounds__(THREADS) void gemm_kernel(MatmulArgs a, int m_tiles
     }
     if (kt < ksteps) step(kt, c0, c1, std::false_type{});
 
-    if (splits > 1) {
-        // Partial sums of this K split go to the workspace in register order ([i][q][thread]: coalesced);
-        // the last split to arrive for the tile adds all of them in split order (deterministic) and
-        // writes the result.  Ordering without L2-wide fences: agent-scope stores go through to L2, every
-        // store of the workgroup has completed (s_waitcnt, barrier) before its arrival is counted, and the
-        // last workgroup reads with agent-scope loads, which bypass its CU's L1.
-        float* tile_part = partials + (int64_t)id * splits * (T::TI * 16 * THREADS);
-        float* mine = tile_part + (int64_t)blockIdx.y * (T::TI * 16 * THREADS);
-#pragma unroll
-        for (int i = 0; i < T::TI; ++i)
-#pragma unroll
-            for (int q = 0; q < 16; ++q)
-                __hip_atomic_store(mine + (i * 16 + q) * THREADS + tid, acc[i][q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        publish_partials();
-        __syncthreads();
-        uint32_t* flag = reinterpret_cast<uint32_t*>(smem);
-        if (tid == 0) *flag = __hip_atomic_fetch_add(&counters[id], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __syncthreads();
-        acquire_partials();
-        if (*flag != (uint32_t)(splits - 1)) return;
-        // G splits' worth of loads are issued before the first add, so the merge costs a few memory
-        // round trips instead of one per split
-        constexpr int G = BM <= 64 ? 8 : 4;
-#pragma unroll
-        for (int i = 0; i < T::TI; ++i) {
-            float sum[16];
-#pragma unroll
-            for (int q = 0; q < 16; ++q) sum[q] = 0.0f;
-            for (int sp0 = 0; sp0 < splits; sp0 += G) {
-                float v[G][16];
-#pragma unroll
-                for (int g = 0; g < G; ++g) {
-                    const int sp = min(sp0 + g, splits - 1);
-                    const float* src = tile_part + (int64_t)sp * (T::TI * 16 * THREADS) + i * 16 * THREADS + tid;
-#pragma unroll
-                    for (int q = 0; q < 16; ++q)
-                        v[g][q] = __hip_atomic_load(src + q * THREADS, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                }
-#pragma unroll
-                for (int g = 0; g < G; ++g)
-                    if (sp0 + g < splits) {
-#pragma unroll
-                        for (int q = 0; q < 16; ++q) sum[q] += v[g][q];
-                    }
-            }
-#pragma unroll
-            for (int q = 0; q < 16; ++q) acc[i][q] = sum[q];
-        }
-        if (tid == 0) __hip_atomic_store(&counters[id], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-
     // acc[i][q] = out[m][n], n = lane & 31, m = 8*(q/4) + 4*(lane/32) + q%4 inside the 32x32 tile
     const int n = n0 + wave * 32 + (lane & 31);
     if (n < a.N) {
@@ -337,9 +282,8 @@ constexpr int MAX_DEVICES = 64;
 // zero-initialised workspace serves both (partial sums never land where the other expects zeroed counters)
 constexpr size_t GEMM_COUNTER_BYTES = GEMV_COUNTER_BYTES;
 
-// K splits for up to 128 rows of x (one tile of x rows): as many workgroups as fit the chip's 256 CUs in
-// one round when the weight has few 256-row tiles; the k steps divide evenly and every split keeps at
-// least 4.
+// Pieces along K for up to 128 rows of x: what the workspace is sized by (as many workgroups of 256 weight rows as fit the
+// chip's 256 CUs in one round; the k steps divide evenly and every piece keeps at least 4), and the most the kernel uses.
 int gemm_splits(int64_t M, int64_t N, int64_t K) {
     if (M > 128) return 1;
     const int64_t tiles = (N + BN - 1) / BN;
@@ -350,28 +294,23 @@ int gemm_splits(int64_t M, int64_t N, int64_t K) {
     return best;
 }
 
-template <bool NESTED, int BM>
+template <bool NESTED>
 hipError_t launch_tile(const MatmulArgs& a, hipStream_t stream) {
-    using T = Tile<BM>;
     static bool ready[MAX_DEVICES] = {};
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
     if (dev < 0 || dev >= MAX_DEVICES) return hipErrorInvalidDevice;
-    auto kern = gemm_kernel<NESTED, BM>;
+    auto kern = gemm_kernel<NESTED>;
     if (!ready[dev]) {
         e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                T::SMEM_BYTES);
+                                Tile::SMEM_BYTES);
         if (e != hipSuccess) return e;
         ready[dev] = true;
     }
     const int m_tiles = (a.M + BM - 1) / BM;
     const int n_tiles = (a.N + BN - 1) / BN;
-    const int splits = gemm_splits(a.M, a.N, a.K);
-    uint32_t* counters = static_cast<uint32_t*>(a.workspace);
-    float* partials = splits > 1 ? reinterpret_cast<float*>(static_cast<uint8_t*>(a.workspace) + GEMM_COUNTER_BYTES) : nullptr;
-    hipLaunchKernelGGL(kern, dim3((unsigned)(m_tiles * n_tiles), (unsigned)splits), dim3(THREADS), T::SMEM_BYTES, stream, a,
-                       m_tiles, n_tiles, splits, counters, partials);
+    hipLaunchKernelGGL(kern, dim3((unsigned)(m_tiles * n_tiles)), dim3(THREADS), Tile::SMEM_BYTES, stream, a, m_tiles, n_tiles);
     return hipGetLastError();
 }
 
@@ -396,12 +335,9 @@ void gemm_plan(int64_t M, int64_t N, int64_t K, int plan[4]) {
 }
 
 hipError_t launch_gemm(const MatmulArgs& a, hipStream_t stream) {
-    // the smallest tile height that covers x with one tile: the weight tile is expanded once per tile of x rows
-    if (a.M <= 64) return a.nested.q ? launch_tile<true, 64>(a, stream) : launch_tile<false, 64>(a, stream);
-    if (a.M <= 128) return a.nested.q ? launch_tile<true, 128>(a, stream) : launch_tile<false, 128>(a, stream);
-    // more rows: the kernel of nf4_gemm_wide.hip, whose x loads address x with 32-bit offsets
-    if ((int64_t)a.M * a.K * 2 < ((int64_t)1 << 32)) return launch_gemm_wide(a, stream);
-    return a.nested.q ? launch_tile<true, 256>(a, stream) : launch_tile<false, 256>(a, stream);
+    if (stream_possible(a.M, a.N, a.K)) return launch_stream(a, false, gemm_splits(a.M, a.N, a.K), stream);
+    if (a.M > 128 && (int64_t)a.M * a.K * 2 < ((int64_t)1 << 32)) return launch_gemm_wide(a, stream);
+    return a.nested.q ? launch_tile<true>(a, stream) : launch_tile<false>(a, stream);
 }
 
 }  // namespace nf4

@@ -1,0 +1,72 @@
+// Which tile the kernel of nf4_gemm_stream.h uses for a call, and its launch.
+#include "nf4_gemv.h"
+
+namespace nf4 {
+namespace stream {
+hipError_t launch_bf16(const MatmulArgs& a, const StreamPlan& p, hipStream_t stream);
+hipError_t launch_bf16_dq(const MatmulArgs& a, const StreamPlan& p, hipStream_t stream);
+hipError_t launch_f16(const MatmulArgs& a, const StreamPlan& p, hipStream_t stream);
+hipError_t launch_f16_dq(const MatmulArgs& a, const StreamPlan& p, hipStream_t stream);
+}  // namespace stream
+namespace {
+
+// The rule is a model of the kernel's time in us: rounds of 256 workgroups (one per CU), each the 64-k steps of its
+// longest k group at 0.45..1 us (by the rows of x per tile; up to 30 % less on a sparsely filled chip); partial tiles that meet
+// in the workspace cost by their size and number.  Over M = 1..128 at fifteen shapes from [600, 1088] to [128256, 4096] its
+// choice takes 0.6 % longer than the best of all choices on average, 9 % at most.  (M <= 16 is judged as 32 rows: the two
+// differ by 0.02 us per step, and a call's sums are then added in one order whether its rows come alone or with others.)
+float step_us(int bm) { return bm <= 32 ? 0.47f : bm == 64 ? 0.67f : 1.0f; }
+float model_us(int64_t wgs, int64_t steps, int bm, int rows, int splits) {
+    const int64_t rounds = (wgs + 255) / 256;
+    const float fill = (float)wgs / (float)(rounds * 256);
+    const float merge = splits == 1 ? 0.0f : 1.0f + (float)(rows * bm) / 32768.0f * (float)(5 + splits);
+    return (float)rounds * ((float)steps * step_us(bm) * (0.7f + 0.3f * fill) + 1.0f) + merge;
+}
+
+size_t plan_bytes(const StreamPlan& p) {
+    if (p.splits == 1) return 0;
+    return GEMV_COUNTER_REGION_BYTES + (size_t)p.m_tiles * p.n_tiles * p.splits * p.wn * 32 * (p.bm < 32 ? 32 : p.bm) * sizeof(float);
+}
+
+}  // namespace
+
+bool stream_possible(int64_t M, int64_t N, int64_t K) {
+    // 32-bit offsets: of x, of a tile's codes, of a weight's blocks
+    return M >= 1 && M <= 128 && N >= 1 && K >= 64 && K % 64 == 0 && K < (1 << 24) && N <= INT32_MAX && N * (K / 64) < ((int64_t)1 << 31);
+}
+
+StreamPlan stream_plan(int64_t M, int64_t N, int64_t K, int max_splits) {
+    StreamPlan best{};
+    float best_us = 0.0f;
+    const int64_t ksteps = K / 64, units = (ksteps + 3) / 4;
+    for (int bm = 32; bm <= 128; bm *= 2) {
+        const int64_t m_tiles = (M + bm - 1) / bm;
+        for (int wn = bm == 128 ? 8 : bm == 64 ? 4 : 2; wn <= 8; wn *= 2) {
+            const int64_t n_tiles = (N + 32 * wn - 1) / (32 * wn);
+            const int wk = 8 / wn;
+            for (int s = 1; s <= max_splits && s <= 8; ++s) {
+                if (s > 1 && (m_tiles * n_tiles * s > 256 || units < s * wk)) break;  // one round, nobody idle
+                const int64_t steps = 4 * ((units + wk * s - 1) / (wk * s));
+                const float us = model_us(m_tiles * n_tiles * s, steps < ksteps ? steps : ksteps, bm, 32 * wn, s);
+                if (!best.bm || us < best_us) {
+                    best = StreamPlan{bm, wn, s, (int)m_tiles, (int)n_tiles};
+                    best_us = us;
+                }
+            }
+        }
+        if (bm >= M) break;
+    }
+    if (M <= 16 && best.bm == 32) best.bm = 16;
+    return best;
+}
+
+size_t stream_workspace_bytes(int64_t M, int64_t N, int64_t K) { return stream_possible(M, N, K) ? plan_bytes(stream_plan(M, N, K, 8)) : 0; }
+
+hipError_t launch_stream(const MatmulArgs& a, bool f16, int max_splits, hipStream_t stream) {
+    StreamPlan p = stream_plan(a.M, a.N, a.K, max_splits);
+    if (plan_bytes(p) > a.workspace_bytes) p = stream_plan(a.M, a.N, a.K, 1);
+    if (f16) return a.nested.q ? stream::launch_f16_dq(a, p, stream) : stream::launch_f16(a, p, stream);
+    return a.nested.q ? stream::launch_bf16_dq(a, p, stream) : stream::launch_bf16(a, p, stream);
+}
+
+}  // namespace nf4

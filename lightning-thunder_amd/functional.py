@@ -542,7 +542,8 @@ def fused_route(x: torch.Tensor, bias, blocksize: int, dtype: torch.dtype, shape
     ``"dequant+linear"`` (dequantize + ``torch.nn.functional.linear``, for dtypes and shapes no kernel here takes).
 
     Mirrors bitsandbytes.matmul_4bit: the fused single-row kernel when the shape allows, else
-    dequantize followed by a dense matmul.
+    dequantize followed by a dense matmul.  ``matmul_nf4`` asks ``_stream_serves`` first: this is the answer for the calls that
+    kernel leaves (and, for up to 128 rows of x, what would serve the others without it).
     """
     N, K = shape
     M = x.numel() // K if K else 0
@@ -575,6 +576,47 @@ def fused_route(x: torch.Tensor, bias, blocksize: int, dtype: torch.dtype, shape
     return "dequant+gemm" if M >= DENSE_ROUTE_MIN_M or K > LONG_K else "gemm"
 
 
+STREAM_MAX_M = 128
+STREAM_LONG_WEIGHT = 1 << 25
+
+
+def _is_plain(*tensors) -> bool:
+    """Can these be handed to a kernel by address?  No: anything that differentiates, transforms, traces or casts -- the
+    fp16 route without a kernel of its own is a torch operation, which does all of that."""
+    if torch.is_autocast_enabled("cuda") or torch._C._len_torch_dispatch_stack() or torch._C._functorch.peek_interpreter_stack() is not None:
+        return False
+    if torch.autograd.forward_ad._current_level >= 0 or torch.overrides._len_torch_function_stack():
+        return False
+    grad = torch.is_grad_enabled()
+    return all(t is None or (type(t) in (torch.Tensor, torch.nn.Parameter) and not (grad and t.requires_grad)) for t in tensors)
+
+
+def _stream_serves(x, qweight, bias, absmax, quant_map, blocksize: int, dtype: torch.dtype, shape) -> bool:
+    """Does ``nf4hip_stream`` serve this call, ahead of ``fused_route``'s answer?
+
+    bf16, 17..128 rows: always (graph replay, cold weights, us, against the former kernels: [4096, 4096] M = 32 / 64 / 128 18.0 / 18.7 /
+    28.3 vs 9.7 / 14.2 / 26.9; [14336, 4096] 24.7 / 27.3 / 35.8 vs 14.5 / 20.0 / 32.9; lm_head [128256, 4096] 112.7 / 124.8 / 171.0 vs
+    77.8 / 98.7 / 139.2).  5..16 rows: where K is no multiple of 512, which the decode kernels need ([5003, 2880] M = 8 18.8 vs
+    9.5), and from 2^25 elements on beyond K = 16384, where those reproduce every weight's rounding and are slow ([8192, 28672]
+    M = 8 / 16 38.7 / 45.0 vs 36.3 / 35.4, nested absmax 45.5 / 51.1 vs 35.4 / 36.3).  Smaller weights stay in the kernel that
+    their epilogue forms run in.
+    fp16, up to 128 rows: always; the alternative writes the dense weight first ([14336, 4096] M = 4: 47 vs 13)."""
+    N, K = shape
+    M = x.numel() // K if K else 0
+    if (not 1 <= M <= STREAM_MAX_M or N <= 0 or x.dtype != dtype or dtype not in (torch.bfloat16, torch.float16)
+            or K % 64 or blocksize not in SUPPORTED_BLOCKSIZES or K % blocksize or K >= 1 << 24 or N * (K // 64) >= 1 << 31
+            or (bias is not None and bias.dtype != dtype)):
+        return False
+    nested = isinstance(absmax, NestedAbsmax)
+    if dtype == torch.bfloat16:
+        if M > 16:
+            return True
+        return M > 4 and (K % 512 != 0 or (K > 16384 and N * K >= STREAM_LONG_WEIGHT))
+    stats = absmax.q if nested else absmax
+    return (_is_plain(x, bias) and (bias is None or bias.shape == (N,)) and (nested or absmax.numel() >= N * K // blocksize)
+            and qweight.numel() >= N * K // 2 and quant_map.numel() >= 16 and all(t is None or t.device == x.device for t in (qweight, bias, stats)))
+
+
 def matmul_nf4(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape) -> torch.Tensor:
     """``x @ dequantize(qweight).T + bias`` with the signature of the reference operator
     ``bnb_matmul_nf4`` (thunder/transforms/quantization.py:34).  ``absmax`` may be a
@@ -584,9 +626,11 @@ def matmul_nf4(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape) -> 
     N, K = shape
     assert x.shape[-1] == K, f"{x.shape=}, rhs {shape=}"
     _require_gpu(x, qweight, quant_map, bias)
+    M = x.numel() // K if K else 0
+    if (M > 4 or x.dtype is not torch.bfloat16) and _stream_serves(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape):
+        return _matmul_nf4_on(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape, "stream")
     nested = isinstance(absmax, NestedAbsmax)
     route = fused_route(x, bias, blocksize, dtype, shape, nested)
-    M = x.numel() // K
     if (route in ("gemm", "dequant+gemm") and M >= CALIBRATE_MIN_M and _calibration_enabled()
             and not torch.cuda.is_current_stream_capturing()):
         key = _route_key(x.device, M, N, K, blocksize, nested, bias is not None)
@@ -607,7 +651,7 @@ NESTED_RECONSTRUCT_MIN_M = 128
 
 
 def _matmul_nf4_on(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape, route: str) -> torch.Tensor:
-    """:func:`matmul_nf4` on a given route (one of ``fused_route``'s answers)."""
+    """:func:`matmul_nf4` on a given route (``"stream"`` or one of ``fused_route``'s answers)."""
     N, K = shape
     if route in ("dequant+linear", "dequant+gemm", "dequant+libgemm"):
         w = dequantize_nf4(qweight, absmax, quant_map, blocksize, dtype, shape).to(x.dtype)
@@ -625,9 +669,15 @@ def _matmul_nf4_on(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape,
     b = None if bias is None else bias.contiguous()
     nblocks = N * K // blocksize
     with _on_device(x.device):
-        out = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
+        out = torch.empty((M, N), dtype=x.dtype, device=x.device)
         stream = _stream()
-        if route in ("gemv", "gemv-chunks"):
+        if route == "stream":
+            need = lib.nf4hip_stream_workspace_bytes(M, N, K)
+            # without scratch (a capture on a stream that has none yet) the kernel does not split K
+            ws = _workspace_pool.get_or_none(x.device, need, stream) if need else None
+            ws_ptr, ws_bytes = (None, 0) if ws is None else (ws.data_ptr(), ws.numel())
+            fn, fn_dq = lib.nf4hip_stream, lib.nf4hip_stream_dq
+        elif route in ("gemv", "gemv-chunks"):
             need = lib.nf4hip_gemv_workspace_bytes(min(M, 16), N, K)
             ws = _gemv_workspace(x.device, need, stream)
             ws_ptr, ws_bytes = ws.data_ptr(), ws.numel()
@@ -650,7 +700,7 @@ def _matmul_nf4_on(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape,
             q, a2, m256, off, nbs = _nested_args(absmax, nblocks)
             for m0 in range(0, M, step):
                 mc = min(step, M - m0)
-                _lib.check(fn_dq(x2.data_ptr() + 2 * m0 * K, _lib.BF16, mc, qweight.data_ptr(), q.data_ptr(), a2.data_ptr(), m256.data_ptr(), off, nbs,
+                _lib.check(fn_dq(x2.data_ptr() + 2 * m0 * K, _DTYPE_CODE[x.dtype], mc, qweight.data_ptr(), q.data_ptr(), a2.data_ptr(), m256.data_ptr(), off, nbs,
                                  quant_map.data_ptr(), bptr, N, K, blocksize, out.data_ptr() + 2 * m0 * N, ws_ptr, ws_bytes, stream))  # fmt: skip
         else:
             _require_gpu(absmax)
@@ -659,7 +709,7 @@ def _matmul_nf4_on(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape,
                 raise ValueError(f"absmax holds {absmax.numel()} entries, need {nblocks}")
             for m0 in range(0, M, step):
                 mc = min(step, M - m0)
-                _lib.check(fn(x2.data_ptr() + 2 * m0 * K, _lib.BF16, mc, qweight.data_ptr(), absmax.data_ptr(), quant_map.data_ptr(), bptr,
+                _lib.check(fn(x2.data_ptr() + 2 * m0 * K, _DTYPE_CODE[x.dtype], mc, qweight.data_ptr(), absmax.data_ptr(), quant_map.data_ptr(), bptr,
                               N, K, blocksize, out.data_ptr() + 2 * m0 * N, ws_ptr, ws_bytes, stream))  # fmt: skip
     return out.reshape(*x.shape[:-1], N)
 
@@ -721,6 +771,10 @@ def matmul_nf4_epilogue(x, qweight, bias, absmax, quant_map, blocksize, dtype, s
     * ``rowscale=(sumsq, eps)``: ``x`` is such an ``xnext``; the sums are multiplied by ``rsqrt(sumsq.sum(-1) / K + eps)``,
       which makes the result ``linear(rms_norm(r) * norm_weight)``.
     * ``silu_pairs``: weight rows 2j / 2j+1 are gate row j / up row j; returns ``silu(gate) * up`` [rows, N/2].
+
+    Each output is what ``matmul_nf4`` and the step would store, bit for bit (``rowscale`` aside), except at 5..16
+    rows on a weight of 2^25 elements and more with K > 16384: there the plain product runs in another kernel
+    (``_stream_serves``), with the same weights and another order of its sums.
 
     Returns None where the library does not serve the case (more than sixteen rows of x, nested absmax, other dtypes,
     one row of x with K > 16384, ...; ``epilogue_served`` answers beforehand): the caller then runs

@@ -1,0 +1,158 @@
+"""``nf4hip_stream``: the fused matmul for up to 128 rows of bf16 or fp16 x, at the edges of its tiles -- rows of x around
+16 / 32 / 64 / 128, ragged weight rows, one k step, a partial unit of four steps, K split over workgroups -- on fp32 and nested
+absmax and larger blocksizes, against a float64 product over the HIP-dequantised weight."""
+
+import ctypes
+
+import pytest
+import torch
+
+DEV = "cuda"
+U = {torch.bfloat16: 2.0**-8, torch.float16: 2.0**-11}  # half an ulp over the value: 8 and 11 significant bits
+A = 1 << 20  # fake, aligned device address: validation dereferences nothing
+
+
+def _weight(ta, N, K, blocksize, nested, dtype, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    w = torch.empty(N, K, device=DEV).normal_(0, 0.02, generator=g).to(dtype)
+    qw, absmax, code = ta.quantize_nf4(w, blocksize)
+    return qw, (ta.compress_absmax(absmax) if nested else absmax), code
+
+
+def _check(y, x, deq, bias):
+    """Each product is exact in fp32; a sum takes at most K / 16 MFMA accumulations and a handful of merges, each within
+    2**-23 of the sum of magnitudes (two roundings); the result is rounded once."""
+    ref, size = x.double() @ deq.double().t(), x.double().abs() @ deq.double().abs().t()
+    if bias is not None:
+        ref, size = ref + bias.double(), size + bias.double().abs()
+    bound = U[y.dtype] * ref.abs() + (x.shape[1] / 16 + 16) * 2.0**-23 * size + 2.0**-24
+    worst = ((y.double() - ref).abs() / bound).max().item()
+    assert worst <= 1.0, f"{worst:.3f} of the bound"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K,blocksize,nested,bias", [
+    (1, 1, 64, 64, False, True), (5, 63, 64, 64, True, False), (16, 64, 192, 64, False, False), (17, 65, 256, 64, True, True),
+    (32, 300, 320, 64, False, True), (33, 129, 1344, 64, True, False), (64, 1000, 2880, 64, False, True), (65, 257, 1024, 128, False, False),
+    (100, 515, 1536, 256, True, True), (128, 4098, 4096, 64, False, True), (128, 96, 28672, 64, True, False), (48, 4096, 4096, 64, True, False),
+    (20, 40000, 512, 64, False, False), (16, 8192, 28672, 64, True, False), (2, 8192, 2048, 2048, False, True),
+])
+def test_stream_matches_float64(ta, dtype, M, N, K, blocksize, nested, bias):
+    print(f"stream M={M} [{N},{K}] bs={blocksize} nested={nested} bias={bias} {dtype}", flush=True)
+    qw, stats, code = _weight(ta, N, K, blocksize, nested, dtype, M + N)
+    g = torch.Generator(device=DEV).manual_seed(K)
+    x = torch.empty(M, K, device=DEV).normal_(0, 1, generator=g).to(dtype)
+    b = torch.empty(N, device=DEV).normal_(0, 1, generator=g).to(dtype) if bias else None
+    deq = ta.dequantize_nf4(qw, stats, code, blocksize, dtype, (N, K))
+    run = lambda: ta.functional._matmul_nf4_on(x, qw, b, stats, code, blocksize, dtype, (N, K), "stream")
+    y = run()
+    _check(y, x, deq, b)
+    assert torch.equal(run(), y)  # the workspace is left as it was found, sums have one order
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M", [16, 32, 64, 128])
+def test_stream_recovers_dequantised_weights(ta, dtype, M):
+    """One-hot rows of x: every output is one product 1.0 * w and must be nf4hip_dequantize's value bit for bit."""
+    print(f"stream one-hot M={M} {dtype}", flush=True)
+    N, K = 272, 1088
+    qw, absmax, code = _weight(ta, N, K, 64, False, dtype, 3)
+    cols = torch.randint(0, K, (M,), generator=torch.Generator().manual_seed(M))
+    x = torch.zeros(M, K, dtype=dtype)
+    x[torch.arange(M), cols] = 1.0
+    y = ta.functional._matmul_nf4_on(x.to(DEV), qw, None, absmax, code, 64, dtype, (N, K), "stream")
+    deq = ta.dequantize_nf4(qw, absmax, code, 64, dtype, (N, K))
+    assert torch.equal(y, deq[:, cols.to(DEV)].t())
+
+
+@pytest.mark.gpu
+def test_stream_infinities_stay_in_their_row(ta):
+    print("stream infinities", flush=True)
+    N, K, M = 300, 2880, 33
+    qw, absmax, code = _weight(ta, N, K, 64, False, torch.float16, 4)
+    x = torch.ones(M, K, dtype=torch.float16, device=DEV)
+    x[5, 7], x[32, K - 1] = float("inf"), float("nan")
+    y = ta.matmul_nf4(x, qw, None, absmax, code, 64, torch.float16, (N, K))
+    others = [m for m in range(M) if m not in (5, 32)]
+    assert y[others].isfinite().all() and y[32].isnan().all() and not y[5].isfinite().any()
+
+
+@pytest.mark.gpu
+def test_stream_capture_without_scratch_and_autograd(ta):
+    print("stream capture / autograd", flush=True)
+    F = ta.functional
+    N, K, M = 512, 4096, 24
+    assert ta._lib.load().nf4hip_stream_workspace_bytes(M, N, K) > 0
+    qw, absmax, code = _weight(ta, N, K, 64, False, torch.float16, 5)
+    x = torch.randn(M, K, device=DEV).half()
+    args = (qw, None, absmax, code, 64, torch.float16, (N, K))
+    deq = ta.dequantize_nf4(qw, absmax, code, 64, torch.float16, (N, K))
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    saved = F._workspace_pool._live
+    try:
+        F._workspace_pool._live = {}
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            y = F.matmul_nf4(x, *args)
+    finally:
+        F._workspace_pool._live = saved
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        _check(y, x, deq, None)
+    # what has to be differentiated goes to the torch operation, as it always has
+    xg = x.clone().requires_grad_(True)
+    F.matmul_nf4(xg, *args).sum().backward()
+    torch.testing.assert_close(xg.grad[0].float(), deq.float().sum(0), rtol=1e-2, atol=1e-2)
+
+
+def test_stream_arguments_and_workspace(ta):
+    """Checked before any HIP call; the workspace holds what the plan can need and is optional."""
+    L = ta._lib
+    lib = L.load()
+
+    def call(x=A, dt=L.F16, M=8, packed=A, absmax=A, lut=A, bias=None, N=64, K=4096, bs=64, out=A, w=None, wb=0):
+        return lib.nf4hip_stream(x, dt, M, packed, absmax, lut, bias, N, K, bs, out, w, wb, None)
+
+    assert call(x=None) == L.E_NULL and call(absmax=None) == L.E_NULL and call(dt=L.F32) == L.E_DTYPE and call(bs=96) == L.E_BLOCKSIZE
+    assert call(M=0) == L.E_SHAPE and call(M=129) == L.E_SHAPE and call(K=96) == L.E_SHAPE and call(K=192, bs=128) == L.E_SHAPE
+    assert call(K=1 << 24) == L.E_SHAPE and call(N=1 << 30) == L.E_SHAPE
+    assert call(out=A + 2) == L.E_ALIGN and call(w=A + 8, wb=1 << 20) == L.E_ALIGN
+    for M in (1, 16, 17, 33, 65, 128):
+        for N, K in ((1, 64), (1024, 4096), (4096, 14336), (128256, 4096), (8192, 28672)):
+            need = lib.nf4hip_stream_workspace_bytes(M, N, K)
+            assert need == 0 or 65536 * 4 < need <= 65536 * 4 + 256 * 256 * 128 * 4
+    assert lib.nf4hip_stream_workspace_bytes(129, 64, 64) == 0 and lib.nf4hip_stream_workspace_bytes(8, 64, 96) == 0
+    _ = ctypes
+
+
+def test_stream_serves(ta):
+    F = ta.functional
+    bf, hf = torch.bfloat16, torch.float16
+
+    def serves(M, N, K, dtype=bf, xdtype=None, bs=64, bias=None, nested=False, x=None):
+        n = N * K // bs
+        stats = F.NestedAbsmax(torch.empty(n, dtype=torch.uint8), None, None, 0.0) if nested else torch.empty(n)
+        x = torch.empty(M, K, dtype=xdtype or dtype) if x is None else x
+        return F._stream_serves(x, torch.empty(N * K // 2, 1, dtype=torch.uint8), bias, stats, torch.empty(16), bs, dtype, (N, K))
+
+    assert not serves(16, 64, 4096) and serves(17, 64, 4096) and serves(128, 64, 4096) and not serves(129, 64, 4096)
+    assert serves(5, 64, 1344) and not serves(4, 64, 1344) and not serves(17, 64, 1376) and not serves(17, 64, 192, bs=128)
+    assert serves(5, 8192, 28672, nested=True) and serves(16, 8192, 28672) and not serves(5, 1000, 28672) and not serves(4, 8192, 28672, nested=True)
+    assert not serves(17, 64, 4096, bias=torch.empty(64)) and not serves(17, 64, 4096, xdtype=hf)
+    assert serves(1, 64, 4096, hf) and serves(128, 64, 4096, hf) and not serves(0, 64, 4096, hf)
+    assert not serves(1, 64, 4096, torch.float32)
+    # what differentiates or transforms stays with the torch operation
+    xg = torch.empty(2, 4096, dtype=hf, requires_grad=True)
+    assert not serves(2, 64, 4096, hf, x=xg)
+    with torch.no_grad():
+        assert serves(2, 64, 4096, hf, x=xg)
+    with torch.autograd.forward_ad.dual_level():
+        assert not serves(2, 64, 4096, hf)
+    seen = []
+    torch.func.vmap(lambda row: (seen.append(serves(1, 64, 4096, hf, x=row)), row)[1])(torch.zeros(2, 1, 4096, dtype=hf))
+    assert seen == [False]
+    assert not serves(2, 64, 4096, hf, bias=torch.empty(1, 64, dtype=hf))

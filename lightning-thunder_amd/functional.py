@@ -142,7 +142,7 @@ class _on_device:
 
 def _require_gpu(*tensors: torch.Tensor) -> None:
     for t in tensors:
-        if t is not None and t.device.type != "cuda":
+        if t is not None and not t.is_cuda:
             raise RuntimeError(f"NF4 HIP ops need GPU tensors, got a tensor on {t.device}")
 
 
@@ -621,8 +621,9 @@ def matmul_nf4(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape) -> 
     """``x @ dequantize(qweight).T + bias`` with the signature of the reference operator
     ``bnb_matmul_nf4`` (thunder/transforms/quantization.py:34).  ``absmax`` may be a
     :class:`NestedAbsmax`."""
-    shape = tuple(int(s) for s in shape)
-    assert len(shape) == 2
+    if type(shape) is not tuple or len(shape) != 2 or type(shape[0]) is not int or type(shape[1]) is not int:
+        shape = tuple(int(s) for s in shape)
+        assert len(shape) == 2
     N, K = shape
     assert x.shape[-1] == K, f"{x.shape=}, rhs {shape=}"
     _require_gpu(x, qweight, quant_map, bias)
@@ -651,7 +652,10 @@ NESTED_RECONSTRUCT_MIN_M = 128
 
 
 def _matmul_nf4_on(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape, route: str) -> torch.Tensor:
-    """:func:`matmul_nf4` on a given route (``"stream"`` or one of ``fused_route``'s answers)."""
+    """:func:`matmul_nf4` on a given route (``"stream"`` or one of ``fused_route``'s answers).
+
+    A decode call on a small weight is as long as this function: views, conversions and a device context that change nothing
+    are not asked for ([4096, 4096], one row, 5 us of kernel: ``matmul_nf4`` 14.9 -> 10.4 us, of which the ctypes call is 4.5)."""
     N, K = shape
     if route in ("dequant+linear", "dequant+gemm", "dequant+libgemm"):
         w = dequantize_nf4(qweight, absmax, quant_map, blocksize, dtype, shape).to(x.dtype)
@@ -659,59 +663,65 @@ def _matmul_nf4_on(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape,
             return linear_bf16(x, w, bias)  # the hand-written dense kernel
         return torch.nn.functional.linear(x, w, bias)
 
+    device = x.device
+    if device.index != torch._C._cuda_getDevice():
+        with torch.cuda.device(device):
+            return _matmul_nf4_on(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape, route)
     lib = _lib.load()
-    x2 = _aligned(x.reshape(-1, K))
+    flat = x.dim() == 2
+    x2 = _aligned(x if flat else x.reshape(-1, K))
     M = x2.shape[0]
     qweight = _aligned(qweight)
     if qweight.numel() < N * K // 2:
         raise ValueError(f"qweight holds {qweight.numel()} bytes, shape {shape} needs {N * K // 2}")
-    quant_map = _aligned(quant_map.to(torch.float32))
+    quant_map = _aligned(quant_map if quant_map.dtype is torch.float32 else quant_map.to(torch.float32))
     b = None if bias is None else bias.contiguous()
     nblocks = N * K // blocksize
-    with _on_device(x.device):
-        out = torch.empty((M, N), dtype=x.dtype, device=x.device)
-        stream = _stream()
-        if route == "stream":
-            need = lib.nf4hip_stream_workspace_bytes(M, N, K)
-            # without scratch (a capture on a stream that has none yet) the kernel does not split K
-            ws = _workspace_pool.get_or_none(x.device, need, stream) if need else None
-            ws_ptr, ws_bytes = (None, 0) if ws is None else (ws.data_ptr(), ws.numel())
-            fn, fn_dq = lib.nf4hip_stream, lib.nf4hip_stream_dq
-        elif route in ("gemv", "gemv-chunks"):
-            need = lib.nf4hip_gemv_workspace_bytes(min(M, 16), N, K)
-            ws = _gemv_workspace(x.device, need, stream)
-            ws_ptr, ws_bytes = ws.data_ptr(), ws.numel()
-            fn, fn_dq = lib.nf4hip_gemv, lib.nf4hip_gemv_dq
-        else:
-            need = lib.nf4hip_gemm_workspace_bytes(M, N, K)  # K split over workgroups: partial tiles and counters
-            ws = _gemv_workspace(x.device, need, stream) if need else None
-            ws_ptr, ws_bytes = (None, 0) if ws is None else (ws.data_ptr(), ws.numel())
-            fn, fn_dq = lib.nf4hip_gemm, lib.nf4hip_gemm_dq
-        bptr = None if b is None else b.data_ptr()
-        # row chunks of x and out: one call, or 16 rows at a time (rows are contiguous, K and N even,
-        # so every chunk starts 16-byte aligned when the whole does and K, N are multiples of 8)
-        step = 16 if route == "gemv-chunks" else M
-        if isinstance(absmax, NestedAbsmax) and route == "gemm" and M > NESTED_RECONSTRUCT_MIN_M:
-            # Many rows of x on nested absmax: the fused GEMM resolves an 8-bit code through two more loads per block and
-            # k step and runs 5-27 % longer than on fp32 absmax; writing the fp32 absmax out first (nf4hip_dq_reconstruct,
-            # 4 bytes per block into a transient buffer, 4-15 us) costs 2-7 %.  Same two roundings, same bits.
-            absmax = reconstruct_absmax(absmax)
-        if isinstance(absmax, NestedAbsmax):
-            q, a2, m256, off, nbs = _nested_args(absmax, nblocks)
-            for m0 in range(0, M, step):
-                mc = min(step, M - m0)
-                _lib.check(fn_dq(x2.data_ptr() + 2 * m0 * K, _DTYPE_CODE[x.dtype], mc, qweight.data_ptr(), q.data_ptr(), a2.data_ptr(), m256.data_ptr(), off, nbs,
-                                 quant_map.data_ptr(), bptr, N, K, blocksize, out.data_ptr() + 2 * m0 * N, ws_ptr, ws_bytes, stream))  # fmt: skip
-        else:
-            _require_gpu(absmax)
-            absmax = _aligned(absmax.to(torch.float32))
-            if absmax.numel() < nblocks:
-                raise ValueError(f"absmax holds {absmax.numel()} entries, need {nblocks}")
-            for m0 in range(0, M, step):
-                mc = min(step, M - m0)
-                _lib.check(fn(x2.data_ptr() + 2 * m0 * K, _DTYPE_CODE[x.dtype], mc, qweight.data_ptr(), absmax.data_ptr(), quant_map.data_ptr(), bptr,
-                              N, K, blocksize, out.data_ptr() + 2 * m0 * N, ws_ptr, ws_bytes, stream))  # fmt: skip
-    return out.reshape(*x.shape[:-1], N)
+    out = x2.new_empty((M, N)) if type(x2) is torch.Tensor else torch.empty((M, N), dtype=x.dtype, device=device)
+    stream = _stream() if _raw_stream is None else _raw_stream(device.index)
+    if route == "stream":
+        need = lib.nf4hip_stream_workspace_bytes(M, N, K)
+        # without scratch (a capture on a stream that has none yet) the kernel does not split K
+        ws = _workspace_pool.get_or_none(device, need, stream) if need else None
+        ws_ptr, ws_bytes = (None, 0) if ws is None else (ws.data_ptr(), ws.numel())
+        fn, fn_dq = lib.nf4hip_stream, lib.nf4hip_stream_dq
+    elif route in ("gemv", "gemv-chunks"):
+        need = lib.nf4hip_gemv_workspace_bytes(min(M, 16), N, K)
+        ws = _gemv_workspace(device, need, stream)
+        ws_ptr, ws_bytes = ws.data_ptr(), ws.numel()
+        fn, fn_dq = lib.nf4hip_gemv, lib.nf4hip_gemv_dq
+    else:
+        need = lib.nf4hip_gemm_workspace_bytes(M, N, K)  # K split over workgroups: partial tiles and counters
+        ws = _gemv_workspace(device, need, stream) if need else None
+        ws_ptr, ws_bytes = (None, 0) if ws is None else (ws.data_ptr(), ws.numel())
+        fn, fn_dq = lib.nf4hip_gemm, lib.nf4hip_gemm_dq
+    bptr = None if b is None else b.data_ptr()
+    # row chunks of x and out: one call, or 16 rows at a time (rows are contiguous, K and N even,
+    # so every chunk starts 16-byte aligned when the whole does and K, N are multiples of 8)
+    step = 16 if route == "gemv-chunks" else M
+    code, x_ptr, out_ptr = _DTYPE_CODE[x.dtype], x2.data_ptr(), out.data_ptr()
+    nested = isinstance(absmax, NestedAbsmax)
+    if nested and route == "gemm" and M > NESTED_RECONSTRUCT_MIN_M:
+        # Many rows of x on nested absmax: the fused GEMM resolves an 8-bit code through two more loads per block and
+        # k step and runs 5-27 % longer than on fp32 absmax; writing the fp32 absmax out first (nf4hip_dq_reconstruct,
+        # 4 bytes per block into a transient buffer, 4-15 us) costs 2-7 %.  Same two roundings, same bits.
+        absmax, nested = reconstruct_absmax(absmax), False
+    if nested:
+        q, a2, m256, off, nbs = _nested_args(absmax, nblocks)
+        for m0 in range(0, M, step):
+            mc = min(step, M - m0)
+            _lib.check(fn_dq(x_ptr + 2 * m0 * K, code, mc, qweight.data_ptr(), q.data_ptr(), a2.data_ptr(), m256.data_ptr(), off, nbs,
+                             quant_map.data_ptr(), bptr, N, K, blocksize, out_ptr + 2 * m0 * N, ws_ptr, ws_bytes, stream))  # fmt: skip
+    else:
+        _require_gpu(absmax)
+        absmax = _aligned(absmax if absmax.dtype is torch.float32 else absmax.to(torch.float32))
+        if absmax.numel() < nblocks:
+            raise ValueError(f"absmax holds {absmax.numel()} entries, need {nblocks}")
+        for m0 in range(0, M, step):
+            mc = min(step, M - m0)
+            _lib.check(fn(x_ptr + 2 * m0 * K, code, mc, qweight.data_ptr(), absmax.data_ptr(), quant_map.data_ptr(), bptr,
+                          N, K, blocksize, out_ptr + 2 * m0 * N, ws_ptr, ws_bytes, stream))  # fmt: skip
+    return out if flat else out.reshape(*x.shape[:-1], N)
 
 
 def linear_possible(x: torch.Tensor, w: torch.Tensor, bias=None) -> bool:

@@ -232,12 +232,14 @@ size_t nf4hip_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K);
 /*
  * The launch plan nf4hip_gemm would use for a shape (no GPU needed): plan[0] rows of x per tile (64, 128 or 256),
  * plan[1] tiles (tiles of x rows x tiles of 256 weight rows), plan[2] pieces a tile is cut into along K (they meet in
- * the workspace), plan[3] workgroups launched.  Up to 128 rows of x this is what the workspace is sized by; the
- * kernel (nf4hip_stream's) lays its own tiles out inside it, cut into no more pieces.  For host code that chooses
+ * the workspace), plan[3] workgroups launched.  Where nf4hip_gemm_streamed says 1 (up to 128 rows of x, more
+ * while tiles of 128 x 256 fill the chip once at most) this is what the workspace is sized by; nf4hip_stream's kernel serves
+ * the call and lays its own tiles out in whatever workspace it is given.  For host code that chooses
  * between this kernel and dequantize + dense GEMM (the choice bitsandbytes.matmul_4bit makes at thunder/transforms/quantization.py:39) without keeping
  * a copy of the launcher's rules.  K must be a multiple of 64.
  */
 int nf4hip_gemm_plan(int64_t M, int64_t N, int64_t K, int32_t plan[4]);
+int nf4hip_gemm_streamed(int64_t M, int64_t N, int64_t K);
 int nf4hip_gemm(const void* x, int x_dtype, int64_t M, const uint8_t* packed, const float* absmax, const float* lut16,
                 const void* bias_or_null, int64_t N, int64_t K, int blocksize, void* out, void* workspace,
                 size_t workspace_bytes, void* stream);

@@ -121,7 +121,7 @@ int matmul_common(MatmulKind kind, const void* x, int x_dtype, int64_t M, const 
             return fail(NF4HIP_E_SHAPE, "nf4hip_gemv: K = %lld > 2^24 with M > 4 (use nf4hip_gemm)", (long long)K);
     } else {
         if (K % 64) return fail(NF4HIP_E_SHAPE, "%s: K = %lld is not a multiple of 64", name, (long long)K);
-        if (kind == STREAM && !nf4::stream_possible(M, N, K))
+        if (kind == STREAM && (M > 128 || !nf4::stream_possible(M, N, K)))
             return fail(NF4HIP_E_SHAPE, "%s: M = %lld, N = %lld, K = %lld: more than 128 rows, or a weight too large for 32-bit offsets", name,
                         (long long)M, (long long)N, (long long)K);
     }
@@ -413,6 +413,8 @@ int nf4hip_gemm(const void* x, int x_dtype, int64_t M, const uint8_t* packed, co
     return matmul_common(GEMM, x, x_dtype, M, packed, absmax, nullptr, lut16, bias_or_null, N, K, blocksize, out,
                          workspace, workspace_bytes, stream);
 }
+
+int nf4hip_gemm_streamed(int64_t M, int64_t N, int64_t K) { return nf4::stream_serves_gemm(M, N, K) ? 1 : 0; }
 
 size_t nf4hip_stream_workspace_bytes(int64_t M, int64_t N, int64_t K) { return nf4::stream_workspace_bytes(M, N, K); }
 

@@ -91,12 +91,13 @@ bool gemv_epilogue_possible(const MatmulArgs& a);  // does the kernel that serve
 int gemv_norm_parts(int64_t M, int64_t N, int64_t K);  // partial sums per row of x an EPI_RESID_NORM call writes (0: not served)
 size_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K);
 hipError_t launch_gemm(const MatmulArgs& a, hipStream_t stream);
-// up to 128 rows of bf16 or fp16 x (nf4_gemm_stream.hip): rows of x per tile, 32-row weight tiles side by side, workgroups
+// up to 128 rows of bf16 or fp16 x, and more where stream_serves_gemm (nf4_gemm_stream.hip): rows of x per tile, 32-row weight tiles side by side, workgroups
 // that share a tile's K, tiles.  At most `max_splits` of those workgroups, one where a.workspace_bytes does not hold them.
 struct StreamPlan {
     int bm, wn, splits, m_tiles, n_tiles;
 };
 bool stream_possible(int64_t M, int64_t N, int64_t K);
+bool stream_serves_gemm(int64_t M, int64_t N, int64_t K);  // does launch_gemm use it?
 StreamPlan stream_plan(int64_t M, int64_t N, int64_t K, int max_splits);
 size_t stream_workspace_bytes(int64_t M, int64_t N, int64_t K);
 hipError_t launch_stream(const MatmulArgs& a, bool f16, int max_splits, hipStream_t stream);

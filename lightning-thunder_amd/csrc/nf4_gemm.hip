@@ -6,7 +6,7 @@
 // bf16 in registers -- bf16_rne(lut16[code] * absmax), the same value nf4hip_dequantize produces --
 // and contracts them with bf16 MFMA, fp32 accumulation, bf16 output.
 //
-// Up to 128 rows of x: nf4_gemm_stream.hip.  More: nf4_gemm_wide.hip.  The kernel here takes what their 32-bit offsets
+// Up to 128 rows of x, and more while the chip is filled once at most: nf4_gemm_stream.hip.  Else: nf4_gemm_wide.hip.  The kernel here takes what their 32-bit offsets
 // do not reach, x of 4 GB and more or a weight of 2^31 blocks: 64-bit addresses, one workgroup per tile.
 //
 // Tile: 256 rows of x x 256 (n) x 64 (k) per workgroup of 512 threads.  Wave w of 8
@@ -335,7 +335,7 @@ void gemm_plan(int64_t M, int64_t N, int64_t K, int plan[4]) {
 }
 
 hipError_t launch_gemm(const MatmulArgs& a, hipStream_t stream) {
-    if (stream_possible(a.M, a.N, a.K)) return launch_stream(a, false, gemm_splits(a.M, a.N, a.K), stream);
+    if (stream_serves_gemm(a.M, a.N, a.K)) return launch_stream(a, false, a.M <= 128 ? gemm_splits(a.M, a.N, a.K) : 8, stream);
     if (a.M > 128 && (int64_t)a.M * a.K * 2 < ((int64_t)1 << 32)) return launch_gemm_wide(a, stream);
     return a.nested.q ? launch_tile<true>(a, stream) : launch_tile<false>(a, stream);
 }

@@ -1,4 +1,5 @@
-// Fused NF4 matmul for up to 128 rows of bf16 or fp16 x, exact weights (the kernel; launcher and rule: nf4_gemm_stream.hip).
+// Fused NF4 matmul for bf16 or fp16 x of up to 128 rows, and more while the chip is filled once at most, exact weights (the
+// kernel; launcher and rules: nf4_gemm_stream.hip).
 //
 // Replaces the dequantize_4bit + F.linear route of bitsandbytes.matmul_4bit (MatMul4Bit.forward, reached from
 // thunder/transforms/quantization.py:39) between a decode step and a prompt.  What such a call has to move is the weight,

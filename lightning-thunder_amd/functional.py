@@ -645,7 +645,8 @@ def matmul_nf4(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape) -> 
     return _matmul_nf4_on(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape, route)
 
 
-# nested absmax, fused GEMM: beyond this many rows of x the fp32 absmax is written out first (measured, us, nested kernel /
+# nested absmax, fused GEMM: beyond this many rows of x the fp32 absmax is written out first, except where the streaming kernel
+# serves the call, which is 1-5 % longer on nested absmax (measured, us, nested kernel /
 # reconstruct + fp32 kernel / fp32 kernel alone: [8192, 8192] M = 256 64 / 58 / 53, M = 512 107 / 91 / 85, M = 2048 255 / 242 / 235;
 # [28672, 8192] M = 512 242 / 226 / 213, M = 2048 930 / 854 / 837; [8192, 28672] M = 1024 481 / 439 / 425; [1024, 8192] M = 512 38 / 37 / 34)
 NESTED_RECONSTRUCT_MIN_M = 128
@@ -692,7 +693,10 @@ def _matmul_nf4_on(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape,
         fn, fn_dq = lib.nf4hip_gemv, lib.nf4hip_gemv_dq
     else:
         need = lib.nf4hip_gemm_workspace_bytes(M, N, K)  # K split over workgroups: partial tiles and counters
-        ws = _gemv_workspace(device, need, stream) if need else None
+        want = max(need, lib.nf4hip_stream_workspace_bytes(M, N, K)) if lib.nf4hip_gemm_streamed(M, N, K) else need
+        ws = _workspace_pool.get_or_none(device, want, stream) if want else None
+        if ws is None and need:
+            ws = _gemv_workspace(device, need, stream)
         ws_ptr, ws_bytes = (None, 0) if ws is None else (ws.data_ptr(), ws.numel())
         fn, fn_dq = lib.nf4hip_gemm, lib.nf4hip_gemm_dq
     bptr = None if b is None else b.data_ptr()
@@ -701,7 +705,7 @@ def _matmul_nf4_on(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape,
     step = 16 if route == "gemv-chunks" else M
     code, x_ptr, out_ptr = _DTYPE_CODE[x.dtype], x2.data_ptr(), out.data_ptr()
     nested = isinstance(absmax, NestedAbsmax)
-    if nested and route == "gemm" and M > NESTED_RECONSTRUCT_MIN_M:
+    if nested and route == "gemm" and M > NESTED_RECONSTRUCT_MIN_M and not lib.nf4hip_gemm_streamed(M, N, K):
         # Many rows of x on nested absmax: the fused GEMM resolves an 8-bit code through two more loads per block and
         # k step and runs 5-27 % longer than on fp32 absmax; writing the fp32 absmax out first (nf4hip_dq_reconstruct,
         # 4 bytes per block into a transient buffer, 4-15 us) costs 2-7 %.  Same two roundings, same bits.

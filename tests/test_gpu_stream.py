@@ -109,6 +109,49 @@ def test_stream_capture_without_scratch_and_autograd(ta):
     torch.testing.assert_close(xg.grad[0].float(), deq.float().sum(0), rtol=1e-2, atol=1e-2)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,blocksize,nested,bias", [
+    (129, 300, 320, 64, False, True), (200, 65, 2880, 64, True, False), (256, 512, 64, 64, False, False), (1025, 1024, 4096, 64, True, True),
+    (513, 1000, 1536, 128, False, False), (2048, 4096, 2048, 64, False, False), (130, 32768, 2048, 64, True, False), (300, 264, 28672, 64, False, True),
+])
+@pytest.mark.parametrize("scratch", [True, False])
+def test_gemm_streamed_beyond_128_rows(ta, M, N, K, blocksize, nested, bias, scratch):
+    """``nf4hip_gemm`` on the streaming kernel for more than 128 rows of x (several tiles of x rows, K split or not)."""
+    print(f"streamed gemm M={M} [{N},{K}] bs={blocksize} nested={nested} bias={bias} scratch={scratch}", flush=True)
+    F, lib = ta.functional, ta._lib.load()
+    assert lib.nf4hip_gemm_streamed(M, N, K)
+    qw, stats, code = _weight(ta, N, K, blocksize, nested, torch.bfloat16, M + N)
+    g = torch.Generator(device=DEV).manual_seed(K)
+    x = torch.empty(M, K, device=DEV).normal_(0, 1, generator=g).to(torch.bfloat16)
+    b = torch.empty(N, device=DEV).normal_(0, 1, generator=g).to(torch.bfloat16) if bias else None
+    deq = ta.dequantize_nf4(qw, stats, code, blocksize, torch.bfloat16, (N, K))
+    if scratch:
+        run = lambda: F._matmul_nf4_on(x, qw, b, stats, code, blocksize, torch.bfloat16, (N, K), "gemm")
+    else:  # the least the C ABI accepts
+        need = lib.nf4hip_gemm_workspace_bytes(M, N, K)
+        ws = torch.zeros(max(need, 16), dtype=torch.uint8, device=DEV)
+        if nested:
+            stats = ta.reconstruct_absmax(stats)
+
+        def run():
+            out = torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+            ta._lib.check(lib.nf4hip_gemm(x.data_ptr(), 0, M, qw.data_ptr(), stats.data_ptr(), code.data_ptr(), None if b is None else b.data_ptr(), N, K,
+                                          blocksize, out.data_ptr(), ws.data_ptr() if need else None, need, F._stream()))
+            return out
+
+    y = run()
+    _check(y, x, deq, b)
+    assert torch.equal(run(), y)
+
+
+def test_gemm_streamed_rule(ta):
+    """Tiles of 128 x 256 fill the chip once at most (half of it with few k steps); beyond 32-bit offsets never."""
+    served = ta._lib.load().nf4hip_gemm_streamed
+    assert served(128, 1 << 20, 4096) and served(2048, 4096, 4096) and not served(2049, 4096, 4096) and served(256, 32768, 2048)
+    assert not served(257, 32768, 2048) and not served(256, 32768, 1024) and served(256, 16384, 1024) and not served(1 << 18, 64, 8192)
+    assert not served(128, 1 << 26, 4096) and not served(0, 64, 64) and not served(8, 64, 96)
+
+
 def test_stream_arguments_and_workspace(ta):
     """Checked before any HIP call; the workspace holds what the plan can need and is optional."""
     L = ta._lib

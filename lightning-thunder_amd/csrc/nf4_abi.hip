@@ -121,8 +121,8 @@ int matmul_common(MatmulKind kind, const void* x, int x_dtype, int64_t M, const 
             return fail(NF4HIP_E_SHAPE, "nf4hip_gemv: K = %lld > 2^24 with M > 4 (use nf4hip_gemm)", (long long)K);
     } else {
         if (K % 64) return fail(NF4HIP_E_SHAPE, "%s: K = %lld is not a multiple of 64", name, (long long)K);
-        if (kind == STREAM && (M > 128 || !nf4::stream_possible(M, N, K)))
-            return fail(NF4HIP_E_SHAPE, "%s: M = %lld, N = %lld, K = %lld: more than 128 rows, or a weight too large for 32-bit offsets", name,
+        if (kind == STREAM && !nf4::stream_serves_gemm(M, N, K))
+            return fail(NF4HIP_E_SHAPE, "%s: M = %lld, N = %lld, K = %lld: not served (nf4hip_gemm_streamed)", name,
                         (long long)M, (long long)N, (long long)K);
     }
     if (!(kind == GEMV && M <= 4) && K % blocksize)

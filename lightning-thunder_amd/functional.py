@@ -577,6 +577,7 @@ def fused_route(x: torch.Tensor, bias, blocksize: int, dtype: torch.dtype, shape
 
 
 STREAM_MAX_M = 128
+STREAM_F16_MAX_M = 2048
 STREAM_LONG_WEIGHT = 1 << 25
 
 
@@ -600,10 +601,13 @@ def _stream_serves(x, qweight, bias, absmax, quant_map, blocksize: int, dtype: t
     9.5), and from 2^25 elements on beyond K = 16384, where those reproduce every weight's rounding and are slow ([8192, 28672]
     M = 8 / 16 38.7 / 45.0 vs 36.3 / 35.4, nested absmax 45.5 / 51.1 vs 35.4 / 36.3).  Smaller weights stay in the kernel that
     their epilogue forms run in.
-    fp16, up to 128 rows: always; the alternative writes the dense weight first ([14336, 4096] M = 4: 47 vs 13)."""
+    fp16, up to 128 rows: always; the alternative writes the dense weight first ([14336, 4096] M = 4: 47 vs 13).  Up to 2048
+    rows: while the kernel's tiles fill the chip once (M = 256 / 512 / 1024 / 2048 [1024, 4096] 21.0 / 23.6 / 26.8 / 33.2 vs 10.8 / 13.3 /
+    20.8 / 28.5; [4096, 4096] 34.7 / 40.0 / 52.7 / 75.9 vs 20.1 / 27.3 / 50.7 / 72.2; [4096, 14336] 90.6 / 113.9 / 146.8 / 226.1 vs 48.7 / 74.8 /
+    130.2 / 228.4; beyond, nothing was measured)."""
     N, K = shape
     M = x.numel() // K if K else 0
-    if (not 1 <= M <= STREAM_MAX_M or N <= 0 or x.dtype != dtype or dtype not in (torch.bfloat16, torch.float16)
+    if (not 1 <= M <= (STREAM_F16_MAX_M if dtype is torch.float16 else STREAM_MAX_M) or N <= 0 or x.dtype != dtype or dtype not in (torch.bfloat16, torch.float16)
             or K % 64 or blocksize not in SUPPORTED_BLOCKSIZES or K % blocksize or K >= 1 << 24 or N * (K // 64) >= 1 << 31
             or (bias is not None and bias.dtype != dtype)):
         return False
@@ -612,6 +616,8 @@ def _stream_serves(x, qweight, bias, absmax, quant_map, blocksize: int, dtype: t
         if M > 16:
             return True
         return M > 4 and (K % 512 != 0 or (K > 16384 and N * K >= STREAM_LONG_WEIGHT))
+    if M > STREAM_MAX_M and not _lib.load().nf4hip_gemm_streamed(M, N, K):
+        return False
     stats = absmax.q if nested else absmax
     return (_is_plain(x, bias) and (bias is None or bias.shape == (N,)) and (nested or absmax.numel() >= N * K // blocksize)
             and qweight.numel() >= N * K // 2 and quant_map.numel() >= 16 and all(t is None or t.device == x.device for t in (qweight, bias, stats)))

@@ -36,7 +36,7 @@ def _check(y, x, deq, bias):
     (1, 1, 64, 64, False, True), (5, 63, 64, 64, True, False), (16, 64, 192, 64, False, False), (17, 65, 256, 64, True, True),
     (32, 300, 320, 64, False, True), (33, 129, 1344, 64, True, False), (64, 1000, 2880, 64, False, True), (65, 257, 1024, 128, False, False),
     (100, 515, 1536, 256, True, True), (128, 4098, 4096, 64, False, True), (128, 96, 28672, 64, True, False), (48, 4096, 4096, 64, True, False),
-    (20, 40000, 512, 64, False, False), (16, 8192, 28672, 64, True, False), (2, 8192, 2048, 2048, False, True),
+    (20, 40000, 512, 64, False, False), (16, 8192, 28672, 64, True, False), (129, 300, 320, 64, True, True), (1000, 1000, 2880, 64, False, True), (2, 8192, 2048, 2048, False, True),
 ])
 def test_stream_matches_float64(ta, dtype, M, N, K, blocksize, nested, bias):
     print(f"stream M={M} [{N},{K}] bs={blocksize} nested={nested} bias={bias} {dtype}", flush=True)
@@ -161,7 +161,7 @@ def test_stream_arguments_and_workspace(ta):
         return lib.nf4hip_stream(x, dt, M, packed, absmax, lut, bias, N, K, bs, out, w, wb, None)
 
     assert call(x=None) == L.E_NULL and call(absmax=None) == L.E_NULL and call(dt=L.F32) == L.E_DTYPE and call(bs=96) == L.E_BLOCKSIZE
-    assert call(M=0) == L.E_SHAPE and call(M=129) == L.E_SHAPE and call(K=96) == L.E_SHAPE and call(K=192, bs=128) == L.E_SHAPE
+    assert call(M=0) == L.E_SHAPE and call(M=257, N=32768) == L.E_SHAPE and call(K=96) == L.E_SHAPE and call(K=192, bs=128) == L.E_SHAPE
     assert call(K=1 << 24) == L.E_SHAPE and call(N=1 << 30) == L.E_SHAPE
     assert call(out=A + 2) == L.E_ALIGN and call(w=A + 8, wb=1 << 20) == L.E_ALIGN
     for M in (1, 16, 17, 33, 65, 128):
@@ -183,6 +183,7 @@ def test_stream_serves(ta):
         return F._stream_serves(x, torch.empty(N * K // 2, 1, dtype=torch.uint8), bias, stats, torch.empty(16), bs, dtype, (N, K))
 
     assert not serves(16, 64, 4096) and serves(17, 64, 4096) and serves(128, 64, 4096) and not serves(129, 64, 4096)
+    assert serves(2048, 64, 4096, hf) and not serves(2049, 64, 4096, hf) and not serves(512, 32768, 256, hf)
     assert serves(5, 64, 1344) and not serves(4, 64, 1344) and not serves(17, 64, 1376) and not serves(17, 64, 192, bs=128)
     assert serves(5, 8192, 28672, nested=True) and serves(16, 8192, 28672) and not serves(5, 1000, 28672) and not serves(4, 8192, 28672, nested=True)
     assert not serves(17, 64, 4096, bias=torch.empty(64)) and not serves(17, 64, 4096, xdtype=hf)

@@ -13,13 +13,14 @@
 // * Codes go from memory into the wave's own 4 KB slot of LDS and from there into registers, a set of four steps at a time.
 //   Loaded into registers directly, in the layout the fragments need (32 rows x 32 bytes per request instead of 8 rows x
 //   128), they cost the CU's address unit twice the time, and a wave that waits to place a request multiplies nothing:
-//   [8192, 28672], M = 16 50.9 -> 44 us by the layout, -> 38 by fetching four steps' absmax in one request.
+//   [8192, 28672], M = 16, fp32 absmax 51 us then, 45 this way, 38 with a set's requests placed one behind each slice and K
+//   dealt in units instead of ranges.
 // * Producer wave p moves a quarter of x, memory -> LDS, three stages.  Requests of one wave complete in order, so a wave
 //   that fetched both x (from L2) and codes (from HBM) would turn every wait for x into one for the codes before it.
 // * One barrier per stage of x.  The WK partial sums of a tile meet in LDS, in a fixed order; with splits they meet in
 //   the workspace (protocol of nf4_common.h), again in a fixed order.
 //
-// What bounds it (counters and variants, [8192, 28672], M = 16): no unit is busy more than half the time (VALU 37 %, address
+// What bounds it (counters of its first form and variants with parts taken out, [8192, 28672], M = 16): no unit is busy more than half the time (VALU 37 %, address
 // unit 53 %, LDS 22 %, MFMA 14 %); with two consumer waves per SIMD that meet at a barrier the times of fetch (~12 us),
 // expansion (~12) and multiplication with its LDS reads (~16) add up more than they overlap.  Book (64 KB), code slots
 // (32 KB) and x leave no LDS for more waves.

@@ -71,9 +71,11 @@ _map_masters: dict[str, torch.Tensor] = {}
 
 
 def _dynamic_map_values() -> torch.Tensor:
+    """Built on the CPU in fp32 whatever the process's default device and dtype are: the result is kept, and quantised
+    weights depend on its last bits."""
     data: list[float] = []
     for i in range(7):
-        boundaries = torch.linspace(0.1, 1, 2**i + 1)
+        boundaries = torch.linspace(0.1, 1, 2**i + 1, dtype=torch.float32, device="cpu")
         means = (boundaries[:-1] + boundaries[1:]) / 2.0
         scale = 10 ** (-6 + i)
         data += (scale * means).tolist()
@@ -85,8 +87,9 @@ def _dynamic_map_values() -> torch.Tensor:
 
 
 def _dynamic_map_master(device=None) -> torch.Tensor:
-    """The map as this package's own tensor, one per device: read it, never hand it out (``dynamic_map`` gives copies)."""
-    dev = torch.device(device) if device is not None else torch.device("cpu")
+    """The map as this package's own tensor, one per device (default: torch's default device): read it, never hand it
+    out (``dynamic_map`` gives copies)."""
+    dev = torch.device(device) if device is not None else torch.get_default_device()
     if dev.type == "cuda" and dev.index is None:
         dev = torch.device("cuda", torch.cuda.current_device())
     master = _map_masters.get(str(dev))

@@ -195,6 +195,25 @@ def test_python_wrappers_refuse_cpu_tensors(ta):
                       torch.zeros(4), ta.nf4_code(), 64, torch.bfloat16, (4, 64))
 
 
+def test_dynamic_map_ignores_default_device_and_dtype(ta, oracle, monkeypatch):
+    """The kept map is computed on the CPU in fp32; only where a copy without a device goes follows the default device."""
+    import torch
+
+    F = ta.functional
+    monkeypatch.setattr(F, "_map_masters", {})
+    before = torch.get_default_dtype()
+    try:
+        torch.set_default_dtype(torch.bfloat16)
+        with torch.device("meta"):
+            kept = F._dynamic_map_values()
+            assert F.dynamic_map().device.type == "meta" and F.dynamic_map("cpu").device.type == "cpu"
+    finally:
+        torch.set_default_dtype(before)
+    assert kept.device.type == "cpu" and torch.equal(kept, oracle.create_dynamic_map())
+    assert torch.equal(F.dynamic_map(), oracle.create_dynamic_map())
+    assert F.dynamic_map() is not F.dynamic_map()
+
+
 def test_check_raises_with_message(ta):
     lib = ta._lib.load()
     rc = lib.nf4hip_quantize(A, 9, 1, 64, A, A, None)

@@ -101,7 +101,8 @@ bool stream_serves_gemm(int64_t M, int64_t N, int64_t K);  // does launch_gemm u
 StreamPlan stream_plan(int64_t M, int64_t N, int64_t K, int max_splits);
 size_t stream_workspace_bytes(int64_t M, int64_t N, int64_t K);
 hipError_t launch_stream(const MatmulArgs& a, bool f16, int max_splits, hipStream_t stream);
-// more than 128 rows of x: one wave per SIMD, 256 x 256 or 128 x 256 tiles (nf4_gemm_wide.hip)
+// what the streaming kernel does not take, with x below 4 GB: 256 x 256 or 128 x 256 tiles (nf4_gemm_wide.hip)
+bool gemm_wide_possible(int64_t M, int64_t K);
 int gemm_wide_tile_rows(int64_t M, int64_t N, int64_t K);
 hipError_t launch_gemm_wide(const MatmulArgs& a, hipStream_t stream);
 size_t gemm_wide_workspace_bytes(int64_t M, int64_t N, int64_t K);

@@ -6,8 +6,9 @@
 // bf16 in registers -- bf16_rne(lut16[code] * absmax), the same value nf4hip_dequantize produces --
 // and contracts them with bf16 MFMA, fp32 accumulation, bf16 output.
 //
-// Up to 128 rows of x, and more while the chip is filled once at most: nf4_gemm_stream.hip.  Else: nf4_gemm_wide.hip.  The kernel here takes what their 32-bit offsets
-// do not reach, x of 4 GB and more or a weight of 2^31 blocks: 64-bit addresses, one workgroup per tile.
+// Up to 128 rows of x, and more while the chip is filled once at most: nf4_gemm_stream.hip.  Else, and where that kernel's
+// 32-bit offsets into a weight end (K >= 2^24, 2^31 blocks): nf4_gemm_wide.hip.  The kernel here takes what the other two's 32-bit
+// offsets into x do not reach, x of 4 GB and more: 64-bit addresses, one workgroup per tile.
 //
 // Tile: 256 rows of x x 256 (n) x 64 (k) per workgroup of 512 threads.  Wave w of 8
 // owns weight rows 32 w .. + 31 of the tile against all rows of x: eight accumulators of
@@ -317,7 +318,8 @@ hipError_t launch_tile(const MatmulArgs& a, hipStream_t stream) {
 }  // namespace
 
 size_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-    if (M > 128) return M * K * 2 < ((int64_t)1 << 32) ? gemm_wide_workspace_bytes(M, N, K) : 0;
+    if (!stream_serves_gemm(M, N, K)) return gemm_wide_possible(M, K) ? gemm_wide_workspace_bytes(M, N, K) : 0;
+    if (M > 128) return gemm_wide_workspace_bytes(M, N, K);
     const int splits = gemm_splits(M, N, K);
     if (splits == 1) return 0;
     const int64_t bm = M <= 64 ? 64 : 128;
@@ -325,18 +327,19 @@ size_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
 }
 
 void gemm_plan(int64_t M, int64_t N, int64_t K, int plan[4]) {
-    if (M > 128 && M * K * 2 < ((int64_t)1 << 32)) return gemm_wide_plan(M, N, K, plan);
-    const int bm = M <= 64 ? 64 : M <= 128 ? 128 : 256;
+    const bool streamed = stream_serves_gemm(M, N, K);
+    if (streamed ? M > 128 : gemm_wide_possible(M, K)) return gemm_wide_plan(M, N, K, plan);
+    const int bm = !streamed ? BM : M <= 64 ? 64 : 128;
     const int64_t tiles = ((M + bm - 1) / bm) * ((N + BN - 1) / BN);
     plan[0] = bm;
     plan[1] = (int)tiles;
-    plan[2] = gemm_splits(M, N, K);
+    plan[2] = streamed ? gemm_splits(M, N, K) : 1;
     plan[3] = (int)tiles * plan[2];
 }
 
 hipError_t launch_gemm(const MatmulArgs& a, hipStream_t stream) {
     if (stream_serves_gemm(a.M, a.N, a.K)) return launch_stream(a, false, a.M <= 128 ? gemm_splits(a.M, a.N, a.K) : 8, stream);
-    if (a.M > 128 && (int64_t)a.M * a.K * 2 < ((int64_t)1 << 32)) return launch_gemm_wide(a, stream);
+    if (gemm_wide_possible(a.M, a.K)) return launch_gemm_wide(a, stream);
     return a.nested.q ? launch_tile<true>(a, stream) : launch_tile<false>(a, stream);
 }
 

@@ -1,4 +1,4 @@
-// Prefill-shape fused NF4 dequant-matmul for gfx950, more than 128 rows of x.
+// Fused NF4 dequant-matmul for gfx950: long prompts, and what else the kernel of nf4_gemm_stream.h does not take.
 //
 // Replaces the dequantize_4bit + F.linear route of bitsandbytes.matmul_4bit (MatMul4Bit.forward),
 // reached from thunder/transforms/quantization.py:39, like gemm_kernel in nf4_gemm.hip: every wave
@@ -150,15 +150,16 @@ __device__ __forceinline__ void expansion_step(Expansion& x, int t, uint32_t d, 
 //   * The first `full` = rounds * GRID tiles are taken whole, one workgroup each.  Tile numbers (m fastest) are
 //     dealt so that every XCD -- workgroup b runs on XCD b % 8 -- owns a contiguous run of them: the x-row tiles
 //     that share a weight tile meet in one L2.
-//   * The remaining `tail_tiles` (fewer than GRID) would leave CUs idle in a last, partial round, so each of them
-//     can be cut into `pieces` equal pieces along k (in quanta of `gran` k steps, qpt per tile), one workgroup per
+//   * The remaining `tail_tiles` (fewer than GRID) would leave CUs idle in a last, partial round.  Where a call has no
+//     other tiles -- nearly all such calls are nf4_gemm_stream.hip's; what is left are shapes beyond its 32-bit offsets,
+//     K >= 2^24 or a weight of 2^31 blocks -- each of them can be cut into `pieces` equal pieces along k (in quanta of `gran` k steps, qpt per tile), one workgroup per
 //     piece, numbered piece-major (all first pieces, then all second pieces, ...).  The pieces of a tile meet in
 //     the workspace (see the kernel).  pieces == 1: whole tiles.
 struct WideSchedule {
     int m_tiles, n_tiles;
     int full, tail_tiles, pieces;
     int qpt, gran;
-    uint32_t* counters;  // two per tail tile, zero between calls
+    uint32_t* counters;  // one per tail tile, zero between calls
     float* partials;     // one slot of BM x 256 floats per piece
 };
 constexpr int GRID = 256;
@@ -403,73 +404,35 @@ void gemm_wide_kernel(MatmulArgs a, WideSchedule sch) {
 
     // ---- a piece of a tail tile: meet the tile's other pieces in the workspace ----
     // Pieces are numbered in k order; piece c of tail tile t has a slot of its own (t * pieces + c) for its fp32
-    // partial tile in register order ([i][g][q][thread]: coalesced).  Two counters per tile, zero between calls: P
-    // counts published partials, T hands out tickets.
-    //   * Every piece but the last to finish stores its partial, waits until L2 has it (publish_partials), and only
-    //     then counts itself in P.  Whoever raises P to the number of pieces adds all partials from memory, in k
-    //     order, and writes the tile.
-    //   * Two pieces (the common case): the holder of the second ticket looks at P first; if the other partial is
-    //     published already, it adds it to its registers and writes the tile without storing a partial (a + b = b + a
-    //     exactly, so the result does not depend on who finishes last).  Otherwise it proceeds like everyone else.
-    // No workgroup ever waits for another one.
+    // partial tile in register order ([i][g][q][thread]: coalesced).  Every piece stores its partial, waits until L2 has
+    // it (publish_partials), and only then counts itself in the tile's counter (zero between calls).  Whoever raises it to
+    // the number of pieces adds all partials from memory, in k order, and writes the tile.  No workgroup ever waits
+    // for another one.
     bool write_tile = true;
     if (partial) {
         constexpr int SLOT = BM * BN;  // floats
         constexpr int FR = 16 * T::THREADS;  // floats per accumulator fragment
         const int pieces = sch.pieces;
-        uint32_t* cP = sch.counters + 2 * tail_tile;
-        uint32_t* cT = cP + 1;
+        uint32_t* arrived = sch.counters + tail_tile;
         auto slot_of = [&](int c) { return sch.partials + (int64_t)(tail_tile * pieces + c) * SLOT; };
         volatile uint32_t* flag = reinterpret_cast<volatile uint32_t*>(smem + BOOK_BYTES);
-        bool in_registers = false;
-        if (pieces == 2) {
-            if (tid == 0) {
-                const uint32_t ticket = __hip_atomic_fetch_add(cT, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                uint32_t ok = 0;
-                if (ticket == 1) ok = __hip_atomic_load(cP, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 1u;
-                *flag = ok;
-            }
-            __syncthreads();
-            in_registers = *flag != 0;
-            acquire_partials();
-            __syncthreads();
-        }
-        bool from_memory = false;
-        if (!in_registers) {
-            float* mine = slot_of(piece);
+        float* mine = slot_of(piece);
 #pragma unroll
-            for (int i = 0; i < T::TI; ++i)
+        for (int i = 0; i < T::TI; ++i)
 #pragma unroll
-                for (int g = 0; g < NG; ++g)
+            for (int g = 0; g < NG; ++g)
 #pragma unroll
-                    for (int q = 0; q < 16; ++q)
-                        __hip_atomic_store(mine + ((i * NG + g) * 16 + q) * T::THREADS + tid, acc[i][g][q], __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_AGENT);
-            publish_partials();
-            __syncthreads();
-            if (tid == 0) *flag = __hip_atomic_fetch_add(cP, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
-            __syncthreads();
-            from_memory = *flag == (uint32_t)pieces;
-            acquire_partials();
-            __syncthreads();
-        }
-        if (in_registers) {
-            const float* other = slot_of(piece ^ 1);
-            constexpr int B = 4;  // fragments whose loads are in flight together
-#pragma unroll
-            for (int f0 = 0; f0 < T::TI * NG; f0 += B) {
-                float v[B][16];
-#pragma unroll
-                for (int f = 0; f < B; ++f)
-#pragma unroll
-                    for (int q = 0; q < 16; ++q)
-                        v[f][q] = __hip_atomic_load(other + ((f0 + f) * 16 + q) * T::THREADS + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-                for (int f = 0; f < B; ++f)
-#pragma unroll
-                    for (int q = 0; q < 16; ++q) acc[(f0 + f) / NG][(f0 + f) % NG][q] += v[f][q];
-            }
-        } else if (from_memory) {
+                for (int q = 0; q < 16; ++q)
+                    __hip_atomic_store(mine + ((i * NG + g) * 16 + q) * T::THREADS + tid, acc[i][g][q], __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+        publish_partials();
+        __syncthreads();
+        if (tid == 0) *flag = __hip_atomic_fetch_add(arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
+        __syncthreads();
+        write_tile = *flag == (uint32_t)pieces;
+        acquire_partials();
+        __syncthreads();
+        if (write_tile) {
             constexpr int G = 4;  // pieces whose loads are in flight together
 #pragma unroll
             for (int f = 0; f < T::TI * NG; ++f) {
@@ -496,11 +459,7 @@ void gemm_wide_kernel(MatmulArgs a, WideSchedule sch) {
 #pragma unroll
                 for (int q = 0; q < 16; ++q) acc[f / NG][f % NG][q] = sum[q];
             }
-        }
-        write_tile = in_registers || from_memory;
-        if (write_tile && tid == 0) {
-            __hip_atomic_store(cP, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(cT, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (tid == 0) __hip_atomic_store(arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
     if (write_tile) {
@@ -620,11 +579,15 @@ hipError_t launch_tile(const MatmulArgs& a, hipStream_t stream) {
 
 }  // namespace
 
+// 32-bit offsets: of x, and of a k step inside a row of it
+bool gemm_wide_possible(int64_t M, int64_t K) { return M * K * 2 < ((int64_t)1 << 32) && K < (1 << 30); }
+
 // Rows of x per tile (a pure function of the shape).  The 256-row tile expands every weight half as often, the
 // 128-row tile gives twice the workgroups: 256 rows once that makes 160 tiles or more, or when the k loop is long
 // enough for the pieces of a cut-up tile to stay long (tiles x k steps >= 28672, e.g. 128 tiles of K = 14336);
 // measured on both sides of either bound.
 int gemm_wide_tile_rows(int64_t M, int64_t N, int64_t K) {
+    if (M <= 128) return 128;
     const int64_t tiles = ((M + 255) / 256) * ((N + BN - 1) / BN);
     return tiles >= 160 || tiles * (K / BK) >= 28672 ? 256 : 128;
 }

@@ -25,10 +25,6 @@ from ._workspace import WorkspacePool
 
 SUPPORTED_BLOCKSIZES = (64, 128, 256, 512, 1024, 2048, 4096)
 
-# Beyond this K the decode kernels round every weight exactly like the reference's dequantisation
-# (the cheaper "scale the partial sum" arithmetic drifts from it like sqrt(K)); the 5..16-row tile
-# kernel has no such variant, so those calls go to the prefill kernel, which is exact by construction.
-EXACT_K = 8192
 # K beyond which a call that no model above claims goes to dequantize + dense GEMM even for a few rows of x
 LONG_K = 16384
 # From this many rows of x on, HIP dequantize followed by the dense library GEMM is a candidate
@@ -340,9 +336,9 @@ def matmul_nf4_dq(x, qweight, bias, absmax_q, nested_absmax, nested_quant_map, n
 # matmul
 # ------------------------------------------------------------------------------------------------
 
-# 40 MiB covers every Llama-3-8B / 70B projection shape on both fused routes (the largest need is the fused
-# GEMM's 33 MB of partial tiles at [16384, 8192], M = 128), so a stream's buffer is normally allocated once.
-_workspace_pool = WorkspacePool(65 << 20, "NF4 matmul")  # 256 partial tiles of 256 x 256 floats + the counter region
+# 65 MiB -- 256 partial tiles of 256 x 256 floats (nf4hip_linear's two pieces of 128 tiles) and the counter region -- is the
+# most any kernel asks for, so a stream's buffer is allocated once.
+_workspace_pool = WorkspacePool(65 << 20, "NF4 matmul")
 
 
 def _gemv_workspace(device: torch.device, nbytes: int, stream: int | None = None) -> torch.Tensor:
@@ -365,34 +361,6 @@ def _gemm_plan(M: int, N: int, K: int) -> tuple[int, int, int, int]:
     plan = (ctypes.c_int * 4)()
     _lib.check(_lib.load().nf4hip_gemm_plan(M, N, K, ctypes.byref(plan)))
     return plan[0], plan[1], plan[2], plan[3]
-
-
-def _gemm_splits(M: int, N: int, K: int) -> int:
-    """K splits of the fused GEMM kernel for up to 128 rows of x (1 beyond)."""
-    return _gemm_plan(M, N, K)[2] if M <= 128 else 1
-
-
-def _fused_gemm_us(M: int, N: int, K: int) -> float:
-    """Model of the fused GEMM kernel's time for up to 128 rows of x (one tile of x rows): tiles of
-    256 weight rows x K splits run in rounds of 256 workgroups (one per CU), K / 64 / splits steps
-    each; a step takes 0.6 us (64-row tile, M <= 64) or 0.8 us (128-row tile) on a sparsely filled chip
-    and 0.35 / 0.5 us more on a full one; merging the splits adds 9 / 16 us, a launch 3 (measured,
-    M = 64 / 128: [4096, 4096] 19 / 30, [6144, 4096] 20 / 30, [4096, 14336] 31 / 45, [14336, 4096] 26 / 35,
-    [16384, 8192] 40 / 56, [28672, 4096] 37 / 52, lm_head [128256, 4096] 121 / 167 us)."""
-    splits = _gemm_splits(M, N, K)
-    wgs = (N + 255) // 256 * splits
-    rounds = (wgs + 255) // 256
-    fill = min(1.0, wgs / rounds / 256.0)
-    step = 0.6 + 0.35 * fill if M <= 64 else 0.8 + 0.5 * fill
-    merge = 0.0 if splits == 1 else 9.0 if M <= 64 else 16.0
-    return 3.0 + rounds * (K // 64 // splits) * step + merge
-
-
-def _dense_route_us(N: int, K: int) -> float:
-    """Model of the dense route before its GEMM: the dequantize kernel writes 2 bytes per weight at HBM
-    speed, 20 + 0.62 W us for W million weights (measured with the GEMM of 64 rows of x: [14336, 4096]
-    56, [28672, 4096] 108, [16384, 8192] 115, lm_head [128256, 4096] 428 us)."""
-    return 20.0 + 0.62 * N * K / 1e6
 
 
 def _wide_schedule(M: int, N: int, K: int) -> tuple[int, int, int]:
@@ -438,53 +406,17 @@ def _dense_gemm_us(M: int, N: int, K: int) -> float:
 
 
 def _fused_gemm_wins(M: int, N: int, K: int, nested: bool = False) -> bool:
-    """Is the fused GEMM kernel faster than dequantize + dense GEMM?  Both sides are modelled from
-    measurements on MI355X.  Up to 128 rows of x (one tile of x rows, K split over workgroups) the fused kernel's
-    time hardly depends on N while the chip is not full, the dense route's grows with the weight (M = 64, us:
-    [4096, 4096] 19 vs 34, [14336, 4096] 26 vs 55, [4096, 14336] 31 vs 64, [28672, 4096] 37 vs 107).  Beyond that the fused kernel
+    """Is the fused GEMM kernel faster than dequantize + dense GEMM (calls that ``_stream_takes`` leaves)?  Both sides are
+    modelled from measurements on MI355X.  The fused kernel
     runs at 1.0-1.15 PFLOP/s, the library GEMM at up to 1.5, but the dense route first writes the bf16 weight: the
     two cross near 1024 rows of x wherever the fused kernel has a workgroup for most CUs (fused vs dense, us, M =
     512 / 1024 / 2048: [14336, 4096] 71 / 117 / 232 vs 84 / 118 / 198; [28672, 4096] 127 / 239 / 473 vs 155 / 238 / 405; [28672, 8192] 226 /
     442 / 881 vs 291 / 466 / 789; lm_head [128256, 4096] 497 / 978 / 1938 vs 741 / 1099 / 1831; short weights leave the chip
     empty: [4096, 14336] 164 / 174 / 255 vs 107 / 142 / 216, [4096, 4096] 54 / 58 / 79 vs 42 / 52 / 75).  A tie goes to the fused kernel,
     which needs no transient bf16 weight."""
-    if M <= 128:
-        return _fused_gemm_us(M, N, K) < _dense_route_us(N, K)
     # nested absmax: the fp32 absmax is written out ahead of the fused kernel (_matmul_nf4_on), 2-7 % on top; the
     # dequantize pass of the dense route resolves the codes itself at no measurable cost
     return _wide_gemm_us(M, N, K) * (1.05 if nested else 1.0) <= 1.03 * _dense_gemm_us(M, N, K)
-
-
-def _gemv_pass_us(N: int, K: int, nested: bool = False) -> float:
-    """Model of one 16-row pass of the decode kernels over a weight of W million elements, from measurements on MI355X
-    (us): the LDS-staged kernel 7.6 + 0.09 W while one workgroup covers K ([14336, 4096] 12.9, [28672, 4096] 17.6,
-    [32000, 4096] 18.5, lm_head [128256, 4096] 54.7) and 9.5 + 0.108 W with K split over workgroups ([4096, 14336] 16.8,
-    [10240, 8192] 17.0, [28672, 8192] 33.8, [57344, 8192] 60.3); the other decode kernels 12 + 0.105 W.  Which kernel it is, the
-    library says (nf4hip_gemv_plan, no GPU needed)."""
-    w = N * K / 1e6
-    plan = (ctypes.c_int * 4)()
-    if _lib.load().nf4hip_gemv_plan(16, N, K, 64, 1 if nested else 0, ctypes.byref(plan)) == 0 and plan[0] == 5:
-        return 7.6 + 0.09 * w if K <= 4096 else 9.5 + 0.108 * w
-    return 12.0 + 0.105 * w
-
-
-def _chunked_gemv_wins(M: int, N: int, K: int, nested: bool = False) -> bool:
-    """For a few more than 16 rows of x: are ceil(M / 16) passes of the decode kernel over the NF4
-    weight cheaper than the alternatives?  All sides modelled from measurements on MI355X
-    (microseconds, W = weights in millions): a 16-row pass takes _gemv_pass_us; the dense route
-    20 + 0.62 W before its GEMM, and the passes must beat that by 20 %; the fused GEMM kernel, where
-    it applies, _fused_gemm_us.  Measured, passes vs fused GEMM, M = 32 / 48: [28672, 4096] 34.8 / 51.6 vs 43.6 / 40.2;
-    lm_head [128256, 4096] 115.7 / 166.5 vs 124.5 / 126.9; [4096, 14336] 32.6 / 47.4 vs 34.2 / 34.3; [14336, 4096] 24.6 / 36.6 vs
-    26.5 / 26.8; [28672, 8192] 66.4 / 98.1 vs 68.1 / 67.6; [6144, 4096] 18.6 / 27.3 vs 19.4 / 19.8: two passes win, three do not;
-    below 40 M weights never."""
-    n_weights = N * K
-    if M <= 16 or n_weights < 40_000_000:
-        return False
-    passes = (M + 15) // 16
-    t = passes * _gemv_pass_us(N, K, nested)
-    if _fused_gemm_wins(M, N, K) and t >= _fused_gemm_us(M, N, K):
-        return False
-    return t < 0.8 * _dense_route_us(N, K)
 
 
 # Many rows of x: the fused GEMM and dequantize + dense GEMM are within a few per cent of each other over a wide range
@@ -537,48 +469,6 @@ def _measure_route(key: tuple, candidates: dict, launches: int = 3) -> str:
     return best
 
 
-def fused_route(x: torch.Tensor, bias, blocksize: int, dtype: torch.dtype, shape, nested: bool = False) -> str:
-    """Which kernel serves this call: ``"gemv"``, ``"gemv-chunks"`` (the decode kernel once per 16
-    rows of x), ``"gemm"`` (fused), ``"dequant+gemm"`` (HIP dequantize, then the hand-written dense MFMA kernel
-    ``nf4hip_linear``, because that is the faster of the two for many rows of x), ``"dequant+libgemm"`` (HIP
-    dequantize, then the vendor library's GEMM; only when NF4HIP_LIBRARY_GEMM=1 and measured faster) or
-    ``"dequant+linear"`` (dequantize + ``torch.nn.functional.linear``, for dtypes and shapes no kernel here takes).
-
-    Mirrors bitsandbytes.matmul_4bit: the fused single-row kernel when the shape allows, else
-    dequantize followed by a dense matmul.  ``matmul_nf4`` asks ``_stream_serves`` first: this is the answer for the calls that
-    kernel leaves (and, for up to 128 rows of x, what would serve the others without it).
-    """
-    N, K = shape
-    M = x.numel() // K if K else 0
-    fused = (
-        x.dtype == torch.bfloat16
-        and dtype == torch.bfloat16
-        and (bias is None or bias.dtype == torch.bfloat16)
-        and blocksize in SUPPORTED_BLOCKSIZES
-        and M > 0
-        and N > 0
-        and (N * K) % 2 == 0
-    )
-    if not fused:
-        return "dequant+linear"
-    if M <= 4 and K % 32 == 0:
-        return "gemv"  # row-streaming kernel: blocks may straddle rows
-    if K % 64 or K % blocksize:
-        return "dequant+linear"
-    if M <= 16 and K % 512 == 0:
-        return "gemv"  # MFMA tile kernel (its exact-weights variant beyond EXACT_K)
-    if K % 512 == 0 and _chunked_gemv_wins(M, N, K, nested):
-        return "gemv-chunks"  # a few 16-row passes over the 4-bit weights beat writing them out as bf16
-    measured = _route_measured.get(_route_key(x.device, M, N, K, blocksize, nested, bias is not None))
-    if measured is not None:
-        return measured  # both routes were timed on this device for this shape (_measure_route)
-    if _fused_gemm_wins(M, N, K, nested):
-        return "gemm"  # expanding the weight tiles in registers beats writing the bf16 weight out
-    # the fused GEMM kernel streams K sequentially per tile: beyond LONG_K even a few rows of x are
-    # served faster by dequantize + dense GEMM
-    return "dequant+gemm" if M >= DENSE_ROUTE_MIN_M or K > LONG_K else "gemm"
-
-
 STREAM_MAX_M = 128
 STREAM_F16_MAX_M = 2048
 STREAM_LONG_WEIGHT = 1 << 25
@@ -595,8 +485,8 @@ def _is_plain(*tensors) -> bool:
     return all(t is None or (type(t) in (torch.Tensor, torch.nn.Parameter) and not (grad and t.requires_grad)) for t in tensors)
 
 
-def _stream_serves(x, qweight, bias, absmax, quant_map, blocksize: int, dtype: torch.dtype, shape) -> bool:
-    """Does ``nf4hip_stream`` serve this call, ahead of ``fused_route``'s answer?
+def _stream_takes(M: int, N: int, K: int, f16: bool) -> bool:
+    """Does ``nf4hip_stream`` serve M rows of bf16 or fp16 x (K a multiple of 64 and of the blocksize)?
 
     bf16, 17..128 rows: always (graph replay, cold weights, us, against the former kernels: [4096, 4096] M = 32 / 64 / 128 18.0 / 18.7 /
     28.3 vs 9.7 / 14.2 / 26.9; [14336, 4096] 24.7 / 27.3 / 35.8 vs 14.5 / 20.0 / 32.9; lm_head [128256, 4096] 112.7 / 124.8 / 171.0 vs
@@ -607,23 +497,64 @@ def _stream_serves(x, qweight, bias, absmax, quant_map, blocksize: int, dtype: t
     fp16, up to 128 rows: always; the alternative writes the dense weight first ([14336, 4096] M = 4: 47 vs 13).  Up to 2048
     rows: while the kernel's tiles fill the chip once (M = 256 / 512 / 1024 / 2048 [1024, 4096] 21.0 / 23.6 / 26.8 / 33.2 vs 10.8 / 13.3 /
     20.8 / 28.5; [4096, 4096] 34.7 / 40.0 / 52.7 / 75.9 vs 20.1 / 27.3 / 50.7 / 72.2; [4096, 14336] 90.6 / 113.9 / 146.8 / 226.1 vs 48.7 / 74.8 /
-    130.2 / 228.4; beyond, nothing was measured)."""
+    130.2 / 228.4; beyond, nothing was measured).
+    Never beyond the kernel's 32-bit offsets into a weight."""
+    if K >= 1 << 24 or N * (K // 64) >= 1 << 31:
+        return False
+    if f16:
+        return M <= STREAM_MAX_M or (M <= STREAM_F16_MAX_M and bool(_lib.load().nf4hip_gemm_streamed(M, N, K)))
+    return 16 < M <= STREAM_MAX_M or 4 < M <= 16 and (K % 512 != 0 or (K > 16384 and N * K >= STREAM_LONG_WEIGHT))
+
+
+def _weight_complete(x, qweight, bias, absmax, quant_map, n: int, blocksize: int) -> bool:
+    """Are the operands of an fp16 call as large as its n weights need and on one device?  Where not, the route through
+    ``torch.nn.functional.linear`` answers, or raises, as it always has."""
+    nested = isinstance(absmax, NestedAbsmax)
+    return ((nested or absmax.numel() >= n // blocksize) and qweight.numel() >= n // 2 and quant_map.numel() >= 16
+            and all(t is None or t.device == x.device for t in (qweight, bias, absmax.q if nested else absmax)))
+
+
+def _decode_takes(M: int, K: int, blocksize: int) -> bool:
+    """Does ``nf4hip_gemv`` serve M rows of bf16 x?  Up to four rows: the row and quad kernels, whose blocks may straddle
+    weight rows; up to sixteen: the others."""
+    return K % 32 == 0 if M <= 4 else M <= 16 and K % 512 == 0 and K % blocksize == 0
+
+
+def fused_route(x: torch.Tensor, bias, blocksize: int, dtype: torch.dtype, shape, nested: bool = False) -> str:
+    """Which kernel serves this call: ``"gemv"`` (a decode kernel), ``"stream"`` (``nf4hip_stream``: the fused kernel between a
+    decode step and a prompt, and for fp16), ``"gemm"`` (``nf4hip_gemm``, fused), ``"dequant+gemm"`` (HIP dequantize, then the
+    hand-written dense MFMA kernel ``nf4hip_linear``, because that is the faster of the two for many rows of x),
+    ``"dequant+libgemm"`` (HIP dequantize, then the vendor library's GEMM; only when measured faster) or ``"dequant+linear"``
+    (dequantize + ``torch.nn.functional.linear``, for dtypes and shapes no kernel here takes).
+
+    Mirrors bitsandbytes.matmul_4bit: the fused single-row kernel when the shape allows, else
+    dequantize followed by a dense matmul.
+    """
     N, K = shape
     M = x.numel() // K if K else 0
-    if (not 1 <= M <= (STREAM_F16_MAX_M if dtype is torch.float16 else STREAM_MAX_M) or N <= 0 or x.dtype != dtype or dtype not in (torch.bfloat16, torch.float16)
-            or K % 64 or blocksize not in SUPPORTED_BLOCKSIZES or K % blocksize or K >= 1 << 24 or N * (K // 64) >= 1 << 31
-            or (bias is not None and bias.dtype != dtype)):
-        return False
-    nested = isinstance(absmax, NestedAbsmax)
-    if dtype == torch.bfloat16:
-        if M > 16:
-            return True
-        return M > 4 and (K % 512 != 0 or (K > 16384 and N * K >= STREAM_LONG_WEIGHT))
-    if M > STREAM_MAX_M and not _lib.load().nf4hip_gemm_streamed(M, N, K):
-        return False
-    stats = absmax.q if nested else absmax
-    return (_is_plain(x, bias) and (bias is None or bias.shape == (N,)) and (nested or absmax.numel() >= N * K // blocksize)
-            and qweight.numel() >= N * K // 2 and quant_map.numel() >= 16 and all(t is None or t.device == x.device for t in (qweight, bias, stats)))
+    if x.dtype is not dtype or M <= 0 or N <= 0 or blocksize not in SUPPORTED_BLOCKSIZES or (bias is not None and bias.dtype is not dtype):
+        return "dequant+linear"
+    if dtype is torch.float16:
+        serves = (K % 64 == 0 and K % blocksize == 0 and _stream_takes(M, N, K, True) and _is_plain(x, bias)
+                  and (bias is None or bias.shape == (N,)))
+        return "stream" if serves else "dequant+linear"
+    if dtype is not torch.bfloat16 or (N * K) % 2:
+        return "dequant+linear"
+    if M <= 4 and _decode_takes(M, K, blocksize):
+        return "gemv"
+    if K % 64 or K % blocksize:
+        return "dequant+linear"
+    if _stream_takes(M, N, K, False):
+        return "stream"
+    if _decode_takes(M, K, blocksize):
+        return "gemv"
+    measured = _route_measured.get(_route_key(x.device, M, N, K, blocksize, nested, bias is not None))
+    if measured is not None:
+        return measured  # both routes were timed on this device for this shape (_measure_route)
+    if _fused_gemm_wins(M, N, K, nested):
+        return "gemm"  # expanding the weight tiles in registers beats writing the bf16 weight out
+    # (a few rows of x beyond the streaming kernel's offsets: the k loop of a tile is long)
+    return "dequant+gemm" if M >= DENSE_ROUTE_MIN_M or K > LONG_K else "gemm"
 
 
 def matmul_nf4(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape) -> torch.Tensor:
@@ -636,13 +567,13 @@ def matmul_nf4(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape) -> 
     N, K = shape
     assert x.shape[-1] == K, f"{x.shape=}, rhs {shape=}"
     _require_gpu(x, qweight, quant_map, bias)
-    M = x.numel() // K if K else 0
-    if (M > 4 or x.dtype is not torch.bfloat16) and _stream_serves(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape):
-        return _matmul_nf4_on(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape, "stream")
     nested = isinstance(absmax, NestedAbsmax)
     route = fused_route(x, bias, blocksize, dtype, shape, nested)
-    if (route in ("gemm", "dequant+gemm") and M >= CALIBRATE_MIN_M and _calibration_enabled()
+    if route == "stream" and dtype is torch.float16 and not _weight_complete(x, qweight, bias, absmax, quant_map, N * K, blocksize):
+        route = "dequant+linear"
+    if (route in ("gemm", "dequant+gemm") and x.numel() >= CALIBRATE_MIN_M * K and _calibration_enabled()
             and not torch.cuda.is_current_stream_capturing()):
+        M = x.numel() // K
         key = _route_key(x.device, M, N, K, blocksize, nested, bias is not None)
         if key not in _route_measured:
             with _on_device(x.device):
@@ -662,7 +593,7 @@ NESTED_RECONSTRUCT_MIN_M = 128
 
 
 def _matmul_nf4_on(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape, route: str) -> torch.Tensor:
-    """:func:`matmul_nf4` on a given route (``"stream"`` or one of ``fused_route``'s answers).
+    """:func:`matmul_nf4` on a given route (one of ``fused_route``'s answers).
 
     A decode call on a small weight is as long as this function: views, conversions and a device context that change nothing
     are not asked for ([4096, 4096], one row, 5 us of kernel: ``matmul_nf4`` 14.9 -> 10.4 us, of which the ctypes call is 4.5)."""
@@ -695,8 +626,8 @@ def _matmul_nf4_on(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape,
         ws = _workspace_pool.get_or_none(device, need, stream) if need else None
         ws_ptr, ws_bytes = (None, 0) if ws is None else (ws.data_ptr(), ws.numel())
         fn, fn_dq = lib.nf4hip_stream, lib.nf4hip_stream_dq
-    elif route in ("gemv", "gemv-chunks"):
-        need = lib.nf4hip_gemv_workspace_bytes(min(M, 16), N, K)
+    elif route == "gemv":
+        need = lib.nf4hip_gemv_workspace_bytes(M, N, K)
         ws = _gemv_workspace(device, need, stream)
         ws_ptr, ws_bytes = ws.data_ptr(), ws.numel()
         fn, fn_dq = lib.nf4hip_gemv, lib.nf4hip_gemv_dq
@@ -709,9 +640,6 @@ def _matmul_nf4_on(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape,
         ws_ptr, ws_bytes = (None, 0) if ws is None else (ws.data_ptr(), ws.numel())
         fn, fn_dq = lib.nf4hip_gemm, lib.nf4hip_gemm_dq
     bptr = None if b is None else b.data_ptr()
-    # row chunks of x and out: one call, or 16 rows at a time (rows are contiguous, K and N even,
-    # so every chunk starts 16-byte aligned when the whole does and K, N are multiples of 8)
-    step = 16 if route == "gemv-chunks" else M
     code, x_ptr, out_ptr = _DTYPE_CODE[x.dtype], x2.data_ptr(), out.data_ptr()
     nested = isinstance(absmax, NestedAbsmax)
     if nested and route == "gemm" and M > NESTED_RECONSTRUCT_MIN_M and not lib.nf4hip_gemm_streamed(M, N, K):
@@ -721,19 +649,15 @@ def _matmul_nf4_on(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape,
         absmax, nested = reconstruct_absmax(absmax), False
     if nested:
         q, a2, m256, off, nbs = _nested_args(absmax, nblocks)
-        for m0 in range(0, M, step):
-            mc = min(step, M - m0)
-            _lib.check(fn_dq(x_ptr + 2 * m0 * K, code, mc, qweight.data_ptr(), q.data_ptr(), a2.data_ptr(), m256.data_ptr(), off, nbs,
-                             quant_map.data_ptr(), bptr, N, K, blocksize, out_ptr + 2 * m0 * N, ws_ptr, ws_bytes, stream))  # fmt: skip
+        _lib.check(fn_dq(x_ptr, code, M, qweight.data_ptr(), q.data_ptr(), a2.data_ptr(), m256.data_ptr(), off, nbs,
+                         quant_map.data_ptr(), bptr, N, K, blocksize, out_ptr, ws_ptr, ws_bytes, stream))  # fmt: skip
     else:
         _require_gpu(absmax)
         absmax = _aligned(absmax if absmax.dtype is torch.float32 else absmax.to(torch.float32))
         if absmax.numel() < nblocks:
             raise ValueError(f"absmax holds {absmax.numel()} entries, need {nblocks}")
-        for m0 in range(0, M, step):
-            mc = min(step, M - m0)
-            _lib.check(fn(x_ptr + 2 * m0 * K, code, mc, qweight.data_ptr(), absmax.data_ptr(), quant_map.data_ptr(), bptr,
-                          N, K, blocksize, out_ptr + 2 * m0 * N, ws_ptr, ws_bytes, stream))  # fmt: skip
+        _lib.check(fn(x_ptr, code, M, qweight.data_ptr(), absmax.data_ptr(), quant_map.data_ptr(), bptr,
+                      N, K, blocksize, out_ptr, ws_ptr, ws_bytes, stream))  # fmt: skip
     return out if flat else out.reshape(*x.shape[:-1], N)
 
 
@@ -797,7 +721,7 @@ def matmul_nf4_epilogue(x, qweight, bias, absmax, quant_map, blocksize, dtype, s
 
     Each output is what ``matmul_nf4`` and the step would store, bit for bit (``rowscale`` aside), except at 5..16
     rows on a weight of 2^25 elements and more with K > 16384: there the plain product runs in another kernel
-    (``_stream_serves``), with the same weights and another order of its sums.
+    (``_stream_takes``), with the same weights and another order of its sums.
 
     Returns None where the library does not serve the case (more than sixteen rows of x, nested absmax, other dtypes,
     one row of x with K > 16384, ...; ``epilogue_served`` answers beforehand): the caller then runs
@@ -807,7 +731,8 @@ def matmul_nf4_epilogue(x, qweight, bias, absmax, quant_map, blocksize, dtype, s
     M = x2.shape[0]
     if isinstance(absmax, NestedAbsmax) or M > 16 or not x2.is_cuda:
         return None
-    if fused_route(x2, bias, blocksize, dtype, (N, K)) != "gemv":
+    if (x.dtype is not torch.bfloat16 or dtype is not torch.bfloat16 or (bias is not None and bias.dtype is not dtype) or M == 0 or N <= 0
+            or blocksize not in SUPPORTED_BLOCKSIZES or (N * K) % 2 or not _decode_takes(M, K, blocksize)):
         return None
     lib = _lib.load()
     _require_gpu(x2, qweight, quant_map, bias, absmax)

@@ -232,21 +232,21 @@ def test_fused_route_rules(ta):
         return F.fused_route(torch.empty(M, K, dtype=xdtype), bias, bs, dtype, (N, K))
 
     assert route(1, 4096, 4096) == "gemv" and route(4, 64, 1376) == "gemv" and route(16, 4096, 4096) == "gemv"
-    assert route(5, 64, 1376) == "dequant+linear"        # tile kernel needs K % 512, gemm K % 64
-    assert route(8, 64, 1344) == "gemm"                   # fused GEMM kernel below DENSE_ROUTE_MIN_M rows
-    # 17..128 rows: one launch of the fused GEMM (64- or 128-row tile, K split over workgroups) wherever it is
-    # modelled faster than the dense route's dequantize pass -- every projection shape of the Llama models
-    assert route(17, 4096, 4096) == "gemm" and route(128, 4096, 4096) == "gemm"
-    assert route(64, 1024, 4096) == "gemm" and route(65, 1024, 4096) == "dequant+gemm"
-    # 17..32 rows of x on a weight of 40 M elements and more: two passes of the decode kernel (the LDS-staged one at these
-    # shapes) beat the fused GEMM; three do not
-    assert route(17, 14336, 4096) == "gemv-chunks" and route(32, 28672, 4096) == "gemv-chunks" and route(32, 128256, 4096) == "gemv-chunks"
-    assert route(33, 14336, 4096) == "gemm" and route(48, 28672, 4096) == "gemm" and route(128, 14336, 4096) == "gemm"
-    assert route(17, 6144, 4096) == "gemm" and route(32, 4096, 4096) == "gemm"  # below 40 M weights never
-    assert route(128, 4096, 14336) == "gemm"
-    assert route(17, 8192, 28672) == "gemm"               # exact at any K
-    assert route(17, 28672, 4096 + 64) == "gemm"          # the tile kernel needs K % 512, the fused GEMM K % 64
-    assert route(17, 128, 64) == "gemm"                   # tiny: one launch instead of two
+    assert route(5, 64, 1376) == "dequant+linear"        # decode kernels need K % 512 from five rows on, the others K % 64
+    assert route(8, 64, 1344) == "stream" and route(4, 64, 1344) == "gemv"
+    # 17..128 rows: the streaming kernel, whatever the shape
+    for M in (17, 32, 33, 48, 65, 128):
+        for N, K in ((128, 64), (1024, 4096), (4096, 4096), (6144, 4096), (14336, 4096), (28672, 4096 + 64), (128256, 4096), (4096, 14336),
+                     (8192, 28672), (2048, 20480), (1536, 28672), (2048, 20480 + 64)):
+            assert route(M, N, K) == "stream", (M, N, K)
+    assert route(17, 64, 1376) == "dequant+linear" and route(17, 64, 192, bs=128) == "dequant+linear"
+    # 5..16 rows there where the decode kernels' exact variants are slow
+    assert route(16, 8192, 28672) == "stream" and route(5, 8192, 28672) == "stream" and route(4, 8192, 28672) == "gemv"
+    assert route(5, 1000, 28672) == "gemv" and route(16, 8192, 14336) == "gemv"
+    # beyond the streaming kernel's offsets into a weight: the models of the fused kernel's whole tiles and of the dense route
+    # (shapes only; an expanded tensor holds one element)
+    far = lambda M, N, K: F.fused_route(torch.empty(1, dtype=bf).expand(M, K), None, 64, bf, (N, K))
+    assert far(64, 64, 1 << 24) == "dequant+gemm" and far(17, 1 << 20, 1 << 17) == "gemm" and far(16, 64, 1 << 24) == "gemv"
     # more than 128 rows: the fused kernel of nf4_gemm_wide.hip (calls with fewer tiles than CUs cut their tiles
     # along k) up to 1024 rows on every Llama projection shape but the smallest, and at 2048 rows where the models
     # put it within 3 % of dequantize + library GEMM; the library GEMM's higher rate wins beyond
@@ -259,14 +259,13 @@ def test_fused_route_rules(ta):
     assert route(2048, 4096, 4096) == "gemm" and route(2048, 4096, 14336) == "gemm" and route(2048, 128256, 4096) == "gemm"
     assert route(2048, 28672, 4096) == "dequant+gemm" and route(2048, 28672, 8192) == "dequant+gemm"
     assert route(129, 1024, 4096) == "dequant+gemm" and route(512, 1024, 4096) == "gemm" and route(8192, 1024, 4096) == "dequant+gemm"
-    # a few more than 16 rows on a short, very wide weight: the decode kernel once per 16 rows
-    assert route(17, 2048, 20480) == "gemv-chunks" and route(32, 2048, 20480) == "gemv-chunks" and route(33, 2048, 20480) == "gemm"
-    assert route(32, 1536, 28672) == "gemv-chunks" and route(33, 1536, 28672) == "dequant+gemm"
-    assert route(17, 2048, 20480 + 64) == "dequant+gemm"  # the decode kernels need K % 512; 321 k steps do not split
-    assert route(16, 8192, 28672) == "gemv"              # K > 8192: the tile kernel's exact-weights variant
     assert route(1, 8192, 28672) == "gemv"               # row-streaming kernel has an exact variant
     assert route(1, 64, 4096, dtype=torch.float32) == "dequant+linear"
-    assert route(1, 64, 4096, xdtype=torch.float16, dtype=torch.float16) == "dequant+linear"
+    half = torch.float16
+    assert route(1, 64, 4096, xdtype=half, dtype=half) == "stream" and route(128, 64, 4096, xdtype=half, dtype=half) == "stream"
+    assert route(1, 64, 1376, xdtype=half, dtype=half) == "dequant+linear" and route(1, 64, 4096, xdtype=half) == "dequant+linear"
+    assert route(1, 64, 4096, xdtype=half, dtype=half, bias=torch.zeros(64, dtype=half)) == "stream"
+    assert route(1, 64, 4096, xdtype=half, dtype=half, bias=torch.zeros(1, 64, dtype=half)) == "dequant+linear"
     assert route(1, 2, 2) == "dequant+linear"
     assert route(1, 64, 4096, bias=torch.zeros(64)) == "dequant+linear"  # fp32 bias with bf16 x
     _ = ctypes  # (imported for readers who want to poke at the library by hand)
@@ -334,7 +333,6 @@ def test_gemm_plan_is_the_launchers_and_agrees_with_the_workspace(ta):
                     assert wgs == (tiles - cut) + cut * pieces and (K // 64) >= pieces
                     assert need == counter_region + cut * pieces * rows * 256 * 4
                     seen_cut += 1
-                assert F._gemm_splits(M, N, K) == (pieces if M <= 128 else 1)
                 if M > 128:
                     assert F._wide_schedule(M, N, K) == (rows, tiles, pieces)
     assert seen_cut > 50 and seen_whole > 50

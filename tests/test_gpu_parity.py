@@ -360,10 +360,13 @@ def test_split_k_hand_off_holds_over_many_launches(ta):
 
 @pytest.fixture
 def fused_gemm(ta, monkeypatch):
-    """Route every M > 16 call to the fused GEMM kernel (the default router prefers HIP dequantize
-    + the dense library GEMM from 17 rows on)."""
+    """Route every call of more than 128 rows to ``nf4hip_gemm`` (the default router prefers HIP dequantize + a dense GEMM for
+    some shapes); up to 128 rows ``nf4hip_stream`` serves them anyway."""
     monkeypatch.setattr(ta.functional, "DENSE_ROUTE_MIN_M", 1 << 30)
-    monkeypatch.setattr(ta.functional, "_chunked_gemv_wins", lambda M, N, K, nested=False: False)
+
+
+def _fused_route_of(M):
+    return "stream" if M <= 128 else "gemm"
 
 
 @pytest.mark.parametrize("M,N,K", [(200, 128, 4096), (129, 1024, 4096), (3000, 1024, 4096)])
@@ -380,7 +383,7 @@ def test_dense_route(ta, oracle, M, N, K):
 )
 def test_gemm_shapes(ta, oracle, M, N, K, fused_gemm):
     _sync_print(f"gemm M={M} N={N} K={K}")
-    assert ta.functional.fused_route(torch.empty(M, K, dtype=torch.bfloat16), None, 64, torch.bfloat16, (N, K)) == "gemm"
+    assert ta.functional.fused_route(torch.empty(M, K, dtype=torch.bfloat16), None, 64, torch.bfloat16, (N, K)) == _fused_route_of(M)
     _matmul_case(ta, oracle, M, N, K, seed=M + N + K)
 
 
@@ -389,10 +392,10 @@ def test_gemm_shapes(ta, oracle, M, N, K, fused_gemm):
     (300, 28930, 512, {"blocksize": 256}), (512, 28672, 1024, {}), (700, 4 * 28672, 128, {"bias": True}),
 ])
 def test_gemm_route_tall_weights(ta, oracle, M, N, K, kw, fused_gemm):
-    """Tall weights through the fused GEMM kernels (all tile heights, ragged M and N, odd and even numbers
-    of k steps, fewer k steps than pipeline stages); up to 128 rows of x the default router picks them itself."""
+    """Tall weights through the streaming kernel and the fused GEMM kernel (ragged M and N, odd and even numbers
+    of k steps, fewer k steps than pipeline stages)."""
     _sync_print(f"gemm (tall) M={M} N={N} K={K} {kw}")
-    assert ta.functional.fused_route(torch.empty(M, K, dtype=torch.bfloat16), None, kw.get("blocksize", 64), torch.bfloat16, (N, K)) == "gemm"
+    assert ta.functional.fused_route(torch.empty(M, K, dtype=torch.bfloat16), None, kw.get("blocksize", 64), torch.bfloat16, (N, K)) == _fused_route_of(M)
     _matmul_case(ta, oracle, M, N, K, seed=M + K, **kw)
 
 
@@ -419,27 +422,27 @@ def test_gemm_bias_nested_blocksize(ta, oracle, fused_gemm):
         _matmul_case(ta, oracle, 200, 300, K, nested=True, seed=5 + K)
 
 
-@pytest.mark.parametrize("case", ["fp32", "fp16", "K_not_64", "n_lt_block"])
+@pytest.mark.parametrize("case", ["fp32", "fp16", "fp16_K_not_64", "K_not_64", "n_lt_block"])
 def test_fallback_route(ta, oracle, case):
     """Shapes/dtypes outside the fused kernels take HIP dequantize + dense matmul, as
-    bitsandbytes.matmul_4bit does."""
+    bitsandbytes.matmul_4bit does; fp16 only where the streaming kernel does not take the shape."""
     _sync_print(f"fallback {case}")
-    dtype = {"fp32": torch.float32, "fp16": torch.float16}.get(case, torch.bfloat16)
-    N, K = {"K_not_64": (64, 1376), "n_lt_block": (2, 2)}.get(case, (96, 256))
+    dtype = {"fp32": torch.float32, "fp16": torch.float16, "fp16_K_not_64": torch.float16}.get(case, torch.bfloat16)
+    N, K = {"K_not_64": (64, 1376), "fp16_K_not_64": (64, 1376), "n_lt_block": (2, 2)}.get(case, (96, 256))
     w = _weights((N, K), seed=5, dtype=dtype)
     x = _acts((7, K), seed=6, dtype=dtype)
     b = _acts((N,), seed=7, dtype=dtype)
     qw, absmax = oracle.C().quantize(w, 64)
-    assert ta.functional.fused_route(x, b, 64, dtype, (N, K)) == "dequant+linear"
+    assert ta.functional.fused_route(x, b, 64, dtype, (N, K)) == ("stream" if case == "fp16" else "dequant+linear")
     y = ta.matmul_nf4(x.to(DEV), qw.to(DEV), b.to(DEV), absmax.to(DEV), ta.nf4_code(DEV), 64, dtype, (N, K))
     ref = oracle.matmul_4bit_f64(x, qw, b, absmax, oracle.nf4_lut(), 64, dtype, (N, K))
     torch.testing.assert_close(y.cpu().float(), ref.float(), rtol=2e-2, atol=2e-2)
 
 
 def test_matmul_randomized_sweep_large(ta):
-    """Seeded sweep over every route of matmul_nf4 at sizes the CPU oracle would take too long for
+    """Seeded sweep over matmul_nf4 at sizes the CPU oracle would take too long for
     (N up to 40000, K up to 28672, M up to 48: row / quad / tile kernels with their exact and
-    long-list variants, the 16-row chunk route, the dense route), each against a float64-accumulated
+    long-list variants, the streaming kernel), each against a float64-accumulated
     matmul over sampled rows of the HIP-dequantized weight (pinned bit-exact against the oracle by the
     tests above)."""
     rng = torch.Generator().manual_seed(4321)
@@ -474,12 +477,13 @@ def test_matmul_randomized_sweep_large(ta):
             ref = ref + b[rows].double()
         torch.testing.assert_close(y[:, rows].double(), ref, rtol=2e-2, atol=2e-2)
         del w, x, qw, absmax, deq, y
-    assert {"gemv", "gemm", "dequant+gemm"} <= seen
+    assert seen == {"gemv", "stream"}
 
 
 def test_gemm_randomized_sweep(ta, fused_gemm):
-    """Seeded sweep over the fused GEMM kernel alone (forced for every shape): both tile heights, ragged
-    M and N, 1..33 k steps, every blocksize, bias, nested absmax; against a float64-accumulated
+    """Seeded sweep over the streaming kernel (up to 128 rows of x, and through ``nf4hip_gemm`` on most of the shapes beyond)
+    and the fused GEMM kernel (more than 128 tiles with a short K): ragged
+    M and N, 1..33 k steps every blocksize, bias, nested absmax; against a float64-accumulated
     matmul over the HIP-dequantized weight."""
     rng = torch.Generator().manual_seed(8765)
 
@@ -502,7 +506,7 @@ def test_gemm_randomized_sweep(ta, fused_gemm):
         qw, absmax, _ = ta.quantize_nf4(w, blocksize)
         state = ta.compress_absmax(absmax) if nested else absmax
         deq = ta.dequantize_nf4(qw, state, code, blocksize, torch.bfloat16, (N, K))
-        assert ta.functional.fused_route(x, b, blocksize, torch.bfloat16, (N, K)) == "gemm"
+        assert ta.functional.fused_route(x, b, blocksize, torch.bfloat16, (N, K)) == _fused_route_of(M)
         y = ta.matmul_nf4(x, qw, b, state, code, blocksize, torch.bfloat16, (N, K))
         ref = x.double() @ deq.double().t()
         if bias:
@@ -593,13 +597,11 @@ def test_gemv_every_m_on_large_weights(ta, N, K):
 
 
 @pytest.mark.parametrize("nested", [False, True])
-def test_gemv_chunks_route(ta, nested):
-    """17..32 rows of x on a large weight go through the decode kernel 16 rows at a time: a full and
-    a ragged last chunk, with bias, against a float64-accumulated matmul over sampled rows of the
-    HIP-dequantized weight.  (A short, very wide weight: everywhere else one launch of the fused GEMM
-    is faster than two passes.)"""
+def test_stream_route_short_wide_weight(ta, nested):
+    """17..32 rows of x on a short, very wide weight, with bias, against a float64-accumulated matmul over sampled rows of the
+    HIP-dequantized weight; sixteen of the rows alone (the same kernel, beyond K = 16384) give the same bits."""
     N, K = 2048, 20480
-    _sync_print(f"gemv-chunks nested={nested}")
+    _sync_print(f"stream, short wide weight nested={nested}")
     g = torch.Generator(device=DEV).manual_seed(99)
     w = (torch.randn(N, K, generator=g, device=DEV) * 0.02).to(torch.bfloat16)
     qw, absmax, code = ta.quantize_nf4(w)
@@ -609,12 +611,12 @@ def test_gemv_chunks_route(ta, nested):
     bias = torch.randn(N, generator=g, device=DEV).to(torch.bfloat16)
     for M in (17, 20, 31, 32):
         x = torch.randn(M, K, generator=g, device=DEV).to(torch.bfloat16)
-        assert ta.functional.fused_route(x, bias, 64, torch.bfloat16, (N, K)) == "gemv-chunks"
+        assert ta.functional.fused_route(x, bias, 64, torch.bfloat16, (N, K)) == "stream"
+        assert ta.functional.fused_route(x[:16], bias, 64, torch.bfloat16, (N, K)) == "stream"
         y = ta.matmul_nf4(x.reshape(1, M, K), qw, bias, state, code, 64, torch.bfloat16, (N, K))
         assert y.shape == (1, M, N)
         ref = x.double() @ deq[rows].double().t() + bias[rows].double()
         torch.testing.assert_close(y[0][:, rows].double(), ref, rtol=2e-2, atol=2e-2)
-        # a chunk computes what a 16-row call computes
         y16 = ta.matmul_nf4(x[16:32] if M >= 32 else x[:16], qw, bias, state, code, 64, torch.bfloat16, (N, K))
         assert torch.equal(y16, y[0][16:32] if M >= 32 else y[0][:16])
 

@@ -172,31 +172,30 @@ def test_stream_arguments_and_workspace(ta):
     _ = ctypes
 
 
-def test_stream_serves(ta):
+def test_fp16_route(ta):
     F = ta.functional
-    bf, hf = torch.bfloat16, torch.float16
+    hf = torch.float16
 
-    def serves(M, N, K, dtype=bf, xdtype=None, bs=64, bias=None, nested=False, x=None):
-        n = N * K // bs
-        stats = F.NestedAbsmax(torch.empty(n, dtype=torch.uint8), None, None, 0.0) if nested else torch.empty(n)
-        x = torch.empty(M, K, dtype=xdtype or dtype) if x is None else x
-        return F._stream_serves(x, torch.empty(N * K // 2, 1, dtype=torch.uint8), bias, stats, torch.empty(16), bs, dtype, (N, K))
+    def route(M, N, K, x=None, bias=None):
+        return F.fused_route(torch.empty(M, K, dtype=hf) if x is None else x, bias, 64, hf, (N, K))
 
-    assert not serves(16, 64, 4096) and serves(17, 64, 4096) and serves(128, 64, 4096) and not serves(129, 64, 4096)
-    assert serves(2048, 64, 4096, hf) and not serves(2049, 64, 4096, hf) and not serves(512, 32768, 256, hf)
-    assert serves(5, 64, 1344) and not serves(4, 64, 1344) and not serves(17, 64, 1376) and not serves(17, 64, 192, bs=128)
-    assert serves(5, 8192, 28672, nested=True) and serves(16, 8192, 28672) and not serves(5, 1000, 28672) and not serves(4, 8192, 28672, nested=True)
-    assert not serves(17, 64, 4096, bias=torch.empty(64)) and not serves(17, 64, 4096, xdtype=hf)
-    assert serves(1, 64, 4096, hf) and serves(128, 64, 4096, hf) and not serves(0, 64, 4096, hf)
-    assert not serves(1, 64, 4096, torch.float32)
+    assert route(2048, 64, 4096) == "stream" and route(2049, 64, 4096) == "dequant+linear" and route(512, 32768, 256) == "dequant+linear"
     # what differentiates or transforms stays with the torch operation
     xg = torch.empty(2, 4096, dtype=hf, requires_grad=True)
-    assert not serves(2, 64, 4096, hf, x=xg)
+    assert route(2, 64, 4096, xg) == "dequant+linear"
     with torch.no_grad():
-        assert serves(2, 64, 4096, hf, x=xg)
+        assert route(2, 64, 4096, xg) == "stream"
     with torch.autograd.forward_ad.dual_level():
-        assert not serves(2, 64, 4096, hf)
+        assert route(2, 64, 4096) == "dequant+linear"
     seen = []
-    torch.func.vmap(lambda row: (seen.append(serves(1, 64, 4096, hf, x=row)), row)[1])(torch.zeros(2, 1, 4096, dtype=hf))
-    assert seen == [False]
-    assert not serves(2, 64, 4096, hf, bias=torch.empty(1, 64, dtype=hf))
+    torch.func.vmap(lambda row: (seen.append(route(1, 64, 4096, row)), row)[1])(torch.zeros(2, 1, 4096, dtype=hf))
+    assert seen == ["dequant+linear"]
+    # ... and so do weights that are too small or lie elsewhere
+    n = 64 * 4096
+    x, book = torch.empty(2, 4096, dtype=hf), torch.empty(16)
+    whole = dict(qweight=torch.empty(n // 2, 1, dtype=torch.uint8), bias=None, absmax=torch.empty(n // 64), quant_map=book, n=n, blocksize=64)
+    ok = lambda **kw: F._weight_complete(x, **{**whole, **kw})
+    assert ok() and not ok(absmax=torch.empty(n // 64 - 1)) and not ok(qweight=torch.empty(n // 2 - 1, 1, dtype=torch.uint8))
+    assert not ok(quant_map=torch.empty(15)) and not ok(bias=torch.empty(64, dtype=hf, device="meta")) and not ok(absmax=whole["absmax"].to("meta"))
+    nested = lambda device: F.NestedAbsmax(torch.empty(n // 64, dtype=torch.uint8, device=device), None, None, 0.0)
+    assert ok(absmax=nested("cpu")) and not ok(absmax=nested("meta"))

@@ -223,18 +223,17 @@ int nf4hip_gemv_static(const void* x, int x_dtype, int64_t M, const uint8_t* pac
  * bitsandbytes.matmul_4bit (MatMul4Bit.forward), reached from thunder/transforms/quantization.py:39.
  * NF4 codes are expanded to bf16 ( bf16(lut16[c] * absmax) ) on chip and contracted with bf16 MFMA,
  * fp32 accumulation, bf16 output.  Same operand layout and fast-path rules as nf4hip_gemv, except
- * K % 64 == 0 and blocksize == 64 ... 4096 dividing K.  Up to 128 rows of x, K may be split over
- * workgroups that meet in `workspace`: nf4hip_gemm_workspace_bytes(M,N,K) bytes (0 = none needed,
- * NULL accepted), under the rules of nf4hip_gemv's workspace -- zeroed once, left zeroed where that
- * matters, one stream at a time; the two kernels may share one workspace.
+ * K % 64 == 0 and blocksize == 64 ... 4096 dividing K.  K may be split over workgroups that meet in `workspace`:
+ * nf4hip_gemm_workspace_bytes(M,N,K) bytes (0 = none needed, NULL accepted), under the rules of nf4hip_gemv's
+ * workspace -- zeroed once, left zeroed where that matters, one stream at a time; the two kernels may share one
+ * workspace.  Less is refused (NF4HIP_E_WORKSPACE), except up to 128 rows of x where K falls into no 2..8 equal ranges of
+ * 256 k or more that run in 256 workgroups of 256 weight rows: such a call runs without, K then not split.
  */
 size_t nf4hip_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K);
 /*
- * The launch plan nf4hip_gemm would use for a shape (no GPU needed): plan[0] rows of x per tile (64, 128 or 256),
- * plan[1] tiles (tiles of x rows x tiles of 256 weight rows), plan[2] pieces a tile is cut into along K (they meet in
- * the workspace), plan[3] workgroups launched.  Where nf4hip_gemm_streamed says 1 (up to 128 rows of x, more
- * while tiles of 128 x 256 fill the chip once at most) this is what the workspace is sized by; nf4hip_stream's kernel serves
- * the call and lays its own tiles out in whatever workspace it is given.  For host code that chooses
+ * The launch plan nf4hip_gemm uses for a shape (no GPU needed): plan[0] rows of x per tile, plan[1] tiles, plan[2] pieces
+ * a tile is cut into along K (they meet in the workspace), plan[3] workgroups launched.  nf4hip_gemm_streamed: is it
+ * nf4hip_stream's kernel (up to 128 rows of x, more while tiles of 128 x 256 fill the chip once at most)?  For host code that chooses
  * between this kernel and dequantize + dense GEMM (the choice bitsandbytes.matmul_4bit makes at thunder/transforms/quantization.py:39) without keeping
  * a copy of the launcher's rules.  K must be a multiple of 64.
  */
@@ -250,6 +249,12 @@ int nf4hip_gemm(const void* x, int x_dtype, int64_t M, const uint8_t* packed, co
  * the kernels may share one) K may be split over workgroups; with less, or NULL, it is not.  Deterministic either way.
  */
 size_t nf4hip_stream_workspace_bytes(int64_t M, int64_t N, int64_t K);
+/*
+ * What it launches with that workspace (no GPU needed): plan[0] rows of x and plan[1] weight rows per tile, plan[2] workgroups that
+ * share a tile's K, plan[3] workgroups; and the time the launcher's model gives it in microseconds on fp32 absmax (0: not served).
+ */
+int nf4hip_stream_plan(int64_t M, int64_t N, int64_t K, int32_t plan[4]);
+float nf4hip_stream_us(int64_t M, int64_t N, int64_t K);
 int nf4hip_stream(const void* x, int x_dtype, int64_t M, const uint8_t* packed, const float* absmax, const float* lut16,
                   const void* bias_or_null, int64_t N, int64_t K, int blocksize, void* out, void* workspace,
                   size_t workspace_bytes, void* stream);

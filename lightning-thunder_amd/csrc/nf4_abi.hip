@@ -132,7 +132,7 @@ int matmul_common(MatmulKind kind, const void* x, int x_dtype, int64_t M, const 
         return fail(NF4HIP_E_ALIGN, "%s: x / packed / absmax / out not 16-byte aligned, lut16 not 4-byte or bias not 2-byte aligned",
                     name);
     // (nf4hip_stream uses what workspace it is given)
-    const size_t need = kind == GEMV ? nf4::gemv_workspace_bytes(M, N, K) : kind == GEMM ? nf4::gemm_workspace_bytes(M, N, K) : 0;
+    const size_t need = kind == GEMV ? nf4::gemv_workspace_bytes(M, N, K) : kind == GEMM ? nf4::gemm_workspace_required(M, N, K) : 0;
     if (use_static) {
         if (need > (size_t)NF4HIP_STATIC_SCRATCH_BYTES)
             return fail(NF4HIP_E_WORKSPACE,
@@ -144,8 +144,9 @@ int matmul_common(MatmulKind kind, const void* x, int x_dtype, int64_t M, const 
             return fail(NF4HIP_E_WORKSPACE, "%s: workspace of %zu bytes required, got %zu", name, need,
                         workspace ? workspace_bytes : (size_t)0);
         if (!aligned16(workspace)) return fail(NF4HIP_E_ALIGN, "%s: workspace not 16-byte aligned", name);
-    } else if (kind == STREAM && !aligned16(workspace)) {
-        return fail(NF4HIP_E_ALIGN, "%s: workspace not 16-byte aligned", name);
+    } else if (!aligned16(workspace)) {
+        if (kind == STREAM) return fail(NF4HIP_E_ALIGN, "%s: workspace not 16-byte aligned", name);
+        workspace = nullptr;  // a call that goes without one takes any pointer, and uses none it cannot
     }
 
     nf4::MatmulArgs a;
@@ -190,7 +191,7 @@ int matmul_common(MatmulKind kind, const void* x, int x_dtype, int64_t M, const 
     }
     const hipError_t e = kind == GEMV   ? nf4::launch_gemv(a, static_cast<hipStream_t>(stream))
                          : kind == GEMM ? nf4::launch_gemm(a, static_cast<hipStream_t>(stream))
-                                        : nf4::launch_stream(a, x_dtype == NF4HIP_F16, 8, static_cast<hipStream_t>(stream));
+                                        : nf4::launch_stream(a, x_dtype == NF4HIP_F16, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(name, e);
     return NF4HIP_OK;
 }
@@ -415,6 +416,21 @@ int nf4hip_gemm(const void* x, int x_dtype, int64_t M, const uint8_t* packed, co
 }
 
 int nf4hip_gemm_streamed(int64_t M, int64_t N, int64_t K) { return nf4::stream_serves_gemm(M, N, K) ? 1 : 0; }
+
+float nf4hip_stream_us(int64_t M, int64_t N, int64_t K) { return nf4::stream_serves_gemm(M, N, K) ? nf4::stream_us(M, N, K) : 0.0f; }
+
+int nf4hip_stream_plan(int64_t M, int64_t N, int64_t K, int32_t plan[4]) {
+    if (!plan) return fail(NF4HIP_E_NULL, "nf4hip_stream_plan: null pointer");
+    if (!nf4::stream_serves_gemm(M, N, K))
+        return fail(NF4HIP_E_SHAPE, "nf4hip_stream_plan: M = %lld, N = %lld, K = %lld: not served (nf4hip_gemm_streamed)",
+                    (long long)M, (long long)N, (long long)K);
+    const nf4::StreamPlan p = nf4::stream_plan(M, N, K, nf4::STREAM_MAX_SPLITS);
+    plan[0] = p.bm;
+    plan[1] = 32 * p.wn;
+    plan[2] = p.splits;
+    plan[3] = p.m_tiles * p.n_tiles * p.splits;
+    return NF4HIP_OK;
+}
 
 size_t nf4hip_stream_workspace_bytes(int64_t M, int64_t N, int64_t K) { return nf4::stream_workspace_bytes(M, N, K); }
 

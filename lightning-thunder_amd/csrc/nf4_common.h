@@ -90,9 +90,11 @@ void gemv_set_staged(int mode);  // -1 the dispatcher's rule, 0 never, 1 whereve
 bool gemv_epilogue_possible(const MatmulArgs& a);  // does the kernel that serves (M, N, K) take a.epi?
 int gemv_norm_parts(int64_t M, int64_t N, int64_t K);  // partial sums per row of x an EPI_RESID_NORM call writes (0: not served)
 size_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K);
+size_t gemm_workspace_required(int64_t M, int64_t N, int64_t K);  // 0: the call is taken without as well
 hipError_t launch_gemm(const MatmulArgs& a, hipStream_t stream);
 // up to 128 rows of bf16 or fp16 x, and more where stream_serves_gemm (nf4_gemm_stream.hip): rows of x per tile, 32-row weight tiles side by side, workgroups
-// that share a tile's K, tiles.  At most `max_splits` of those workgroups, one where a.workspace_bytes does not hold them.
+// that share a tile's K (at most `max_splits`), tiles.  K is not split where a.workspace_bytes does not hold the partial tiles.
+constexpr int STREAM_MAX_SPLITS = 8;
 struct StreamPlan {
     int bm, wn, splits, m_tiles, n_tiles;
 };
@@ -100,7 +102,8 @@ bool stream_possible(int64_t M, int64_t N, int64_t K);
 bool stream_serves_gemm(int64_t M, int64_t N, int64_t K);  // does launch_gemm use it?
 StreamPlan stream_plan(int64_t M, int64_t N, int64_t K, int max_splits);
 size_t stream_workspace_bytes(int64_t M, int64_t N, int64_t K);
-hipError_t launch_stream(const MatmulArgs& a, bool f16, int max_splits, hipStream_t stream);
+float stream_us(int64_t M, int64_t N, int64_t K);  // its modelled time with that workspace, fp32 absmax
+hipError_t launch_stream(const MatmulArgs& a, bool f16, hipStream_t stream);
 // what the streaming kernel does not take, with x below 4 GB: 256 x 256 or 128 x 256 tiles (nf4_gemm_wide.hip)
 bool gemm_wide_possible(int64_t M, int64_t K);
 int gemm_wide_tile_rows(int64_t M, int64_t N, int64_t K);

@@ -279,20 +279,16 @@ __global__ __launch_bounds__(THREADS) void gemm_kernel(MatmulArgs a, int m_tiles
 }
 
 constexpr int MAX_DEVICES = 64;
-// arrival counters at the head of the workspace: the same region as the decode kernels', so that one
-// zero-initialised workspace serves both (partial sums never land where the other expects zeroed counters)
-constexpr size_t GEMM_COUNTER_BYTES = GEMV_COUNTER_BYTES;
 
-// Pieces along K for up to 128 rows of x: what the workspace is sized by (as many workgroups of 256 weight rows as fit the
-// chip's 256 CUs in one round; the k steps divide evenly and every piece keeps at least 4), and the most the kernel uses.
-int gemm_splits(int64_t M, int64_t N, int64_t K) {
-    if (M > 128) return 1;
-    const int64_t tiles = (N + BN - 1) / BN;
-    const int64_t ksteps = K / BK;
-    int best = 1;
+// Up to 128 rows of x, calls that are taken without the workspace as well, K then not split: those for which none was asked
+// before the streaming kernel served them, because K falls into no 2..8 equal ranges of four 64-k steps or more that run in one
+// round of workgroups of 256 weight rows.  (Beyond 128 rows no such call has a split.)
+bool without_workspace(int64_t M, int64_t N, int64_t K) {
+    if (M > 128) return false;
+    const int64_t tiles = (N + BN - 1) / BN, ksteps = K / BK;
     for (int s = 2; s <= 8; ++s)
-        if (tiles * s <= 256 && ksteps % s == 0 && ksteps / s >= 4) best = s;
-    return best;
+        if (tiles * s <= 256 && ksteps % s == 0 && ksteps / s >= 4) return false;
+    return true;
 }
 
 template <bool NESTED>
@@ -318,27 +314,32 @@ hipError_t launch_tile(const MatmulArgs& a, hipStream_t stream) {
 }  // namespace
 
 size_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-    if (!stream_serves_gemm(M, N, K)) return gemm_wide_possible(M, K) ? gemm_wide_workspace_bytes(M, N, K) : 0;
-    if (M > 128) return gemm_wide_workspace_bytes(M, N, K);
-    const int splits = gemm_splits(M, N, K);
-    if (splits == 1) return 0;
-    const int64_t bm = M <= 64 ? 64 : 128;
-    return GEMM_COUNTER_BYTES + (size_t)((N + BN - 1) / BN) * splits * bm * BN * sizeof(float);
+    if (stream_serves_gemm(M, N, K)) return stream_workspace_bytes(M, N, K);
+    return gemm_wide_possible(M, K) ? gemm_wide_workspace_bytes(M, N, K) : 0;
+}
+
+size_t gemm_workspace_required(int64_t M, int64_t N, int64_t K) {
+    return without_workspace(M, N, K) ? 0 : gemm_workspace_bytes(M, N, K);
 }
 
 void gemm_plan(int64_t M, int64_t N, int64_t K, int plan[4]) {
-    const bool streamed = stream_serves_gemm(M, N, K);
-    if (streamed ? M > 128 : gemm_wide_possible(M, K)) return gemm_wide_plan(M, N, K, plan);
-    const int bm = !streamed ? BM : M <= 64 ? 64 : 128;
-    const int64_t tiles = ((M + bm - 1) / bm) * ((N + BN - 1) / BN);
-    plan[0] = bm;
-    plan[1] = (int)tiles;
-    plan[2] = streamed ? gemm_splits(M, N, K) : 1;
-    plan[3] = (int)tiles * plan[2];
+    if (stream_serves_gemm(M, N, K)) {
+        const StreamPlan p = stream_plan(M, N, K, STREAM_MAX_SPLITS);
+        plan[0] = p.bm;
+        plan[1] = p.m_tiles * p.n_tiles;
+        plan[2] = p.splits;
+    } else if (gemm_wide_possible(M, K)) {
+        return gemm_wide_plan(M, N, K, plan);
+    } else {
+        plan[0] = BM;
+        plan[1] = (int)(((M + BM - 1) / BM) * ((N + BN - 1) / BN));
+        plan[2] = 1;
+    }
+    plan[3] = plan[1] * plan[2];
 }
 
 hipError_t launch_gemm(const MatmulArgs& a, hipStream_t stream) {
-    if (stream_serves_gemm(a.M, a.N, a.K)) return launch_stream(a, false, a.M <= 128 ? gemm_splits(a.M, a.N, a.K) : 8, stream);
+    if (stream_serves_gemm(a.M, a.N, a.K)) return launch_stream(a, false, stream);
     if (gemm_wide_possible(a.M, a.K)) return launch_gemm_wide(a, stream);
     return a.nested.q ? launch_tile<true>(a, stream) : launch_tile<false>(a, stream);
 }

@@ -48,16 +48,18 @@ bool stream_serves_gemm(int64_t M, int64_t N, int64_t K) {
     return M <= 128 || tiles <= (K >= 2048 ? 256 : 128);
 }
 
-StreamPlan stream_plan(int64_t M, int64_t N, int64_t K, int max_splits) {
+namespace {
+
+StreamPlan plan_and_time(int64_t M, int64_t N, int64_t K, int max_splits, float& best_us) {
     StreamPlan best{};
-    float best_us = 0.0f;
+    best_us = 0.0f;
     const int64_t ksteps = K / 64, units = (ksteps + 3) / 4;
     for (int bm = 32; bm <= 128; bm *= 2) {
         const int64_t m_tiles = (M + bm - 1) / bm;
         for (int wn = bm == 128 ? 8 : bm == 64 ? 4 : 2; wn <= 8; wn *= 2) {
             const int64_t n_tiles = (N + 32 * wn - 1) / (32 * wn);
             const int wk = 8 / wn;
-            for (int s = 1; s <= max_splits && s <= 8; ++s) {
+            for (int s = 1; s <= max_splits; ++s) {
                 if (s > 1 && (m_tiles * n_tiles * s > 256 || units < s * wk)) break;  // one round, nobody idle
                 const int64_t steps = 4 * ((units + wk * s - 1) / (wk * s));
                 const float us = model_us(m_tiles * n_tiles * s, steps < ksteps ? steps : ksteps, bm, 32 * wn, s);
@@ -73,10 +75,28 @@ StreamPlan stream_plan(int64_t M, int64_t N, int64_t K, int max_splits) {
     return best;
 }
 
-size_t stream_workspace_bytes(int64_t M, int64_t N, int64_t K) { return stream_possible(M, N, K) ? plan_bytes(stream_plan(M, N, K, 8)) : 0; }
+}  // namespace
 
-hipError_t launch_stream(const MatmulArgs& a, bool f16, int max_splits, hipStream_t stream) {
-    StreamPlan p = stream_plan(a.M, a.N, a.K, max_splits);
+StreamPlan stream_plan(int64_t M, int64_t N, int64_t K, int max_splits) {
+    float us;
+    return plan_and_time(M, N, K, max_splits, us);
+}
+
+// (5 us: what the model leaves out because every choice has it, the start of a launch and its last stores.  Measured / modelled
+// at M = 130, 512, 2048: [1024, 4096] 10.6, 13.6, 28.9 / 10.8, 13.5, 27.4; [4096, 4096] 18.6, 27.7, 74.1 / 18.7, 27.4, 70.0; [4096, 14336]
+// 41.4, 72.9, 218.3 / 43.5, 72.0, 230.0; [14336, 4096] at 130 and 512 40.9, 65.8 / 44.5, 67.6.)
+float stream_us(int64_t M, int64_t N, int64_t K) {
+    float us;
+    plan_and_time(M, N, K, STREAM_MAX_SPLITS, us);
+    return us + 5.0f;
+}
+
+size_t stream_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+    return stream_possible(M, N, K) ? plan_bytes(stream_plan(M, N, K, STREAM_MAX_SPLITS)) : 0;
+}
+
+hipError_t launch_stream(const MatmulArgs& a, bool f16, hipStream_t stream) {
+    StreamPlan p = stream_plan(a.M, a.N, a.K, STREAM_MAX_SPLITS);
     if (plan_bytes(p) > a.workspace_bytes) p = stream_plan(a.M, a.N, a.K, 1);
     if (f16) return a.nested.q ? stream::launch_f16_dq(a, p, stream) : stream::launch_f16(a, p, stream);
     return a.nested.q ? stream::launch_bf16_dq(a, p, stream) : stream::launch_bf16(a, p, stream);

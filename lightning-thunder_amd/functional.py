@@ -363,14 +363,6 @@ def _gemm_plan(M: int, N: int, K: int) -> tuple[int, int, int, int]:
     return plan[0], plan[1], plan[2], plan[3]
 
 
-def _wide_schedule(M: int, N: int, K: int) -> tuple[int, int, int]:
-    """(rows of x per tile, tiles, pieces per tile) of the fused GEMM kernel for more than 128 rows of x: the 256-row
-    tile from 160 tiles on or when tiles x k steps >= 28672, else the 128-row tile; a call with fewer tiles than the 256
-    CUs cuts every tile into up to 8 equal pieces along k that meet in the workspace."""
-    bm, tiles, pieces, _ = _gemm_plan(M, N, K)
-    return bm, tiles, pieces
-
-
 def _wide_gemm_us(M: int, N: int, K: int) -> float:
     """Model of the fused GEMM kernel for more than 128 rows of x (csrc/nf4_gemm_wide.hip): workgroups (one per tile
     or piece of a tile) run in rounds of 256, K / 64 / pieces steps each; a step of the 256-row tile takes 1.85 us
@@ -379,8 +371,7 @@ def _wide_gemm_us(M: int, N: int, K: int) -> float:
     [4096, 4096] M = 256 / 512 / 1024 / 2048: 30 / 36 / 53 / 75 vs 29 / 37 / 53 / 76; [1024, 4096] M = 256 / 2048: 25 / 34
     vs 27 / 37; [4096, 14336] M = 256 / 512 / 2048: 52 / 77 / 229 vs 49 / 77 / 233; [8192, 28672] M = 512: 230 vs 233;
     [14336, 4096] M = 512 / 1024 / 2048: 69 / 113 / 220 vs 68 / 124 / 237; lm_head [128256, 4096] M = 2048: 1940 vs 1890."""
-    bm, tiles, pieces = _wide_schedule(M, N, K)
-    wgs = tiles * pieces
+    bm, _, pieces, wgs = _gemm_plan(M, N, K)
     rounds = (wgs + 255) // 256
     fill = wgs / (rounds * 256.0)
     step = (1.85 if bm == 256 else 1.0) * (0.6 + 0.4 * fill)
@@ -406,8 +397,11 @@ def _dense_gemm_us(M: int, N: int, K: int) -> float:
 
 
 def _fused_gemm_wins(M: int, N: int, K: int, nested: bool = False) -> bool:
-    """Is the fused GEMM kernel faster than dequantize + dense GEMM (calls that ``_stream_takes`` leaves)?  Both sides are
-    modelled from measurements on MI355X.  The fused kernel
+    """Is ``nf4hip_gemm`` faster than dequantize + dense GEMM (calls that ``_stream_takes`` leaves)?  Both sides are
+    modelled from measurements on MI355X.  While the streaming kernel serves the call, its launcher's own model stands against
+    what ``nf4hip_linear`` takes behind the dequantize pass, 3-18 % longer than the library GEMM the dense model describes (fused
+    measured / modelled vs dense route, us: M = 1457 [3616, 14528] 203 / 213 vs 183, M = 2957 [2235, 10944] 163 / 169 vs 171, M = 2392
+    [1332, 17344] 141 / 146 vs 186, M = 2691 [664, 9088] 57 / 60 vs 94).  Beyond, the fused kernel
     runs at 1.0-1.15 PFLOP/s, the library GEMM at up to 1.5, but the dense route first writes the bf16 weight: the
     two cross near 1024 rows of x wherever the fused kernel has a workgroup for most CUs (fused vs dense, us, M =
     512 / 1024 / 2048: [14336, 4096] 71 / 117 / 232 vs 84 / 118 / 198; [28672, 4096] 127 / 239 / 473 vs 155 / 238 / 405; [28672, 8192] 226 /
@@ -416,7 +410,10 @@ def _fused_gemm_wins(M: int, N: int, K: int, nested: bool = False) -> bool:
     which needs no transient bf16 weight."""
     # nested absmax: the fp32 absmax is written out ahead of the fused kernel (_matmul_nf4_on), 2-7 % on top; the
     # dequantize pass of the dense route resolves the codes itself at no measurable cost
-    return _wide_gemm_us(M, N, K) * (1.05 if nested else 1.0) <= 1.03 * _dense_gemm_us(M, N, K)
+    nested_factor = 1.05 if nested else 1.0
+    if _lib.load().nf4hip_gemm_streamed(M, N, K):
+        return _lib.load().nf4hip_stream_us(M, N, K) * nested_factor <= 1.15 * _dense_gemm_us(M, N, K)
+    return _wide_gemm_us(M, N, K) * nested_factor <= 1.03 * _dense_gemm_us(M, N, K)
 
 
 # Many rows of x: the fused GEMM and dequantize + dense GEMM are within a few per cent of each other over a wide range
@@ -633,10 +630,7 @@ def _matmul_nf4_on(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape,
         fn, fn_dq = lib.nf4hip_gemv, lib.nf4hip_gemv_dq
     else:
         need = lib.nf4hip_gemm_workspace_bytes(M, N, K)  # K split over workgroups: partial tiles and counters
-        want = max(need, lib.nf4hip_stream_workspace_bytes(M, N, K)) if lib.nf4hip_gemm_streamed(M, N, K) else need
-        ws = _workspace_pool.get_or_none(device, want, stream) if want else None
-        if ws is None and need:
-            ws = _gemv_workspace(device, need, stream)
+        ws = _workspace_pool.get_or_none(device, need, stream) if need else None
         ws_ptr, ws_bytes = (None, 0) if ws is None else (ws.data_ptr(), ws.numel())
         fn, fn_dq = lib.nf4hip_gemm, lib.nf4hip_gemm_dq
     bptr = None if b is None else b.data_ptr()
@@ -649,15 +643,18 @@ def _matmul_nf4_on(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape,
         absmax, nested = reconstruct_absmax(absmax), False
     if nested:
         q, a2, m256, off, nbs = _nested_args(absmax, nblocks)
-        _lib.check(fn_dq(x_ptr, code, M, qweight.data_ptr(), q.data_ptr(), a2.data_ptr(), m256.data_ptr(), off, nbs,
-                         quant_map.data_ptr(), bptr, N, K, blocksize, out_ptr, ws_ptr, ws_bytes, stream))  # fmt: skip
+        rc = fn_dq(x_ptr, code, M, qweight.data_ptr(), q.data_ptr(), a2.data_ptr(), m256.data_ptr(), off, nbs,
+                   quant_map.data_ptr(), bptr, N, K, blocksize, out_ptr, ws_ptr, ws_bytes, stream)  # fmt: skip
     else:
         _require_gpu(absmax)
         absmax = _aligned(absmax if absmax.dtype is torch.float32 else absmax.to(torch.float32))
         if absmax.numel() < nblocks:
             raise ValueError(f"absmax holds {absmax.numel()} entries, need {nblocks}")
-        _lib.check(fn(x_ptr, code, M, qweight.data_ptr(), absmax.data_ptr(), quant_map.data_ptr(), bptr,
-                      N, K, blocksize, out_ptr, ws_ptr, ws_bytes, stream))  # fmt: skip
+        rc = fn(x_ptr, code, M, qweight.data_ptr(), absmax.data_ptr(), quant_map.data_ptr(), bptr,
+                N, K, blocksize, out_ptr, ws_ptr, ws_bytes, stream)  # fmt: skip
+    if rc == _lib.E_WORKSPACE and ws is None:
+        _gemv_workspace(device, need, stream)  # raises: a capture on a stream that has none
+    _lib.check(rc)
     return out if flat else out.reshape(*x.shape[:-1], N)
 
 

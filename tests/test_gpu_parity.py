@@ -317,8 +317,8 @@ def test_gemv_repeatable_and_workspace_reuse(ta, oracle):
 
 def test_split_k_hand_off_holds_over_many_launches(ta):
     """2000 launches on ONE workspace, alternating between four calls whose partial sums cross workgroups (decode
-    tile kernel with K split eight ways, row kernel with a long K, fused GEMM with K split, fused GEMM with cut-up
-    tiles): every result must equal the first of its kind bit for bit and every arrival counter must be back at
+    tile kernel with K split eight ways, row kernel with a long K, streaming kernel with one tile of x rows and with
+    several): every result must equal the first of its kind bit for bit and every arrival counter must be back at
     zero.  The comparison runs on the device; the host looks at the verdict every 100 launches and stops at the
     first mismatch."""
     _sync_print("split-K hand-off, 2000 launches on one workspace")
@@ -326,7 +326,7 @@ def test_split_k_hand_off_holds_over_many_launches(ta):
     code = ta.nf4_code(DEV)
     g = torch.Generator(device=DEV).manual_seed(7)
     calls = []
-    for kind, M, N, K in [("gemv", 16, 6144, 4096), ("gemv", 1, 512, 32768), ("gemm", 64, 1024, 4096), ("gemm", 512, 1024, 4096)]:
+    for kind, M, N, K in [("gemv", 16, 6144, 4096), ("gemv", 1, 512, 32768), ("gemm", 64, 1024, 4096), ("gemm", 256, 1024, 8192)]:
         n = N * K
         packed = torch.randint(0, 256, (n // 2,), dtype=torch.uint8, device=DEV, generator=g)
         absmax = torch.rand(n // 64, device=DEV, generator=g) * 0.05 + 0.01
@@ -369,11 +369,19 @@ def _fused_route_of(M):
     return "stream" if M <= 128 else "gemm"
 
 
-@pytest.mark.parametrize("M,N,K", [(200, 128, 4096), (129, 1024, 4096), (3000, 1024, 4096)])
+@pytest.mark.parametrize("M,N,K", [(9000, 260, 512), (4100, 1024, 1024)])
 def test_dense_route(ta, oracle, M, N, K):
     """Default route for many rows of x: nf4hip_dequantize + dense GEMM."""
     _sync_print(f"dequant+gemm M={M} N={N} K={K}")
     assert ta.functional.fused_route(torch.empty(M, K, dtype=torch.bfloat16), None, 64, torch.bfloat16, (N, K)) == "dequant+gemm"
+    _matmul_case(ta, oracle, M, N, K, seed=M + N + K + 1)
+
+
+@pytest.mark.parametrize("M,N,K", [(200, 128, 4096), (129, 1024, 4096), (3000, 1024, 4096)])
+def test_dense_route_forced(ta, oracle, M, N, K, monkeypatch):
+    """The same route on shapes whose own route is the fused kernel."""
+    _sync_print(f"dequant+gemm (forced) M={M} N={N} K={K}")
+    monkeypatch.setattr(ta.functional, "fused_route", lambda *a, **k: "dequant+gemm")
     _matmul_case(ta, oracle, M, N, K, seed=M + N + K + 1)
 
 

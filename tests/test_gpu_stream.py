@@ -2,8 +2,6 @@
 16 / 32 / 64 / 128, ragged weight rows, one k step, a partial unit of four steps, K split over workgroups -- on fp32 and nested
 absmax and larger blocksizes, against a float64 product over the HIP-dequantised weight."""
 
-import ctypes
-
 import pytest
 import torch
 
@@ -127,21 +125,44 @@ def test_gemm_streamed_beyond_128_rows(ta, M, N, K, blocksize, nested, bias, scr
     deq = ta.dequantize_nf4(qw, stats, code, blocksize, torch.bfloat16, (N, K))
     if scratch:
         run = lambda: F._matmul_nf4_on(x, qw, b, stats, code, blocksize, torch.bfloat16, (N, K), "gemm")
-    else:  # the least the C ABI accepts
-        need = lib.nf4hip_gemm_workspace_bytes(M, N, K)
-        ws = torch.zeros(max(need, 16), dtype=torch.uint8, device=DEV)
+    else:  # the streaming kernel takes any plan without
         if nested:
             stats = ta.reconstruct_absmax(stats)
 
         def run():
             out = torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
-            ta._lib.check(lib.nf4hip_gemm(x.data_ptr(), 0, M, qw.data_ptr(), stats.data_ptr(), code.data_ptr(), None if b is None else b.data_ptr(), N, K,
-                                          blocksize, out.data_ptr(), ws.data_ptr() if need else None, need, F._stream()))
+            ta._lib.check(lib.nf4hip_stream(x.data_ptr(), 0, M, qw.data_ptr(), stats.data_ptr(), code.data_ptr(), None if b is None else b.data_ptr(), N, K,
+                                            blocksize, out.data_ptr(), None, 0, F._stream()))
             return out
 
     y = run()
     _check(y, x, deq, b)
     assert torch.equal(run(), y)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,split", [(24, 512, 64 * 47, True), (100, 300, 64 * 61, True), (300, 1000, 1024, False)])
+def test_gemm_without_the_workspace(ta, M, N, K, split):
+    """Calls that nf4hip_gemm takes without the workspace it asks for (K in no equal ranges) or that need none: NULL, too small a
+    one, one that is not aligned and one that was not asked for, which stay as they are."""
+    print(f"gemm without workspace M={M} [{N},{K}]", flush=True)
+    F, lib, L = ta.functional, ta._lib.load(), ta._lib
+    need = lib.nf4hip_gemm_workspace_bytes(M, N, K)
+    assert (need > 0) == split and lib.nf4hip_gemm_streamed(M, N, K)
+    qw, absmax, code = _weight(ta, N, K, 64, False, torch.bfloat16, M + N)
+    x = torch.randn(M, K, device=DEV, generator=torch.Generator(device=DEV).manual_seed(K)).to(torch.bfloat16)
+    deq = ta.dequantize_nf4(qw, absmax, code, 64, torch.bfloat16, (N, K))
+    ws = torch.full((4 << 20,), 0x5A, dtype=torch.uint8, device=DEV)
+    assert need < ws.numel() - 16
+    cases = [(None, 0), (ws.data_ptr(), 4096), (ws.data_ptr() + 2, ws.numel() - 16)] + ([] if split else [(ws.data_ptr(), ws.numel())])
+    first = None
+    for ptr, nbytes in cases:
+        out = torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+        L.check(lib.nf4hip_gemm(x.data_ptr(), L.BF16, M, qw.data_ptr(), absmax.data_ptr(), code.data_ptr(), None, N, K, 64, out.data_ptr(), ptr, nbytes,
+                                F._stream()))
+        first = out if first is None else first
+        assert torch.equal(out, first) and bool((ws == 0x5A).all())
+    _check(first, x, deq, None)
 
 
 def test_gemm_streamed_rule(ta):
@@ -169,7 +190,6 @@ def test_stream_arguments_and_workspace(ta):
             need = lib.nf4hip_stream_workspace_bytes(M, N, K)
             assert need == 0 or 65536 * 4 < need <= 65536 * 4 + 256 * 256 * 128 * 4
     assert lib.nf4hip_stream_workspace_bytes(129, 64, 64) == 0 and lib.nf4hip_stream_workspace_bytes(8, 64, 96) == 0
-    _ = ctypes
 
 
 def test_fp16_route(ta):

@@ -8,7 +8,8 @@ Lifetime rules, chosen for callers that capture HIP graphs:
   buffer is retired (kept alive), not released.
 * Nothing is allocated while the stream is capturing.  ``torch.zeros`` there would record a memset node
   (unreliable in replayed graphs on this target) and tie the buffer to the capture's private pool; the
-  call raises instead and tells the caller to warm up or to :meth:`reserve` first.
+  call raises instead and tells the caller to warm up or to :meth:`reserve` first.  A caller that can go on
+  without a buffer asks :meth:`get_or_none`.
 * Buffers start at ``floor_bytes``, large enough for every Llama-3-8B / 70B projection shape, so growth is
   the exception.
 

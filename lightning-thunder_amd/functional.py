@@ -16,6 +16,7 @@ from __future__ import annotations
 import ctypes
 import math
 import os
+import warnings
 from dataclasses import dataclass
 
 import torch
@@ -617,22 +618,17 @@ def _matmul_nf4_on(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape,
     nblocks = N * K // blocksize
     out = x2.new_empty((M, N)) if type(x2) is torch.Tensor else torch.empty((M, N), dtype=x.dtype, device=device)
     stream = _stream() if _raw_stream is None else _raw_stream(device.index)
-    if route == "stream":
-        need = lib.nf4hip_stream_workspace_bytes(M, N, K)
-        # without scratch (a capture on a stream that has none yet) the kernel does not split K
-        ws = _workspace_pool.get_or_none(device, need, stream) if need else None
-        ws_ptr, ws_bytes = (None, 0) if ws is None else (ws.data_ptr(), ws.numel())
-        fn, fn_dq = lib.nf4hip_stream, lib.nf4hip_stream_dq
-    elif route == "gemv":
+    if route == "gemv":
         need = lib.nf4hip_gemv_workspace_bytes(M, N, K)
         ws = _gemv_workspace(device, need, stream)
-        ws_ptr, ws_bytes = ws.data_ptr(), ws.numel()
         fn, fn_dq = lib.nf4hip_gemv, lib.nf4hip_gemv_dq
-    else:
-        need = lib.nf4hip_gemm_workspace_bytes(M, N, K)  # K split over workgroups: partial tiles and counters
+    else:  # K split over workgroups: partial tiles and counters.  Under capture, on a stream that has none yet, what can do without does
+        if x.dtype is torch.float16:
+            need, fn, fn_dq = lib.nf4hip_stream_workspace_bytes(M, N, K), lib.nf4hip_stream, lib.nf4hip_stream_dq
+        else:
+            need, fn, fn_dq = lib.nf4hip_gemm_workspace_bytes(M, N, K), lib.nf4hip_gemm, lib.nf4hip_gemm_dq
         ws = _workspace_pool.get_or_none(device, need, stream) if need else None
-        ws_ptr, ws_bytes = (None, 0) if ws is None else (ws.data_ptr(), ws.numel())
-        fn, fn_dq = lib.nf4hip_gemm, lib.nf4hip_gemm_dq
+    ws_ptr, ws_bytes = (None, 0) if ws is None else (ws.data_ptr(), ws.numel())
     bptr = None if b is None else b.data_ptr()
     code, x_ptr, out_ptr = _DTYPE_CODE[x.dtype], x2.data_ptr(), out.data_ptr()
     nested = isinstance(absmax, NestedAbsmax)
@@ -652,8 +648,13 @@ def _matmul_nf4_on(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape,
             raise ValueError(f"absmax holds {absmax.numel()} entries, need {nblocks}")
         rc = fn(x_ptr, code, M, qweight.data_ptr(), absmax.data_ptr(), quant_map.data_ptr(), bptr,
                 N, K, blocksize, out_ptr, ws_ptr, ws_bytes, stream)  # fmt: skip
-    if rc == _lib.E_WORKSPACE and ws is None:
-        _gemv_workspace(device, need, stream)  # raises: a capture on a stream that has none
+    if ws is None and need:
+        if rc == _lib.E_WORKSPACE:
+            _gemv_workspace(device, need, stream)  # raises: a capture on a stream that has none
+        if rc == 0:
+            warnings.warn(f"NF4 matmul: [{N}, {K}] captured on a stream without a workspace, so K is not split over workgroups: a slower "
+                          "kernel than the eager call's. Run the call once on this stream before the capture, or call reserve_workspace().",
+                          stacklevel=3)
     _lib.check(rc)
     return out if flat else out.reshape(*x.shape[:-1], N)
 

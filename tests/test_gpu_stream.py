@@ -78,6 +78,33 @@ def test_stream_infinities_stay_in_their_row(ta):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,refused", [(24, 512, 4096, True), (128, 4096, 14336, True), (8, 300, 2880, True), (256, 1024, 8192, True),
+                                           (24, 512, 64 * 47, False)])
+def test_capture_on_a_stream_without_a_workspace(ta, monkeypatch, M, N, K, refused):
+    """bf16 calls that would record a slower plan than the eager call's are refused, with the way out in the message; those that
+    were always taken without a workspace, and fp16, which has no other kernel, go on and say so.  (The stream is only said
+    to be capturing.)"""
+    print(f"capture without workspace M={M} [{N},{K}]", flush=True)
+    F = ta.functional
+    for dtype in (torch.bfloat16, torch.float16):
+        qw, absmax, code = _weight(ta, N, K, 64, False, dtype, 5)
+        x = torch.randn(M, K, device=DEV).to(dtype)
+        deq = ta.dequantize_nf4(qw, absmax, code, 64, dtype, (N, K))
+        call = lambda: F.matmul_nf4(x, qw, None, absmax, code, 64, dtype, (N, K))
+        with monkeypatch.context() as m:
+            m.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+            m.setattr(F._workspace_pool, "_live", {})
+            if refused and dtype == torch.bfloat16:
+                with pytest.raises(RuntimeError, match="reserve_workspace"):
+                    call()
+            else:
+                with pytest.warns(UserWarning, match="without a workspace"):
+                    y = call()
+                _check(y, x, deq, None)
+        _check(call(), x, deq, None)
+
+
+@pytest.mark.gpu
 def test_stream_capture_without_scratch_and_autograd(ta):
     print("stream capture / autograd", flush=True)
     F = ta.functional

@@ -43,6 +43,11 @@ def test_no_allocation_while_capturing(pool_mod, monkeypatch):
         pool.get(cpu, 4096, stream=1)                    # growth during capture is refused ...
     assert pool.get(cpu, 512, stream=1) is ws            # ... and the existing buffer is untouched
     assert pool.stats()["retired"] == 0
+    # a caller that can do without: what there is, or nothing; outside a capture as get()
+    assert pool.get_or_none(cpu, 512, stream=1) is ws and pool.get_or_none(cpu, 4096, stream=1) is None
+    assert pool.get_or_none(cpu, 10, stream=2) is None and pool.stats()["live"] == 1
+    capturing["on"] = False
+    assert pool.get_or_none(cpu, 10, stream=2).numel() == 1024
 
 
 def test_functional_pool_covers_llama_shapes(ta):

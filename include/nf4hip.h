@@ -232,29 +232,31 @@ int nf4hip_gemv_static(const void* x, int x_dtype, int64_t M, const uint8_t* pac
 size_t nf4hip_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K);
 /*
  * The launch plan nf4hip_gemm uses for a shape (no GPU needed): plan[0] rows of x per tile, plan[1] tiles, plan[2] pieces
- * a tile is cut into along K (they meet in the workspace), plan[3] workgroups launched.  nf4hip_gemm_streamed: is it
- * nf4hip_stream's kernel (up to 128 rows of x, more while tiles of 128 x 256 fill the chip once at most)?  For host code that chooses
+ * a tile is cut into along K (they meet in the workspace), plan[3] workgroups launched.  nf4hip_gemm_us: the time the launcher's
+ * model gives the call in microseconds, on fp32 absmax.  nf4hip_gemm_streamed: is it nf4hip_stream's kernel (up to 128 rows of x,
+ * on most weights more while tiles of 128 x 256 fill the chip once at most)?  For host code that chooses
  * between this kernel and dequantize + dense GEMM (the choice bitsandbytes.matmul_4bit makes at thunder/transforms/quantization.py:39) without keeping
  * a copy of the launcher's rules.  K must be a multiple of 64.
  */
 int nf4hip_gemm_plan(int64_t M, int64_t N, int64_t K, int32_t plan[4]);
+float nf4hip_gemm_us(int64_t M, int64_t N, int64_t K);
 int nf4hip_gemm_streamed(int64_t M, int64_t N, int64_t K);
 int nf4hip_gemm(const void* x, int x_dtype, int64_t M, const uint8_t* packed, const float* absmax, const float* lut16,
                 const void* bias_or_null, int64_t N, int64_t K, int blocksize, void* out, void* workspace,
                 size_t workspace_bytes, void* stream);
 /*
- * The same product, wherever nf4hip_gemm_streamed says 1, for bf16 or fp16 x (then bias and out are fp16 too), every weight rounded to x's type as
+ * The same product, wherever nf4hip_stream_served says 1 (at least where nf4hip_gemm_streamed does), for bf16 or fp16 x (then bias and out are fp16 too), every weight rounded to x's type as
  * nf4hip_dequantize rounds it: the kernel between the decode step and the prompt, and for fp16 also at decode shapes.
  * K % 64 == 0, blocksize dividing K.  With nf4hip_stream_workspace_bytes(M, N, K) bytes of workspace (rules of nf4hip_gemv's;
  * the kernels may share one) K may be split over workgroups; with less, or NULL, it is not.  Deterministic either way.
  */
+int nf4hip_stream_served(int64_t M, int64_t N, int64_t K);
 size_t nf4hip_stream_workspace_bytes(int64_t M, int64_t N, int64_t K);
 /*
  * What it launches with that workspace (no GPU needed): plan[0] rows of x and plan[1] weight rows per tile, plan[2] workgroups that
- * share a tile's K, plan[3] workgroups; and the time the launcher's model gives it in microseconds on fp32 absmax (0: not served).
+ * share a tile's K, plan[3] workgroups.
  */
 int nf4hip_stream_plan(int64_t M, int64_t N, int64_t K, int32_t plan[4]);
-float nf4hip_stream_us(int64_t M, int64_t N, int64_t K);
 int nf4hip_stream(const void* x, int x_dtype, int64_t M, const uint8_t* packed, const float* absmax, const float* lut16,
                   const void* bias_or_null, int64_t N, int64_t K, int blocksize, void* out, void* workspace,
                   size_t workspace_bytes, void* stream);

@@ -67,12 +67,13 @@ SYMBOLS = {
     "nf4hip_gemv_plan": (_i32, [_i64, _i64, _i64, _i32, _i32, ctypes.POINTER(_i32 * 4)]),
     "nf4hip_gemm_workspace_bytes": (_sz, [_i64, _i64, _i64]),
     "nf4hip_gemm_plan": (_i32, [_i64, _i64, _i64, ctypes.POINTER(_i32 * 4)]),
+    "nf4hip_gemm_us": (_f32, [_i64, _i64, _i64]),
     "nf4hip_gemm_streamed": (_i32, [_i64, _i64, _i64]),
     "nf4hip_gemm": (_i32, _MATMUL),
     "nf4hip_gemm_dq": (_i32, _MATMUL_DQ),
     "nf4hip_stream_workspace_bytes": (_sz, [_i64, _i64, _i64]),
     "nf4hip_stream_plan": (_i32, [_i64, _i64, _i64, ctypes.POINTER(_i32 * 4)]),
-    "nf4hip_stream_us": (_f32, [_i64, _i64, _i64]),
+    "nf4hip_stream_served": (_i32, [_i64, _i64, _i64]),
     "nf4hip_stream": (_i32, _MATMUL),
     "nf4hip_stream_dq": (_i32, _MATMUL_DQ),
     "nf4hip_linear_workspace_bytes": (_sz, [_i64, _i64, _i64]),

@@ -121,8 +121,8 @@ int matmul_common(MatmulKind kind, const void* x, int x_dtype, int64_t M, const 
             return fail(NF4HIP_E_SHAPE, "nf4hip_gemv: K = %lld > 2^24 with M > 4 (use nf4hip_gemm)", (long long)K);
     } else {
         if (K % 64) return fail(NF4HIP_E_SHAPE, "%s: K = %lld is not a multiple of 64", name, (long long)K);
-        if (kind == STREAM && !nf4::stream_serves_gemm(M, N, K))
-            return fail(NF4HIP_E_SHAPE, "%s: M = %lld, N = %lld, K = %lld: not served (nf4hip_gemm_streamed)", name,
+        if (kind == STREAM && !nf4::stream_served(M, N, K))
+            return fail(NF4HIP_E_SHAPE, "%s: M = %lld, N = %lld, K = %lld: not served (nf4hip_stream_served)", name,
                         (long long)M, (long long)N, (long long)K);
     }
     if (!(kind == GEMV && M <= 4) && K % blocksize)
@@ -417,12 +417,14 @@ int nf4hip_gemm(const void* x, int x_dtype, int64_t M, const uint8_t* packed, co
 
 int nf4hip_gemm_streamed(int64_t M, int64_t N, int64_t K) { return nf4::stream_serves_gemm(M, N, K) ? 1 : 0; }
 
-float nf4hip_stream_us(int64_t M, int64_t N, int64_t K) { return nf4::stream_serves_gemm(M, N, K) ? nf4::stream_us(M, N, K) : 0.0f; }
+float nf4hip_gemm_us(int64_t M, int64_t N, int64_t K) { return M <= 0 || N <= 0 || K <= 0 || K % 64 ? 0.0f : nf4::gemm_us(M, N, K); }
+
+int nf4hip_stream_served(int64_t M, int64_t N, int64_t K) { return nf4::stream_served(M, N, K) ? 1 : 0; }
 
 int nf4hip_stream_plan(int64_t M, int64_t N, int64_t K, int32_t plan[4]) {
     if (!plan) return fail(NF4HIP_E_NULL, "nf4hip_stream_plan: null pointer");
-    if (!nf4::stream_serves_gemm(M, N, K))
-        return fail(NF4HIP_E_SHAPE, "nf4hip_stream_plan: M = %lld, N = %lld, K = %lld: not served (nf4hip_gemm_streamed)",
+    if (!nf4::stream_served(M, N, K))
+        return fail(NF4HIP_E_SHAPE, "nf4hip_stream_plan: M = %lld, N = %lld, K = %lld: not served (nf4hip_stream_served)",
                     (long long)M, (long long)N, (long long)K);
     const nf4::StreamPlan p = nf4::stream_plan(M, N, K, nf4::STREAM_MAX_SPLITS);
     plan[0] = p.bm;

@@ -92,13 +92,14 @@ int gemv_norm_parts(int64_t M, int64_t N, int64_t K);  // partial sums per row o
 size_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K);
 size_t gemm_workspace_required(int64_t M, int64_t N, int64_t K);  // 0: the call is taken without as well
 hipError_t launch_gemm(const MatmulArgs& a, hipStream_t stream);
-// up to 128 rows of bf16 or fp16 x, and more where stream_serves_gemm (nf4_gemm_stream.hip): rows of x per tile, 32-row weight tiles side by side, workgroups
+// up to 128 rows of bf16 or fp16 x, and more where stream_served (nf4_gemm_stream.hip): rows of x per tile, 32-row weight tiles side by side, workgroups
 // that share a tile's K (at most `max_splits`), tiles.  K is not split where a.workspace_bytes does not hold the partial tiles.
 constexpr int STREAM_MAX_SPLITS = 8;
 struct StreamPlan {
     int bm, wn, splits, m_tiles, n_tiles;
 };
 bool stream_possible(int64_t M, int64_t N, int64_t K);
+bool stream_served(int64_t M, int64_t N, int64_t K);       // does launch_stream take it?
 bool stream_serves_gemm(int64_t M, int64_t N, int64_t K);  // does launch_gemm use it?
 StreamPlan stream_plan(int64_t M, int64_t N, int64_t K, int max_splits);
 size_t stream_workspace_bytes(int64_t M, int64_t N, int64_t K);
@@ -107,11 +108,14 @@ hipError_t launch_stream(const MatmulArgs& a, bool f16, hipStream_t stream);
 // what the streaming kernel does not take, with x below 4 GB: 256 x 256 or 128 x 256 tiles (nf4_gemm_wide.hip)
 bool gemm_wide_possible(int64_t M, int64_t K);
 int gemm_wide_tile_rows(int64_t M, int64_t N, int64_t K);
+bool gemm_wide_cuts_long_tiles(int64_t M, int64_t N, int64_t K);  // in 256-row tiles, each in pieces along K?
+float gemm_wide_us(int64_t M, int64_t N, int64_t K);              // modelled time, fp32 absmax
 hipError_t launch_gemm_wide(const MatmulArgs& a, hipStream_t stream);
 size_t gemm_wide_workspace_bytes(int64_t M, int64_t N, int64_t K);
 // The launch plan of the fused GEMM for a shape, as the launchers compute it: plan[0] rows of x per tile (64, 128,
 // 256), plan[1] tiles (tiles of x rows times tiles of 256 weight rows), plan[2] pieces a tile is cut into along K,
 // plan[3] workgroups launched.
+float gemm_us(int64_t M, int64_t N, int64_t K);  // of what launch_gemm launches
 void gemm_wide_plan(int64_t M, int64_t N, int64_t K, int plan[4]);
 void gemm_plan(int64_t M, int64_t N, int64_t K, int plan[4]);
 // which decode kernel serves a call without an epilogue (GEMV_KERNEL_* of nf4_gemv.h) and its arithmetic mode (ARITH_*)

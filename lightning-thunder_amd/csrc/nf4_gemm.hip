@@ -6,9 +6,9 @@
 // bf16 in registers -- bf16_rne(lut16[code] * absmax), the same value nf4hip_dequantize produces --
 // and contracts them with bf16 MFMA, fp32 accumulation, bf16 output.
 //
-// Up to 128 rows of x, and more while the chip is filled once at most: nf4_gemm_stream.hip.  Else, and where that kernel's
-// 32-bit offsets into a weight end (K >= 2^24, 2^31 blocks): nf4_gemm_wide.hip.  The kernel here takes what the other two's 32-bit
-// offsets into x do not reach, x of 4 GB and more: 64-bit addresses, one workgroup per tile.
+// Up to 128 rows of x, and on most weights more while the chip is filled once at most: nf4_gemm_stream.hip (stream_serves_gemm).
+// Else, and where that kernel's 32-bit offsets into a weight end (K >= 2^24, 2^31 blocks): nf4_gemm_wide.hip.  The kernel here takes
+// what the other two's 32-bit offsets into x do not reach, x of 4 GB and more: 64-bit addresses, one workgroup per tile.
 //
 // Tile: 256 rows of x x 256 (n) x 64 (k) per workgroup of 512 threads.  Wave w of 8
 // owns weight rows 32 w .. + 31 of the tile against all rows of x: eight accumulators of
@@ -336,6 +336,11 @@ void gemm_plan(int64_t M, int64_t N, int64_t K, int plan[4]) {
         plan[2] = 1;
     }
     plan[3] = plan[1] * plan[2];
+}
+
+// (The general kernel's whole 256-row tiles as if the other kernel took them: nothing chooses by this.)
+float gemm_us(int64_t M, int64_t N, int64_t K) {
+    return stream_serves_gemm(M, N, K) ? stream_us(M, N, K) : gemm_wide_us(M, N, K);
 }
 
 hipError_t launch_gemm(const MatmulArgs& a, hipStream_t stream) {

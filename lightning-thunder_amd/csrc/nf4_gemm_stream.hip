@@ -42,10 +42,19 @@ bool stream_possible(int64_t M, int64_t N, int64_t K) {
 // [14336, 4096] 50.0 / 40.9, 73.4 / 65.8 (224 tiles), 216.6 / 253.6.  Beyond one round that kernel's 256-row tiles expand every
 // weight half as often: [28672, 4096] M = 256 75.1 / 65.3 (224 tiles), M = 384 112.5 / 118.1 (336).  With few k steps and a nearly
 // full chip the two are level ([32000, 1024] M = 130..256, 250 tiles: 25.8, 25.5, 26.7 / 25.8, 26.0, 27.4).
-bool stream_serves_gemm(int64_t M, int64_t N, int64_t K) {
+bool stream_served(int64_t M, int64_t N, int64_t K) {
     if (!stream_possible(M, N, K)) return false;
     const int64_t tiles = ((M + 127) / 128) * ((N + 255) / 256);
     return M <= 128 || tiles <= (K >= 2048 ? 256 : 128);
+}
+
+// Of these, nf4hip_gemm leaves to that kernel what it takes in 256-row tiles cut along K (at most 128 of them, K >= 14336) when its
+// model is ahead: the 128-row tiles here expand every weight twice as often and often have no split left to fill the chip with.
+// Over 80 such shapes the choice takes 0.2 % longer than the better of the two on average, 6 % at most (always here: 7 %, 36 %); wide /
+// here: M = 986 [4384, 27520] 243 / 330, M = 1343 [4864, 26560] 358 / 413, M = 2005 [3236, 20224] 271 / 295, M = 315 [8768, 27648] 250 / 206.
+bool stream_serves_gemm(int64_t M, int64_t N, int64_t K) {
+    if (!stream_served(M, N, K)) return false;
+    return M <= 128 || !gemm_wide_cuts_long_tiles(M, N, K) || stream_us(M, N, K) <= gemm_wide_us(M, N, K);
 }
 
 namespace {

@@ -151,8 +151,7 @@ __device__ __forceinline__ void expansion_step(Expansion& x, int t, uint32_t d, 
 //     dealt so that every XCD -- workgroup b runs on XCD b % 8 -- owns a contiguous run of them: the x-row tiles
 //     that share a weight tile meet in one L2.
 //   * The remaining `tail_tiles` (fewer than GRID) would leave CUs idle in a last, partial round.  Where a call has no
-//     other tiles -- nearly all such calls are nf4_gemm_stream.hip's; what is left are shapes beyond its 32-bit offsets,
-//     K >= 2^24 or a weight of 2^31 blocks -- each of them can be cut into `pieces` equal pieces along k (in quanta of `gran` k steps, qpt per tile), one workgroup per
+//     other tiles (most such calls are nf4_gemm_stream.hip's; those that come here have long rows, K >= 14336), each of them can be cut into `pieces` equal pieces along k (in quanta of `gran` k steps, qpt per tile), one workgroup per
 //     piece, numbered piece-major (all first pieces, then all second pieces, ...).  The pieces of a tile meet in
 //     the workspace (see the kernel).  pieces == 1: whole tiles.
 struct WideSchedule {
@@ -606,6 +605,25 @@ void gemm_wide_plan(int64_t M, int64_t N, int64_t K, int plan[4]) {
     plan[1] = s.m_tiles * s.n_tiles;
     plan[2] = s.pieces;
     plan[3] = s.full + s.tail_tiles * s.pieces;
+}
+
+bool gemm_wide_cuts_long_tiles(int64_t M, int64_t N, int64_t K) {
+    return gemm_wide_possible(M, K) && gemm_wide_tile_rows(M, N, K) == 256 && wide_schedule(M, N, K, 256, ~(size_t)0).pieces > 1;
+}
+
+// Workgroups (one per tile or piece of a tile) run in rounds of 256, K / 64 / pieces steps each; a step of the 256-row tile takes
+// 1.85 us on a full chip, of the 128-row tile 1.0 us, up to 40 % less on a sparsely filled one; 12 us of launch, prologue and
+// epilogue; pieces that meet in the workspace add 6 us (128-row tile) or 12 us.  Measured / modelled: [14336, 4096] M = 1024, 2048
+// 113, 220 / 124, 237; lm_head [128256, 4096] M = 2048 1940 / 1890; in pieces [4864, 26560] M = 1343 358 / 390, [3236, 20224] M = 2005 271 / 294,
+// [4096, 24064] M = 1249 237 / 249.
+float gemm_wide_us(int64_t M, int64_t N, int64_t K) {
+    int plan[4];
+    gemm_wide_plan(M, N, K, plan);
+    const int64_t rounds = ((int64_t)plan[3] + 255) / 256;
+    const float fill = (float)plan[3] / (float)(rounds * 256);
+    const float step = (plan[0] == 256 ? 1.85f : 1.0f) * (0.6f + 0.4f * fill);
+    const float merge = plan[2] == 1 ? 0.0f : plan[0] == 128 ? 6.0f : 12.0f;
+    return 12.0f + (float)rounds * (float)(K / BK / plan[2]) * step + merge;
 }
 
 hipError_t launch_gemm_wide(const MatmulArgs& a, hipStream_t stream) {

@@ -364,22 +364,6 @@ def _gemm_plan(M: int, N: int, K: int) -> tuple[int, int, int, int]:
     return plan[0], plan[1], plan[2], plan[3]
 
 
-def _wide_gemm_us(M: int, N: int, K: int) -> float:
-    """Model of the fused GEMM kernel for more than 128 rows of x (csrc/nf4_gemm_wide.hip): workgroups (one per tile
-    or piece of a tile) run in rounds of 256, K / 64 / pieces steps each; a step of the 256-row tile takes 1.85 us
-    on a full chip, of the 128-row tile 1.0 us, up to 40 % less on a sparsely filled one; 12 us of launch, prologue
-    and epilogue; pieces that meet in the workspace add 6 us (128-row tile) or 12 us.  Measured / modelled, us:
-    [4096, 4096] M = 256 / 512 / 1024 / 2048: 30 / 36 / 53 / 75 vs 29 / 37 / 53 / 76; [1024, 4096] M = 256 / 2048: 25 / 34
-    vs 27 / 37; [4096, 14336] M = 256 / 512 / 2048: 52 / 77 / 229 vs 49 / 77 / 233; [8192, 28672] M = 512: 230 vs 233;
-    [14336, 4096] M = 512 / 1024 / 2048: 69 / 113 / 220 vs 68 / 124 / 237; lm_head [128256, 4096] M = 2048: 1940 vs 1890."""
-    bm, _, pieces, wgs = _gemm_plan(M, N, K)
-    rounds = (wgs + 255) // 256
-    fill = wgs / (rounds * 256.0)
-    step = (1.85 if bm == 256 else 1.0) * (0.6 + 0.4 * fill)
-    merge = 0.0 if pieces == 1 else 6.0 if bm == 128 else 12.0
-    return 12.0 + rounds * (K // 64 // pieces) * step + merge
-
-
 def _dense_gemm_us(M: int, N: int, K: int) -> float:
     """Model of the dense route for more than 128 rows of x, kernel time: the dequantize pass (10 us with the gap to the
     GEMM + 0.45 us per million weights) plus the library GEMM, 3 us + flops / rate with 1 / rate = 1 / cap(M) + 85 / t in s per PFLOP: cap
@@ -399,22 +383,19 @@ def _dense_gemm_us(M: int, N: int, K: int) -> float:
 
 def _fused_gemm_wins(M: int, N: int, K: int, nested: bool = False) -> bool:
     """Is ``nf4hip_gemm`` faster than dequantize + dense GEMM (calls that ``_stream_takes`` leaves)?  Both sides are
-    modelled from measurements on MI355X.  While the streaming kernel serves the call, its launcher's own model stands against
-    what ``nf4hip_linear`` takes behind the dequantize pass, 3-18 % longer than the library GEMM the dense model describes (fused
-    measured / modelled vs dense route, us: M = 1457 [3616, 14528] 203 / 213 vs 183, M = 2957 [2235, 10944] 163 / 169 vs 171, M = 2392
-    [1332, 17344] 141 / 146 vs 186, M = 2691 [664, 9088] 57 / 60 vs 94).  Beyond, the fused kernel
-    runs at 1.0-1.15 PFLOP/s, the library GEMM at up to 1.5, but the dense route first writes the bf16 weight: the
-    two cross near 1024 rows of x wherever the fused kernel has a workgroup for most CUs (fused vs dense, us, M =
-    512 / 1024 / 2048: [14336, 4096] 71 / 117 / 232 vs 84 / 118 / 198; [28672, 4096] 127 / 239 / 473 vs 155 / 238 / 405; [28672, 8192] 226 /
-    442 / 881 vs 291 / 466 / 789; lm_head [128256, 4096] 497 / 978 / 1938 vs 741 / 1099 / 1831; short weights leave the chip
-    empty: [4096, 14336] 164 / 174 / 255 vs 107 / 142 / 216, [4096, 4096] 54 / 58 / 79 vs 42 / 52 / 75).  A tie goes to the fused kernel,
+    modelled from measurements on MI355X, the fused one by its launcher (``nf4hip_gemm_us``).  While the streaming kernel
+    serves the call, that stands against what ``nf4hip_linear`` takes behind the dequantize pass, 3-18 % longer than the
+    library GEMM the dense model describes (fused measured / modelled vs dense route, us: M = 1457 [3616, 14528] 203 / 213 vs 183,
+    M = 2957 [2235, 10944] 163 / 169 vs 171, M = 2392 [1332, 17344] 141 / 146 vs 186, M = 2691 [664, 9088] 57 / 60 vs 94).  Beyond, the
+    fused kernel runs at 1.0-1.15 PFLOP/s, the library GEMM at up to 1.5, but the dense route first writes the bf16 weight: the two
+    cross near 1024 rows of x (fused vs dense, us, M = 1024 / 2048: [14336, 4096] 117 / 232 vs 118 / 198; [28672, 4096] 239 / 473 vs 238 /
+    405; [28672, 8192] 442 / 881 vs 466 / 789; lm_head [128256, 4096] 978 / 1938 vs 1099 / 1831).  A tie goes to the fused kernel,
     which needs no transient bf16 weight."""
     # nested absmax: the fp32 absmax is written out ahead of the fused kernel (_matmul_nf4_on), 2-7 % on top; the
     # dequantize pass of the dense route resolves the codes itself at no measurable cost
-    nested_factor = 1.05 if nested else 1.0
-    if _lib.load().nf4hip_gemm_streamed(M, N, K):
-        return _lib.load().nf4hip_stream_us(M, N, K) * nested_factor <= 1.15 * _dense_gemm_us(M, N, K)
-    return _wide_gemm_us(M, N, K) * nested_factor <= 1.03 * _dense_gemm_us(M, N, K)
+    lib = _lib.load()
+    margin = 1.15 if lib.nf4hip_gemm_streamed(M, N, K) else 1.03
+    return lib.nf4hip_gemm_us(M, N, K) * (1.05 if nested else 1.0) <= margin * _dense_gemm_us(M, N, K)
 
 
 # Many rows of x: the fused GEMM and dequantize + dense GEMM are within a few per cent of each other over a wide range
@@ -500,7 +481,7 @@ def _stream_takes(M: int, N: int, K: int, f16: bool) -> bool:
     if K >= 1 << 24 or N * (K // 64) >= 1 << 31:
         return False
     if f16:
-        return M <= STREAM_MAX_M or (M <= STREAM_F16_MAX_M and bool(_lib.load().nf4hip_gemm_streamed(M, N, K)))
+        return M <= STREAM_MAX_M or (M <= STREAM_F16_MAX_M and bool(_lib.load().nf4hip_stream_served(M, N, K)))
     return 16 < M <= STREAM_MAX_M or 4 < M <= 16 and (K % 512 != 0 or (K > 16384 and N * K >= STREAM_LONG_WEIGHT))
 
 

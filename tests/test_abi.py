@@ -263,7 +263,7 @@ def test_fused_route_rules(ta):
     # that says so is that kernel's own
     for M, N, K in ((129, 1024, 4096), (192, 1024, 4096), (129, 512, 4096), (768, 512, 4096), (129, 2048, 2048), (1536, 2048, 2048), (192, 5003 + 1, 2880)):
         assert F._lib.load().nf4hip_gemm_streamed(M, N, K) and route(M, N, K) == "gemm", (M, N, K)
-        assert F._lib.load().nf4hip_stream_us(M, N, K) < F._dense_gemm_us(M, N, K)
+        assert F._lib.load().nf4hip_gemm_us(M, N, K) < F._dense_gemm_us(M, N, K)
     assert route(1457, 3616, 14528) == "dequant+gemm"  # twelve by fifteen tiles, 70 % of the CUs: the dense route is ahead
     assert route(1, 8192, 28672) == "gemv"               # row-streaming kernel has an exact variant
     assert route(1, 64, 4096, dtype=torch.float32) == "dequant+linear"
@@ -331,10 +331,10 @@ def test_gemm_plan_is_the_launchers_and_agrees_with_the_workspace(ta):
                     assert lib.nf4hip_stream_plan(M, N, K, ctypes.byref(stream)) == 0
                     width = stream[1]
                     assert (rows, pieces, wgs) == (stream[0], stream[2], stream[3]) and rows in (16, 32, 64, 128) and width in (64, 128, 256)
-                    assert need == lib.nf4hip_stream_workspace_bytes(M, N, K) and lib.nf4hip_stream_us(M, N, K) > 5
+                    assert need == lib.nf4hip_stream_workspace_bytes(M, N, K) and lib.nf4hip_gemm_us(M, N, K) > 5
                 else:
                     width = 256
-                    assert rows in (128, 256) and lib.nf4hip_stream_us(M, N, K) == 0
+                    assert rows in (128, 256) and lib.nf4hip_gemm_us(M, N, K) > 12
                 assert tiles == ((M + rows - 1) // rows) * ((N + width - 1) // width) and 1 <= pieces <= 8 and wgs == tiles * pieces
                 if pieces == 1:
                     assert need == 0
@@ -348,6 +348,7 @@ def test_gemm_plan_is_the_launchers_and_agrees_with_the_workspace(ta):
     assert lib.nf4hip_gemm_plan(64, 64, 100, ctypes.byref(plan)) == L.E_SHAPE
     assert lib.nf4hip_gemm_plan(64, 64, 64, None) == L.E_NULL
     assert lib.nf4hip_stream_plan(64, 64, 100, ctypes.byref(plan)) == L.E_SHAPE and lib.nf4hip_stream_plan(64, 64, 64, None) == L.E_NULL
+    assert lib.nf4hip_gemm_us(64, 64, 100) == 0 and lib.nf4hip_gemm_us(0, 64, 64) == 0
 
 
 def test_gemm_insists_on_the_workspace_of_its_plan(ta):

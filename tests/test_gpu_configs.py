@@ -242,7 +242,7 @@ def test_lm_head_router_takes_fused_kernel(ta, oracle, weights, M):
     (256, 1024, 8192, False, 32, 2),
     (1024, 4096, 4096, True, 128, 2),    # nested absmax
     (2048, 4096, 14336, False, 128, 1),
-    (512, 8192, 28672, False, 128, 2),
+    (200, 8192, 28672, False, 128, 4),
     (512, 4096, 14336, False, 128, 4),
     (130, 264, 2048 + 64, False, 32, 1),  # 33 k steps
 ])

@@ -1,6 +1,6 @@
-"""``nf4hip_gemm`` beyond the streaming kernel's 32-bit offsets: rows of K >= 2^24 (the kernel of nf4_gemm_wide.hip with its
-tiles cut along K, pieces that meet in the workspace) and x of 4 GB and more (the general kernel of nf4_gemm.hip), against a
-float64 product over the HIP-dequantised weight."""
+"""``nf4hip_gemm`` on large calls: the kernel of nf4_gemm_wide.hip with its tiles cut along K, pieces that meet in the workspace
+(256-row tiles on long rows, 128-row tiles from K = 2^24 on), and the general kernel of nf4_gemm.hip (x of 4 GB and more), against
+a float64 product over the HIP-dequantised weight."""
 
 import pytest
 import torch
@@ -84,6 +84,35 @@ def test_cut_tiles_at_k_of_2_to_24(ta, M, N, K, nested, bias):
                                        (ta.reconstruct_absmax(stats) if nested else stats)[r * (K // 64):(r + 1) * (K // 64)], code, 64, torch.bfloat16,
                                        (1, K)) for r in rows])
     _check(first[:, rows], x, deq, None if b is None else b[rows], 4096)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,nested,pieces", [(512, 8192, 28672, False, 4), (1249, 4096, 24064, True, 3), (2005, 3236, 20224, False, 2),
+                                                 (986, 4384, 27520 + 64, False, 3)])
+def test_cut_256_row_tiles(ta, M, N, K, nested, pieces):
+    """Ragged M and N, an odd number of k steps (pieces of unequal length); five calls on one workspace give the same bits."""
+    print(f"cut 256-row tiles M={M} [{N},{K}] nested={nested}", flush=True)
+    lib = ta._lib.load()
+    tiles = ((M + 255) // 256) * ((N + 255) // 256)
+    assert not lib.nf4hip_gemm_streamed(M, N, K) and ta.functional._gemm_plan(M, N, K) == (256, tiles, pieces, tiles * pieces)
+    need = lib.nf4hip_gemm_workspace_bytes(M, N, K)
+    assert need == COUNTERS + tiles * pieces * 256 * 256 * 4
+    packed, stats, code = _weight(ta, N, K, nested, M)
+    g = torch.Generator(device=DEV).manual_seed(N)
+    x = torch.empty(M, K, device=DEV).normal_(0, 1, generator=g).to(torch.bfloat16)
+    b = torch.empty(N, device=DEV).normal_(0, 1, generator=g).to(torch.bfloat16)
+    out = torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+    assert _gemm(ta, x, packed, stats, code, b, N, K, out, None, 0) == ta._lib.E_WORKSPACE
+    ws = torch.full((need + 4096,), 0x5A, dtype=torch.uint8, device=DEV)
+    ws[:COUNTERS] = 0
+    first = None
+    for _ in range(5):
+        out.fill_(float("nan"))
+        ta._lib.check(_gemm(ta, x, packed, stats, code, b, N, K, out, ws, need))
+        first = out.clone() if first is None else first
+        assert torch.equal(out, first)
+    assert not ws[:COUNTERS].any() and bool((ws[need:] == 0x5A).all())
+    _check(first, x, ta.dequantize_nf4(packed, stats, code, 64, torch.bfloat16, (N, K)), b, K // 16)
 
 
 @pytest.mark.gpu

@@ -193,8 +193,13 @@ def test_gemm_without_the_workspace(ta, M, N, K, split):
 
 
 def test_gemm_streamed_rule(ta):
-    """Tiles of 128 x 256 fill the chip once at most (half of it with few k steps); beyond 32-bit offsets never."""
-    served = ta._lib.load().nf4hip_gemm_streamed
+    """Tiles of 128 x 256 fill the chip once at most (half of it with few k steps); beyond 32-bit offsets never.  Of these
+    nf4hip_gemm leaves long rows to the other kernel's 256-row tiles in pieces where their models say so."""
+    lib = ta._lib.load()
+    served = lib.nf4hip_stream_served
+    for M, N, K, streamed in ((986, 4384, 27520, 0), (1343, 4864, 26560, 0), (2005, 3236, 20224, 0), (512, 8192, 28672, 0), (315, 8768, 27648, 1),
+                              (2048, 4096, 14336, 1), (512, 4096, 14336, 1), (302, 19800, 12672, 1), (129, 8192, 28672, 1)):
+        assert served(M, N, K) and lib.nf4hip_gemm_streamed(M, N, K) == streamed, (M, N, K)
     assert served(128, 1 << 20, 4096) and served(2048, 4096, 4096) and not served(2049, 4096, 4096) and served(256, 32768, 2048)
     assert not served(257, 32768, 2048) and not served(256, 32768, 1024) and served(256, 16384, 1024) and not served(1 << 18, 64, 8192)
     assert not served(128, 1 << 26, 4096) and not served(0, 64, 64) and not served(8, 64, 96)

@@ -564,11 +564,16 @@ def matmul_nf4(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape) -> 
     return _matmul_nf4_on(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape, route)
 
 
-# nested absmax, fused GEMM: beyond this many rows of x the fp32 absmax is written out first, except where the streaming kernel
-# serves the call, which is 1-5 % longer on nested absmax (measured, us, nested kernel /
-# reconstruct + fp32 kernel / fp32 kernel alone: [8192, 8192] M = 256 64 / 58 / 53, M = 512 107 / 91 / 85, M = 2048 255 / 242 / 235;
-# [28672, 8192] M = 512 242 / 226 / 213, M = 2048 930 / 854 / 837; [8192, 28672] M = 1024 481 / 439 / 425; [1024, 8192] M = 512 38 / 37 / 34)
+# Nested absmax beyond this many rows of x: the fp32 absmax may be written out first (nf4hip_dq_reconstruct, 4 bytes per block into
+# a transient buffer, 2-15 us; same two roundings, same bits).  Always ahead of the kernel of nf4_gemm_wide.hip, which resolves an 8-bit
+# code through two more loads per block and k step (us, nested kernel / reconstruct + fp32 kernel / fp32 kernel alone: [28672, 8192]
+# M = 512 242 / 226 / 213, M = 2048 930 / 854 / 837; [8192, 28672] M = 1024 481 / 439 / 425).  The streaming kernel loads the
+# statistics of four k steps at a time where blocksize is 64 and K a multiple of 256, and hardly at all from blocksize 256 on (M = 320
+# [7040, 11264] 77.5 / 80.5 / 74.2, M = 1403 [4164, 10240] 147.1 / 147.8 / 141.9); in between, per step and lane, which a call has to be
+# long for to pay another launch (K % 256 != 0: M = 2047 [2816, 12352] 205 / 182 / 179, M = 602 [3016, 5056] 41.0 / 38.7 / 32.8, M = 200
+# [1024, 2880] 12.4 / 13.2, M = 140 [600, 1088] 7.6 / 9.6; blocksize 128: M = 1403 [4164, 10240] 163 / 150, M = 200 [4096, 4096] 23.3 / 23.9).
 NESTED_RECONSTRUCT_MIN_M = 128
+NESTED_RECONSTRUCT_MIN_US = 30
 
 
 def _matmul_nf4_on(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape, route: str) -> torch.Tensor:
@@ -613,10 +618,9 @@ def _matmul_nf4_on(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape,
     bptr = None if b is None else b.data_ptr()
     code, x_ptr, out_ptr = _DTYPE_CODE[x.dtype], x2.data_ptr(), out.data_ptr()
     nested = isinstance(absmax, NestedAbsmax)
-    if nested and route == "gemm" and M > NESTED_RECONSTRUCT_MIN_M and not lib.nf4hip_gemm_streamed(M, N, K):
-        # Many rows of x on nested absmax: the fused GEMM resolves an 8-bit code through two more loads per block and
-        # k step and runs 5-27 % longer than on fp32 absmax; writing the fp32 absmax out first (nf4hip_dq_reconstruct,
-        # 4 bytes per block into a transient buffer, 4-15 us) costs 2-7 %.  Same two roundings, same bits.
+    if (nested and route != "gemv" and M > NESTED_RECONSTRUCT_MIN_M
+            and (not (route == "stream" or lib.nf4hip_gemm_streamed(M, N, K))
+                 or ((blocksize == 128 or K % 256) and lib.nf4hip_gemm_us(M, N, K) > NESTED_RECONSTRUCT_MIN_US))):
         absmax, nested = reconstruct_absmax(absmax), False
     if nested:
         q, a2, m256, off, nbs = _nested_args(absmax, nblocks)

@@ -192,6 +192,29 @@ def test_gemm_without_the_workspace(ta, M, N, K, split):
     _check(first, x, deq, None)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,blocksize,written", [(700, 3000, 5056, 64, True), (700, 3000, 5120, 64, False), (700, 3000, 5120, 128, True),
+                                                     (700, 3000, 5120, 256, False), (200, 300, 2880, 64, False), (128, 3000, 5056, 64, False),
+                                                     (512, 8192, 28672, 64, True)])
+def test_nested_absmax_written_out(ta, monkeypatch, M, N, K, blocksize, written):
+    """More than 128 rows of x on nested absmax: the fp32 absmax is written out first where the kernel that serves the call reads
+    the nested form value by value; the bits are those of the kernel on the nested form."""
+    print(f"nested absmax M={M} [{N},{K}] bs={blocksize}", flush=True)
+    F, L, lib = ta.functional, ta._lib, ta._lib.load()
+    qw, nq, code = _weight(ta, N, K, blocksize, True, torch.bfloat16, 9)
+    x = torch.randn(M, K, device=DEV).to(torch.bfloat16)
+    calls, real = [], F.reconstruct_absmax
+    monkeypatch.setattr(F, "reconstruct_absmax", lambda nq: calls.append(1) or real(nq))
+    y = F._matmul_nf4_on(x, qw, None, nq, code, blocksize, torch.bfloat16, (N, K), "gemm")
+    assert bool(calls) == written
+    need = lib.nf4hip_gemm_workspace_bytes(M, N, K)
+    ws = torch.zeros(max(need, 16), dtype=torch.uint8, device=DEV)
+    out = torch.empty_like(y)
+    L.check(lib.nf4hip_gemm_dq(x.data_ptr(), L.BF16, M, qw.data_ptr(), nq.q.data_ptr(), nq.absmax2.data_ptr(), nq.map256.data_ptr(), nq.offset, nq.blocksize,
+                               code.data_ptr(), None, N, K, blocksize, out.data_ptr(), ws.data_ptr(), need, F._stream()))
+    assert torch.equal(out, y)
+
+
 def test_gemm_streamed_rule(ta):
     """Tiles of 128 x 256 fill the chip once at most (half of it with few k steps); beyond 32-bit offsets never.  Of these
     nf4hip_gemm leaves long rows to the other kernel's 256-row tiles in pieces where their models say so."""

@@ -402,14 +402,17 @@ def _fused_gemm_wins(M: int, N: int, K: int, nested: bool = False) -> bool:
 # of shapes, and which one leads moves with the board (clocks under a power limit, the library's GEMM heuristics).  The
 # time models above are the answer where nothing can be measured (on the CPU, under stream capture); otherwise the
 # first call of a shape on a device times both routes once -- a few launches each -- and every later call takes the
-# faster one.  NF4HIP_CALIBRATE=0 switches the measurement off.
+# faster one.  fp16 in the range of the streaming kernel: that kernel against dequantize + the library's GEMM, which no model
+# predicts (it is 2.3 times to 0.86 times as fast from 1000 rows on: M = 1375 [512, 24320] 60 vs 138 us, M = 1388 [4284, 15168] 229 vs 197, M = 1003
+# [4224, 3904] 60 vs 52; below 1000 rows the kernel was ahead on every shape tried, and is the answer where nothing is measured).
+# NF4HIP_CALIBRATE=0 switches the measurement off.
 CALIBRATE_MIN_M = 129
 _route_measured: dict[tuple, str] = {}
 
 
-def _route_key(device: torch.device, M: int, N: int, K: int, blocksize: int, nested: bool, has_bias: bool) -> tuple:
+def _route_key(device: torch.device, M: int, N: int, K: int, blocksize: int, nested: bool, has_bias: bool, f16: bool = False) -> tuple:
     index = device.index if device.index is not None else (torch.cuda.current_device() if device.type == "cuda" else -1)
-    return (device.type, index, M, N, K, blocksize, nested, has_bias)
+    return (device.type, index, M, N, K, blocksize, nested, has_bias, f16)
 
 
 def _calibration_enabled() -> bool:
@@ -427,7 +430,7 @@ def _measure_route(key: tuple, candidates: dict, launches: int = 3) -> str:
     """Time every candidate (a callable per route name) on the current stream: one untimed call, then ``launches``
     calls between two events; remember and return the fastest.  The vendor library's GEMM ("dequant+libgemm") has to
     beat the best hand-written route by more than 3 %; a candidate within 2 % of the best that needs no transient
-    bf16 weight ("gemm") is preferred."""
+    dense weight ("gemm", "stream") is preferred."""
     times = {}
     for name, fn in candidates.items():
         fn()
@@ -442,8 +445,9 @@ def _measure_route(key: tuple, candidates: dict, launches: int = 3) -> str:
     own = {name: t for name, t in times.items() if name != "dequant+libgemm"}
     if best == "dequant+libgemm" and own and min(own.values()) <= 1.03 * times[best]:
         best = min(own, key=own.get)
-    if "gemm" in times and times["gemm"] <= 1.02 * times[best]:
-        best = "gemm"
+    for fused in ("gemm", "stream"):
+        if fused in times and times[fused] <= 1.02 * times[best]:
+            best = fused
     _route_measured[key] = best
     return best
 
@@ -474,9 +478,9 @@ def _stream_takes(M: int, N: int, K: int, f16: bool) -> bool:
     M = 8 / 16 38.7 / 45.0 vs 36.3 / 35.4, nested absmax 45.5 / 51.1 vs 35.4 / 36.3).  Smaller weights stay in the kernel that
     their epilogue forms run in.
     fp16, up to 128 rows: always; the alternative writes the dense weight first ([14336, 4096] M = 4: 47 vs 13).  Up to 2048
-    rows: while the kernel's tiles fill the chip once (M = 256 / 512 / 1024 / 2048 [1024, 4096] 21.0 / 23.6 / 26.8 / 33.2 vs 10.8 / 13.3 /
-    20.8 / 28.5; [4096, 4096] 34.7 / 40.0 / 52.7 / 75.9 vs 20.1 / 27.3 / 50.7 / 72.2; [4096, 14336] 90.6 / 113.9 / 146.8 / 226.1 vs 48.7 / 74.8 /
-    130.2 / 228.4; beyond, nothing was measured).
+    rows, while the kernel's tiles fill the chip once: a candidate, measured against that route per shape (M = 256 / 512 / 1024 / 2048
+    [1024, 4096] 21.0 / 23.6 / 26.8 / 33.2 vs 10.8 / 13.3 / 20.8 / 28.5; [4096, 4096] 34.7 / 40.0 / 52.7 / 75.9 vs 20.1 / 27.3 / 50.7 / 72.2;
+    [4096, 14336] 90.6 / 113.9 / 146.8 / 226.1 vs 48.7 / 74.8 / 130.2 / 228.4; beyond 2048, nothing was).
     Never beyond the kernel's 32-bit offsets into a weight."""
     if K >= 1 << 24 or N * (K // 64) >= 1 << 31:
         return False
@@ -516,7 +520,9 @@ def fused_route(x: torch.Tensor, bias, blocksize: int, dtype: torch.dtype, shape
     if dtype is torch.float16:
         serves = (K % 64 == 0 and K % blocksize == 0 and _stream_takes(M, N, K, True) and _is_plain(x, bias)
                   and (bias is None or bias.shape == (N,)))
-        return "stream" if serves else "dequant+linear"
+        if not serves:
+            return "dequant+linear"
+        return "stream" if M <= STREAM_MAX_M else _route_measured.get(_route_key(x.device, M, N, K, blocksize, nested, bias is not None, True), "stream")
     if dtype is not torch.bfloat16 or (N * K) % 2:
         return "dequant+linear"
     if M <= 4 and _decode_takes(M, K, blocksize):
@@ -550,13 +556,13 @@ def matmul_nf4(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape) -> 
     route = fused_route(x, bias, blocksize, dtype, shape, nested)
     if route == "stream" and dtype is torch.float16 and not _weight_complete(x, qweight, bias, absmax, quant_map, N * K, blocksize):
         route = "dequant+linear"
-    if (route in ("gemm", "dequant+gemm") and x.numel() >= CALIBRATE_MIN_M * K and _calibration_enabled()
+    if (route in ("gemm", "dequant+gemm", "stream") and x.numel() >= CALIBRATE_MIN_M * K and _calibration_enabled()
             and not torch.cuda.is_current_stream_capturing()):
-        M = x.numel() // K
-        key = _route_key(x.device, M, N, K, blocksize, nested, bias is not None)
+        M, f16 = x.numel() // K, route == "stream"  # (bf16 is streamed up to 128 rows only)
+        key = _route_key(x.device, M, N, K, blocksize, nested, bias is not None, f16)
         if key not in _route_measured:
             with _on_device(x.device):
-                names = ["gemm", "dequant+gemm"] + (["dequant+libgemm"] if _library_gemm_allowed() else [])
+                names = ["stream", "dequant+linear"] if f16 else ["gemm", "dequant+gemm"] + (["dequant+libgemm"] if _library_gemm_allowed() else [])
                 route = _measure_route(key, {
                     name: (lambda name=name: _matmul_nf4_on(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape, name))
                     for name in names

@@ -76,6 +76,50 @@ def test_library_gemm_can_be_kept_out_and_needs_a_margin(ta, oracle, monkeypatch
     assert pick({"gemm": 1.10, "dequant+gemm": 1.05, "dequant+libgemm": 1.00}) == "dequant+libgemm"
     assert pick({"gemm": 1.03, "dequant+gemm": 1.02, "dequant+libgemm": 1.00}) == "gemm"
     assert pick({"gemm": 1.00, "dequant+gemm": 1.01}) == "gemm"
+    assert pick({"stream": 1.03, "dequant+linear": 1.00}) == "dequant+linear" and pick({"stream": 1.01, "dequant+linear": 1.00}) == "stream"
+
+
+def test_fp16_prompts_are_measured_against_the_library_route(ta, monkeypatch):
+    """More than 128 rows of fp16 x: the first call of a shape times the streaming kernel against dequantize + linear, later
+    calls follow; what a kernel cannot be handed by address is not timed and takes the torch operation, whatever was measured; up to
+    128 rows nothing is."""
+    print("route calibration: fp16", flush=True)
+    F = ta.functional
+    monkeypatch.setenv("NF4HIP_CALIBRATE", "1")
+    monkeypatch.setattr(F, "_route_measured", {})
+    M, N, K = 1388, 516, 2048
+    hf = torch.float16
+    g = torch.Generator(device=DEV).manual_seed(3)
+    qw, absmax, code = ta.quantize_nf4((torch.randn(N, K, device=DEV, generator=g) * 0.02).to(hf))
+    x = torch.randn(M, K, device=DEV, generator=g).to(hf)
+    ref = x.double() @ ta.dequantize_nf4(qw, absmax, code, 64, hf, (N, K)).double().t()
+    ran = []
+    real = F._matmul_nf4_on
+    monkeypatch.setattr(F, "_matmul_nf4_on", lambda *a: (ran.append(a[-1]), real(*a))[1])
+    call = lambda x: F.matmul_nf4(x, qw, None, absmax, code, 64, hf, (N, K))
+    xg = x.clone().requires_grad_(True)
+    call(xg)
+    assert ran == ["dequant+linear"] and not F._route_measured
+    for few in (1, 128):
+        call(x[:few])
+    assert ran[1:] == ["stream", "stream"] and not F._route_measured
+    ran.clear()
+    y = call(x)
+    key = F._route_key(x.device, M, N, K, 64, False, False, True)
+    picked = F._route_measured[key]
+    assert list(F._route_measured) == [key] and picked in ("stream", "dequant+linear") and ran[-1] == picked
+    assert ran.count("stream") >= 4 and ran.count("dequant+linear") >= 4 and set(ran) == {"stream", "dequant+linear"}
+    torch.testing.assert_close(y.double(), ref, rtol=2e-2, atol=2e-2)
+    for measured in ("stream", "dequant+linear"):
+        F._route_measured[key] = measured
+        ran.clear()
+        call(x), call(xg)
+        assert ran == [measured, "dequant+linear"]
+    monkeypatch.setenv("NF4HIP_CALIBRATE", "0")
+    F._route_measured.clear()
+    ran.clear()
+    call(x)
+    assert ran == ["stream"] and not F._route_measured
 
 
 def test_no_measurement_under_stream_capture_or_when_switched_off(ta, oracle, monkeypatch):

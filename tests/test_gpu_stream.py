@@ -2,6 +2,8 @@
 16 / 32 / 64 / 128, ragged weight rows, one k step, a partial unit of four steps, K split over workgroups -- on fp32 and nested
 absmax and larger blocksizes, against a float64 product over the HIP-dequantised weight."""
 
+import ctypes
+
 import pytest
 import torch
 
@@ -15,6 +17,12 @@ def _weight(ta, N, K, blocksize, nested, dtype, seed):
     w = torch.empty(N, K, device=DEV).normal_(0, 0.02, generator=g).to(dtype)
     qw, absmax, code = ta.quantize_nf4(w, blocksize)
     return qw, (ta.compress_absmax(absmax) if nested else absmax), code
+
+
+def _plan(ta, M, N, K):
+    plan = (ctypes.c_int * 4)()
+    ta._lib.check(ta._lib.load().nf4hip_stream_plan(M, N, K, ctypes.byref(plan)))
+    return tuple(plan)
 
 
 def _check(y, x, deq, bias):
@@ -47,6 +55,67 @@ def test_stream_matches_float64(ta, dtype, M, N, K, blocksize, nested, bias):
     y = run()
     _check(y, x, deq, b)
     assert torch.equal(run(), y)  # the workspace is left as it was found, sums have one order
+
+
+# (M, N, K, rows of x per tile, weight rows per tile, K splits): every tile the kernel is built for, with K a multiple of 256 (four
+# absmax per load where blocksize is 64) and not (a partial unit), with one workgroup per tile and with K split; ragged M and N, and
+# units of K that the k groups share unevenly where more than one group shares them.
+TILES = [
+    (11, 16, 2176, 16, 64, 1), (3, 16, 16960, 16, 64, 6), (4, 16, 2304, 16, 64, 1), (13, 16, 16640, 16, 64, 6),
+    (9, 16765, 1088, 16, 128, 1), (2, 5448, 6208, 16, 128, 5), (1, 16412, 1280, 16, 128, 1), (15, 5656, 6400, 16, 128, 5),
+    (7, 33001, 1088, 16, 256, 1), (5, 17122, 4224, 16, 256, 3), (10, 33001, 1024, 16, 256, 1), (6, 16686, 4352, 16, 256, 3),
+    (19, 16, 2176, 32, 64, 1), (17, 16, 17472, 32, 64, 6), (29, 16, 2304, 32, 64, 1), (19, 16, 16896, 32, 64, 6),
+    (33, 8764, 1088, 32, 128, 1), (1373, 67, 6976, 32, 128, 5), (34, 8332, 1280, 32, 128, 1), (1358, 65, 6912, 32, 128, 5),
+    (31, 33001, 1088, 32, 256, 1), (79, 5517, 4160, 32, 256, 3), (21, 33001, 1024, 32, 256, 1), (71, 6274, 4352, 32, 256, 3),
+    (36, 16940, 1152, 64, 128, 1), (1402, 129, 6976, 64, 128, 5), (35, 17382, 1280, 64, 128, 1), (1382, 134, 6656, 64, 128, 5),
+    (47, 33001, 1088, 64, 256, 1), (1249, 774, 4160, 64, 256, 3), (61, 33001, 1024, 64, 256, 1), (34, 17161, 4352, 64, 256, 3),
+    (101, 33001, 1088, 128, 256, 1), (99, 16972, 2752, 128, 256, 3), (125, 33001, 1024, 128, 256, 1), (851, 2345, 2816, 128, 256, 3),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("nested", [False, True])
+@pytest.mark.parametrize("M,N,K,rows,width,splits", TILES)
+def test_every_tile(ta, dtype, nested, M, N, K, rows, width, splits):
+    print(f"tile {rows}x{width} / {splits}: M={M} [{N},{K}] nested={nested} {dtype}", flush=True)
+    L, lib = ta._lib, ta._lib.load()
+    need = lib.nf4hip_stream_workspace_bytes(M, N, K)
+    assert _plan(ta, M, N, K)[:3] == (rows, width, splits) and (need > 0) == (splits > 1)
+    qw, stats, code = _weight(ta, N, K, 64, nested, dtype, M + N)
+    x = torch.empty(M, K, device=DEV).normal_(0, 1, generator=torch.Generator(device=DEV).manual_seed(K)).to(dtype)
+    b = torch.empty(N, device=DEV).normal_(0, 1, generator=torch.Generator(device=DEV).manual_seed(N)).to(dtype)
+    deq = ta.dequantize_nf4(qw, stats, code, 64, dtype, (N, K))
+    ws = torch.zeros(need + 4096, dtype=torch.uint8, device=DEV)
+    head = (x.data_ptr(), L.F16 if dtype == torch.float16 else L.BF16, M, qw.data_ptr())
+    first = None
+    for _ in range(2):
+        out = torch.full((M + 1, N), float("nan"), dtype=dtype, device=DEV)
+        tail = (code.data_ptr(), b.data_ptr(), N, K, 64, out.data_ptr(), ws.data_ptr() if need else None, need, ta.functional._stream())
+        if nested:
+            L.check(lib.nf4hip_stream_dq(*head, stats.q.data_ptr(), stats.absmax2.data_ptr(), stats.map256.data_ptr(), stats.offset, stats.blocksize, *tail))
+        else:
+            L.check(lib.nf4hip_stream(*head, stats.data_ptr(), *tail))
+        _check(out[:M], x, deq, b)
+        assert out[M].isnan().all() and not ws[:65536 * 4].any() and not ws[need:].any()
+        first = out if first is None else first
+        assert torch.equal(out[:M], first[:M])
+
+
+def test_every_tile_is_listed(ta):
+    """The list above names the tiles the library plans (checked without a GPU), each with and without a split of K, whole and
+    partial units."""
+    seen = set()
+    for M, N, K, rows, width, splits in TILES:
+        assert _plan(ta, M, N, K)[:3] == (rows, width, splits), (M, N, K, _plan(ta, M, N, K))
+        seen.add((rows, width, K % 256 == 0, splits > 1))
+    tiles = [(16, 64), (16, 128), (16, 256), (32, 64), (32, 128), (32, 256), (64, 128), (64, 256), (128, 256)]
+    assert seen == {(*tile, whole, split) for tile in tiles for whole in (False, True) for split in (False, True)}
+    g = torch.Generator().manual_seed(0)
+    for _ in range(2000):  # ... and no other
+        M, N, K = (int(2.0 ** (lo + (hi - lo) * torch.rand(1, generator=g).item())) for lo, hi in ((0, 12), (0, 17), (0, 9)))
+        if ta._lib.load().nf4hip_stream_served(M, N, 64 * K):
+            assert _plan(ta, M, N, 64 * K)[:2] in tiles
 
 
 @pytest.mark.gpu

@@ -407,11 +407,13 @@ def test_gemm_route_tall_weights(ta, oracle, M, N, K, kw, fused_gemm):
     _matmul_case(ta, oracle, M, N, K, seed=M + K, **kw)
 
 
-def test_gemm_recovers_dequantized_weight_bit_exact(ta, oracle, fused_gemm):
-    """x = identity makes every output a single product 1.0 * w: the fused kernel's in-LDS
-    dequantisation must equal nf4hip_dequantize bit for bit."""
-    _sync_print("gemm identity")
-    N, K = 256, 512
+@pytest.mark.parametrize("N,streamed", [(256, 1), (9000, 0)])
+def test_gemm_recovers_dequantized_weight_bit_exact(ta, oracle, fused_gemm, N, streamed):
+    """x = identity makes every output a single product 1.0 * w: the expansion in either fused kernel
+    (nf4_gemm_stream.h, nf4_gemm_wide.hip) must equal nf4hip_dequantize bit for bit."""
+    _sync_print(f"gemm identity N={N}")
+    K = 512
+    assert ta._lib.load().nf4hip_gemm_streamed(K, N, K) == streamed
     w = _weights((N, K), seed=9)
     qw, absmax = oracle.C().quantize(w, 64)
     x = torch.eye(K, dtype=torch.bfloat16)
@@ -420,7 +422,7 @@ def test_gemm_recovers_dequantized_weight_bit_exact(ta, oracle, fused_gemm):
     assert torch.equal(y.cpu().t().contiguous().view(torch.int16), deq.view(torch.int16))
 
 
-def test_gemm_bias_nested_blocksize(ta, oracle, fused_gemm):
+def test_gemm_bias_nested_blocksize(ta, oracle, fused_gemm, monkeypatch):
     _sync_print("gemm bias/nested/blocksize")
     _matmul_case(ta, oracle, 64, 256, 1024, bias=True, seed=1)
     _matmul_case(ta, oracle, 64, 256, 1024, nested=True, seed=2)
@@ -428,6 +430,11 @@ def test_gemm_bias_nested_blocksize(ta, oracle, fused_gemm):
     for K in (64, 128, 192, 256, 320):  # 1..5 k steps: the nested absmax look-ups are staged across steps
         _matmul_case(ta, oracle, 40, 300, K, nested=True, bias=True, seed=4 + K)
         _matmul_case(ta, oracle, 200, 300, K, nested=True, seed=5 + K)
+        assert not ta._lib.load().nf4hip_gemm_streamed(200, 16900, K)  # the same steps in the other kernel, on either form of absmax
+        _matmul_case(ta, oracle, 200, 16900, K, seed=6 + K)
+        with monkeypatch.context() as m:
+            m.setattr(ta.functional, "NESTED_RECONSTRUCT_MIN_M", 1 << 30)
+            _matmul_case(ta, oracle, 200, 16900, K, nested=True, seed=7 + K)
 
 
 @pytest.mark.parametrize("case", ["fp32", "fp16", "fp16_K_not_64", "K_not_64", "n_lt_block"])

@@ -1,5 +1,5 @@
 // Fused NF4 matmul for bf16 or fp16 x of up to 128 rows, and more while the chip is filled once at most, exact weights (the
-// kernel; launcher and rules: nf4_gemm_stream.hip).
+// kernel; launcher, time model and rules: nf4_gemm_stream.hip).
 //
 // Replaces the dequantize_4bit + F.linear route of bitsandbytes.matmul_4bit (MatMul4Bit.forward, reached from
 // thunder/transforms/quantization.py:39) between a decode step and a prompt.  What such a call has to move is the weight,
@@ -20,10 +20,11 @@
 // * One barrier per stage of x.  The WK partial sums of a tile meet in LDS, in a fixed order; with splits they meet in
 //   the workspace (protocol of nf4_common.h), again in a fixed order.
 //
-// What bounds it (counters of its first form and variants with parts taken out, [8192, 28672], M = 16): no unit is busy more than half the time (VALU 37 %, address
-// unit 53 %, LDS 22 %, MFMA 14 %); with two consumer waves per SIMD that meet at a barrier the times of fetch (~12 us),
-// expansion (~12) and multiplication with its LDS reads (~16) add up more than they overlap.  Book (64 KB), code slots
-// (32 KB) and x leave no LDS for more waves.
+// What bounds it (counters, [8192, 28672], M = 16; share of the kernel's cycles): no unit is busy throughout -- address unit 60 % (in 27 % held
+// by the cache), VALU 48 %, LDS 34 %, MFMA 20 %; [14336, 4096], M = 64: 39, 25, 20, 16 %; [4096, 14336], M = 512 (128 x 256 tiles): 44, 36, 38,
+// 47 %.  Two consumer waves per SIMD that meet at a barrier add up the times of fetch (~12 us of the first), expansion (~12) and
+// multiplication with its LDS reads (~16; the parts from variants with the others taken out of an earlier form) more than they overlap
+// them.  Book (64 KB), code slots (32 KB) and x leave no LDS for more waves.  With M <= 16 half of every MFMA and x read is duplicate rows.
 // Measured against what served these calls before (graph replay, cold weights, us): M = 32 [4096, 4096] 18.0 -> 9.7,
 // [14336, 4096] 24.7 -> 14.5, [28672, 4096] 33.2 -> 21.4, lm_head [128256, 4096] 112.7 -> 77.8; M = 64 [4096, 4096] 18.7 -> 14.2,
 // [14336, 4096] 27.3 -> 20.0, lm_head 124.8 -> 98.7; fp16 (dequantize + library GEMM before) [14336, 4096] M = 4 47 -> 13.

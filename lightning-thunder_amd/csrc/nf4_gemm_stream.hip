@@ -36,10 +36,10 @@ bool stream_possible(int64_t M, int64_t N, int64_t K) {
            N * (K / 64) < ((int64_t)1 << 31) && M * K * 2 < ((int64_t)1 << 32);
 }
 
-// More than 128 rows of x: while tiles of 128 x 256 fill the chip once at most.  Measured against the kernel of nf4_gemm_wide.hip
-// (its own tiles and pieces; graph replay, cold weights, us, wide / here), M = 130, 512, 2048: [1024, 4096] 25.4 / 10.6, 26.1 / 13.6,
-// 34.6 / 28.9; [4096, 4096] 28.7 / 18.6, 35.6 / 27.7, 76.8 / 74.1 (256 tiles); [4096, 14336] 52.5 / 41.4, 80.4 / 72.9, 224.5 / 218.3;
-// [14336, 4096] 50.0 / 40.9, 73.4 / 65.8 (224 tiles), 216.6 / 253.6.  Beyond one round that kernel's 256-row tiles expand every
+// More than 128 rows of x: while tiles of 128 x 256 fill the chip once at most.  Measured against the kernel of
+// nf4_gemm_wide.hip (its own tiles and pieces; graph replay, cold weights, us, wide / here), M = 130, 512, 2048: [1024, 4096] 25.4 / 10.6,
+// 26.1 / 13.6, 34.6 / 28.9; [4096, 4096] 28.7 / 18.6, 35.6 / 27.7, 76.8 / 74.1 (256 tiles); [4096, 14336] 52.5 / 41.4, 80.4 / 72.9, 224.5 /
+// 218.3; [14336, 4096] 50.0 / 40.9, 73.4 / 65.8 (224 tiles), 216.6 / 253.6.  Beyond one round that kernel's 256-row tiles expand every
 // weight half as often: [28672, 4096] M = 256 75.1 / 65.3 (224 tiles), M = 384 112.5 / 118.1 (336).  With few k steps and a nearly
 // full chip the two are level ([32000, 1024] M = 130..256, 250 tiles: 25.8, 25.5, 26.7 / 25.8, 26.0, 27.4).
 bool stream_served(int64_t M, int64_t N, int64_t K) {

@@ -245,8 +245,9 @@ int nf4hip_gemm(const void* x, int x_dtype, int64_t M, const uint8_t* packed, co
                 const void* bias_or_null, int64_t N, int64_t K, int blocksize, void* out, void* workspace,
                 size_t workspace_bytes, void* stream);
 /*
- * The same product, wherever nf4hip_stream_served says 1 (at least where nf4hip_gemm_streamed does), for bf16 or fp16 x (then bias and out are fp16 too), every weight rounded to x's type as
- * nf4hip_dequantize rounds it: the kernel between the decode step and the prompt, and for fp16 also at decode shapes.
+ * The same product, wherever nf4hip_stream_served says 1 (at least where nf4hip_gemm_streamed does), for bf16 or fp16 x
+ * (then bias and out are fp16 too), every weight rounded to x's type as nf4hip_dequantize rounds it: the kernel between
+ * the decode step and the prompt, and for fp16 also at decode shapes.
  * K % 64 == 0, blocksize dividing K.  With nf4hip_stream_workspace_bytes(M, N, K) bytes of workspace (rules of nf4hip_gemv's;
  * the kernels may share one) K may be split over workgroups; with less, or NULL, it is not.  Deterministic either way.
  */

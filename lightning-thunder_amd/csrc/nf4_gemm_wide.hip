@@ -151,7 +151,8 @@ __device__ __forceinline__ void expansion_step(Expansion& x, int t, uint32_t d, 
 //     dealt so that every XCD -- workgroup b runs on XCD b % 8 -- owns a contiguous run of them: the x-row tiles
 //     that share a weight tile meet in one L2.
 //   * The remaining `tail_tiles` (fewer than GRID) would leave CUs idle in a last, partial round.  Where a call has no
-//     other tiles (most such calls are nf4_gemm_stream.hip's; those that come here have long rows, K >= 14336), each of them can be cut into `pieces` equal pieces along k (in quanta of `gran` k steps, qpt per tile), one workgroup per
+//     other tiles (most such calls are nf4_gemm_stream.hip's; those that come here have long rows, K >= 14336), each of
+//     them can be cut into `pieces` equal pieces along k (in quanta of `gran` k steps, qpt per tile), one workgroup per
 //     piece, numbered piece-major (all first pieces, then all second pieces, ...).  The pieces of a tile meet in
 //     the workspace (see the kernel).  pieces == 1: whole tiles.
 struct WideSchedule {

@@ -706,6 +706,9 @@ hipError_t allow_lds(K kern, size_t bytes) {
 
 }  // namespace
 
+// (for decode_chain.hip)
+extern "C" int nf4hip_decode_fail(const char* text) { return fail(text); }
+
 extern "C" {
 
 __attribute__((visibility("default"))) const char* nf4hip_decode_last_error(void) { return g_err; }

@@ -172,7 +172,9 @@ class Llama(nn.Module):
         H, Hkv, eps = cfg.n_head, cfg.n_kv_head, cfg.norm_eps
         x = self.wte(idx)[:, 0, :].contiguous()
         if cfg.linear_epilogues and cfg.fused_projections and cfg.gate_up_interleaved and x.shape[0] <= 16:
-            out = self._decode_step_epilogues(x, pos, kcache, vcache)
+            out = self._decode_step_chain(x, pos, kcache, vcache)
+            if out is None:
+                out = self._decode_step_epilogues(x, pos, kcache, vcache)
             if out is not None:
                 return out
         delta = None
@@ -190,6 +192,38 @@ class Llama(nn.Module):
             gate_up = m.gate_up_proj(h) if cfg.fused_projections else torch.cat((m.gate_proj(h), m.up_proj(h)), dim=-1)
             delta = m.down_proj(glue.silu_mul(gate_up, pairs=cfg.fused_projections and cfg.gate_up_interleaved))
         return self.lm_head(glue.add_rmsnorm(x, delta, self.norm_f.weight, eps))
+
+    def _decode_step_chain(self, x, pos, kcache, vcache):
+        """The single-token forward as one kernel: the operator calls of ``_decode_step_epilogues``, on a ``glue.DecodeChain`` in the
+        place of activations, which collects them and launches them together.  Returns None (before anything is launched)
+        unless every linear runs as the 4-bit operator with fp32 absmax, without a bias, at shapes the kernel takes."""
+        from . import glue
+        from .transforms import quantization as Q
+
+        cfg = self.cfg
+        B, d, hd, eps = x.shape[0], cfg.d_model, cfg.head_dim, cfg.norm_eps
+        shape = (cfg.n_layer, B, cfg.n_kv_head, cfg.max_seq, 128)
+        if hd != 128 or tuple(kcache.shape) != shape or tuple(vcache.shape) != shape:
+            return None
+        lins = [l for blk in self.blocks for l in (blk.attn.qkv_proj, blk.attn.o_proj, blk.mlp.gate_up_proj, blk.mlp.down_proj)] + [self.lm_head]
+        shapes = [((cfg.n_head + 2 * cfg.n_kv_head) * hd, d), (cfg.n_head * hd, d), (2 * cfg.d_ff, d), (d, cfg.d_ff)] * cfg.n_layer + [(cfg.vocab, d)]
+        planned = [_planned_nf4(l) for l in lins]
+        if any(a is None or a[1] is not None or a[4] != 64 or a[5] != torch.bfloat16 or tuple(a[6]) != s for a, s in zip(planned, shapes)):
+            return None
+        norms = [w for blk in self.blocks for w in (blk.norm_1.weight, blk.norm_2.weight)] + [self.norm_f.weight]
+        if not glue.decode_chain_takes(x, [(a[0], a[2], a[3]) for a in planned], norms, pos, self.rope_cos, self.rope_sin, kcache, vcache, cfg.n_head,
+                                       cfg.d_ff, cfg.vocab):
+            return None
+        ep = Q.hip_matmul_nf4_epilogue
+        chain = glue.DecodeChain(x, norms[0], eps, pos, self.rope_cos, self.rope_sin, kcache, vcache, cfg.n_head, cfg.n_kv_head)
+        r = xn = ss = chain
+        for i in range(cfg.n_layer):
+            qkv, o, gate_up, down = planned[4 * i: 4 * i + 4]
+            y = chain.attention(ep(xn, *qkv, rowscale=(ss, eps)) if i else chain.linear(*qkv))
+            r, xn, ss = ep(y, *o, resid_norm=(r, norms[2 * i + 1]))
+            h = ep(xn, *gate_up, rowscale=(ss, eps), silu_pairs=True)
+            r, xn, ss = ep(h, *down, resid_norm=(r, norms[2 * i + 2]))
+        return ep(xn, *planned[-1], rowscale=(ss, eps)).launch()
 
     def _decode_step_epilogues(self, x, pos, kcache, vcache):
         """The single-token forward with the neighbours of every linear done in that linear's epilogue

@@ -1,8 +1,10 @@
-"""Decode-step glue: ctypes binding of ``libnf4hip_decode.so`` (C ABI in ``include/nf4hip_decode.h``).
+"""Decode-step glue: ctypes binding of ``libnf4hip_decode.so`` (C ABI in ``include/nf4hip_decode.h`` and
+``include/nf4hip_decode_chain.h``).
 
 Three kernels for the work between the 4-bit linears of a Llama decode step -- residual add +
 RMSNorm, rotary embedding + KV-cache update + grouped-query attention, SiLU(gate) * up -- and a row
-argmax for greedy sampling, used by ``decode.Llama`` / ``decode.greedy_decode`` when ``LlamaConfig.hip_glue`` is set.  The reference leaves this work to its other
+argmax for greedy sampling, used by ``decode.Llama`` / ``decode.greedy_decode`` when ``LlamaConfig.hip_glue`` is set; and
+``decode_chain``, the whole step as one kernel.  The reference leaves this work to its other
 executors (thunder/executors/sdpaex.py, nvFuser / torch.compile fusions); it is not part of the
 bitsandbytes path.  There is no CPU fallback: without the built library these functions raise.
 """
@@ -29,6 +31,12 @@ SYMBOLS = {
     "nf4hip_decode_silu_mul": (_i32, [_vp, _i64, _i64, _vp, _vp]),
     "nf4hip_decode_silu_mul_pairs": (_i32, [_vp, _i64, _i64, _vp, _vp]),
     "nf4hip_decode_argmax": (_i32, [_vp, _i64, _i64, _vp, _vp, _vp]),
+}
+# include/nf4hip_decode_chain.h
+CHAIN_SYMBOLS = {
+    "nf4hip_decode_chain_workspace_bytes": (ctypes.c_size_t, [_i64, _i64, _i64, _i32, _i32, _i64, _i64, _i64]),
+    "nf4hip_decode_chain": (_i32, [_vp, _vp, _vp, _vp, _f32, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _i32, _i64, _i64, _i64, _i32, _vp, _vp,
+                                   ctypes.c_size_t, _vp]),
 }
 
 _lib = None
@@ -59,7 +67,7 @@ def load(path: str | None = None) -> ctypes.CDLL:
                 "There is no CPU fallback."
             )
         lib = ctypes.CDLL(p)
-        for name, (restype, argtypes) in SYMBOLS.items():
+        for name, (restype, argtypes) in {**SYMBOLS, **CHAIN_SYMBOLS}.items():
             fn = getattr(lib, name)
             fn.restype, fn.argtypes = restype, argtypes
         if path is None:
@@ -139,6 +147,91 @@ def silu_mul(gate_up: torch.Tensor, pairs: bool = False) -> torch.Tensor:
     fn = lib.nf4hip_decode_silu_mul_pairs if pairs else lib.nf4hip_decode_silu_mul
     with torch.cuda.device(gate_up.device):
         _check(lib, fn(gate_up.data_ptr(), rows, dff, out.data_ptr(), _stream(gate_up)))
+    return out
+
+
+def decode_chain_takes(x, linears, norms, pos, cos, sin, kcache, vcache, n_head: int, d_ff: int, vocab: int) -> bool:
+    """Would ``decode_chain`` take these operands on their device?  (Everything lies on it, 16-byte aligned, in the types and
+    layouts that the kernel reads, and the library has a plan for the shapes.)"""
+    n_layer, B, Hkv, max_seq, _ = kcache.shape
+    weights = [t for lin in linears for t in lin]
+    if not all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.device == x.device and t.is_contiguous() and t.data_ptr() % 16 == 0
+               for t in [x, cos, sin, kcache, vcache, *norms, *weights]):
+        return False
+    if any(t.dtype != torch.bfloat16 for t in (x, kcache, vcache, *norms)) or any(t.dtype != torch.float32 for lin in linears for t in lin[1:]):
+        return False
+    if not (pos.device == x.device and pos.dtype == torch.int64 and pos.numel() == 1) or any(t.dtype != torch.float32 or t.shape != (max_seq, 128) for t in (cos, sin)):
+        return False
+    with torch.cuda.device(x.device):
+        return load().nf4hip_decode_chain_workspace_bytes(B, n_layer, x.shape[1], n_head, Hkv, d_ff, vocab, max_seq) > 0
+
+
+class DecodeChain:
+    """Stands for every activation of a decode step that runs as one kernel: given as ``x`` to ``hip_matmul_nf4_epilogue`` it
+    takes down the linear and the norm weight behind it and is the result as well; ``launch`` runs the step
+    (``decode_chain``).  The order is the decoder's: per layer QKV, attention, output projection, gate-up, down, then the head."""
+
+    def __init__(self, x, norm_first, eps, pos, cos, sin, kcache, vcache, n_head: int, n_kv_head: int):
+        self.args = (eps, pos, cos, sin, kcache, vcache, n_head, n_kv_head)
+        self.x, self.linears, self.norms, self.shapes = x, [], [norm_first], []
+
+    def linear(self, qweight, bias, absmax, quant_map, blocksize, dtype, shape, rowscale=None, silu_pairs=False, resid_norm=None):
+        if bias is not None or blocksize != 64 or dtype != torch.bfloat16:
+            raise ValueError("a decode chain takes 4-bit bf16 linears in blocks of 64, without a bias")
+        self.linears.append((qweight, absmax, quant_map))
+        self.shapes.append(tuple(shape))
+        if resid_norm is None:
+            return self
+        self.norms.append(resid_norm[1])
+        return self, self, self
+
+    def attention(self, qkv):
+        return self
+
+    def launch(self) -> torch.Tensor:
+        return decode_chain(self.x, self.linears, self.norms, *self.args, self.shapes[3][1], self.shapes[-1][0])
+
+
+def decode_chain(x: torch.Tensor, linears, norms, eps: float, pos: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, kcache: torch.Tensor,
+                 vcache: torch.Tensor, n_head: int, n_kv_head: int, d_ff: int, vocab: int, max_workgroups: int = 0) -> torch.Tensor:
+    """A whole decode step from the embedded tokens ``x`` [B, d] to the logits [B, vocab] (``nf4hip_decode_chain``).
+
+    ``linears``: (qweight, absmax, quant_map) of every layer's QKV, output, gate-up and down projection in that order, then of the
+    output head; ``norms``: the two norm weights of every layer in order, then the final one.  ``kcache`` / ``vcache``
+    [n_layer, B, n_kv_head, max_seq, 128].  Two launches on the current stream; the scratch is this call's own (under
+    capture it belongs to the graph)."""
+    lib = load()
+    _bf16_cuda(x, kcache, vcache, *norms)
+    n_layer, B, Hkv, max_seq, hd = kcache.shape
+    d = x.shape[1]
+    if x.shape != (B, n_head * hd) or vcache.shape != kcache.shape or Hkv != n_kv_head or len(linears) != 4 * n_layer + 1 or len(norms) != 2 * n_layer + 1:
+        raise ValueError(f"{x.shape=} {kcache.shape=} {vcache.shape=}, {len(linears)} linears and {len(norms)} norms do not fit {n_head=} {n_kv_head=}")
+    if not (pos.is_cuda and pos.dtype == torch.int64 and pos.numel() == 1):
+        raise ValueError("pos must be a one-element int64 tensor on the GPU")
+    for t in (cos, sin):
+        if not (t.is_cuda and t.dtype == torch.float32 and t.is_contiguous() and t.shape == (max_seq, hd)):
+            raise ValueError(f"rotary tables must be contiguous fp32 [{max_seq}, {hd}] on the GPU")
+    shapes = [((n_head + 2 * n_kv_head) * hd, d), (d, d), (2 * d_ff, d), (d, d_ff)] * n_layer + [(vocab, d)]
+    for (qweight, absmax, quant_map), (n, k) in zip(linears, shapes):
+        if not (qweight.is_cuda and qweight.is_contiguous() and qweight.numel() * qweight.element_size() >= n * k // 2
+                and absmax.dtype == torch.float32 and absmax.is_contiguous() and absmax.numel() >= n * k // 64
+                and quant_map.dtype == torch.float32 and quant_map.is_contiguous() and quant_map.numel() >= 16):
+            raise ValueError(f"a 4-bit weight does not hold [{n}, {k}] in blocks of 64")
+    for w in norms:
+        if w.numel() != d:
+            raise ValueError(f"norm weight of {w.numel()} elements, expected {d}")
+    layers = []
+    for i in range(n_layer):
+        layers += [t.data_ptr() for lin in linears[4 * i: 4 * i + 4] for t in lin] + [norms[2 * i + 1].data_ptr(), norms[2 * i + 2].data_ptr()]
+    layer_ptrs = (ctypes.c_void_p * len(layers))(*layers)
+    head_ptrs = (ctypes.c_void_p * 3)(*(t.data_ptr() for t in linears[-1]))
+    out = torch.empty((B, vocab), dtype=torch.bfloat16, device=x.device)
+    with torch.cuda.device(x.device):
+        need = lib.nf4hip_decode_chain_workspace_bytes(B, n_layer, d, n_head, n_kv_head, d_ff, vocab, max_seq)
+        ws = torch.empty(max(need, 1), dtype=torch.uint8, device=x.device)
+        _check(lib, lib.nf4hip_decode_chain(x.data_ptr(), layer_ptrs, head_ptrs, norms[0].data_ptr(), float(eps), pos.data_ptr(), cos.data_ptr(),
+                                            sin.data_ptr(), kcache.data_ptr(), vcache.data_ptr(), B, n_layer, d, n_head, n_kv_head, d_ff, vocab, max_seq,
+                                            max_workgroups, out.data_ptr(), ws.data_ptr(), ws.numel(), _stream(x)))
     return out
 
 

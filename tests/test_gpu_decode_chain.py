@@ -1,0 +1,217 @@
+"""The decode step as one kernel (nf4hip_decode_chain): ABI checks without a GPU; on the GPU against the PyTorch step of the same
+quantized model, and bit for bit against itself with fewer workgroups, in a replayed graph and beside other steps."""
+
+import ctypes
+import importlib
+import math
+import os
+import re
+
+import pytest
+import torch
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module")
+def glue():
+    return importlib.import_module("lightning-thunder_amd.glue")
+
+
+@pytest.fixture(scope="module")
+def D():
+    return importlib.import_module("lightning-thunder_amd.decode")
+
+
+def test_symbols_and_argument_errors(glue):
+    text = re.sub(r"/\*.*?\*/", "", open(os.path.join(ROOT, "include", "nf4hip_decode_chain.h")).read(), flags=re.S)
+    declared = sorted(set(re.findall(r"\b(nf4hip_decode_\w+)\s*\(", text)))
+    assert declared == sorted(glue.CHAIN_SYMBOLS)
+    lib = glue.load()
+    need = lib.nf4hip_decode_chain_workspace_bytes
+    assert need(1, 32, 4096, 32, 8, 14336, 128256, 640) > 0 and need(16, 1, 2048, 16, 4, 4096, 32000, 4096) > 0
+    # 17 sequences, head size 64, eight query heads per kv head, K > 4096, d_ff no multiple of 256 or beyond 16384, vocab no multiple of 8
+    for shape in [(17, 2, 4096, 32, 8, 14336, 32000, 640), (1, 2, 2048, 32, 8, 8192, 32000, 640), (1, 2, 4096, 32, 4, 14336, 32000, 640),
+                  (1, 2, 8192, 64, 16, 28672, 32000, 640), (1, 2, 4096, 32, 8, 14400, 32000, 640), (1, 2, 4096, 32, 8, 16640, 32000, 640),
+                  (1, 2, 4096, 32, 8, 14336, 32001, 640), (1, 0, 4096, 32, 8, 14336, 32000, 640)]:
+        assert need(*shape) == 0, shape
+    A = 4096  # non-null, 16-byte aligned fake device address: validation never dereferences
+    err = lambda: lib.nf4hip_decode_last_error().decode()
+
+    def call(layers=(A,) * 14, head=(A,) * 3, x=A, batch=1, ws_bytes=1 << 40):
+        return lib.nf4hip_decode_chain(x, (ctypes.c_void_p * 14)(*layers), (ctypes.c_void_p * 3)(*head), A, 1e-5, A, A, A, A, A, batch, 1, 4096, 32, 8,
+                                       14336, 32000, 640, 0, A, A, ws_bytes, None)
+
+    assert call(x=None) == -1 and "null" in err()
+    assert call(batch=17) == -1 and "not served" in err()
+    assert call(ws_bytes=4096) == -1 and "workspace" in err()
+    assert call(x=A + 2) == -1 and "aligned" in err()
+    assert call(layers=(A,) * 13 + (None,)) == -1 and "null" in err()
+    assert call(head=(A, A + 8, A)) == -1 and "aligned" in err()
+
+
+def _model(D, ta, batch, layers, d, d_ff, vocab, max_seq, seed=1):
+    cfg = D.LlamaConfig(n_layer=layers, d_model=d, n_head=d // 128, n_kv_head=d // 512, d_ff=d_ff, vocab=vocab, max_seq=max_seq,
+                        fused_projections=True, hip_glue=True, gate_up_interleaved=True)
+    model = ta.jit(D.build_llama(cfg, device=DEV, seed=seed), transforms=[ta.BitsAndBytesLinearQuant4bit()])
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    kc, vc = D.new_caches(cfg, batch, DEV)
+    kc.normal_(generator=g)
+    vc.normal_(generator=g)
+    tok = torch.randint(0, vocab, (batch, 1), generator=g, device=DEV)
+    return cfg, model, kc, vc, tok
+
+
+@pytest.fixture
+def chain_calls(glue, monkeypatch):
+    """Counts the calls of glue.decode_chain and caps their workgroups."""
+    calls = {"n": 0, "workgroups": 0}
+    real = glue.decode_chain
+
+    def counted(*args, **kw):
+        calls["n"] += 1
+        return real(*args, max_workgroups=calls["workgroups"], **kw)
+
+    monkeypatch.setattr(glue, "decode_chain", counted)
+    return calls
+
+
+# batch, layers, d_model, d_ff, vocab, max_seq, position: 1, 2 and more rows of x (two ways to operands), one to four K ranges of the down
+# projection (the last of them shorter), parts of K that are not whole, rows that are no whole tile, no cached key, one key, ragged
+# ranges of keys
+SHAPES = [(1, 2, 4096, 14336, 8000, 128, 0), (1, 2, 1024, 2304, 1000, 640, 333), (7, 2, 1024, 4096, 1000, 640, 17), (2, 2, 1024, 2304, 1000, 640, 1), (3, 2, 2048, 5632, 8008, 640, 17), (5, 1, 4096, 16384, 1000, 640, 333),
+          (9, 2, 2048, 4096, 1000, 2048, 2047), (16, 2, 4096, 8448, 8000, 640, 639), (16, 1, 4096, 12288, 1000, 300, 16)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,layers,d,d_ff,vocab,max_seq,p", SHAPES)
+def test_chain_against_the_pytorch_step(D, ta, chain_calls, batch, layers, d, d_ff, vocab, max_seq, p):
+    print(f"chain {batch=} {layers=} {d=} {d_ff=} {vocab=} {max_seq=} {p=}", flush=True)
+    cfg, model, kc, vc, tok = _model(D, ta, batch, layers, d, d_ff, vocab, max_seq)
+    pos = torch.full((1,), p, device=DEV, dtype=torch.long)
+    kr, vr = kc.clone(), vc.clone()
+    with torch.no_grad():
+        out = model(tok, pos, kc, vc)
+        assert chain_calls["n"] == 1
+        cfg.hip_glue = False
+        ref = model(tok, pos, kr, vr)
+    rel = lambda a, b: ((a.float() - b.float()).norm() / b.float().norm()).item()
+    # bf16 activations rounded in another order, layer after layer: 0.012 * sqrt(layers) measured between the forms of the step
+    bound = 0.03 * math.sqrt(layers)
+    assert rel(out, ref) < bound
+    for c, r in ((kc, kr), (vc, vr)):
+        assert rel(c[:, :, :, p], r[:, :, :, p]) < bound
+        c[:, :, :, p] = 0
+        r[:, :, :, p] = 0
+        assert torch.equal(c, r)  # no other row is written
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,p", [(1, 0), (1, 512), (5, 3), (8, 576), (9, 100), (16, 639)])
+def test_same_bits_as_launch_by_launch_at_8b_shapes(D, ta, chain_calls, monkeypatch, batch, p):
+    """Every sum is taken in the order of the kernels that the step of one launch per linear runs there."""
+    print(f"chain bits {batch=} {p=}", flush=True)
+    cfg, model, kc, vc, tok = _model(D, ta, batch, 2, 4096, 14336, 32000, 640)
+    pos = torch.full((1,), p, device=DEV, dtype=torch.long)
+    kr, vr = kc.clone(), vc.clone()
+    with torch.no_grad():
+        out = model(tok, pos, kc, vc)
+        assert chain_calls["n"] == 1
+        monkeypatch.setattr(D.Llama, "_decode_step_chain", lambda *a: None)
+        ref = model(tok, pos, kr, vr)
+    assert chain_calls["n"] == 1
+    assert torch.equal(out, ref) and torch.equal(kc, kr) and torch.equal(vc, vr)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,layers,d,d_ff,p", [(1, 2, 4096, 14336, 300), (1, 2, 2048, 5632, 40), (5, 2, 2048, 5632, 300), (3, 2, 4096, 14336, 300), (16, 1, 4096, 8192, 37), (2, 35, 1024, 2048, 77)])
+def test_fewer_workgroups_same_bits(D, ta, chain_calls, batch, layers, d, d_ff, p):
+    """Tasks are dealt by the shape alone; (35 layers are two launches)."""
+    print(f"chain workgroups {batch=} {layers=} {d=} {d_ff=}", flush=True)
+    cfg, model, kc, vc, tok = _model(D, ta, batch, layers, d, d_ff, 1000, 640)
+    pos = torch.full((1,), p, device=DEV, dtype=torch.long)
+    ref = None
+    for workgroups in (0, 255, 37, 3, 1):
+        chain_calls["workgroups"] = workgroups
+        k, v = kc.clone(), vc.clone()
+        with torch.no_grad():
+            got = (model(tok, pos, k, v), k, v)
+        if ref is None:
+            ref = got
+            assert not ref[0].isnan().any()
+        assert all(torch.equal(a, b) for a, b in zip(got, ref)), workgroups
+    assert chain_calls["n"] == 5
+
+
+@pytest.mark.gpu
+def test_chain_graph_replays_and_streams(D, ta, chain_calls):
+    """Replays with new tokens and positions equal the eager step, with eager steps between them; steps of three models at a time on
+    as many streams give what they give alone."""
+    cfg, model, kc, vc, tok = _model(D, ta, 8, 2, 2048, 5632, 1000, 640)
+    pos = torch.full((1,), 100, device=DEV, dtype=torch.long)
+    ke, ve = kc.clone(), vc.clone()
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.no_grad(), torch.cuda.stream(side):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):  # (no call on this stream before: the step brings its own scratch)
+            out = model(tok, pos, kc, vc)
+    torch.cuda.synchronize()
+    for i in range(12):
+        t = torch.randint(0, 1000, (8, 1), device=DEV)
+        tok.copy_(t)
+        pos.fill_(100 + 7 * i)
+        graph.replay()
+        with torch.no_grad():
+            eager = model(t, torch.full((1,), 100 + 7 * i, device=DEV, dtype=torch.long), ke, ve)
+        assert torch.equal(eager, out) and torch.equal(ke, kc) and torch.equal(ve, vc), i
+
+    models = [_model(D, ta, b, 2, 2048, 5632, 1000, 640, seed=b) for b in (1, 4, 9)]
+    streams = [torch.cuda.Stream() for _ in models]
+    pos.fill_(200)
+    with torch.no_grad():
+        alone = [m(t, pos, k.clone(), v.clone()) for _, m, k, v, t in models]
+        torch.cuda.synchronize()
+        for _ in range(5):
+            got = []
+            for s, (_, m, k, v, t) in zip(streams, models):
+                with torch.cuda.stream(s):
+                    got.append(m(t, pos, k.clone(), v.clone()))
+            torch.cuda.synchronize()
+            assert all(torch.equal(a, b) for a, b in zip(got, alone))
+
+
+@pytest.mark.gpu
+def test_chain_position_outside_the_cache_and_other_routes(D, ta, chain_calls):
+    cfg, model, kc, vc, tok = _model(D, ta, 2, 1, 1024, 2048, 1000, 64)
+    k, v = kc.clone(), vc.clone()
+    with torch.no_grad():
+        for p in (64, -1):
+            model(tok, torch.full((1,), p, device=DEV, dtype=torch.long), k, v)
+    torch.cuda.synchronize()
+    assert torch.equal(k, kc) and torch.equal(v, vc) and chain_calls["n"] == 2
+    # caches in another layout, seventeen sequences: the step of several launches, as before
+    pos = torch.full((1,), 5, device=DEV, dtype=torch.long)
+    apart = torch.zeros((1, 2, 2, 64, 256), device=DEV, dtype=torch.bfloat16)
+    with torch.no_grad(), pytest.raises(ValueError):
+        model(tok, pos, apart[..., :128], apart[..., 128:])
+    kb, vb = D.new_caches(cfg, 17, DEV)
+    with torch.no_grad():
+        assert model(tok[:1].expand(17, 1).contiguous(), pos, kb, vb).shape == (17, 1000)
+    assert chain_calls["n"] == 2
+
+
+@pytest.mark.gpu
+def test_chain_infinities_and_nan(D, ta, chain_calls):
+    """A value of +inf in one sequence's cache stays in that sequence, and a NaN there makes its logits NaN, without a wait that lasts."""
+    cfg, model, kc, vc, tok = _model(D, ta, 4, 2, 1024, 2048, 1000, 64)
+    pos = torch.full((1,), 40, device=DEV, dtype=torch.long)
+    with torch.no_grad():
+        ref = model(tok, pos, kc.clone(), vc.clone())
+        for bad in (float("inf"), float("nan")):
+            v = vc.clone()
+            v[0, 1, 0, 3, 5] = bad
+            out = model(tok, pos, kc.clone(), v)
+            assert out[1].isnan().all()  # (an infinite residual has an infinite rms)
+            assert torch.equal(out[[0, 2, 3]], ref[[0, 2, 3]])

@@ -275,7 +275,7 @@ int nf4hip_dq_compress(const float* absmax, int64_t nblocks, int nested_blocksiz
     if (!aligned16(absmax) || !aligned16(absmax_q) || !aligned16(absmax2) || !aligned4(map256))
         return fail(NF4HIP_E_ALIGN, "nf4hip_dq_compress: absmax / absmax_q / absmax2 not 16-byte aligned or map256 not 4-byte aligned");
     const hipError_t e =
-        nf4::launch_dq_compress(absmax, nblocks, nl, map256, offset, nullptr, absmax_q, absmax2, static_cast<hipStream_t>(stream));
+        nf4::launch_dq_compress(absmax, nblocks, nl, map256, offset, absmax_q, absmax2, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail("nf4hip_dq_compress", e);
     return NF4HIP_OK;
 }

@@ -76,9 +76,8 @@ hipError_t launch_quantize_dq(const void* w, int w_dtype, int64_t n, int block_l
 hipError_t launch_dequantize(const uint8_t* packed, const float* absmax, const NestedAbsmax& nested,
                              const float* lut16, int64_t n, int block_log2, void* out, int out_dtype,
                              hipStream_t stream);
-// offset_ptr: where the offset lies on the device, or NULL: it is `offset`
 hipError_t launch_dq_compress(const float* absmax, int64_t nblocks, int nested_log2, const float* map256,
-                              float offset, const float* offset_ptr, uint8_t* q, float* absmax2, hipStream_t stream);
+                              float offset, uint8_t* q, float* absmax2, hipStream_t stream);
 hipError_t launch_dq_reconstruct(const NestedAbsmax& nested, int64_t nblocks, float* absmax, hipStream_t stream);
 
 // Head of every matmul workspace: the split-K arrival counters (zero between calls).

@@ -25,11 +25,13 @@ namespace {
 //
 // [-1, 1] is cut into 32 cells of width 1/16; adjacent thresholds are at least 0.08 apart, so a cell
 // holds at most one of them, and code = (thresholds below the cell) + (s > the cell's threshold).
-// Lane c of a wave keeps cell c & 31 in two registers and every lane fetches its cell with
-// ds_bpermute: 6 VALU operations per element instead of a 4-level tree of compares and selects.
-// The cell index comes from fma(s, 16, 16) rounded to fp32; a value within rounding distance of a
-// cell boundary may land in the neighbouring cell, which gives the same code because no threshold
-// is closer than 1.6e-3 to a boundary.
+// Both numbers of a cell are one 64-bit LDS word; 32 words are one word per bank, so a wave's reads
+// never conflict.  The cell's byte offset comes out of two additions: fma(s, 0.5, 0.5 - 2^-9) clamped
+// to [0, 1] (NaN and negatives 0), plus 2^15, whose last bit is 2^-8: the low mantissa bits then hold
+// floor(128 s + 128) and the cell is that without its last three bits.  s = 1 may round up into word
+// 32, which is the last cell once more (the words behind it only pad the mask's range).  A value within
+// rounding distance of a cell boundary may land in the neighbouring cell, which gives the same code
+// because no threshold is closer than 1.6e-3 to a boundary.
 __device__ __constant__ const uint32_t CELL_THR[32] = {
     0x7F800000u, 0x7F800000u, 0xBF591CD9u, 0x7F800000u, 0x7F800000u, 0x7F800000u, 0xBF1C5270u, 0x7F800000u,
     0xBEEB8480u, 0x7F800000u, 0xBEADEA76u, 0x7F800000u, 0xBE703CECu, 0xBE0D38BCu, 0x7F800000u, 0xBD3A7871u,
@@ -38,116 +40,137 @@ __device__ __constant__ const uint32_t CELL_THR[32] = {
 __device__ __constant__ const uint32_t CELL_BASE[32] = {0, 0, 0,  1,  1,  1,  1,  2,  2,  3,  3,  4,  4,  5,  6,  6,
                                                         7, 8, 9,  9,  10, 11, 11, 12, 12, 13, 13, 14, 14, 14, 15, 15};
 
-struct CodeCells {
-    uint32_t thr;   // CELL_THR[lane & 31]
-    uint32_t base;  // CELL_BASE[lane & 31]
+constexpr int CODE_CELLS = 64;
+
+// Appends the code of s to the codes in `word`.
+__device__ __forceinline__ uint32_t append_code(uint32_t word, float s, const uint2* cells) {
+    const float u = __builtin_amdgcn_fmed3f(__builtin_fmaf(s, 0.5f, 0.5f - 0x1p-9f), 0.0f, 1.0f) + 0x1p15f;
+    const uint2 cell = cells[(__float_as_uint(u) >> 3) & (CODE_CELLS - 1)];
+    return (word << 4) + cell.y + (s > __uint_as_float(cell.x) ? 1u : 0u);
+}
+
+// 8 elements as they lie in memory
+template <int DTYPE>
+struct Raw8 {
+    uint32_t d[DTYPE == F32 ? 8 : 4];
 };
 
-__device__ __forceinline__ uint32_t nf4_code(float s, const CodeCells& cc) {
-    // NaN and negatives convert to 0, values above 31 are clamped
-    const uint32_t cell = min((uint32_t)__builtin_fmaf(s, 16.0f, 16.0f), 31u);
-    const float t = __uint_as_float((uint32_t)__builtin_amdgcn_ds_bpermute((int)(cell << 2), (int)cc.thr));
-    const uint32_t b = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(cell << 2), (int)cc.base);
-    return b + (s > t ? 1u : 0u);
-}
-
-__device__ __forceinline__ float load_elem(const void* w, int dtype, int64_t i) {
-    if (dtype == BF16) return bf16_bits_to_f32(reinterpret_cast<const uint16_t*>(w)[i]);
-    if (dtype == F16) return __half2float(reinterpret_cast<const __half*>(w)[i]);
-    return reinterpret_cast<const float*>(w)[i];
-}
-
-// Load the 8 elements [e0, e0+8) as fp32; elements at or beyond n read as 0.
-__device__ __forceinline__ void load8(const void* w, int dtype, int64_t e0, int64_t n, float v[8]) {
-    if (e0 + 8 <= n) {
-        if (dtype == F32) {
-            const float4 a = reinterpret_cast<const float4*>(w)[e0 / 4];
-            const float4 b = reinterpret_cast<const float4*>(w)[e0 / 4 + 1];
-            v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
-            v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-        } else {
-            const uint4 q = reinterpret_cast<const uint4*>(w)[e0 / 8];
-            const uint32_t d[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                if (dtype == BF16) {
-                    v[2 * j] = __uint_as_float(d[j] << 16);
-                    v[2 * j + 1] = __uint_as_float(d[j] & 0xffff0000u);
-                } else {
-                    v[2 * j] = __half2float(__ushort_as_half((unsigned short)(d[j] & 0xffffu)));
-                    v[2 * j + 1] = __half2float(__ushort_as_half((unsigned short)(d[j] >> 16)));
-                }
-            }
-        }
-    } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = (e0 + j < n) ? load_elem(w, dtype, e0 + j) : 0.0f;
+template <int DTYPE>
+__device__ __forceinline__ Raw8<DTYPE> load8(const void* w, int64_t e0) {
+    Raw8<DTYPE> r;
+    const uint4 a = load16_stream(static_cast<const char*>(w) + e0 * (DTYPE == F32 ? 4 : 2));
+    r.d[0] = a.x; r.d[1] = a.y; r.d[2] = a.z; r.d[3] = a.w;
+    if (DTYPE == F32) {
+        const uint4 b = load16_stream(static_cast<const float*>(w) + e0 + 4);
+        r.d[4] = b.x; r.d[5] = b.y; r.d[6] = b.z; r.d[7] = b.w;
     }
+    return r;
+}
+
+// the same where the array may end inside: elements at or beyond n read as 0
+template <int DTYPE>
+__device__ __forceinline__ Raw8<DTYPE> load8_edge(const void* w, int64_t e0, int64_t n) {
+    if (e0 + 8 <= n) return load8<DTYPE>(w, e0);
+    Raw8<DTYPE> r = {};
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        if (e0 + j >= n) continue;
+        if (DTYPE == F32)
+            r.d[j] = static_cast<const uint32_t*>(w)[e0 + j];
+        else
+            r.d[j / 2] |= (uint32_t)static_cast<const uint16_t*>(w)[e0 + j] << (16 * (j & 1));
+    }
+    return r;
+}
+
+template <int DTYPE>
+__device__ __forceinline__ float element(const Raw8<DTYPE>& r, int j) {
+    if (DTYPE == F32) return __uint_as_float(r.d[j]);
+    if (DTYPE == BF16) return __uint_as_float(j & 1 ? r.d[j / 2] & 0xffff0000u : r.d[j / 2] << 16);
+    return __half2float(__ushort_as_half((unsigned short)(r.d[j / 2] >> (16 * (j & 1)))));
+}
+
+template <int CTRL>
+__device__ __forceinline__ float max_dpp(float m) {
+    return fmaxf(m, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(m), CTRL, 0xf, 0xf, true)));
+}
+
+// Maximum over `lanes` (a power of two, 64 at most) adjacent lanes: within 16 by DPP, an operand modifier of the maximum
+// itself, where a shuffle is an LDS round trip.
+__device__ __forceinline__ float group_max(float m, int lanes) {
+    if (lanes > 1) m = max_dpp<0xB1>(m);   // quad_perm [1, 0, 3, 2]
+    if (lanes > 2) m = max_dpp<0x4E>(m);   // quad_perm [2, 3, 0, 1]
+    if (lanes > 4) m = max_dpp<0x141>(m);  // row_half_mirror
+    if (lanes > 8) m = max_dpp<0x140>(m);  // row_mirror
+    for (int off = 16; off < lanes; off <<= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
+    return m;
 }
 
 // A workgroup covers Q_SLOTS consecutive spans of THREADS * 8 elements (a span holds whole
-// quantisation blocks); a thread owns 8 consecutive elements of each span.  The loads of all spans
-// are in flight before the first reduction.
+// quantisation blocks); a thread owns 8 consecutive elements of each span.
+//
+// Bound by HBM (the weight read once, a quarter of it written) once the loads of all spans are in flight before the first
+// is used: they are taken as raw words, behind one branch for the whole workgroup, and converted afterwards.  With the
+// bounds check and the conversion around each load a span waited for the one before it, and with the cells fetched by
+// two ds_bpermute each span's arithmetic came on top: [28672, 8192] bf16 took
+// 117-128 us, now 97 (602 MB: 6.2 TB/s).
+// Spans per workgroup (same shape): 1 / 2 / 4 / 8 took 110 / 97 / 92-96 / 101 us.
 constexpr int Q_SLOTS = 4;
 
-template <int THREADS>
-__global__ __launch_bounds__(THREADS) void quantize_kernel(const void* __restrict__ w, int dtype, int64_t n,
-                                                           int block_log2, uint8_t* __restrict__ packed,
-                                                           float* __restrict__ absmax) {
+template <int THREADS, int DTYPE>
+__global__ __launch_bounds__(THREADS) void quantize_kernel(const void* __restrict__ w, int64_t n, int block_log2,
+                                                           uint8_t* __restrict__ packed, float* __restrict__ absmax) {
     __shared__ float wave_max[Q_SLOTS][THREADS / 64];
+    __shared__ uint2 cells[CODE_CELLS];
     const int tid = threadIdx.x;
     const int group = 1 << (block_log2 - 3);  // lanes per quantisation block
-    const CodeCells cc = {CELL_THR[tid & 31], CELL_BASE[tid & 31]};
-    float v[Q_SLOTS][8];
-    float m[Q_SLOTS];
+    const int64_t first = (int64_t)blockIdx.x * (Q_SLOTS * THREADS * 8) + tid * 8;
+    const bool whole = ((int64_t)blockIdx.x + 1) * (Q_SLOTS * THREADS * 8) <= n;
+    Raw8<DTYPE> raw[Q_SLOTS];
+    if (whole) {
+#pragma unroll
+        for (int c = 0; c < Q_SLOTS; ++c) raw[c] = load8<DTYPE>(w, first + c * (THREADS * 8));
+    } else {
+#pragma unroll
+        for (int c = 0; c < Q_SLOTS; ++c) raw[c] = load8_edge<DTYPE>(w, first + c * (THREADS * 8), n);
+    }
+    if (tid < CODE_CELLS)
+        cells[tid] = tid < 32 ? make_uint2(CELL_THR[tid], CELL_BASE[tid]) : make_uint2(0x7F800000u, 15u);
+    __syncthreads();
 #pragma unroll
     for (int c = 0; c < Q_SLOTS; ++c) {
-        const int64_t e0 = (((int64_t)blockIdx.x * Q_SLOTS + c) * THREADS + tid) * 8;
-        load8(w, dtype, e0, n, v[c]);
-    }
-    const int in_wave = group < 64 ? group : 64;
+        float v[8];
 #pragma unroll
-    for (int c = 0; c < Q_SLOTS; ++c) {
-        float mm = 0.0f;
+        for (int j = 0; j < 8; ++j) v[j] = element<DTYPE>(raw[c], j);
+        float m = 0.0f;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) mm = fmaxf(mm, fabsf(v[c][j]));
-        // max over the lanes of one quantisation block
-        for (int off = 1; off < in_wave; off <<= 1) mm = fmaxf(mm, __shfl_xor(mm, off, 64));
-        m[c] = mm;
-    }
-    if (group > 64) {  // uniform branch: blocks of 1024, 2048 or 4096 elements span several waves
-#pragma unroll
-        for (int c = 0; c < Q_SLOTS; ++c)
-            if ((tid & 63) == 0) wave_max[c][tid >> 6] = m[c];
-        __syncthreads();
-        const int waves = group >> 6;
-        const int first = (tid >> 6) & ~(waves - 1);
-#pragma unroll
-        for (int c = 0; c < Q_SLOTS; ++c)
-            for (int j = 0; j < waves; ++j) m[c] = fmaxf(m[c], wave_max[c][first + j]);
-    }
-#pragma unroll
-    for (int c = 0; c < Q_SLOTS; ++c) {
-        const int64_t e0 = (((int64_t)blockIdx.x * Q_SLOTS + c) * THREADS + tid) * 8;
-        // every lane computes its codes (the cell lookup reads other lanes' registers, so no lane
-        // may drop out before it); lanes past the end hold zeros and store nothing
-        const float inv = __fdiv_rn(1.0f, m[c]);
+        for (int j = 0; j < 8; ++j) m = fmaxf(m, fabsf(v[j]));
+        m = group_max(m, group < 64 ? group : 64);
+        if (group > 64) {  // uniform branch: blocks of 1024, 2048 or 4096 elements span several waves
+            if ((tid & 63) == 0) wave_max[c][tid >> 6] = m;
+            __syncthreads();
+            const int waves = group >> 6;
+            const int w0 = (tid >> 6) & ~(waves - 1);
+            for (int j = 0; j < waves; ++j) m = fmaxf(m, wave_max[c][w0 + j]);
+        }
+        const float inv = __fdiv_rn(1.0f, m);
         uint32_t word = 0;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t hi = nf4_code(__fmul_rn(v[c][2 * j], inv), cc);
-            const uint32_t lo = nf4_code(__fmul_rn(v[c][2 * j + 1], inv), cc);
-            word |= ((hi << 4) | lo) << (8 * j);
+        for (int j = 3; j >= 0; --j) {  // byte j: element 2j in the high half
+            word = append_code(word, __fmul_rn(v[2 * j], inv), cells);
+            word = append_code(word, __fmul_rn(v[2 * j + 1], inv), cells);
         }
-        if (e0 >= n) continue;
-        if ((tid & (group - 1)) == 0) absmax[e0 >> block_log2] = m[c];
-        if (e0 + 8 <= n) {
-            reinterpret_cast<uint32_t*>(packed)[e0 / 8] = word;
-        } else {
-            const int64_t nbytes = (n + 1) / 2;
+        const int64_t e0 = first + c * (THREADS * 8);
+        if (whole || e0 < n) {
+            if ((tid & (group - 1)) == 0) absmax[e0 >> block_log2] = m;
+            if (whole || e0 + 8 <= n) {
+                reinterpret_cast<uint32_t*>(packed)[e0 / 8] = word;
+            } else {
+                const int64_t nbytes = (n + 1) / 2;
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                if (e0 / 2 + j < nbytes) packed[e0 / 2 + j] = (uint8_t)(word >> (8 * j));
+                for (int j = 0; j < 4; ++j)
+                    if (e0 / 2 + j < nbytes) packed[e0 / 2 + j] = (uint8_t)(word >> (8 * j));
+            }
         }
     }
 }
@@ -241,23 +264,35 @@ __global__ __launch_bounds__(256) void dequantize_kernel(const uint8_t* __restri
 }
 
 // offset = mean of absmax, float64 sum rounded to fp32 once: up to DQ_SUMS workgroups add a contiguous range each (absmax
-// was just written and comes from the caches), one adds their sums.  The second kernel also writes the two tables a
-// double-quantised weight carries (NULL: not wanted), which saves their copies a launch each.  [28672, 8192]: 11 us for
-// both; the same sum taken inside the quantize kernel made that kernel 16-25 us longer (float64 registers).
+// was just written and comes from the caches), and whoever needs the offset adds their sums (dq_offset below).  A thread
+// adds its values in the order in which they lie; full rounds of 1024 values are loaded DQ_ROUNDS at a time.
+// [28672, 8192]: 5.3 us; loaded a round at a time, with a second kernel for the offset, 11.  The same sum taken inside the quantize kernel made that kernel 16-25 us longer (float64
+// registers).
+constexpr int DQ_ROUNDS = 8;
+
 __global__ __launch_bounds__(256) void dq_sum_kernel(const float* __restrict__ absmax, int64_t nblocks, int64_t per,
                                                      double* __restrict__ sums) {
     __shared__ double wave_sum[4];
     const int tid = threadIdx.x;
     const int64_t first = (int64_t)blockIdx.x * per, last = min(first + per, nblocks);
+    const int rounds = (int)((last - first) / 1024);
     double t = 0.0;
-#pragma unroll 4
-    for (int64_t i = first + tid * 4; i < last; i += 1024) {
-        if (i + 4 <= last) {
-            const float4 f = *reinterpret_cast<const float4*>(absmax + i);
-            t += ((double)f.x + (double)f.y) + ((double)f.z + (double)f.w);
-        } else {
-            for (int64_t k = i; k < last; ++k) t += (double)absmax[k];
-        }
+    const float4* p = reinterpret_cast<const float4*>(absmax + first) + tid;
+    for (int r = 0; r < rounds; r += DQ_ROUNDS) {
+        float4 f[DQ_ROUNDS];
+#pragma unroll
+        for (int c = 0; c < DQ_ROUNDS; ++c)
+            if (r + c < rounds) f[c] = p[(r + c) * 256];
+#pragma unroll
+        for (int c = 0; c < DQ_ROUNDS; ++c)
+            if (r + c < rounds) t += ((double)f[c].x + (double)f[c].y) + ((double)f[c].z + (double)f[c].w);
+    }
+    const int64_t i = first + (int64_t)rounds * 1024 + tid * 4;
+    if (i + 4 <= last) {
+        const float4 f = *reinterpret_cast<const float4*>(absmax + i);
+        t += ((double)f.x + (double)f.y) + ((double)f.z + (double)f.w);
+    } else {
+        for (int64_t k = i; k < last; ++k) t += (double)absmax[k];
     }
     for (int off = 1; off < 64; off <<= 1) t += __shfl_xor(t, off, 64);
     if ((tid & 63) == 0) wave_sum[tid >> 6] = t;
@@ -268,21 +303,39 @@ __global__ __launch_bounds__(256) void dq_sum_kernel(const float* __restrict__ a
 __device__ __constant__ const uint32_t NF4_CODE_BITS[16] = {
     0xBF800000u, 0xBF3239B1u, 0xBF066B30u, 0xBECA32A0u, 0xBE91A24Du, 0xBE3D353Fu, 0xBDBA7871u, 0x00000000u,
     0x3DA2FAFFu, 0x3E24CAE3u, 0x3E7C04DDu, 0x3EAD033Au, 0x3EE1A4B8u, 0x3F1007ABu, 0x3F3913B3u, 0x3F800000u};
-__global__ __launch_bounds__(DQ_SUMS) void dq_offset_kernel(const double* __restrict__ sums, int count, int64_t nblocks,
-                                                            float* __restrict__ offset, const float* __restrict__ map256,
-                                                            float* __restrict__ map_out, float* __restrict__ code_out) {
-    __shared__ double wave_sum[DQ_SUMS / 64];
+// What the offset of a compressed absmax comes from and where it and the two tables that a double-quantised weight
+// carries go (the tables NULL: not wanted).  `sums` NULL: the offset is `value` and nothing is written.
+struct DqOffset {
+    const double* sums;
+    float* out;
+    float* map_out;
+    float* code_out;
+    int count;
+    float value;
+};
+
+// Adds the workgroups' sums, in the same order in every workgroup: butterflies over 64 of them, then those one by one.
+template <int THREADS>
+__device__ __forceinline__ void dq_wave_sums(const DqOffset& o, double* wave_sum) {
     const int tid = threadIdx.x;
-    double t = tid < count ? sums[tid] : 0.0;
-    if (map_out && tid < 256) map_out[tid] = map256[tid];
-    if (code_out && tid < 16) code_out[tid] = __uint_as_float(NF4_CODE_BITS[tid]);
-    for (int off = 1; off < 64; off <<= 1) t += __shfl_xor(t, off, 64);
-    if ((tid & 63) == 0) wave_sum[tid >> 6] = t;
-    __syncthreads();
-    if (tid == 0) {
-        for (int j = 1; j < DQ_SUMS / 64; ++j) t += wave_sum[j];
-        *offset = (float)(t / (double)nblocks);
-    }
+    if (tid >= DQ_SUMS) return;
+    constexpr int EACH = THREADS < DQ_SUMS ? DQ_SUMS / THREADS : 1;
+    double t[EACH];
+#pragma unroll
+    for (int i = 0; i < EACH; ++i) t[i] = tid + i * THREADS < o.count ? o.sums[tid + i * THREADS] : 0.0;
+    for (int off = 1; off < 64; off <<= 1)
+#pragma unroll
+        for (int i = 0; i < EACH; ++i) t[i] += __shfl_xor(t[i], off, 64);
+#pragma unroll
+    for (int i = 0; i < EACH; ++i)
+        if ((tid & 63) == 0) wave_sum[(tid + i * THREADS) >> 6] = t[i];
+}
+
+__device__ __forceinline__ float dq_offset(const double* wave_sum, int64_t nblocks) {
+    double t = wave_sum[0];
+#pragma unroll
+    for (int j = 1; j < DQ_SUMS / 64; ++j) t += wave_sum[j];
+    return (float)(t / (double)nblocks);
 }
 
 // r = absmax - offset; absmax2 = max|r| over a nested block; then the nearest entry of the 256-entry map (lowest index on
@@ -292,95 +345,167 @@ __global__ __launch_bounds__(DQ_SUMS) void dq_offset_kernel(const double* __rest
 // The nearest entry of an ascending map is found by bisection: rounded distances fl(s - map[j]) fall towards s from
 // either side (rounding is monotonic), so the minimum lies at the last entry <= s or the first one > s.  Equal rounded
 // distances are settled as the scan over all entries would: the left candidate wins a tie, and from there the index
-// goes down while the distance stays the same.  A map that is not ascending and finite takes that scan.  Bisection: 9
-// LDS reads per value instead of 256 reads, subtractions and compares; [28672, 8192] (3.7 M values) 93 us before, now 14.
+// goes down while the distance stays the same.  A map that is not ascending and finite takes that scan.  The
+// bisection walks a tree in level order (node n's children are 2n and 2n + 1), in which a level's entries lie side by
+// side: the upper seven levels read without bank conflicts, and a step is a compare, an add with its carry and a shift.
+// 11 LDS reads per value instead of 256 reads, subtractions and compares (93 us for the 3.7 M values of [28672, 8192]).
+//
+// The offset is added up by every workgroup itself from the DQ_SUMS partial sums (4 KB from a cache), which saves a launch
+// between the sums and this kernel; the first workgroup writes it and the tables out.  DQ_SPANS spans of THREADS * 4
+// values per workgroup, so that the map, its check and the offset are paid once for all of them and the values' loads are
+// in flight meanwhile, and the searches of DQ_SPANS * 4 values go down their tree together: [28672, 8192] 14 us (15.6 with
+// four spans); [4096, 4096] 6 us, where a search after the other took 8.6.
+constexpr int DQ_SPANS = 2;
+
 template <int THREADS>
 __global__ __launch_bounds__(THREADS) void dq_compress_kernel(const float* __restrict__ absmax, int64_t nblocks,
                                                               int nested_log2, const float* __restrict__ map256,
-                                                              float offset_value, const float* __restrict__ offset_ptr,
-                                                              uint8_t* __restrict__ q, float* __restrict__ absmax2) {
+                                                              DqOffset o, uint8_t* __restrict__ q,
+                                                              float* __restrict__ absmax2) {
     __shared__ float map[256];
-    __shared__ float wave_max[THREADS / 64];
-    __shared__ int zero_code;
+    __shared__ float tree[256];
+    __shared__ float wave_max[DQ_SPANS][THREADS / 64];
+    __shared__ double wave_sum[DQ_SUMS / 64];
+    __shared__ int wave_zero[4], wave_rising[4];
     const int tid = threadIdx.x;
-    const int64_t i0 = ((int64_t)blockIdx.x * THREADS + tid) * 4;
-    float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (i0 + 4 <= nblocks) {
-        const float4 f = *reinterpret_cast<const float4*>(absmax + i0);
-        v[0] = f.x; v[1] = f.y; v[2] = f.z; v[3] = f.w;
+    const int64_t first = ((int64_t)blockIdx.x * (DQ_SPANS * THREADS) + tid) * 4;
+    float v[DQ_SPANS][4];
+    if (((int64_t)blockIdx.x + 1) * (DQ_SPANS * THREADS * 4) <= nblocks) {
+#pragma unroll
+        for (int c = 0; c < DQ_SPANS; ++c) {
+            const float4 f = *reinterpret_cast<const float4*>(absmax + first + c * (THREADS * 4));
+            v[c][0] = f.x; v[c][1] = f.y; v[c][2] = f.z; v[c][3] = f.w;
+        }
     } else {
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
-            if (i0 + c < nblocks) v[c] = absmax[i0 + c];
-    }
-    const float offset = offset_ptr ? *offset_ptr : offset_value;
-    if (tid < 256) map[tid] = map256[tid];
-    if (tid == 0) zero_code = 256;  // sentinel: the map holds no 0.0 (then an all-zero block stores code 0)
-    __syncthreads();
-    if (tid < 256 && map[tid] == 0.0f) atomicMin(&zero_code, tid);
-    const bool ascending =
-        __syncthreads_and(tid >= 255 ? isfinite(map[0]) && isfinite(map[255]) : map[tid] <= map[tid + 1]);
-
-    float m = 0.0f;
+        for (int c = 0; c < DQ_SPANS; ++c)
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        v[c] = __fsub_rn(v[c], offset);
-        if (i0 + c < nblocks) m = fmaxf(m, fabsf(v[c]));
-    }
-    const int group = 1 << (nested_log2 - 2);  // lanes per nested block
-    for (int off = 1; off < (group < 64 ? group : 64); off <<= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
-    if (group > 64) {  // uniform branch: the nested block spans several waves
-        if ((tid & 63) == 0) wave_max[tid >> 6] = m;
-        __syncthreads();
-        const int waves = group >> 6, first = (tid >> 6) & ~(waves - 1);
-        for (int j = 0; j < waves; ++j) m = fmaxf(m, wave_max[first + j]);
-    }
-    if (i0 >= nblocks) return;
-    if ((tid & (group - 1)) == 0) absmax2[i0 >> nested_log2] = m;
-
-    const float inv = __fdiv_rn(1.0f, m);
-    uint32_t code[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        const float s = __fmul_rn(v[c], inv);
-        if (m == 0.0f) {
-            code[c] = zero_code == 256 ? 0 : zero_code;
-        } else if (!isfinite(s)) {
-            code[c] = 0;  // no distance is below infinity
-        } else if (ascending) {
-            int pos = 0;  // entries <= s (255 at most)
-#pragma unroll
-            for (int step = 128; step; step >>= 1)
-                if (map[pos + step - 1] <= s) pos += step;
-            const float right = fabsf(__fsub_rn(s, map[pos]));
-            int best = pos;
-            if (pos > 0) {
-                const float left = fabsf(__fsub_rn(s, map[pos - 1]));
-                if (left <= right) {
-                    best = pos - 1;
-                    while (best > 0 && fabsf(__fsub_rn(s, map[best - 1])) == left) --best;
-                }
+            for (int k = 0; k < 4; ++k) {
+                const int64_t i = first + c * (THREADS * 4) + k;
+                v[c][k] = i < nblocks ? absmax[i] : 0.0f;
             }
-            code[c] = best;
-        } else {
-            float bestd = INFINITY;
-            int best = 0;
-            for (int j = 0; j < 256; ++j) {
-                const float d = fabsf(__fsub_rn(s, map[j]));
-                if (d < bestd) {
-                    bestd = d;
-                    best = j;
-                }
-            }
-            code[c] = best;
+    }
+    if (tid < 256) {  // whole waves
+        const int node = max(tid, 1);  // node n of level l is entry (2 (n - 2^l) + 1) 2^(7 - l) - 1
+        const float entry = map256[tid], next = map256[min(tid + 1, 255)];
+        tree[tid] = map256[((2 * node + 1) << (7 - (31 - __clz(node)))) - 257];
+        map[tid] = entry;
+        const uint64_t zeros = __ballot(entry == 0.0f);
+        const bool rising = entry <= next && (isfinite(entry) || (tid != 0 && tid != 255));
+        const bool all_rising = __ballot(rising) == ~0ull;
+        if ((tid & 63) == 0) {
+            wave_zero[tid >> 6] = zeros ? tid + __ffsll((unsigned long long)zeros) - 1 : 256;
+            wave_rising[tid >> 6] = all_rising;
         }
     }
-    if (i0 + 4 <= nblocks) {
-        *reinterpret_cast<uint32_t*>(q + i0) = code[0] | (code[1] << 8) | (code[2] << 16) | (code[3] << 24);
+    if (o.sums) dq_wave_sums<THREADS>(o, wave_sum);
+    __syncthreads();
+    const bool ascending = wave_rising[0] & wave_rising[1] & wave_rising[2] & wave_rising[3];
+    // the map may hold no 0.0: then an all-zero block stores code 0
+    const int first_zero = min(min(wave_zero[0], wave_zero[1]), min(wave_zero[2], wave_zero[3]));
+    const int zero = first_zero == 256 ? 0 : first_zero;
+    const float offset = o.sums ? dq_offset(wave_sum, nblocks) : o.value;
+    if (o.sums && blockIdx.x == 0) {
+        if (tid == 0) *o.out = offset;
+        if (o.map_out && tid < 256) o.map_out[tid] = map[tid];
+        if (o.code_out && tid < 16) o.code_out[tid] = __uint_as_float(NF4_CODE_BITS[tid]);
+    }
+
+    const int group = 1 << (nested_log2 - 2);  // lanes per nested block
+    float m[DQ_SPANS];
+#pragma unroll
+    for (int c = 0; c < DQ_SPANS; ++c) {
+        const int64_t i0 = first + c * (THREADS * 4);
+        m[c] = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            v[c][k] = __fsub_rn(v[c][k], offset);
+            if (i0 + k < nblocks) m[c] = fmaxf(m[c], fabsf(v[c][k]));
+        }
+        m[c] = group_max(m[c], group < 64 ? group : 64);
+        if (group > 64) {  // uniform branch: the nested block spans several waves
+            if ((tid & 63) == 0) wave_max[c][tid >> 6] = m[c];
+            __syncthreads();
+            const int waves = group >> 6, w0 = (tid >> 6) & ~(waves - 1);
+            for (int j = 0; j < waves; ++j) m[c] = fmaxf(m[c], wave_max[c][w0 + j]);
+        }
+        if (i0 < nblocks && (tid & (group - 1)) == 0) absmax2[i0 >> nested_log2] = m[c];
+        const float inv = __fdiv_rn(1.0f, m[c]);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[c][k] = __fmul_rn(v[c][k], inv);
+    }
+
+    int best[DQ_SPANS][4] = {};
+    if (ascending) {  // the same for the whole workgroup
+        // entries <= s (255 at most; 0 for NaN), the searches of all values side by side: each level is an LDS round trip
+#pragma unroll
+        for (int c = 0; c < DQ_SPANS; ++c)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) best[c][k] = 1;
+#pragma unroll
+        for (int level = 0; level < 8; ++level)
+#pragma unroll
+            for (int c = 0; c < DQ_SPANS; ++c)
+#pragma unroll
+                for (int k = 0; k < 4; ++k) best[c][k] = 2 * best[c][k] + (tree[best[c][k]] <= v[c][k] ? 1 : 0);
+#pragma unroll
+        for (int c = 0; c < DQ_SPANS; ++c)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) best[c][k] -= 256;
+        float left[DQ_SPANS][4];
+#pragma unroll
+        for (int c = 0; c < DQ_SPANS; ++c)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int pos = best[c][k], before = pos > 0 ? pos - 1 : 0;
+                const float right = fabsf(__fsub_rn(v[c][k], map[pos]));
+                left[c][k] = fabsf(__fsub_rn(v[c][k], map[before]));
+                if (left[c][k] <= right) best[c][k] = before;
+                else left[c][k] = -1.0f;  // no distance: nothing further to the left is as near
+            }
+        bool tied = false;  // an entry further to the left is as near: duplicates, or entries closer than fp32 tells apart
+#pragma unroll
+        for (int c = 0; c < DQ_SPANS; ++c)
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                tied |= best[c][k] > 0 && fabsf(__fsub_rn(v[c][k], map[max(best[c][k], 1) - 1])) == left[c][k];
+        if (tied) {
+#pragma unroll
+            for (int c = 0; c < DQ_SPANS; ++c)
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    while (best[c][k] > 0 && fabsf(__fsub_rn(v[c][k], map[best[c][k] - 1])) == left[c][k]) --best[c][k];
+        }
     } else {
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
-            if (i0 + c < nblocks) q[i0 + c] = (uint8_t)code[c];
+        for (int c = 0; c < DQ_SPANS; ++c)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                float bestd = INFINITY;
+                for (int j = 0; j < 256; ++j) {
+                    const float d = fabsf(__fsub_rn(v[c][k], map[j]));
+                    if (d < bestd) {
+                        bestd = d;
+                        best[c][k] = j;
+                    }
+                }
+            }
+    }
+
+#pragma unroll
+    for (int c = 0; c < DQ_SPANS; ++c) {
+        const int64_t i0 = first + c * (THREADS * 4);
+        uint32_t code[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)  // infinity and NaN: no distance is below infinity, the code stays 0
+            code[k] = m[c] == 0.0f ? zero : isfinite(v[c][k]) ? best[c][k] : 0;
+        if (i0 + 4 <= nblocks) {
+            *reinterpret_cast<uint32_t*>(q + i0) = code[0] | (code[1] << 8) | (code[2] << 16) | (code[3] << 24);
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (i0 + k < nblocks) q[i0 + k] = (uint8_t)code[k];
+        }
     }
 }
 
@@ -392,18 +517,43 @@ __global__ __launch_bounds__(256) void dq_reconstruct_kernel(NestedAbsmax nq, in
 
 }  // namespace
 
+namespace {
+
+template <int DTYPE>
+void enqueue_quantize(const void* w, int64_t n, int block_log2, uint8_t* packed, float* absmax, hipStream_t stream) {
+    const int threads = block_log2 == 12 ? 512 : 256;  // a span holds a whole block
+    const int64_t per = (int64_t)threads * 8 * Q_SLOTS;
+    const dim3 grid((unsigned)((n + per - 1) / per));
+    if (threads == 512)
+        hipLaunchKernelGGL((quantize_kernel<512, DTYPE>), grid, dim3(512), 0, stream, w, n, block_log2, packed, absmax);
+    else
+        hipLaunchKernelGGL((quantize_kernel<256, DTYPE>), grid, dim3(256), 0, stream, w, n, block_log2, packed, absmax);
+}
+
+hipError_t enqueue_compress(const float* absmax, int64_t nblocks, int nested_log2, const float* map256, const DqOffset& o,
+                            uint8_t* q, float* absmax2, hipStream_t stream) {
+    // a span holds whole nested blocks: 1024 values, or 4096 for the two largest nested block sizes
+    const int threads = nested_log2 <= 10 ? 256 : 1024;
+    const int64_t per = (int64_t)threads * 4 * DQ_SPANS;
+    const dim3 grid((unsigned)((nblocks + per - 1) / per));
+    if (threads == 256)
+        hipLaunchKernelGGL(dq_compress_kernel<256>, grid, dim3(256), 0, stream, absmax, nblocks, nested_log2, map256, o, q, absmax2);
+    else
+        hipLaunchKernelGGL(dq_compress_kernel<1024>, grid, dim3(1024), 0, stream, absmax, nblocks, nested_log2, map256, o, q, absmax2);
+    return hipGetLastError();
+}
+
+}  // namespace
+
 hipError_t launch_quantize(const void* w, int w_dtype, int64_t n, int block_log2, uint8_t* packed, float* absmax,
                            hipStream_t stream) {
     if (n == 0) return hipSuccess;
-    if (block_log2 == 12) {
-        const int64_t grid = (n + 4096 * Q_SLOTS - 1) / (4096 * Q_SLOTS);
-        hipLaunchKernelGGL(quantize_kernel<512>, dim3((unsigned)grid), dim3(512), 0, stream, w, w_dtype, n, block_log2,
-                           packed, absmax);
-    } else {
-        const int64_t grid = (n + 2048 * Q_SLOTS - 1) / (2048 * Q_SLOTS);
-        hipLaunchKernelGGL(quantize_kernel<256>, dim3((unsigned)grid), dim3(256), 0, stream, w, w_dtype, n, block_log2,
-                           packed, absmax);
-    }
+    if (w_dtype == BF16)
+        enqueue_quantize<BF16>(w, n, block_log2, packed, absmax, stream);
+    else if (w_dtype == F16)
+        enqueue_quantize<F16>(w, n, block_log2, packed, absmax, stream);
+    else
+        enqueue_quantize<F32>(w, n, block_log2, packed, absmax, stream);
     return hipGetLastError();
 }
 
@@ -418,9 +568,7 @@ hipError_t launch_quantize_dq(const void* w, int w_dtype, int64_t n, int block_l
     const int count = (int)((nblocks + per - 1) / per);
     hipLaunchKernelGGL(dq_sum_kernel, dim3((unsigned)count), dim3(256), 0, stream, absmax, nblocks, per, sums);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    hipLaunchKernelGGL(dq_offset_kernel, dim3(1), dim3(DQ_SUMS), 0, stream, sums, count, nblocks, offset, map256, map_out, code_out);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    return launch_dq_compress(absmax, nblocks, nested_log2, map256, 0.0f, offset, q, absmax2, stream);
+    return enqueue_compress(absmax, nblocks, nested_log2, map256, {sums, offset, map_out, code_out, count, 0.0f}, q, absmax2, stream);
 }
 
 hipError_t launch_dequantize(const uint8_t* packed, const float* absmax, const NestedAbsmax& nested,
@@ -449,18 +597,9 @@ hipError_t launch_dequantize(const uint8_t* packed, const float* absmax, const N
 }
 
 hipError_t launch_dq_compress(const float* absmax, int64_t nblocks, int nested_log2, const float* map256,
-                              float offset, const float* offset_ptr, uint8_t* q, float* absmax2, hipStream_t stream) {
+                              float offset, uint8_t* q, float* absmax2, hipStream_t stream) {
     if (nblocks == 0) return hipSuccess;
-    // a workgroup holds whole nested blocks: 1024 values, or 4096 for the two largest nested block sizes
-    const int threads = nested_log2 <= 10 ? 256 : 1024;
-    const dim3 grid((unsigned)((nblocks + 4 * threads - 1) / (4 * threads)));
-    if (threads == 256)
-        hipLaunchKernelGGL(dq_compress_kernel<256>, grid, dim3(256), 0, stream, absmax, nblocks, nested_log2, map256, offset,
-                           offset_ptr, q, absmax2);
-    else
-        hipLaunchKernelGGL(dq_compress_kernel<1024>, grid, dim3(1024), 0, stream, absmax, nblocks, nested_log2, map256, offset,
-                           offset_ptr, q, absmax2);
-    return hipGetLastError();
+    return enqueue_compress(absmax, nblocks, nested_log2, map256, {nullptr, nullptr, nullptr, nullptr, 0, offset}, q, absmax2, stream);
 }
 
 hipError_t launch_dq_reconstruct(const NestedAbsmax& nested, int64_t nblocks, float* absmax, hipStream_t stream) {

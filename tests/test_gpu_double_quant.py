@@ -81,6 +81,36 @@ def test_quantize_dq(ta, oracle, dtype, n, blocksize, nested):
     assert torch.equal(qw.cpu(), qw_o) and torch.equal(q.cpu(), q_o) and torch.equal(a2.cpu(), a2_o)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("blocksize", [64, 512, 1024, 4096])
+def test_quantize_workgroup_edges(ta, oracle, dtype, blocksize):
+    """The last workgroup whole, one element short, one element over; thresholds and their neighbours, infinities, NaN and
+    denormals in a whole workgroup and in the ragged one."""
+    thr = torch.tensor([(0xBF591CD9 - (1 << 32)), 0x3D22FAFF, 0x3F5C89D9], dtype=torch.int32).view(torch.float32)
+    one = torch.tensor([1.0, -1.0, float("inf"), float("nan"), float("-inf"), 1e-39, 0.0, -0.0])
+    special = torch.cat([thr, torch.nextafter(thr, one[:1]), torch.nextafter(thr, one[1:2]), one])
+    span = 8192 if blocksize < 4096 else 16384
+    for n in (span - 1, span, span + 1, 2 * span, 3 * span + 9):
+        print(f"quantize edges {dtype} {blocksize} n={n}", flush=True)
+        w = torch.rand(n, generator=torch.Generator().manual_seed(n)) * 2 - 1
+        for at in (0, blocksize - 20, n - len(special)):
+            w[at:at + len(special)] = special
+        w[2 * blocksize:3 * blocksize] = 0.0
+        w = w.to(dtype)
+        qw, absmax, _ = ta.quantize_nf4(w.to(DEV), blocksize)
+        qw_o, absmax_o = oracle.C().quantize(w, blocksize)
+        assert torch.equal(absmax.cpu(), absmax_o) and torch.equal(qw.cpu().flatten(), qw_o.flatten()), n
+
+
+def test_offset_of_more_values_than_one_round_of_loads(ta):
+    """4.8 M blocks: every workgroup of the sum takes more full rounds than it loads at a time, and a remainder."""
+    n = 64 * (512 * 9300 + 5)
+    w = torch.randn(n, device=DEV, dtype=torch.bfloat16)
+    off = ta.functional.quantize_nf4_dq(w)[4]
+    absmax = ta.quantize_nf4(w)[1]
+    assert off.item() == float(absmax.cpu().double().mean().to(torch.float32))
+
+
 @pytest.mark.parametrize("n,blocksize,nested", [(7, 64, 256), (8192 + 8, 64, 64), (8192 * 5 + 3, 256, 256), (100_000, 64, 4096)])
 def test_dequantize_nested_sizes(ta, oracle, n, blocksize, nested):
     print(f"dequantize nested n={n} {blocksize}/{nested}", flush=True)

@@ -175,11 +175,17 @@ __global__ __launch_bounds__(THREADS) void quantize_kernel(const void* __restric
     }
 }
 
+// Two values as bf16, rounded to nearest even, in one instruction.
+__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
+    typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+    typedef float f32x2_t __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{lo, hi}, bf16x2_t));
+}
+
 // Eight elements of output from one 32-bit word of codes.
-template <bool STREAM>
-__device__ __forceinline__ void dequant8_store(uint32_t word, float s, const float* lut, void* out, int out_dtype,
-                                               int64_t e0, int64_t n) {
-    const bool full = e0 + 8 <= n;
+template <bool STREAM, int OUT>
+__device__ __forceinline__ void dequant8_store(uint32_t word, float s, const float* lut, void* out, int64_t e0,
+                                               bool full, int64_t n) {
     float v[8];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -187,69 +193,92 @@ __device__ __forceinline__ void dequant8_store(uint32_t word, float s, const flo
         v[2 * j] = __fmul_rn(lut[byte >> 4], s);
         v[2 * j + 1] = __fmul_rn(lut[byte & 15u], s);
     }
-    if (out_dtype == F32) {
+    if (OUT == F32) {
         float* o = reinterpret_cast<float*>(out);
         if (full) {
             store16<STREAM>(o + e0, __float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3]));
             store16<STREAM>(o + e0 + 4, __float_as_uint(v[4]), __float_as_uint(v[5]), __float_as_uint(v[6]), __float_as_uint(v[7]));
         } else {
+#pragma unroll
             for (int j = 0; j < 8; ++j)
                 if (e0 + j < n) o[e0 + j] = v[j];
         }
     } else {
-        uint32_t h[8];
+        uint32_t h[4];
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
-            h[j] = out_dtype == BF16 ? f32_to_bf16_bits(v[j]) : (uint32_t)__half_as_ushort(__float2half_rn(v[j]));
+        for (int j = 0; j < 4; ++j) {
+            if (OUT == BF16) {
+                h[j] = pack_bf16(v[2 * j], v[2 * j + 1]);
+            } else {
+                // the product is rounded to fp32 first: without this a mixed-precision multiply-add would do both at once
+                asm("" : "+v"(v[2 * j]), "+v"(v[2 * j + 1]));
+                h[j] = (uint32_t)__half_as_ushort(__float2half_rn(v[2 * j])) |
+                       (uint32_t)__half_as_ushort(__float2half_rn(v[2 * j + 1])) << 16;
+            }
+        }
         uint16_t* o = reinterpret_cast<uint16_t*>(out);
         if (full) {
-            store16<STREAM>(o + e0, h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16));
+            store16<STREAM>(o + e0, h[0], h[1], h[2], h[3]);
         } else {
+#pragma unroll
             for (int j = 0; j < 8; ++j)
-                if (e0 + j < n) o[e0 + j] = (uint16_t)h[j];
+                if (e0 + j < n) o[e0 + j] = (uint16_t)(h[j / 2] >> (16 * (j & 1)));
         }
     }
 }
 
 // A workgroup covers DQ_SLOTS consecutive spans of 2048 elements; a thread owns 8 consecutive
-// elements of each span, so every load and store of a wave is contiguous, and the loads of all
-// spans are in flight before the first store.
-// Nested absmax: the 8-bit code and the second-level absmax of every span are requested together with the codes and the
-// map is copied into LDS meanwhile, so that no load waits for another.  With the map looked up in global memory
-// (code -> map entry -> value, two dependent loads per span) the kernel took 175 us for the 592 MB of a [28672, 8192]
-// weight (3.4 TB/s); now 101 us (5.9 TB/s).
+// elements of each span, so every load and store of a wave is contiguous.  Bound by HBM, mostly by the writes.
+//
+// The loads of all spans are in flight before the first is used: codes first (they come from the farthest), then the
+// statistics, with one branch for the whole workgroup instead of one around each load.  An output that does not fit the
+// last-level cache (STREAM) has its codes read past the cache too; behind a smaller one they may stay there.
+// 16-bit outputs are packed by one conversion per two values.
+// us, with a check around every load and the codes always read past the cache -> now: [14336, 4096] bf16 39.5 -> 34.9 (of
+// which about 12 is the call), fp32 107 -> 102; nested [28672, 8192] bf16 112 -> 109.  Statistics first: 118 for the last.
+// Spans per workgroup 1 / 2 / 4 / 8: 132 / 134 / 115 / 120.
+// Nested absmax: the map is copied into LDS meanwhile, so that no load waits for another.  With the map looked up in
+// global memory (code -> map entry -> value, two dependent loads per span) the kernel took 175 us for that weight.
 constexpr int DQ_SLOTS = 4;
 
-template <bool NESTED, bool STREAM>
+template <bool NESTED, bool STREAM, int OUT>
 __global__ __launch_bounds__(256) void dequantize_kernel(const uint8_t* __restrict__ packed,
                                                          const float* __restrict__ absmax, NestedAbsmax nq,
                                                          const float* __restrict__ lut16, int64_t n, int block_log2,
-                                                         void* __restrict__ out, int out_dtype) {
+                                                         void* __restrict__ out) {
     __shared__ float lut[16];
     __shared__ float map[NESTED ? 256 : 1];
     const int tid = threadIdx.x;
+    const int64_t first = (int64_t)blockIdx.x * (DQ_SLOTS * 2048) + tid * 8;
+    const bool whole = ((int64_t)blockIdx.x + 1) * (DQ_SLOTS * 2048) <= n;
     const float lut_entry = lut16[tid & 15], map_entry = NESTED ? nq.map256[tid] : 0.0f;
     uint32_t word[DQ_SLOTS], q[DQ_SLOTS];
     float s[DQ_SLOTS];  // absmax, or with nested absmax the second-level value
+    if (whole) {
+#pragma unroll
+        for (int c = 0; c < DQ_SLOTS; ++c)
+            word[c] = STREAM ? __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(packed) + ((first + c * 2048) >> 3)) : reinterpret_cast<const uint32_t*>(packed)[(first + c * 2048) >> 3];
+    } else {
+        const int64_t nbytes = (n + 1) / 2;
+#pragma unroll
+        for (int c = 0; c < DQ_SLOTS; ++c) {
+            const int64_t e0 = first + c * 2048;
+            word[c] = 0;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (e0 / 2 + j < nbytes) word[c] |= (uint32_t)packed[e0 / 2 + j] << (8 * j);
+        }
+    }
 #pragma unroll
     for (int c = 0; c < DQ_SLOTS; ++c) {
-        const int64_t e0 = (((int64_t)blockIdx.x * DQ_SLOTS + c) * 256 + tid) * 8;
-        word[c] = q[c] = 0;
-        s[c] = 0.0f;
-        if (e0 >= n) continue;
-        const int64_t blk = e0 >> block_log2;
+        // lanes past the end read the last block's statistics, which they do not use
+        const int64_t e0 = first + c * 2048, blk = (whole || e0 < n ? e0 : n - 1) >> block_log2;
         if (NESTED) {
             q[c] = nq.q[blk];
             s[c] = nq.absmax2[blk >> nq.nested_log2];
         } else {
+            q[c] = 0;
             s[c] = absmax[blk];
-        }
-        if (e0 + 8 <= n) {
-            word[c] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(packed) + e0 / 8);
-        } else {
-            const int64_t nbytes = (n + 1) / 2;
-            for (int j = 0; j < 4; ++j)
-                if (e0 / 2 + j < nbytes) word[c] |= (uint32_t)packed[e0 / 2 + j] << (8 * j);
         }
     }
     if (tid < 16) lut[tid] = lut_entry;
@@ -257,9 +286,9 @@ __global__ __launch_bounds__(256) void dequantize_kernel(const uint8_t* __restri
     __syncthreads();
 #pragma unroll
     for (int c = 0; c < DQ_SLOTS; ++c) {
-        const int64_t e0 = (((int64_t)blockIdx.x * DQ_SLOTS + c) * 256 + tid) * 8;
+        const int64_t e0 = first + c * 2048;
         const float scale = NESTED ? __fadd_rn(__fmul_rn(map[q[c]], s[c]), nq.offset) : s[c];  // as nested_absmax
-        if (e0 < n) dequant8_store<STREAM>(word[c], scale, lut, out, out_dtype, e0, n);
+        if (whole || e0 < n) dequant8_store<STREAM, OUT>(word[c], scale, lut, out, e0, whole || e0 + 8 <= n, n);
     }
 }
 
@@ -571,28 +600,33 @@ hipError_t launch_quantize_dq(const void* w, int w_dtype, int64_t n, int block_l
     return enqueue_compress(absmax, nblocks, nested_log2, map256, {sums, offset, map_out, code_out, count, 0.0f}, q, absmax2, stream);
 }
 
+namespace {
+
+template <bool STREAM, int OUT>
+void enqueue_dequantize(const uint8_t* packed, const float* absmax, const NestedAbsmax& nested, const float* lut16,
+                        int64_t n, int block_log2, void* out, hipStream_t stream) {
+    const dim3 grid((unsigned)((n + 2048 * DQ_SLOTS - 1) / (2048 * DQ_SLOTS))), threads(256);
+    if (nested.q)
+        hipLaunchKernelGGL((dequantize_kernel<true, STREAM, OUT>), grid, threads, 0, stream, packed, absmax, nested, lut16, n, block_log2, out);
+    else
+        hipLaunchKernelGGL((dequantize_kernel<false, STREAM, OUT>), grid, threads, 0, stream, packed, absmax, nested, lut16, n, block_log2, out);
+}
+
+}  // namespace
+
 hipError_t launch_dequantize(const uint8_t* packed, const float* absmax, const NestedAbsmax& nested,
                              const float* lut16, int64_t n, int block_log2, void* out, int out_dtype,
                              hipStream_t stream) {
     if (n == 0) return hipSuccess;
-    const int64_t grid = (n + 2048 * DQ_SLOTS - 1) / (2048 * DQ_SLOTS);
     // An output that fits in the 256 MB last-level cache is written with ordinary stores, so that the
     // GEMM that usually follows finds it there; a larger one cannot stay anyway and is streamed
     // (non-temporal stores: 20 % faster on their own, 5 % slower for that GEMM).
     const int64_t out_bytes = n * (out_dtype == F32 ? 4 : 2);
     const bool stream_out = out_bytes > ((int64_t)192 << 20);
-    const dim3 g((unsigned)grid), b(256);
-    if (nested.q) {
-        if (stream_out)
-            hipLaunchKernelGGL((dequantize_kernel<true, true>), g, b, 0, stream, packed, absmax, nested, lut16, n, block_log2, out, out_dtype);
-        else
-            hipLaunchKernelGGL((dequantize_kernel<true, false>), g, b, 0, stream, packed, absmax, nested, lut16, n, block_log2, out, out_dtype);
-    } else {
-        if (stream_out)
-            hipLaunchKernelGGL((dequantize_kernel<false, true>), g, b, 0, stream, packed, absmax, nested, lut16, n, block_log2, out, out_dtype);
-        else
-            hipLaunchKernelGGL((dequantize_kernel<false, false>), g, b, 0, stream, packed, absmax, nested, lut16, n, block_log2, out, out_dtype);
-    }
+    const auto enqueue = out_dtype == F32    ? (stream_out ? enqueue_dequantize<true, F32> : enqueue_dequantize<false, F32>)
+                         : out_dtype == BF16 ? (stream_out ? enqueue_dequantize<true, BF16> : enqueue_dequantize<false, BF16>)
+                                             : (stream_out ? enqueue_dequantize<true, F16> : enqueue_dequantize<false, F16>);
+    enqueue(packed, absmax, nested, lut16, n, block_log2, out, stream);
     return hipGetLastError();
 }
 

@@ -1,4 +1,4 @@
-"""ctypes binding of ``libnf4hip.so`` (C ABI in ``include/nf4hip.h``).
+"""ctypes binding of ``libnf4hip.so`` (C ABI in ``include/nf4hip.h``), and ``nf4hip_host.so``, which calls its matmuls natively.
 
 The library is built in-tree (``lightning-thunder_amd/libnf4hip.so``) by
 ``__graft_entry__.build()`` / ``make -C lightning-thunder_amd/csrc``.  There is no CPU fallback:
@@ -8,6 +8,8 @@ if the library is missing or its ABI version differs, every op raises.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import threading
 
@@ -30,6 +32,8 @@ _ERROR_NAMES = {
 }
 
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libnf4hip.so")
+
+HOST_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "nf4hip_host.so")
 
 # every symbol include/nf4hip.h declares: name -> (restype, argtypes)
 _vp, _i32, _i64, _f32, _sz = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64, ctypes.c_float, ctypes.c_size_t
@@ -82,6 +86,10 @@ SYMBOLS = {
 }
 
 
+# matmul entry points the native host side (csrc/host_call.cpp) calls: name -> the query for its workspace
+HOST_CALLS = {"nf4hip_gemv": "nf4hip_gemv_workspace_bytes", "nf4hip_gemm": "nf4hip_gemm_workspace_bytes", "nf4hip_stream": "nf4hip_stream_workspace_bytes"}
+
+
 class NF4HipError(RuntimeError):
     """A call into libnf4hip.so returned a negative status."""
 
@@ -117,9 +125,21 @@ def load(path: str | None = None) -> ctypes.CDLL:
         got = lib.nf4hip_abi_version()
         if got != ABI_VERSION:
             raise RuntimeError(f"{p}: ABI version {got}, host code expects {ABI_VERSION}")
+        address = lambda name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value  # noqa: E731
+        lib.host_matmul = _load_host().matmul
+        lib.host_calls = {name: (address(name), address(need)) for name, need in HOST_CALLS.items()}
         if path is None:
             _lib = lib
         return lib
+
+
+def _load_host():
+    if not os.path.exists(HOST_PATH):
+        raise RuntimeError(f"{HOST_PATH} not found: the extension has not been built (`make -C lightning-thunder_amd/csrc`)")
+    loader = importlib.machinery.ExtensionFileLoader("nf4hip_host", HOST_PATH)
+    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("nf4hip_host", loader))
+    loader.exec_module(module)
+    return module
 
 
 def check(rc: int) -> None:

@@ -42,6 +42,10 @@ class WorkspacePool:
             idx = torch.cuda.current_device() if device.type == "cuda" else -1
         return idx, current_stream_handle(idx) if stream is None else stream
 
+    def peek(self, device_index: int, stream: int) -> torch.Tensor | None:
+        """The buffer that (device, stream) has, of whatever length."""
+        return self._live.get((device_index, stream))
+
     def get(self, device: torch.device, nbytes: int, stream: int | None = None) -> torch.Tensor:
         """The zero-initialised buffer of (device, stream), at least ``nbytes`` long."""
         key = self._key(device, stream)

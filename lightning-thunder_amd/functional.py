@@ -585,8 +585,10 @@ NESTED_RECONSTRUCT_MIN_US = 30
 def _matmul_nf4_on(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape, route: str) -> torch.Tensor:
     """:func:`matmul_nf4` on a given route (one of ``fused_route``'s answers).
 
-    A decode call on a small weight is as long as this function: views, conversions and a device context that change nothing
-    are not asked for ([4096, 4096], one row, 5 us of kernel: ``matmul_nf4`` 14.9 -> 10.4 us, of which the ctypes call is 4.5)."""
+    A decode call on a small weight is as long as this function, so what needs no conversion is handed to the library in one native
+    step (csrc/host_call.cpp; [4096, 4096], one row, 4.6 us of kernel: ``matmul_nf4`` 9.5 -> 5.3 us, of which the launch is 2.9).  What that
+    step does not take -- nested statistics, views, other types, a stream without a workspace, tensors inside a transform -- comes
+    back and is served below."""
     N, K = shape
     if route in ("dequant+linear", "dequant+gemm", "dequant+libgemm"):
         w = dequantize_nf4(qweight, absmax, quant_map, blocksize, dtype, shape).to(x.dtype)
@@ -599,6 +601,14 @@ def _matmul_nf4_on(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape,
         with torch.cuda.device(device):
             return _matmul_nf4_on(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape, route)
     lib = _lib.load()
+    stream = _stream() if _raw_stream is None else _raw_stream(device.index)
+    entry = "nf4hip_gemv" if route == "gemv" else "nf4hip_stream" if x.dtype is torch.float16 else "nf4hip_gemm"
+    out = lib.host_matmul(*lib.host_calls[entry], x, qweight, absmax, quant_map, bias, N, K, blocksize,
+                          _workspace_pool.peek(device.index, stream), stream)  # fmt: skip
+    if out is not None:
+        if type(out) is int:
+            _lib.check(out)
+        return out
     flat = x.dim() == 2
     x2 = _aligned(x if flat else x.reshape(-1, K))
     M = x2.shape[0]
@@ -609,7 +619,6 @@ def _matmul_nf4_on(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape,
     b = None if bias is None else bias.contiguous()
     nblocks = N * K // blocksize
     out = x2.new_empty((M, N)) if type(x2) is torch.Tensor else torch.empty((M, N), dtype=x.dtype, device=device)
-    stream = _stream() if _raw_stream is None else _raw_stream(device.index)
     if route == "gemv":
         need = lib.nf4hip_gemv_workspace_bytes(M, N, K)
         ws = _gemv_workspace(device, need, stream)

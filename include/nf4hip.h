@@ -102,6 +102,16 @@ int nf4hip_quantize_dq(const void* w, int w_dtype, int64_t n, int blocksize, int
                        uint8_t* packed, uint8_t* absmax_q, float* absmax2, float* offset, float* map_out_or_null,
                        float* code_out_or_null, void* workspace, size_t workspace_bytes, void* stream);
 
+/*
+ * The second half of nf4hip_quantize_dq, for a caller that launches nf4hip_quantize as soon as it has that kernel's outputs
+ * and prepares the rest meanwhile: absmax (fp32 [nblocks], 16-byte aligned) is compressed, everything else as there.
+ * `workspace`: NF4HIP_DQ_STATISTICS_WORKSPACE_BYTES, 16-byte aligned, in any state.
+ */
+#define NF4HIP_DQ_STATISTICS_WORKSPACE_BYTES 4096
+int nf4hip_dq_statistics(const float* absmax, int64_t nblocks, int nested_blocksize, const float* map256, uint8_t* absmax_q,
+                         float* absmax2, float* offset, float* map_out_or_null, float* code_out_or_null, void* workspace,
+                         size_t workspace_bytes, void* stream);
+
 /* Same as nf4hip_dequantize with absmax given in nested form. */
 int nf4hip_dequantize_dq(const uint8_t* packed, const uint8_t* absmax_q, const float* absmax2, const float* map256,
                          float offset, int nested_blocksize, const float* lut16, int64_t n, int blocksize, void* out,

@@ -19,6 +19,8 @@ BF16, F16, F32 = 0, 1, 2
 
 STATIC_SCRATCH_BYTES = 4 << 20  # NF4HIP_STATIC_SCRATCH_BYTES
 
+DQ_STATISTICS_WORKSPACE_BYTES = 4096  # NF4HIP_DQ_STATISTICS_WORKSPACE_BYTES
+
 E_NULL, E_DTYPE, E_BLOCKSIZE, E_SHAPE, E_ALIGN, E_WORKSPACE, E_HIP = -1, -2, -3, -4, -5, -6, -7
 
 _ERROR_NAMES = {
@@ -56,6 +58,7 @@ SYMBOLS = {
     "nf4hip_quantize": (_i32, [_vp, _i32, _i64, _i32, _vp, _vp, _vp]),
     "nf4hip_quantize_dq_workspace_bytes": (_sz, [_i64, _i32]),
     "nf4hip_quantize_dq": (_i32, [_vp, _i32, _i64, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
+    "nf4hip_dq_statistics": (_i32, [_vp, _i64, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
     "nf4hip_dequantize": (_i32, [_vp, _vp, _vp, _i64, _i32, _vp, _i32, _vp]),
     "nf4hip_dq_compress": (_i32, [_vp, _i64, _i32, _vp, _f32, _vp, _vp, _vp]),
     "nf4hip_dq_reconstruct": (_i32, [_vp, _vp, _vp, _f32, _i64, _i32, _vp, _vp]),

@@ -242,8 +242,32 @@ int nf4hip_quantize_dq(const void* w, int w_dtype, int64_t n, int blocksize, int
         return fail(NF4HIP_E_WORKSPACE, "%s: workspace of %zu bytes required, got %zu", name, need, workspace ? workspace_bytes : (size_t)0);
     if (!aligned16(workspace)) return fail(NF4HIP_E_ALIGN, "%s: workspace not 16-byte aligned", name);
     float* absmax = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + nf4::DQ_SUMS * sizeof(double));
-    const hipError_t e = nf4::launch_quantize_dq(w, w_dtype, n, bl, nl, map256, packed, absmax, static_cast<double*>(workspace), offset,
-                                                 absmax_q, absmax2, map_out_or_null, code_out_or_null, static_cast<hipStream_t>(stream));
+    hipError_t e = nf4::launch_quantize(w, w_dtype, n, bl, packed, absmax, static_cast<hipStream_t>(stream));
+    if (e == hipSuccess)
+        e = nf4::launch_dq_statistics(absmax, (n + blocksize - 1) / blocksize, nl, map256, static_cast<double*>(workspace), offset, absmax_q,
+                                      absmax2, map_out_or_null, code_out_or_null, static_cast<hipStream_t>(stream));
+    if (e != hipSuccess) return hip_fail(name, e);
+    return NF4HIP_OK;
+}
+
+int nf4hip_dq_statistics(const float* absmax, int64_t nblocks, int nested_blocksize, const float* map256, uint8_t* absmax_q,
+                         float* absmax2, float* offset, float* map_out_or_null, float* code_out_or_null, void* workspace,
+                         size_t workspace_bytes, void* stream) {
+    static_assert(NF4HIP_DQ_STATISTICS_WORKSPACE_BYTES == nf4::DQ_SUMS * sizeof(double), "the partial sums");
+    const char* name = "nf4hip_dq_statistics";
+    if (nblocks <= 0) return fail(NF4HIP_E_SHAPE, "%s: nblocks = %lld is not positive", name, (long long)nblocks);
+    const int nl = block_log2(nested_blocksize);
+    if (nl < 0) return fail(NF4HIP_E_BLOCKSIZE, "%s: nested_blocksize %d unsupported", name, nested_blocksize);
+    if (!absmax || !map256 || !absmax_q || !absmax2 || !offset) return fail(NF4HIP_E_NULL, "%s: null pointer", name);
+    if (!aligned16(absmax) || !aligned16(absmax_q) || !aligned16(absmax2) || !aligned4(map256) || !aligned4(offset) ||
+        !aligned4(map_out_or_null) || !aligned4(code_out_or_null))
+        return fail(NF4HIP_E_ALIGN, "%s: absmax / absmax_q / absmax2 not 16-byte aligned or a table not 4-byte aligned", name);
+    if (!workspace || workspace_bytes < NF4HIP_DQ_STATISTICS_WORKSPACE_BYTES)
+        return fail(NF4HIP_E_WORKSPACE, "%s: workspace of %d bytes required, got %zu", name, NF4HIP_DQ_STATISTICS_WORKSPACE_BYTES,
+                    workspace ? workspace_bytes : (size_t)0);
+    if (!aligned16(workspace)) return fail(NF4HIP_E_ALIGN, "%s: workspace not 16-byte aligned", name);
+    const hipError_t e = nf4::launch_dq_statistics(absmax, nblocks, nl, map256, static_cast<double*>(workspace), offset, absmax_q, absmax2,
+                                                   map_out_or_null, code_out_or_null, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(name, e);
     return NF4HIP_OK;
 }

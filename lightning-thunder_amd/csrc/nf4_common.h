@@ -68,11 +68,10 @@ struct DenseArgs {
 // hipError_t of the launch.
 hipError_t launch_quantize(const void* w, int w_dtype, int64_t n, int block_log2, uint8_t* packed, float* absmax,
                            hipStream_t stream);
-// `sums`: DQ_SUMS float64; `absmax`: scratch here, one fp32 per block
+// offset = mean(absmax), then launch_dq_compress with it; `sums`: DQ_SUMS float64
 constexpr int DQ_SUMS = 512;
-hipError_t launch_quantize_dq(const void* w, int w_dtype, int64_t n, int block_log2, int nested_log2, const float* map256,
-                              uint8_t* packed, float* absmax, double* sums, float* offset, uint8_t* q, float* absmax2,
-                              float* map_out, float* code_out, hipStream_t stream);
+hipError_t launch_dq_statistics(const float* absmax, int64_t nblocks, int nested_log2, const float* map256, double* sums,
+                                float* offset, uint8_t* q, float* absmax2, float* map_out, float* code_out, hipStream_t stream);
 hipError_t launch_dequantize(const uint8_t* packed, const float* absmax, const NestedAbsmax& nested,
                              const float* lut16, int64_t n, int block_log2, void* out, int out_dtype,
                              hipStream_t stream);

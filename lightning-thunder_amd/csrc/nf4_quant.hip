@@ -586,17 +586,15 @@ hipError_t launch_quantize(const void* w, int w_dtype, int64_t n, int block_log2
     return hipGetLastError();
 }
 
-hipError_t launch_quantize_dq(const void* w, int w_dtype, int64_t n, int block_log2, int nested_log2, const float* map256,
-                              uint8_t* packed, float* absmax, double* sums, float* offset, uint8_t* q, float* absmax2,
-                              float* map_out, float* code_out, hipStream_t stream) {
-    const int64_t nblocks = (n + (1 << block_log2) - 1) >> block_log2;
-    hipError_t e = launch_quantize(w, w_dtype, n, block_log2, packed, absmax, stream);
-    if (e != hipSuccess) return e;
+hipError_t launch_dq_statistics(const float* absmax, int64_t nblocks, int nested_log2, const float* map256, double* sums,
+                                float* offset, uint8_t* q, float* absmax2, float* map_out, float* code_out, hipStream_t stream) {
+    if (nblocks == 0) return hipSuccess;
     // a workgroup of the sum takes at least 4096 values
     const int64_t per = max((int64_t)4096, ((nblocks + DQ_SUMS - 1) / DQ_SUMS + 3) & ~(int64_t)3);
     const int count = (int)((nblocks + per - 1) / per);
     hipLaunchKernelGGL(dq_sum_kernel, dim3((unsigned)count), dim3(256), 0, stream, absmax, nblocks, per, sums);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
     return enqueue_compress(absmax, nblocks, nested_log2, map256, {sums, offset, map_out, code_out, count, 0.0f}, q, absmax2, stream);
 }
 

@@ -306,15 +306,18 @@ def quantize_nf4_dq(w: torch.Tensor, blocksize: int = 64, nested_blocksize: int 
     dev, n = w.device, w.numel()
     nblocks = (n + blocksize - 1) // blocksize
     with _on_device(dev):
+        # the long kernel first: what the others need is prepared while it runs ([28672, 8192]: 138 -> 129.5 us)
+        stream, sums = _stream(), _lib.DQ_STATISTICS_WORKSPACE_BYTES
         qw = torch.empty(((n + 1) // 2, 1), dtype=torch.uint8, device=dev)
+        scratch = torch.empty(sums + 4 * nblocks, dtype=torch.uint8, device=dev)  # partial sums, absmax in fp32: nobody keeps them
+        absmax = scratch.data_ptr() + sums
+        _lib.check(lib.nf4hip_quantize(w.data_ptr(), _DTYPE_CODE[w.dtype], n, blocksize, qw.data_ptr(), absmax, stream))
         q = torch.empty(nblocks, dtype=torch.uint8, device=dev)
         absmax2 = torch.empty(((nblocks + nested_blocksize - 1) // nested_blocksize,), dtype=torch.float32, device=dev)
         map256, code, offset = (torch.empty(k, dtype=torch.float32, device=dev) for k in (256, 16, 1))
-        need = lib.nf4hip_quantize_dq_workspace_bytes(n, blocksize)
-        scratch = torch.empty(need, dtype=torch.uint8, device=dev)  # absmax in fp32, which nobody keeps
-        _lib.check(lib.nf4hip_quantize_dq(w.data_ptr(), _DTYPE_CODE[w.dtype], n, blocksize, nested_blocksize, _dynamic_map_master(dev).data_ptr(),
-                                          qw.data_ptr(), q.data_ptr(), absmax2.data_ptr(), offset.data_ptr(), map256.data_ptr(),
-                                          code.data_ptr(), scratch.data_ptr(), need, _stream()))
+        _lib.check(lib.nf4hip_dq_statistics(absmax, nblocks, nested_blocksize, _dynamic_map_master(dev).data_ptr(), q.data_ptr(),
+                                            absmax2.data_ptr(), offset.data_ptr(), map256.data_ptr(), code.data_ptr(), scratch.data_ptr(),
+                                            sums, stream))
         _offset_value(offset)  # one read back, behind all three kernels: the matmuls' C ABI takes the offset by value
     return qw, q, absmax2, map256, offset, code
 

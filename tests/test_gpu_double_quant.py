@@ -102,6 +102,33 @@ def test_quantize_workgroup_edges(ta, oracle, dtype, blocksize):
         assert torch.equal(absmax.cpu(), absmax_o) and torch.equal(qw.cpu().flatten(), qw_o.flatten()), n
 
 
+def test_statistics_in_one_call_or_two(ta):
+    """nf4hip_quantize_dq is nf4hip_quantize and nf4hip_dq_statistics, which functional.quantize_nf4_dq launches apart; what the
+    second refuses."""
+    L = ta._lib
+    lib = L.load()
+    n, stream = 64 * 5003, torch.cuda.current_stream().cuda_stream
+    w = torch.randn(n, device=DEV, dtype=torch.bfloat16)
+    want = ta.functional.quantize_nf4_dq(w)
+    D = ta.functional.dynamic_map(w.device)
+    got = [torch.empty_like(t) for t in want]
+    need = lib.nf4hip_quantize_dq_workspace_bytes(n, 64)
+    ws = torch.empty(need, dtype=torch.uint8, device=DEV)
+    qw, q, a2, m256, off, code = (t.data_ptr() for t in got)
+    L.check(lib.nf4hip_quantize_dq(w.data_ptr(), L.BF16, n, 64, 256, D.data_ptr(), qw, q, a2, off, m256, code, ws.data_ptr(), need, stream))
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    absmax = torch.rand(5003, device=DEV)
+
+    def statistics(absmax=absmax.data_ptr(), n=5003, nested=256, offset=off, ws_bytes=L.DQ_STATISTICS_WORKSPACE_BYTES):
+        return lib.nf4hip_dq_statistics(absmax, n, nested, D.data_ptr(), q, a2, offset, None, None, ws.data_ptr(), ws_bytes, stream)
+
+    assert statistics() == 0 and statistics(n=0) == L.E_SHAPE and statistics(nested=96) == L.E_BLOCKSIZE
+    assert statistics(offset=None) == L.E_NULL and statistics(absmax=absmax.data_ptr() + 4) == L.E_ALIGN
+    assert statistics(ws_bytes=L.DQ_STATISTICS_WORKSPACE_BYTES - 1) == L.E_WORKSPACE
+    torch.cuda.synchronize()
+    assert got[4].item() == float(absmax.cpu().double().mean().to(torch.float32))
+
+
 def test_offset_of_more_values_than_one_round_of_loads(ta):
     """4.8 M blocks: every workgroup of the sum takes more full rounds than it loads at a time, and a remainder."""
     n = 64 * (512 * 9300 + 5)

@@ -55,13 +55,14 @@ struct Raw8 {
     uint32_t d[DTYPE == F32 ? 8 : 4];
 };
 
-template <int DTYPE>
+template <int DTYPE, bool STREAM>
 __device__ __forceinline__ Raw8<DTYPE> load8(const void* w, int64_t e0) {
     Raw8<DTYPE> r;
-    const uint4 a = load16_stream(static_cast<const char*>(w) + e0 * (DTYPE == F32 ? 4 : 2));
+    const uint4* p = reinterpret_cast<const uint4*>(static_cast<const char*>(w) + e0 * (DTYPE == F32 ? 4 : 2));
+    const uint4 a = STREAM ? load16_stream(p) : *p;
     r.d[0] = a.x; r.d[1] = a.y; r.d[2] = a.z; r.d[3] = a.w;
     if (DTYPE == F32) {
-        const uint4 b = load16_stream(static_cast<const float*>(w) + e0 + 4);
+        const uint4 b = STREAM ? load16_stream(p + 1) : p[1];
         r.d[4] = b.x; r.d[5] = b.y; r.d[6] = b.z; r.d[7] = b.w;
     }
     return r;
@@ -70,7 +71,7 @@ __device__ __forceinline__ Raw8<DTYPE> load8(const void* w, int64_t e0) {
 // the same where the array may end inside: elements at or beyond n read as 0
 template <int DTYPE>
 __device__ __forceinline__ Raw8<DTYPE> load8_edge(const void* w, int64_t e0, int64_t n) {
-    if (e0 + 8 <= n) return load8<DTYPE>(w, e0);
+    if (e0 + 8 <= n) return load8<DTYPE, false>(w, e0);
     Raw8<DTYPE> r = {};
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -113,13 +114,14 @@ __device__ __forceinline__ float group_max(float m, int lanes) {
 // is used: they are taken as raw words, behind one branch for the whole workgroup, and converted afterwards.  With the
 // bounds check and the conversion around each load a span waited for the one before it, and with the cells fetched by
 // two ds_bpermute each span's arithmetic came on top: [28672, 8192] bf16 took
-// 117-128 us, now 97 (602 MB: 6.2 TB/s).
+// 126 us, now 92-96 (602 MB: 6.3-6.5 TB/s).
 // Spans per workgroup (same shape): 1 / 2 / 4 / 8 took 110 / 97 / 92-96 / 101 us.
 constexpr int Q_SLOTS = 4;
 
 template <int THREADS, int DTYPE>
 __global__ __launch_bounds__(THREADS) void quantize_kernel(const void* __restrict__ w, int64_t n, int block_log2,
-                                                           uint8_t* __restrict__ packed, float* __restrict__ absmax) {
+                                                           uint8_t* __restrict__ packed, float* __restrict__ absmax,
+                                                           bool stream_in) {
     __shared__ float wave_max[Q_SLOTS][THREADS / 64];
     __shared__ uint2 cells[CODE_CELLS];
     const int tid = threadIdx.x;
@@ -127,9 +129,12 @@ __global__ __launch_bounds__(THREADS) void quantize_kernel(const void* __restric
     const int64_t first = (int64_t)blockIdx.x * (Q_SLOTS * THREADS * 8) + tid * 8;
     const bool whole = ((int64_t)blockIdx.x + 1) * (Q_SLOTS * THREADS * 8) <= n;
     Raw8<DTYPE> raw[Q_SLOTS];
-    if (whole) {
+    if (whole && stream_in) {
 #pragma unroll
-        for (int c = 0; c < Q_SLOTS; ++c) raw[c] = load8<DTYPE>(w, first + c * (THREADS * 8));
+        for (int c = 0; c < Q_SLOTS; ++c) raw[c] = load8<DTYPE, true>(w, first + c * (THREADS * 8));
+    } else if (whole) {
+#pragma unroll
+        for (int c = 0; c < Q_SLOTS; ++c) raw[c] = load8<DTYPE, false>(w, first + c * (THREADS * 8));
     } else {
 #pragma unroll
         for (int c = 0; c < Q_SLOTS; ++c) raw[c] = load8_edge<DTYPE>(w, first + c * (THREADS * 8), n);
@@ -234,8 +239,9 @@ __device__ __forceinline__ void dequant8_store(uint32_t word, float s, const flo
 // statistics, with one branch for the whole workgroup instead of one around each load.  An output that does not fit the
 // last-level cache (STREAM) has its codes read past the cache too; behind a smaller one they may stay there.
 // 16-bit outputs are packed by one conversion per two values.
+// A streamed output's first store waits for the last load (lm_head 213 -> 210 us; nested 215 -> 209).
 // us, with a check around every load and the codes always read past the cache -> now: [14336, 4096] bf16 39.5 -> 34.9 (of
-// which about 12 is the call), fp32 107 -> 102; nested [28672, 8192] bf16 112 -> 109.  Statistics first: 118 for the last.
+// which about 12 is the call), fp32 107 -> 102; nested [28672, 8192] bf16 99 -> 95 back to back.  Statistics first: 106 for the last.
 // Spans per workgroup 1 / 2 / 4 / 8: 132 / 134 / 115 / 120.
 // Nested absmax: the map is copied into LDS meanwhile, so that no load waits for another.  With the map looked up in
 // global memory (code -> map entry -> value, two dependent loads per span) the kernel took 175 us for that weight.
@@ -283,6 +289,7 @@ __global__ __launch_bounds__(256) void dequantize_kernel(const uint8_t* __restri
     }
     if (tid < 16) lut[tid] = lut_entry;
     if (NESTED) map[tid] = map_entry;
+    if (STREAM) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no store ahead of the last load
     __syncthreads();
 #pragma unroll
     for (int c = 0; c < DQ_SLOTS; ++c) {
@@ -553,10 +560,14 @@ void enqueue_quantize(const void* w, int64_t n, int block_log2, uint8_t* packed,
     const int threads = block_log2 == 12 ? 512 : 256;  // a span holds a whole block
     const int64_t per = (int64_t)threads * 8 * Q_SLOTS;
     const dim3 grid((unsigned)((n + per - 1) / per));
+    // A weight that does not fit the 256 MB last-level cache is read past it; of a smaller one that was just written, or is read
+    // again, much is still there
+    // (us back to back, past the cache / through it: [14336, 4096] bf16 29.1 / 25.7, fp32 53.0 / 42.3; [28672, 8192] bf16 96 / 109).
+    const bool stream_in = n * (DTYPE == F32 ? 4 : 2) > ((int64_t)256 << 20);
     if (threads == 512)
-        hipLaunchKernelGGL((quantize_kernel<512, DTYPE>), grid, dim3(512), 0, stream, w, n, block_log2, packed, absmax);
+        hipLaunchKernelGGL((quantize_kernel<512, DTYPE>), grid, dim3(512), 0, stream, w, n, block_log2, packed, absmax, stream_in);
     else
-        hipLaunchKernelGGL((quantize_kernel<256, DTYPE>), grid, dim3(256), 0, stream, w, n, block_log2, packed, absmax);
+        hipLaunchKernelGGL((quantize_kernel<256, DTYPE>), grid, dim3(256), 0, stream, w, n, block_log2, packed, absmax, stream_in);
 }
 
 hipError_t enqueue_compress(const float* absmax, int64_t nblocks, int nested_log2, const float* map256, const DqOffset& o,

@@ -134,8 +134,14 @@ def test_offset_of_more_values_than_one_round_of_loads(ta):
     n = 64 * (512 * 9300 + 5)
     w = torch.randn(n, device=DEV, dtype=torch.bfloat16)
     off = ta.functional.quantize_nf4_dq(w)[4]
-    absmax = ta.quantize_nf4(w)[1]
+    qw, absmax, code = ta.quantize_nf4(w)
     assert off.item() == float(absmax.cpu().double().mean().to(torch.float32))
+    # beyond the last-level cache weight and output are streamed past it: what a part alone, which is not, gives
+    m = 64 * 100_003
+    part = ta.quantize_nf4(w[-m:].clone())
+    assert torch.equal(part[0].flatten(), qw.flatten()[-m // 2:]) and torch.equal(part[1], absmax[-100_003:])
+    dense = ta.dequantize_nf4(qw, absmax, code, 64, torch.bfloat16, (n,))
+    assert torch.equal(dense[-m:], ta.dequantize_nf4(*part, 64, torch.bfloat16, (m,)))
 
 
 @pytest.mark.parametrize("n,blocksize,nested", [(7, 64, 256), (8192 + 8, 64, 64), (8192 * 5 + 3, 256, 256), (100_000, 64, 4096)])

@@ -585,9 +585,8 @@ def llama_decode(torch, ta, n_new: int) -> dict:
     out = {
         "model": "Llama-3-8B architecture (32 layers, d 4096, 32q/8kv heads, FFN 14336, vocab 128256), random init, "
                  "all 161 linears NF4 (QKV and gate/up fused, gate and up rows interleaved), prompt 512, greedy, HIP-graph decode step; "
-                 "decode_tok_per_s: residual add + RMSNorm + SiLU*up in the epilogues of the NF4 decode kernels (up to sixteen rows of x), "
-                 "rotary + cache + attention and sampling as HIP glue kernels; _separate_glue: all of that work as HIP glue kernels "
-                 "between the linears; _torch_glue: as PyTorch ops",
+                 "decode_tok_per_s: the whole step as one kernel, sampling as a second (beyond sixteen sequences as _separate_glue); _separate_glue: all "
+                 "work between the linears as HIP glue kernels; _torch_glue: as PyTorch ops",
         "new_tokens": n_new,
         "linear_weight_bytes_per_token": int(nweights * 0.5625),
         "hbm_bound_tok_per_s_batch1": round(HBM_PEAK_GBS * 1e9 / (nweights * 0.5625), 1),
@@ -597,9 +596,8 @@ def llama_decode(torch, ta, n_new: int) -> dict:
         prompt = torch.randint(0, cfg.vocab, (B, 512), generator=g, device=dev)
         D.greedy_decode(jm, cfg, prompt, n_new=1, use_graph=False)  # untimed: library start-up, GEMM heuristics
         res, toks = {}, {}
-        # the single-token step with residual add / RMSNorm / SiLU * up done by the epilogues of the NF4 decode kernels
-        # where those take them (up to sixteen rows of x; rotary + cache + attention and sampling as HIP glue kernels), with
-        # all of that work as HIP glue kernels of its own, and with plain PyTorch ops in its place
+        # the single-token step as one kernel (up to sixteen sequences), with all work between the linears as HIP glue
+        # kernels, and with plain PyTorch ops in their place
         for key, glue, epi in (("", True, True), ("_separate_glue", True, False), ("_torch_glue", False, False)):
             if (B > 8 and not glue) or (B > 16 and glue and not epi):
                 continue  # beyond sixteen rows of x the linears run as GEMMs, without epilogues: the first variant is the second

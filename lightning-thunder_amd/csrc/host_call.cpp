@@ -68,6 +68,7 @@ PyObject* matmul(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if (x->dim() < 1 || x->size(-1) != K || x->numel() == 0) Py_RETURN_NONE;
     const int64_t M = x->numel() / K;
     if (qweight->numel() < N * K / 2 || absmax->numel() < N * K / blocksize) Py_RETURN_NONE;
+    if (bias && bias->numel() != N) Py_RETURN_NONE;
     const at::Tensor* ws = nullptr;
     if (const size_t bytes = need(M, N, K)) {
         ws = args[10] == Py_None ? nullptr : plain(args[10], at::kByte);

@@ -518,7 +518,8 @@ def fused_route(x: torch.Tensor, bias, blocksize: int, dtype: torch.dtype, shape
     """
     N, K = shape
     M = x.numel() // K if K else 0
-    if x.dtype is not dtype or M <= 0 or N <= 0 or blocksize not in SUPPORTED_BLOCKSIZES or (bias is not None and bias.dtype is not dtype):
+    # (a bias of another size than N is torch's to broadcast or to refuse: the kernels read one value per weight row)
+    if x.dtype is not dtype or M <= 0 or N <= 0 or blocksize not in SUPPORTED_BLOCKSIZES or (bias is not None and (bias.dtype is not dtype or bias.numel() != N)):
         return "dequant+linear"
     if dtype is torch.float16:
         serves = (K % 64 == 0 and K % blocksize == 0 and _stream_takes(M, N, K, True) and _is_plain(x, bias)
@@ -663,10 +664,11 @@ def _matmul_nf4_on(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape,
 
 
 def linear_possible(x: torch.Tensor, w: torch.Tensor, bias=None) -> bool:
-    """Does ``linear_bf16`` take these operands (bf16, K a multiple of 64 and at least 128)?"""
+    """Does ``linear_bf16`` take these operands (bf16, K a multiple of 64 and at least 128, a bias of N values or none)?"""
     K = w.shape[-1]
     return (x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and (bias is None or bias.dtype == torch.bfloat16)
-            and w.dim() == 2 and x.shape[-1] == K and K % 64 == 0 and K >= 128 and x.numel() > 0 and w.numel() > 0)
+            and w.dim() == 2 and (bias is None or bias.numel() == w.shape[0])
+            and x.shape[-1] == K and K % 64 == 0 and K >= 128 and x.numel() > 0 and w.numel() > 0)
 
 
 def linear_bf16(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
@@ -674,8 +676,8 @@ def linear_bf16(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
     (``nf4hip_linear``): the GEMM that follows ``dequantize_nf4`` on the dequantize + linear route of
     bitsandbytes.matmul_4bit (MatMul4Bit.forward, reached from thunder/transforms/quantization.py:39).  ``w`` is [N, K]."""
     if not linear_possible(x, w, bias):
-        raise ValueError(f"linear_bf16: bf16 operands with K a multiple of 64 (>= 128) only, got x {tuple(x.shape)} {x.dtype}, "
-                         f"w {tuple(w.shape)} {w.dtype}")
+        raise ValueError(f"linear_bf16: bf16 operands with K a multiple of 64 (>= 128) and a bias of N values or none only, got x {tuple(x.shape)} "
+                         f"{x.dtype}, w {tuple(w.shape)} {w.dtype}, bias {None if bias is None else tuple(bias.shape)}")
     _require_gpu(x, w, bias)
     lib = _lib.load()
     N, K = w.shape
@@ -732,8 +734,8 @@ def matmul_nf4_epilogue(x, qweight, bias, absmax, quant_map, blocksize, dtype, s
     M = x2.shape[0]
     if isinstance(absmax, NestedAbsmax) or M > 16 or not x2.is_cuda:
         return None
-    if (x.dtype is not torch.bfloat16 or dtype is not torch.bfloat16 or (bias is not None and bias.dtype is not dtype) or M == 0 or N <= 0
-            or blocksize not in SUPPORTED_BLOCKSIZES or (N * K) % 2 or not _decode_takes(M, K, blocksize)):
+    if (x.dtype is not torch.bfloat16 or dtype is not torch.bfloat16 or (bias is not None and (bias.dtype is not dtype or bias.numel() != N))
+            or M == 0 or N <= 0 or blocksize not in SUPPORTED_BLOCKSIZES or (N * K) % 2 or not _decode_takes(M, K, blocksize)):
         return None
     lib = _lib.load()
     _require_gpu(x2, qweight, quant_map, bias, absmax)

@@ -5,7 +5,7 @@
 // interpreter, 5.3 this way, of which the launch is 2.9; a module around it 12.9 and 8.8.
 //
 // Only what can be handed over as it lies is taken: plain contiguous 16-byte aligned tensors of the expected types and
-// sizes, no transform, mode or capture of dispatch around them.  Anything else returns None and goes through the
+// sizes on x's device, no transform, mode or capture of dispatch around them.  Anything else returns None and goes through the
 // interpreter, which converts, copies or raises as ever.
 #define PY_SSIZE_T_CLEAN
 #include <ATen/ATen.h>
@@ -67,12 +67,14 @@ PyObject* matmul(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if (!x || !qweight || !absmax || !quant_map || (!bias && args[6] != Py_None)) Py_RETURN_NONE;
     if (x->dim() < 1 || x->size(-1) != K || x->numel() == 0) Py_RETURN_NONE;
     const int64_t M = x->numel() / K;
-    if (qweight->numel() < N * K / 2 || absmax->numel() < N * K / blocksize) Py_RETURN_NONE;
+    if (qweight->numel() < N * K / 2 || absmax->numel() < (N * K + blocksize - 1) / blocksize || quant_map->numel() < 16) Py_RETURN_NONE;
     if (bias && bias->numel() != N) Py_RETURN_NONE;
+    for (const at::Tensor* t : {qweight, absmax, quant_map, bias})
+        if (t && t->get_device() != x->get_device()) Py_RETURN_NONE;
     const at::Tensor* ws = nullptr;
     if (const size_t bytes = need(M, N, K)) {
         ws = args[10] == Py_None ? nullptr : plain(args[10], at::kByte);
-        if (!ws || (size_t)ws->numel() < bytes) Py_RETURN_NONE;
+        if (!ws || (size_t)ws->numel() < bytes || ws->get_device() != x->get_device()) Py_RETURN_NONE;
     }
 
     c10::SmallVector<int64_t, 5> sizes(x->sizes().begin(), x->sizes().end());

@@ -146,12 +146,33 @@ def _require_gpu(*tensors: torch.Tensor) -> None:
             raise RuntimeError(f"NF4 HIP ops need GPU tensors, got a tensor on {t.device}")
 
 
+def _require_device(device: torch.device, *tensors: torch.Tensor) -> None:
+    for t in tensors:
+        if t is not None and t.device != device:
+            raise RuntimeError(f"NF4 HIP ops need all operands on one device, got a tensor on {t.device} beside one on {device}")
+
+
 def _aligned(t: torch.Tensor) -> torch.Tensor:
     """Contiguous and 16-byte aligned view or copy of ``t``."""
     t = t.contiguous()
     if t.data_ptr() % 16:
         t = t.clone(memory_format=torch.contiguous_format)
     return t
+
+
+def _code_book(quant_map: torch.Tensor) -> torch.Tensor:
+    """``quant_map`` as the kernels read it: sixteen fp32 values."""
+    if quant_map.numel() < 16:
+        raise ValueError(f"quant_map holds {quant_map.numel()} values, need 16")
+    return _aligned(quant_map if quant_map.dtype is torch.float32 else quant_map.to(torch.float32))
+
+
+def _plain_absmax(absmax: torch.Tensor, nblocks: int, device: torch.device) -> torch.Tensor:
+    """fp32 statistics of ``nblocks`` blocks as the kernels read them."""
+    _require_device(device, absmax)
+    if absmax.numel() < nblocks:
+        raise ValueError(f"absmax holds {absmax.numel()} entries, need {nblocks}")
+    return _aligned(absmax if absmax.dtype is torch.float32 else absmax.to(torch.float32))
 
 
 def _check_blocksize(blocksize: int) -> None:
@@ -198,21 +219,19 @@ def dequantize_nf4(qweight, absmax, quant_map, blocksize, dtype, shape) -> torch
     qweight = _aligned(qweight)
     if qweight.numel() < (n + 1) // 2:
         raise ValueError(f"qweight holds {qweight.numel()} bytes, shape {shape} needs {(n + 1) // 2}")
-    quant_map = _aligned(quant_map.to(torch.float32))
+    _require_device(qweight.device, quant_map)
+    quant_map = _code_book(quant_map)
     nblocks = (n + blocksize - 1) // blocksize
     with _on_device(qweight.device):
         out = torch.empty(shape, dtype=dtype, device=qweight.device)
         if isinstance(absmax, NestedAbsmax):
-            nq = _nested_args(absmax, nblocks)
+            nq = _nested_args(absmax, nblocks, qweight.device)
             _lib.check(
                 lib.nf4hip_dequantize_dq(qweight.data_ptr(), nq[0].data_ptr(), nq[1].data_ptr(), nq[2].data_ptr(), nq[3], nq[4],
                                          quant_map.data_ptr(), n, blocksize, out.data_ptr(), _DTYPE_CODE[dtype], _stream())
             )  # fmt: skip
         else:
-            _require_gpu(absmax)
-            absmax = _aligned(absmax.to(torch.float32))
-            if absmax.numel() < nblocks:
-                raise ValueError(f"absmax holds {absmax.numel()} entries, need {nblocks}")
+            absmax = _plain_absmax(absmax, nblocks, qweight.device)
             _lib.check(
                 lib.nf4hip_dequantize(qweight.data_ptr(), absmax.data_ptr(), quant_map.data_ptr(), n, blocksize,
                                       out.data_ptr(), _DTYPE_CODE[dtype], _stream())
@@ -225,10 +244,14 @@ def dequantize_nf4(qweight, absmax, quant_map, blocksize, dtype, shape) -> torch
 # ------------------------------------------------------------------------------------------------
 
 
-def _nested_args(nq: NestedAbsmax, nblocks: int):
-    _require_gpu(nq.q, nq.absmax2, nq.map256)
+def _nested_args(nq: NestedAbsmax, nblocks: int, device: torch.device):
+    """Nested statistics of ``nblocks`` blocks as the kernels read them."""
+    _require_device(device, nq.q, nq.absmax2, nq.map256)
     if nq.q.numel() < nblocks:
         raise ValueError(f"nested absmax holds {nq.q.numel()} codes, need {nblocks}")
+    if nq.absmax2.numel() * nq.blocksize < nblocks or nq.map256.numel() < 256:
+        raise ValueError(f"nested absmax holds {nq.absmax2.numel()} values for blocks of {nq.blocksize} and a map of {nq.map256.numel()}, need "
+                         f"values for {nblocks} codes and a map of 256")
     return (_aligned(nq.q), _aligned(nq.absmax2.to(torch.float32)), _aligned(nq.map256.to(torch.float32)), float(nq.offset), int(nq.blocksize))
 
 
@@ -237,6 +260,10 @@ def compress_absmax(absmax: torch.Tensor, nested_blocksize: int = 256, map256: t
     The mean is taken in float64 and rounded to fp32 once, so it does not depend on reduction order."""
     _check_blocksize(nested_blocksize)
     _require_gpu(absmax)
+    if map256 is not None:
+        _require_device(absmax.device, map256)
+        if map256.numel() < 256:
+            raise ValueError(f"map256 holds {map256.numel()} values, need 256")
     lib = _lib.load()
     absmax = _aligned(absmax.to(torch.float32))
     nb = absmax.numel()
@@ -254,7 +281,8 @@ def compress_absmax(absmax: torch.Tensor, nested_blocksize: int = 256, map256: t
 def reconstruct_absmax(nq: NestedAbsmax) -> torch.Tensor:
     lib = _lib.load()
     nb = nq.q.numel()
-    q, a2, m, off, bs = _nested_args(nq, nb)
+    _require_gpu(nq.q)
+    q, a2, m, off, bs = _nested_args(nq, nb, nq.q.device)
     with _on_device(q.device):
         out = torch.empty(nb, dtype=torch.float32, device=q.device)
         _lib.check(lib.nf4hip_dq_reconstruct(q.data_ptr(), a2.data_ptr(), m.data_ptr(), off, nb, bs, out.data_ptr(), _stream()))
@@ -619,9 +647,10 @@ def _matmul_nf4_on(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape,
     qweight = _aligned(qweight)
     if qweight.numel() < N * K // 2:
         raise ValueError(f"qweight holds {qweight.numel()} bytes, shape {shape} needs {N * K // 2}")
-    quant_map = _aligned(quant_map if quant_map.dtype is torch.float32 else quant_map.to(torch.float32))
+    _require_device(device, qweight, quant_map, bias)
+    quant_map = _code_book(quant_map)
     b = None if bias is None else bias.contiguous()
-    nblocks = N * K // blocksize
+    nblocks = -(-N * K // blocksize)  # (up to four rows of x a block may straddle weight rows, and the last may be cut off)
     out = x2.new_empty((M, N)) if type(x2) is torch.Tensor else torch.empty((M, N), dtype=x.dtype, device=device)
     if route == "gemv":
         need = lib.nf4hip_gemv_workspace_bytes(M, N, K)
@@ -642,14 +671,11 @@ def _matmul_nf4_on(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape,
                  or ((blocksize == 128 or K % 256) and lib.nf4hip_gemm_us(M, N, K) > NESTED_RECONSTRUCT_MIN_US))):
         absmax, nested = reconstruct_absmax(absmax), False
     if nested:
-        q, a2, m256, off, nbs = _nested_args(absmax, nblocks)
+        q, a2, m256, off, nbs = _nested_args(absmax, nblocks, device)
         rc = fn_dq(x_ptr, code, M, qweight.data_ptr(), q.data_ptr(), a2.data_ptr(), m256.data_ptr(), off, nbs,
                    quant_map.data_ptr(), bptr, N, K, blocksize, out_ptr, ws_ptr, ws_bytes, stream)  # fmt: skip
     else:
-        _require_gpu(absmax)
-        absmax = _aligned(absmax if absmax.dtype is torch.float32 else absmax.to(torch.float32))
-        if absmax.numel() < nblocks:
-            raise ValueError(f"absmax holds {absmax.numel()} entries, need {nblocks}")
+        absmax = _plain_absmax(absmax, nblocks, device)
         rc = fn(x_ptr, code, M, qweight.data_ptr(), absmax.data_ptr(), quant_map.data_ptr(), bptr,
                 N, K, blocksize, out_ptr, ws_ptr, ws_bytes, stream)  # fmt: skip
     if ws is None and need:
@@ -738,11 +764,11 @@ def matmul_nf4_epilogue(x, qweight, bias, absmax, quant_map, blocksize, dtype, s
             or M == 0 or N <= 0 or blocksize not in SUPPORTED_BLOCKSIZES or (N * K) % 2 or not _decode_takes(M, K, blocksize)):
         return None
     lib = _lib.load()
-    _require_gpu(x2, qweight, quant_map, bias, absmax)
+    _require_device(x2.device, qweight, quant_map, bias)
     x2, qweight = _aligned(x2), _aligned(qweight)
-    quant_map, absmax = _aligned(quant_map.to(torch.float32)), _aligned(absmax.to(torch.float32))
-    if qweight.numel() < N * K // 2 or absmax.numel() < N * K // blocksize:
-        raise ValueError(f"qweight / absmax hold {qweight.numel()} / {absmax.numel()} entries, too few for {shape}")
+    if qweight.numel() < N * K // 2:
+        raise ValueError(f"qweight holds {qweight.numel()} bytes, too few for {shape}")
+    quant_map, absmax = _code_book(quant_map), _plain_absmax(absmax, -(-N * K // blocksize), x2.device)
     b = None if bias is None else bias.contiguous()
     epi = _lib.Epilogue()
     keep = []  # tensors whose addresses the struct holds

@@ -203,7 +203,8 @@ class Llama(nn.Module):
         cfg = self.cfg
         B, d, hd, eps = x.shape[0], cfg.d_model, cfg.head_dim, cfg.norm_eps
         shape = (cfg.n_layer, B, cfg.n_kv_head, cfg.max_seq, 128)
-        if hd != 128 or tuple(kcache.shape) != shape or tuple(vcache.shape) != shape:
+        # (a list of one tensor per layer is served launch by launch)
+        if hd != 128 or any(not isinstance(c, torch.Tensor) or tuple(c.shape) != shape for c in (kcache, vcache)):
             return None
         lins = [l for blk in self.blocks for l in (blk.attn.qkv_proj, blk.attn.o_proj, blk.mlp.gate_up_proj, blk.mlp.down_proj)] + [self.lm_head]
         shapes = [((cfg.n_head + 2 * cfg.n_kv_head) * hd, d), (cfg.n_head * hd, d), (2 * cfg.d_ff, d), (d, cfg.d_ff)] * cfg.n_layer + [(cfg.vocab, d)]

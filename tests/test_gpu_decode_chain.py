@@ -215,3 +215,25 @@ def test_chain_infinities_and_nan(D, ta, chain_calls):
             out = model(tok, pos, kc.clone(), v)
             assert out[1].isnan().all()  # (an infinite residual has an infinite rms)
             assert torch.equal(out[[0, 2, 3]], ref[[0, 2, 3]])
+
+
+def test_caches_of_one_tensor_per_layer_are_left_to_the_launches(D):
+    cfg = D.LlamaConfig(n_layer=2, d_model=1024, n_head=8, n_kv_head=2, d_ff=256, vocab=64, max_seq=16, fused_projections=True, hip_glue=True,
+                        gate_up_interleaved=True)
+    model = D.build_llama(cfg, device="cpu")
+    kc, vc = D.new_caches(cfg, 1, "cpu")
+    for k, v in ((list(kc), list(vc)), (tuple(kc), vc), (kc, list(vc))):
+        assert model._decode_step_chain(torch.zeros(1, 1024, dtype=torch.bfloat16), torch.zeros(1, dtype=torch.long), k, v) is None
+
+
+@pytest.mark.gpu
+def test_caches_of_one_tensor_per_layer(D, ta, chain_calls, monkeypatch):
+    cfg, model, kc, vc, tok = _model(D, ta, 5, 2, 1024, 2048, 1000, 64)
+    pos = torch.full((1,), 30, device=DEV, dtype=torch.long)
+    kl, vl = [c.clone() for c in kc], [c.clone() for c in vc]
+    with torch.no_grad():
+        got = model(tok, pos, kl, vl)
+        assert chain_calls["n"] == 0
+        monkeypatch.setattr(D.Llama, "_decode_step_chain", lambda *a: None)
+        ref = model(tok, pos, kc, vc)
+    assert torch.equal(got, ref) and torch.equal(torch.stack(kl), kc) and torch.equal(torch.stack(vl), vc)

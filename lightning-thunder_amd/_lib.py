@@ -12,6 +12,7 @@ import importlib.machinery
 import importlib.util
 import os
 import threading
+import warnings
 
 ABI_VERSION = 6
 
@@ -129,20 +130,30 @@ def load(path: str | None = None) -> ctypes.CDLL:
         if got != ABI_VERSION:
             raise RuntimeError(f"{p}: ABI version {got}, host code expects {ABI_VERSION}")
         address = lambda name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value  # noqa: E731
-        lib.host_matmul = _load_host().matmul
+        lib.host_matmul = _load_host_matmul()
         lib.host_calls = {name: (address(name), address(need)) for name, need in HOST_CALLS.items()}
         if path is None:
             _lib = lib
         return lib
 
 
-def _load_host():
-    if not os.path.exists(HOST_PATH):
-        raise RuntimeError(f"{HOST_PATH} not found: the extension has not been built (`make -C lightning-thunder_amd/csrc`)")
-    loader = importlib.machinery.ExtensionFileLoader("nf4hip_host", HOST_PATH)
-    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("nf4hip_host", loader))
-    loader.exec_module(module)
-    return module
+def _load_host_matmul():
+    """``matmul`` of nf4hip_host.so.  That library only shortens the host side of a call: where it is missing, or was built
+    against another torch, a warning says so and every matmul goes through the interpreter, to the same kernels."""
+    import torch
+
+    try:
+        if not os.path.exists(HOST_PATH):
+            raise ImportError(f"{HOST_PATH} not found")
+        loader = importlib.machinery.ExtensionFileLoader("nf4hip_host", HOST_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("nf4hip_host", loader))
+        loader.exec_module(module)
+        if not torch.__version__.startswith(module.torch_version):
+            raise ImportError(f"{HOST_PATH} was built for torch {module.torch_version}, this is {torch.__version__}")
+        return module.matmul
+    except ImportError as e:
+        warnings.warn(f"{e}: NF4 matmul calls take the slower way through the interpreter (`make -C lightning-thunder_amd/csrc`)", stacklevel=3)
+        return lambda *args: None
 
 
 def check(rc: int) -> None:

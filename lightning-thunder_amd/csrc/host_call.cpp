@@ -13,6 +13,7 @@
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/version.h>
 
 #include <cstdint>
 
@@ -101,4 +102,11 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "nf4hip_host", nullptr, -1, methods
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit_nf4hip_host() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit_nf4hip_host() {
+    PyObject* const m = PyModule_Create(&module);
+    if (m && PyModule_AddStringConstant(m, "torch_version", TORCH_VERSION) < 0) {
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
+}

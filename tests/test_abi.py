@@ -366,3 +366,20 @@ def test_gemm_insists_on_the_workspace_of_its_plan(ta):
         assert gemm(M, N, K, None, 0) == L.E_WORKSPACE and gemm(M, N, K, A, need - 1) == L.E_WORKSPACE and str(need) in _err(ta)
         assert gemm(M, N, K, A + 8, need) == L.E_ALIGN
     assert lib.nf4hip_gemm_workspace_bytes(512, 4096, 4096) == 0  # 256 workgroups without a split of K
+
+
+def test_without_the_native_host_side(ta, monkeypatch, tmp_path):
+    """nf4hip_host.so missing, unreadable or built for another torch: a warning, and the library loads with everything but that."""
+    import torch
+
+    L = ta._lib
+    (tmp_path / "broken.so").write_bytes(b"not a library")
+    for path, version, why in ((tmp_path / "none.so", torch.__version__, "not found"), (tmp_path / "broken.so", torch.__version__, "broken.so"),
+                               (L.HOST_PATH, "1.0.0", "built for torch")):
+        with monkeypatch.context() as m:
+            m.setattr(L, "HOST_PATH", str(path))
+            m.setattr(torch, "__version__", version)
+            with pytest.warns(UserWarning, match=why):
+                lib = L.load(L.LIB_PATH)
+        assert lib.host_matmul(*range(12)) is None and lib.nf4hip_abi_version() == L.ABI_VERSION and set(lib.host_calls) == set(L.HOST_CALLS)
+    assert L.load(L.LIB_PATH).host_matmul(0, 0, *[None] * 5, 1, 1, 64, None, 0) is None  # (the native step itself: nothing to call)

@@ -619,8 +619,8 @@ def _matmul_nf4_on(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape,
 
     A decode call on a small weight is as long as this function, so what needs no conversion is handed to the library in one native
     step (csrc/host_call.cpp; [4096, 4096], one row, 4.6 us of kernel: ``matmul_nf4`` 9.5 -> 5.3 us, of which the launch is 2.9).  What that
-    step does not take -- nested statistics, views, other types, a stream without a workspace, tensors inside a transform -- comes
-    back and is served below."""
+    step does not take -- views, other types, a stream without a workspace, tensors inside a transform -- comes back and is
+    served below, as are nested statistics, which it is not asked for."""
     N, K = shape
     if route in ("dequant+linear", "dequant+gemm", "dequant+libgemm"):
         w = dequantize_nf4(qweight, absmax, quant_map, blocksize, dtype, shape).to(x.dtype)
@@ -634,13 +634,15 @@ def _matmul_nf4_on(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape,
             return _matmul_nf4_on(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape, route)
     lib = _lib.load()
     stream = _stream() if _raw_stream is None else _raw_stream(device.index)
-    entry = "nf4hip_gemv" if route == "gemv" else "nf4hip_stream" if x.dtype is torch.float16 else "nf4hip_gemm"
-    out = lib.host_matmul(*lib.host_calls[entry], x, qweight, absmax, quant_map, bias, N, K, blocksize,
-                          _workspace_pool.peek(device.index, stream), stream)  # fmt: skip
-    if out is not None:
-        if type(out) is int:
-            _lib.check(out)
-        return out
+    nested = isinstance(absmax, NestedAbsmax)
+    if not nested:
+        entry = "nf4hip_gemv" if route == "gemv" else "nf4hip_stream" if x.dtype is torch.float16 else "nf4hip_gemm"
+        out = lib.host_matmul(*lib.host_calls[entry], x, qweight, absmax, quant_map, bias, N, K, blocksize,
+                              _workspace_pool.peek(device.index, stream), stream)  # fmt: skip
+        if out is not None:
+            if type(out) is int:
+                _lib.check(out)
+            return out
     flat = x.dim() == 2
     x2 = _aligned(x if flat else x.reshape(-1, K))
     M = x2.shape[0]
@@ -665,7 +667,6 @@ def _matmul_nf4_on(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape,
     ws_ptr, ws_bytes = (None, 0) if ws is None else (ws.data_ptr(), ws.numel())
     bptr = None if b is None else b.data_ptr()
     code, x_ptr, out_ptr = _DTYPE_CODE[x.dtype], x2.data_ptr(), out.data_ptr()
-    nested = isinstance(absmax, NestedAbsmax)
     if (nested and route != "gemv" and M > NESTED_RECONSTRUCT_MIN_M
             and (not (route == "stream" or lib.nf4hip_gemm_streamed(M, N, K))
                  or ((blocksize == 128 or K % 256) and lib.nf4hip_gemm_us(M, N, K) > NESTED_RECONSTRUCT_MIN_US))):

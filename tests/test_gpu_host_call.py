@@ -60,6 +60,16 @@ def test_same_bits(ta, both, dtype, lead, N, K, biased):
     assert taken == 1 or lead == (192,)
 
 
+def test_nested_statistics_are_not_asked_about(ta, monkeypatch):
+    asked = []
+    monkeypatch.setattr(ta._lib.load(), "host_matmul", lambda *args: asked.append(1))
+    qw, *nested, code = ta.functional.quantize_nf4_dq((torch.randn(512, 1024, device=DEV) * 0.02).bfloat16())
+    for M in (1, 45):
+        x = torch.randn(M, 1024, device=DEV).bfloat16()
+        ta.functional.matmul_nf4_dq(x, qw, None, *nested, code, 64, 256, torch.bfloat16, (512, 1024))
+    assert not asked
+
+
 def test_not_taken(ta, both):
     N, K = 512, 1024
     qw, absmax, code = _weight(ta, N, K)

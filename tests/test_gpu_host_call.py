@@ -44,20 +44,21 @@ def both(ta, monkeypatch):
     (torch.bfloat16, (2, 8), 4096, 4096, True),     # three dimensions
     (torch.bfloat16, (), 512, 1024, False),         # a vector
     (torch.bfloat16, (45,), 5003, 2880, True),      # streaming kernel
-    (torch.bfloat16, (192,), 512, 1024, False),     # prompt
+    (torch.bfloat16, (192,), 512, 1024, False),     # prompt, kept on the fused route
     (torch.float16, (4,), 1024, 1024, True),
 ])  # fmt: skip
-def test_same_bits(ta, both, dtype, lead, N, K, biased):
+def test_same_bits(ta, both, monkeypatch, dtype, lead, N, K, biased):
     print(f"host call {dtype} {lead} [{N}, {K}]", flush=True)
     qw, absmax, code = _weight(ta, N, K, dtype)
     x = torch.randn(*lead, K, device=DEV).to(dtype)
     bias = torch.randn(N, device=DEV).to(dtype) if biased else None
     args = (qw, bias, absmax, code, 64, dtype, (N, K))
-    ta.matmul_nf4(x, *args)  # (the stream's scratch, the measured route)
+    if lead == (192,):  # (whatever the dense route's time is on this card)
+        monkeypatch.setitem(ta.functional._route_measured, ta.functional._route_key(x.device, 192, N, K, 64, False, False), "gemm")
+    ta.matmul_nf4(x, *args)  # (the stream's scratch)
     a, taken, b = both(lambda: ta.matmul_nf4(x, *args))
     assert torch.equal(a, b) and a.shape == (*lead, N) and a.dtype is dtype and a.is_contiguous()
-    # (where a prompt's measured route writes the dense weight, nothing is asked)
-    assert taken == 1 or lead == (192,)
+    assert taken == 1
 
 
 def test_nested_statistics_are_not_asked_about(ta, monkeypatch):

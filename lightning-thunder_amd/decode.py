@@ -194,14 +194,12 @@ class Llama(nn.Module):
         return self.lm_head(glue.add_rmsnorm(x, delta, self.norm_f.weight, eps))
 
     def _decode_step_chain(self, x, pos, kcache, vcache):
-        """The single-token forward as one kernel: the operator calls of ``_decode_step_epilogues``, on a ``glue.DecodeChain`` in the
-        place of activations, which collects them and launches them together.  Returns None (before anything is launched)
-        unless every linear runs as the 4-bit operator with fp32 absmax, without a bias, at shapes the kernel takes."""
+        """The single-token forward as one kernel (``glue.decode_chain``).  Returns None (before anything is launched) unless every
+        linear runs as the 4-bit operator with fp32 absmax, without a bias, at shapes the kernel takes."""
         from . import glue
-        from .transforms import quantization as Q
 
         cfg = self.cfg
-        B, d, hd, eps = x.shape[0], cfg.d_model, cfg.head_dim, cfg.norm_eps
+        B, d, hd = x.shape[0], cfg.d_model, cfg.head_dim
         shape = (cfg.n_layer, B, cfg.n_kv_head, cfg.max_seq, 128)
         # (a list of one tensor per layer is served launch by launch)
         if hd != 128 or any(not isinstance(c, torch.Tensor) or tuple(c.shape) != shape for c in (kcache, vcache)):
@@ -211,20 +209,12 @@ class Llama(nn.Module):
         planned = [_planned_nf4(l) for l in lins]
         if any(a is None or a[1] is not None or a[4] != 64 or a[5] != torch.bfloat16 or tuple(a[6]) != s for a, s in zip(planned, shapes)):
             return None
+        linears = [(a[0], a[2], a[3]) for a in planned]
         norms = [w for blk in self.blocks for w in (blk.norm_1.weight, blk.norm_2.weight)] + [self.norm_f.weight]
-        if not glue.decode_chain_takes(x, [(a[0], a[2], a[3]) for a in planned], norms, pos, self.rope_cos, self.rope_sin, kcache, vcache, cfg.n_head,
-                                       cfg.d_ff, cfg.vocab):
+        if not glue.decode_chain_takes(x, linears, norms, pos, self.rope_cos, self.rope_sin, kcache, vcache, cfg.n_head, cfg.d_ff, cfg.vocab):
             return None
-        ep = Q.hip_matmul_nf4_epilogue
-        chain = glue.DecodeChain(x, norms[0], eps, pos, self.rope_cos, self.rope_sin, kcache, vcache, cfg.n_head, cfg.n_kv_head)
-        r = xn = ss = chain
-        for i in range(cfg.n_layer):
-            qkv, o, gate_up, down = planned[4 * i: 4 * i + 4]
-            y = chain.attention(ep(xn, *qkv, rowscale=(ss, eps)) if i else chain.linear(*qkv))
-            r, xn, ss = ep(y, *o, resid_norm=(r, norms[2 * i + 1]))
-            h = ep(xn, *gate_up, rowscale=(ss, eps), silu_pairs=True)
-            r, xn, ss = ep(h, *down, resid_norm=(r, norms[2 * i + 2]))
-        return ep(xn, *planned[-1], rowscale=(ss, eps)).launch()
+        return glue.decode_chain(x, linears, norms, cfg.norm_eps, pos, self.rope_cos, self.rope_sin, kcache, vcache, cfg.n_head, cfg.n_kv_head,
+                                 cfg.d_ff, cfg.vocab)
 
     def _decode_step_epilogues(self, x, pos, kcache, vcache):
         """The single-token forward with the neighbours of every linear done in that linear's epilogue

@@ -166,32 +166,6 @@ def decode_chain_takes(x, linears, norms, pos, cos, sin, kcache, vcache, n_head:
         return load().nf4hip_decode_chain_workspace_bytes(B, n_layer, x.shape[1], n_head, Hkv, d_ff, vocab, max_seq) > 0
 
 
-class DecodeChain:
-    """Stands for every activation of a decode step that runs as one kernel: given as ``x`` to ``hip_matmul_nf4_epilogue`` it
-    takes down the linear and the norm weight behind it and is the result as well; ``launch`` runs the step
-    (``decode_chain``).  The order is the decoder's: per layer QKV, attention, output projection, gate-up, down, then the head."""
-
-    def __init__(self, x, norm_first, eps, pos, cos, sin, kcache, vcache, n_head: int, n_kv_head: int):
-        self.args = (eps, pos, cos, sin, kcache, vcache, n_head, n_kv_head)
-        self.x, self.linears, self.norms, self.shapes = x, [], [norm_first], []
-
-    def linear(self, qweight, bias, absmax, quant_map, blocksize, dtype, shape, rowscale=None, silu_pairs=False, resid_norm=None):
-        if bias is not None or blocksize != 64 or dtype != torch.bfloat16:
-            raise ValueError("a decode chain takes 4-bit bf16 linears in blocks of 64, without a bias")
-        self.linears.append((qweight, absmax, quant_map))
-        self.shapes.append(tuple(shape))
-        if resid_norm is None:
-            return self
-        self.norms.append(resid_norm[1])
-        return self, self, self
-
-    def attention(self, qkv):
-        return self
-
-    def launch(self) -> torch.Tensor:
-        return decode_chain(self.x, self.linears, self.norms, *self.args, self.shapes[3][1], self.shapes[-1][0])
-
-
 def decode_chain(x: torch.Tensor, linears, norms, eps: float, pos: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, kcache: torch.Tensor,
                  vcache: torch.Tensor, n_head: int, n_kv_head: int, d_ff: int, vocab: int, max_workgroups: int = 0) -> torch.Tensor:
     """A whole decode step from the embedded tokens ``x`` [B, d] to the logits [B, vocab] (``nf4hip_decode_chain``).

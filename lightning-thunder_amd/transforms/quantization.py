@@ -18,7 +18,7 @@ from collections.abc import Sequence
 
 import torch
 
-from .. import extend, functional, glue
+from .. import extend, functional
 from ..trace import (
     STATIC_MEMORY_LOCATION,
     TensorProxy,
@@ -111,10 +111,7 @@ def hip_matmul_nf4_epilogue_impl(x, qweight, bias, absmax, quant_map, blocksize,
     """``hip_matmul_nf4`` with the decoder layer's neighbouring step done in the kernel's epilogue
     (``functional.matmul_nf4_epilogue``).  Where the kernels do not serve the case (more than sixteen rows of x, nested
     absmax, a shape outside their rules) the operator runs ``hip_matmul_nf4`` and the step by itself, with the same
-    roundings of stored tensors, so that it always returns what its meta function describes.  A ``glue.DecodeChain`` as ``x``
-    takes the call down, to run it with the rest of its decode step."""
-    if isinstance(x, glue.DecodeChain):
-        return x.linear(qweight, bias, absmax, quant_map, blocksize, dtype, shape, rowscale, silu_pairs, resid_norm)
+    roundings of stored tensors, so that it always returns what its meta function describes."""
     got = functional.matmul_nf4_epilogue(x, qweight, bias, absmax, quant_map, blocksize, dtype, shape, rowscale=rowscale,
                                          silu_pairs=silu_pairs, resid_norm=resid_norm)
     if got is not None:

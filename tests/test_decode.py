@@ -84,14 +84,15 @@ def test_quantized_decode_graph_equals_eager(D, ta, fused, batch):
 
 
 @pytest.mark.gpu
-def test_llama3_8b_full_size_decode(D, ta):
+def test_llama3_8b_full_size_decode(D, ta, monkeypatch):
     """The benchmark's model at full size, as the benchmark builds it: 32 layers, d = 4096, 32 / 8 heads, FFN 14336,
     vocab 128256, Q/K/V and gate/up as one linear each with gate and up rows interleaved, every linear NF4-quantized
-    through the transform, prompts of 512 random token ids, batch 1 and 8.  Both single-token steps are run: the one
-    whose tok/s the benchmark reports (``linear_epilogues``: residual add, RMSNorm and SiLU * up in the epilogues of the
-    decode kernels, five launches per layer) and the one with that work as glue kernels of their own.  For each, the
-    HIP-graph replay of the step must give the tokens of the eager loop, token for token; the two steps must give each
-    other's tokens unless the logits they disagree on are a tie within the matmul's tolerance.
+    through the transform, prompts of 512 random token ids, batch 1 and 8.  All three single-token steps are run: the one
+    whose tok/s the benchmark reports (the whole step as one kernel), the one that models take which that kernel does not serve
+    (residual add, RMSNorm and SiLU * up in the epilogues of the decode kernels, five launches per layer) and the one with that
+    work as glue kernels of their own.  For each, the HIP-graph replay of the step must give the tokens of the eager loop, token
+    for token; the others must give the first one's tokens unless the logits they disagree on are a tie within the matmul's
+    tolerance.
 
     Logits (prefill, then one decode step on the caches the prefill wrote) are judged against the SAME model in
     fp32 -- dequantized weights, fp32 activations, plain PyTorch -- next to a plain PyTorch bf16 model on the same
@@ -132,24 +133,30 @@ def test_llama3_8b_full_size_decode(D, ta):
         assert rms_a <= 1.5 * rms_b + 1e-3, f"{what}: rms error {rms_a:.4f} vs PyTorch bf16 {rms_b:.4f}"
         assert max_a <= 1.5 * max_b + 1e-2, f"{what}: max error {max_a:.4f} vs PyTorch bf16 {max_b:.4f}"
 
-    def launches_of_a_step(batch):
-        """How many times the step calls the epilogue operator (counted on one eager step)."""
+    def calls_of_a_step(batch):
+        """How many times the step calls the one-kernel step and the epilogue operator (counted on one eager step)."""
         from importlib import import_module
 
-        Q = import_module("lightning-thunder_amd.transforms.quantization")
-        real, n = Q.hip_matmul_nf4_epilogue, [0]
+        Q, glue = import_module("lightning-thunder_amd.transforms.quantization"), import_module("lightning-thunder_amd.glue")
+        n = {"chain": 0, "epilogue": 0}
 
-        def counting(*a, **k):
-            n[0] += 1
-            return real(*a, **k)
+        def counting(key, real):
+            def call(*a, **k):
+                n[key] += 1
+                return real(*a, **k)
 
-        Q.hip_matmul_nf4_epilogue = counting
-        try:
+            return call
+
+        with monkeypatch.context() as m:
+            m.setattr(Q, "hip_matmul_nf4_epilogue", counting("epilogue", Q.hip_matmul_nf4_epilogue))
+            m.setattr(glue, "decode_chain", counting("chain", glue.decode_chain))
             kc, vc = D.new_caches(cfg, batch, dev)
             jm(torch.zeros(batch, 1, dtype=torch.long, device=dev), torch.zeros(1, dtype=torch.long, device=dev), kc, vc)
-        finally:
-            Q.hip_matmul_nf4_epilogue = real
-        return n[0]
+        return n["chain"], n["epilogue"]
+
+    # the step under test is the one it claims to be: one call for all of it; 4 x 32 + 1 epilogue calls, less the first QKV; neither
+    steps = {"one kernel": (1, 0), "epilogues": (0, 32 * 4), "separate glue kernels": (0, 0)}
+    chain_step = D.Llama._decode_step_chain
 
     g = torch.Generator().manual_seed(4001)
     for batch in (1, 8):
@@ -163,48 +170,49 @@ def test_llama3_8b_full_size_decode(D, ta):
         tok = c.argmax(-1, keepdim=True)
         b1, c1 = ref(tok, pos1, kr, vr), ref32(tok, pos1, k32, v32)
         tokens, step_logits = {}, {}
-        for epilogues in (True, False):
-            cfg.linear_epilogues = epilogues
-            what = "epilogues" if epilogues else "separate glue kernels"
+        for what, calls in steps.items():
+            cfg.linear_epilogues = what != "separate glue kernels"
+            monkeypatch.setattr(D.Llama, "_decode_step_chain", chain_step if what == "one kernel" else lambda *a: None)
             print(f"  batch {batch}, {what}", flush=True)
-            # the step under test is the one it claims to be: 4 x 32 + 1 epilogue calls, less the first QKV, or none
-            assert launches_of_a_step(batch) == (32 * 4 if epilogues else 0)
+            assert calls_of_a_step(batch) == calls
             eager, s0 = D.greedy_decode(jm, cfg, prompt, n_new=8, use_graph=False)
             graph, s1 = D.greedy_decode(jm, cfg, prompt, n_new=8, use_graph=True)
             assert s1["graph"] and not s0["graph"]
             assert torch.equal(eager, graph), f"{what}: graph replay and eager decode disagree"
             assert int(eager.min()) >= 0 and int(eager.max()) < cfg.vocab
-            tokens[epilogues] = eager
+            tokens[what] = eager
             kc, vc = D.new_caches(cfg, batch, dev)
             a = jm(prompt, pos, kc, vc)
-            if epilogues:
+            if what == "one kernel":
                 judge(a, b, c, f"prefill, batch {batch}")
-            step_logits[epilogues] = jm(tok, pos1, kc, vc)
-            judge(step_logits[epilogues], b1, c1, f"decode step ({what}), batch {batch}")
+            step_logits[what] = jm(tok, pos1, kc, vc)
+            judge(step_logits[what], b1, c1, f"decode step ({what}), batch {batch}")
         cfg.linear_epilogues = True
-        # the two steps against each other: the same tokens, except where a sequence's two best logits are closer
+        monkeypatch.setattr(D.Llama, "_decode_step_chain", chain_step)
+        # the steps against the first: the same tokens, except where a sequence's two best logits are closer
         # than the two evaluations are to each other (from there on the sequences differ and are not compared)
         # (their logits differ like two correct bf16 evaluations of 32 layers do: by no more than twice PyTorch's own
         # bf16 error against fp32)
-        between = float((step_logits[True].float() - step_logits[False].float()).pow(2).mean().sqrt())
         torch_err = float((b1.float() - c1.float()).pow(2).mean().sqrt())
-        print(f"  batch {batch}: rms between the two steps' logits {between:.4f}, PyTorch bf16 vs fp32 {torch_err:.4f}", flush=True)
-        assert between <= 2.0 * torch_err, f"the two steps' logits differ by {between:.4f} rms (PyTorch bf16 vs fp32: {torch_err:.4f})"
-        for s in range(batch):
-            ta_, tb_ = tokens[True][s], tokens[False][s]
-            if torch.equal(ta_, tb_):
-                continue
-            i = int((ta_ != tb_).nonzero()[0])
-            assert i >= 1, "the first token comes from the prefill, which the two steps share"
-            # replay both variants on the common prefix and look at the logits of the two candidates
-            seq = torch.cat([prompt[s:s + 1], ta_[None, :i]], dim=1)
-            kc, vc = D.new_caches(cfg, 1, dev)
-            jm(seq[:, :-1], torch.arange(seq.shape[1] - 1, device=dev), kc, vc)
-            lg = jm(seq[:, -1:], torch.full((1,), seq.shape[1] - 1, device=dev, dtype=torch.long), kc, vc).float()[0]
-            gap = abs(float(lg[ta_[i]] - lg[tb_[i]]))
-            print(f"  batch {batch} sequence {s}: the two steps part at token {i}, logit gap {gap:.4f}", flush=True)
-            # a tie: the candidates' logits are no further apart than evaluations are from each other.  `between` is
-            # the rms of one logit's difference between two evaluations; the difference of TWO logits (candidate a
-            # minus candidate b) then varies by sqrt(2) * between from one evaluation to another, the steps disagree
-            # when the true gap is inside that, and the gap is measured here by a third evaluation: 3 sigma of that.
-            assert gap <= 3.0 * 2.0 ** 0.5 * between, f"sequence {s}: the two steps disagree at token {i} with a logit gap of {gap:.4f}"
+        for other in ("epilogues", "separate glue kernels"):
+            between = float((step_logits["one kernel"].float() - step_logits[other].float()).pow(2).mean().sqrt())
+            print(f"  batch {batch}: rms between the logits of one kernel and {other} {between:.4f}, PyTorch bf16 vs fp32 {torch_err:.4f}", flush=True)
+            assert between <= 2.0 * torch_err, f"the two steps' logits differ by {between:.4f} rms (PyTorch bf16 vs fp32: {torch_err:.4f})"
+            for s in range(batch):
+                ta_, tb_ = tokens["one kernel"][s], tokens[other][s]
+                if torch.equal(ta_, tb_):
+                    continue
+                i = int((ta_ != tb_).nonzero()[0])
+                assert i >= 1, "the first token comes from the prefill, which the two steps share"
+                # replay both variants on the common prefix and look at the logits of the two candidates
+                seq = torch.cat([prompt[s:s + 1], ta_[None, :i]], dim=1)
+                kc, vc = D.new_caches(cfg, 1, dev)
+                jm(seq[:, :-1], torch.arange(seq.shape[1] - 1, device=dev), kc, vc)
+                lg = jm(seq[:, -1:], torch.full((1,), seq.shape[1] - 1, device=dev, dtype=torch.long), kc, vc).float()[0]
+                gap = abs(float(lg[ta_[i]] - lg[tb_[i]]))
+                print(f"  batch {batch} sequence {s}: the two steps part at token {i}, logit gap {gap:.4f}", flush=True)
+                # a tie: the candidates' logits are no further apart than evaluations are from each other.  `between` is
+                # the rms of one logit's difference between two evaluations; the difference of TWO logits (candidate a
+                # minus candidate b) then varies by sqrt(2) * between from one evaluation to another, the steps disagree
+                # when the true gap is inside that, and the gap is measured here by a third evaluation: 3 sigma of that.
+                assert gap <= 3.0 * 2.0 ** 0.5 * between, f"sequence {s}: the two steps disagree at token {i} with a logit gap of {gap:.4f}"

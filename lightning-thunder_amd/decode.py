@@ -204,17 +204,23 @@ class Llama(nn.Module):
         # (a list of one tensor per layer is served launch by launch)
         if hd != 128 or any(not isinstance(c, torch.Tensor) or tuple(c.shape) != shape for c in (kcache, vcache)):
             return None
-        lins = [l for blk in self.blocks for l in (blk.attn.qkv_proj, blk.attn.o_proj, blk.mlp.gate_up_proj, blk.mlp.down_proj)] + [self.lm_head]
-        shapes = [((cfg.n_head + 2 * cfg.n_kv_head) * hd, d), (cfg.n_head * hd, d), (2 * cfg.d_ff, d), (d, cfg.d_ff)] * cfg.n_layer + [(cfg.vocab, d)]
-        planned = [_planned_nf4(l) for l in lins]
-        if any(a is None or a[1] is not None or a[4] != 64 or a[5] != torch.bfloat16 or tuple(a[6]) != s for a, s in zip(planned, shapes)):
+        # one query of the library and the first linear that does not fit are all that an eager step of another model pays
+        if not glue.decode_chain_served(x.device, B, cfg.n_layer, d, cfg.n_head, cfg.n_kv_head, cfg.d_ff, cfg.vocab, cfg.max_seq):
             return None
-        linears = [(a[0], a[2], a[3]) for a in planned]
+        shapes = ((cfg.n_head + 2 * cfg.n_kv_head) * hd, d), (cfg.n_head * hd, d), (2 * cfg.d_ff, d), (d, cfg.d_ff)
+        linears = []
+        for blk in [*self.blocks, None]:
+            lins = (blk.attn.qkv_proj, blk.attn.o_proj, blk.mlp.gate_up_proj, blk.mlp.down_proj) if blk is not None else (self.lm_head,)
+            for lin, want in zip(lins, shapes if blk is not None else ((cfg.vocab, d),)):
+                a = _planned_nf4(lin)
+                if a is None or a[1] is not None or a[4] != 64 or a[5] != torch.bfloat16 or tuple(a[6]) != want:
+                    return None
+                linears.append((a[0], a[2], a[3]))
         norms = [w for blk in self.blocks for w in (blk.norm_1.weight, blk.norm_2.weight)] + [self.norm_f.weight]
         if not glue.decode_chain_takes(x, linears, norms, pos, self.rope_cos, self.rope_sin, kcache, vcache, cfg.n_head, cfg.d_ff, cfg.vocab):
             return None
         return glue.decode_chain(x, linears, norms, cfg.norm_eps, pos, self.rope_cos, self.rope_sin, kcache, vcache, cfg.n_head, cfg.n_kv_head,
-                                 cfg.d_ff, cfg.vocab)
+                                 cfg.d_ff, cfg.vocab, checked=True)
 
     def _decode_step_epilogues(self, x, pos, kcache, vcache):
         """The single-token forward with the neighbours of every linear done in that linear's epilogue

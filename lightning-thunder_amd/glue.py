@@ -150,50 +150,70 @@ def silu_mul(gate_up: torch.Tensor, pairs: bool = False) -> torch.Tensor:
     return out
 
 
+def decode_chain_served(device: torch.device, batch: int, n_layer: int, d_model: int, n_head: int, n_kv_head: int, d_ff: int, vocab: int,
+                        max_seq: int) -> bool:
+    """Has ``decode_chain`` a plan for these shapes on ``device``?"""
+    with torch.cuda.device(device):
+        return load().nf4hip_decode_chain_workspace_bytes(batch, n_layer, d_model, n_head, n_kv_head, d_ff, vocab, max_seq) > 0
+
+
+def _chain_misfit(x, linears, norms, pos, cos, sin, kcache, vcache, n_head: int, n_kv_head: int, d_ff: int, vocab: int) -> str | None:
+    """What, if anything, keeps these operands from being read as a decode step of these sizes."""
+    n_layer, B, Hkv, max_seq, hd = kcache.shape
+    d = x.shape[1]
+    if x.shape != (B, n_head * hd) or vcache.shape != kcache.shape or Hkv != n_kv_head or len(linears) != 4 * n_layer + 1 or len(norms) != 2 * n_layer + 1:
+        return f"{x.shape=} {kcache.shape=} {vcache.shape=}, {len(linears)} linears and {len(norms)} norms do not fit {n_head=} {n_kv_head=}"
+    if not (pos.device == x.device and pos.dtype == torch.int64 and pos.numel() == 1):
+        return "pos must be a one-element int64 tensor on the GPU"
+    for t in (cos, sin):
+        if not (t.device == x.device and t.dtype == torch.float32 and t.is_contiguous() and t.shape == (max_seq, hd)):
+            return f"rotary tables must be contiguous fp32 [{max_seq}, {hd}] on the GPU"
+    shapes = [((n_head + 2 * n_kv_head) * hd, d), (d, d), (2 * d_ff, d), (d, d_ff)] * n_layer + [(vocab, d)]
+    for (qweight, absmax, quant_map), (n, k) in zip(linears, shapes):
+        if not (qweight.is_contiguous() and qweight.numel() * qweight.element_size() >= n * k // 2
+                and absmax.dtype == torch.float32 and absmax.is_contiguous() and absmax.numel() >= n * k // 64
+                and quant_map.dtype == torch.float32 and quant_map.is_contiguous() and quant_map.numel() >= 16):
+            return f"a 4-bit weight does not hold [{n}, {k}] in blocks of 64"
+        if qweight.device != x.device or absmax.device != x.device or quant_map.device != x.device:
+            return "a 4-bit weight lies on another device"
+    for w in norms:
+        if w.numel() != d:
+            return f"norm weight of {w.numel()} elements, expected {d}"
+    for t in (kcache, vcache, *norms):
+        if t.device != x.device:
+            return "a cache or a norm weight lies on another device"
+    return None
+
+
 def decode_chain_takes(x, linears, norms, pos, cos, sin, kcache, vcache, n_head: int, d_ff: int, vocab: int) -> bool:
-    """Would ``decode_chain`` take these operands on their device?  (Everything lies on it, 16-byte aligned, in the types and
+    """Would ``decode_chain`` take these operands on their device?  (Everything lies on it, 16-byte aligned, in the types, sizes and
     layouts that the kernel reads, and the library has a plan for the shapes.)"""
     n_layer, B, Hkv, max_seq, _ = kcache.shape
-    weights = [t for lin in linears for t in lin]
-    if not all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.device == x.device and t.is_contiguous() and t.data_ptr() % 16 == 0
-               for t in [x, cos, sin, kcache, vcache, *norms, *weights]):
+    if not x.is_cuda or not decode_chain_served(x.device, B, n_layer, x.shape[1], n_head, Hkv, d_ff, vocab, max_seq):
         return False
-    if any(t.dtype != torch.bfloat16 for t in (x, kcache, vcache, *norms)) or any(t.dtype != torch.float32 for lin in linears for t in lin[1:]):
+    bf16 = [x, kcache, vcache, *norms]
+    if not all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.data_ptr() % 16 == 0 for t in [*bf16, cos, sin, *(t for lin in linears for t in lin)]):
         return False
-    if not (pos.device == x.device and pos.dtype == torch.int64 and pos.numel() == 1) or any(t.dtype != torch.float32 or t.shape != (max_seq, 128) for t in (cos, sin)):
-        return False
-    with torch.cuda.device(x.device):
-        return load().nf4hip_decode_chain_workspace_bytes(B, n_layer, x.shape[1], n_head, Hkv, d_ff, vocab, max_seq) > 0
+    return (all(t.dtype == torch.bfloat16 and t.is_contiguous() for t in bf16)
+            and _chain_misfit(x, linears, norms, pos, cos, sin, kcache, vcache, n_head, Hkv, d_ff, vocab) is None)
 
 
 def decode_chain(x: torch.Tensor, linears, norms, eps: float, pos: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, kcache: torch.Tensor,
-                 vcache: torch.Tensor, n_head: int, n_kv_head: int, d_ff: int, vocab: int, max_workgroups: int = 0) -> torch.Tensor:
+                 vcache: torch.Tensor, n_head: int, n_kv_head: int, d_ff: int, vocab: int, max_workgroups: int = 0, checked: bool = False) -> torch.Tensor:
     """A whole decode step from the embedded tokens ``x`` [B, d] to the logits [B, vocab] (``nf4hip_decode_chain``).
 
     ``linears``: (qweight, absmax, quant_map) of every layer's QKV, output, gate-up and down projection in that order, then of the
     output head; ``norms``: the two norm weights of every layer in order, then the final one.  ``kcache`` / ``vcache``
     [n_layer, B, n_kv_head, max_seq, 128].  Two launches on the current stream; the scratch is this call's own (under
-    capture it belongs to the graph)."""
+    capture it belongs to the graph).  ``checked``: ``decode_chain_takes`` has just said yes to these operands."""
     lib = load()
-    _bf16_cuda(x, kcache, vcache, *norms)
-    n_layer, B, Hkv, max_seq, hd = kcache.shape
+    if not checked:
+        _bf16_cuda(x, kcache, vcache, *norms)
+        misfit = _chain_misfit(x, linears, norms, pos, cos, sin, kcache, vcache, n_head, n_kv_head, d_ff, vocab)
+        if misfit is not None:
+            raise ValueError(misfit)
+    n_layer, B, _, max_seq, _ = kcache.shape
     d = x.shape[1]
-    if x.shape != (B, n_head * hd) or vcache.shape != kcache.shape or Hkv != n_kv_head or len(linears) != 4 * n_layer + 1 or len(norms) != 2 * n_layer + 1:
-        raise ValueError(f"{x.shape=} {kcache.shape=} {vcache.shape=}, {len(linears)} linears and {len(norms)} norms do not fit {n_head=} {n_kv_head=}")
-    if not (pos.is_cuda and pos.dtype == torch.int64 and pos.numel() == 1):
-        raise ValueError("pos must be a one-element int64 tensor on the GPU")
-    for t in (cos, sin):
-        if not (t.is_cuda and t.dtype == torch.float32 and t.is_contiguous() and t.shape == (max_seq, hd)):
-            raise ValueError(f"rotary tables must be contiguous fp32 [{max_seq}, {hd}] on the GPU")
-    shapes = [((n_head + 2 * n_kv_head) * hd, d), (d, d), (2 * d_ff, d), (d, d_ff)] * n_layer + [(vocab, d)]
-    for (qweight, absmax, quant_map), (n, k) in zip(linears, shapes):
-        if not (qweight.is_cuda and qweight.is_contiguous() and qweight.numel() * qweight.element_size() >= n * k // 2
-                and absmax.dtype == torch.float32 and absmax.is_contiguous() and absmax.numel() >= n * k // 64
-                and quant_map.dtype == torch.float32 and quant_map.is_contiguous() and quant_map.numel() >= 16):
-            raise ValueError(f"a 4-bit weight does not hold [{n}, {k}] in blocks of 64")
-    for w in norms:
-        if w.numel() != d:
-            raise ValueError(f"norm weight of {w.numel()} elements, expected {d}")
     layers = []
     for i in range(n_layer):
         layers += [t.data_ptr() for lin in linears[4 * i: 4 * i + 4] for t in lin] + [norms[2 * i + 1].data_ptr(), norms[2 * i + 2].data_ptr()]

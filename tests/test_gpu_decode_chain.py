@@ -237,3 +237,16 @@ def test_caches_of_one_tensor_per_layer(D, ta, chain_calls, monkeypatch):
         monkeypatch.setattr(D.Llama, "_decode_step_chain", lambda *a: None)
         ref = model(tok, pos, kc, vc)
     assert torch.equal(got, ref) and torch.equal(torch.stack(kl), kc) and torch.equal(torch.stack(vl), vc)
+
+
+def test_a_model_that_is_refused_is_asked_about_once(D, glue, monkeypatch):
+    """Shapes first: a model that the kernel does not serve pays one query per eager step, not a look at every weight."""
+    cfg = D.LlamaConfig(n_layer=2, d_model=1024, n_head=8, n_kv_head=8, d_ff=256, vocab=64, max_seq=16, fused_projections=True, hip_glue=True,
+                        gate_up_interleaved=True)
+    model = D.build_llama(cfg, device="cpu")
+    kc, vc = D.new_caches(cfg, 1, "cpu")
+    asked = []
+    monkeypatch.setattr(glue, "decode_chain_served", lambda *a: asked.append(a[1:]))
+    monkeypatch.setattr(D, "_planned_nf4", lambda lin: pytest.fail("a weight was looked at"))
+    assert model._decode_step_chain(torch.zeros(1, 1024, dtype=torch.bfloat16), torch.zeros(1, dtype=torch.long), kc, vc) is None
+    assert asked == [(1, 2, 1024, 8, 8, 256, 64, 16)]

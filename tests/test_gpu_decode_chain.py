@@ -36,6 +36,9 @@ def test_symbols_and_argument_errors(glue):
                   (1, 2, 8192, 64, 16, 28672, 32000, 640), (1, 2, 4096, 32, 8, 14400, 32000, 640), (1, 2, 4096, 32, 8, 16640, 32000, 640),
                   (1, 2, 4096, 32, 8, 14336, 32001, 640), (1, 0, 4096, 32, 8, 14336, 32000, 640)]:
         assert need(*shape) == 0, shape
+    # the longest caches whose scores fit LDS: 2880 keys in each of eight, four and two ranges
+    for batch, longest in ((1, 23033), (4, 23033), (8, 11517), (16, 5759)):
+        assert need(batch, 1, 4096, 32, 8, 14336, 8000, longest) > 0 and need(batch, 1, 4096, 32, 8, 14336, 8000, longest + 1) == 0, batch
     A = 4096  # non-null, 16-byte aligned fake device address: validation never dereferences
     err = lambda: lib.nf4hip_decode_last_error().decode()
 
@@ -122,6 +125,34 @@ def test_same_bits_as_launch_by_launch_at_8b_shapes(D, ta, chain_calls, monkeypa
         ref = model(tok, pos, kr, vr)
     assert chain_calls["n"] == 1
     assert torch.equal(out, ref) and torch.equal(kc, kr) and torch.equal(vc, vr)
+
+
+# ranges of keys that reach into the second part of the scores' LDS (from 2048 keys on): just so, in the middle, the longest that there are;
+# whole rounds of 192 keys and 160 values and one more  (vocabulary: one where the launches' head takes its sums in the same order)
+LONG = [(1, 23033, 16384), (1, 23033, 16392), (1, 23033, 20011), (1, 23033, 23032), (5, 13817, 13816), (8, 11517, 11516), (16, 5759, 384), (16, 5759, 386),
+        (16, 5759, 4097), (16, 5759, 5758)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,max_seq,p", LONG)
+def test_long_contexts_same_bits_as_launch_by_launch(D, ta, chain_calls, monkeypatch, batch, max_seq, p):
+    print(f"chain long {batch=} {max_seq=} {p=}", flush=True)
+    cfg, model, kc, vc, tok = _model(D, ta, batch, 1, 4096, 14336, 32000, max_seq)
+    pos = torch.full((1,), p, device=DEV, dtype=torch.long)
+    kr, vr = kc.clone(), vc.clone()
+    step = D.Llama._decode_step_chain
+    seen = []
+    for q in (p // 2, p - 1):  # (a key that counts, early and late)
+        for k, v in ((kc, vc), (kr, vr)):
+            k[:, -1:, :, q], v[:, -1:, :, q] = 3.0, 50.0
+        with torch.no_grad():
+            monkeypatch.setattr(D.Llama, "_decode_step_chain", step)
+            out = model(tok, pos, kc, vc)
+            monkeypatch.setattr(D.Llama, "_decode_step_chain", lambda *a: None)
+            ref = model(tok, pos, kr, vr)
+        assert torch.equal(out, ref) and torch.equal(kc, kr) and torch.equal(vc, vr)
+        seen.append(out)
+    assert chain_calls["n"] == 2 and not torch.equal(seen[0][-1], seen[1][-1])
 
 
 @pytest.mark.gpu

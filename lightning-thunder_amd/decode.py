@@ -195,7 +195,7 @@ class Llama(nn.Module):
 
     def _decode_step_chain(self, x, pos, kcache, vcache):
         """The single-token forward as one kernel (``glue.decode_chain``).  Returns None (before anything is launched) unless every
-        linear runs as the 4-bit operator with fp32 absmax, without a bias, at shapes the kernel takes."""
+        linear runs as the 4-bit operator with fp32 absmax, without a bias, at shapes that the kernel takes and gains on."""
         from . import glue
 
         cfg = self.cfg
@@ -206,6 +206,8 @@ class Llama(nn.Module):
             return None
         # one query of the library and the first linear that does not fit are all that an eager step of another model pays
         if not glue.decode_chain_served(x.device, B, cfg.n_layer, d, cfg.n_head, cfg.n_kv_head, cfg.d_ff, cfg.vocab, cfg.max_seq):
+            return None
+        if not glue.decode_chain_pays(B, cfg.n_layer, d, cfg.n_head, cfg.max_seq):
             return None
         shapes = ((cfg.n_head + 2 * cfg.n_kv_head) * hd, d), (cfg.n_head * hd, d), (2 * cfg.d_ff, d), (d, cfg.d_ff)
         linears = []

@@ -68,7 +68,8 @@ def _model(D, ta, batch, layers, d, d_ff, vocab, max_seq, seed=1):
 
 @pytest.fixture
 def chain_calls(glue, monkeypatch):
-    """Counts the calls of glue.decode_chain and caps their workgroups."""
+    """Counts the calls of glue.decode_chain and caps their workgroups; every step that the kernel serves is one, also where launches
+    are faster."""
     calls = {"n": 0, "workgroups": 0}
     real = glue.decode_chain
 
@@ -77,6 +78,7 @@ def chain_calls(glue, monkeypatch):
         return real(*args, max_workgroups=calls["workgroups"], **kw)
 
     monkeypatch.setattr(glue, "decode_chain", counted)
+    monkeypatch.setattr(glue, "decode_chain_pays", lambda *a: True)
     return calls
 
 
@@ -281,3 +283,21 @@ def test_a_model_that_is_refused_is_asked_about_once(D, glue, monkeypatch):
     monkeypatch.setattr(D, "_planned_nf4", lambda lin: pytest.fail("a weight was looked at"))
     assert model._decode_step_chain(torch.zeros(1, 1024, dtype=torch.bfloat16), torch.zeros(1, dtype=torch.long), kc, vc) is None
     assert asked == [(1, 2, 1024, 8, 8, 256, 64, 16)]
+
+
+def test_rule_of_use(D, glue, monkeypatch):
+    """Where both steps were timed, the rule names the faster one (cases within 2 % left out)."""
+    # batch, layers, d_model, max_seq
+    faster = [(b, l, 4096, 640) for b in (1, 3, 8, 16) for l in (2, 8, 32)] + [(b, 8, d, 640) for b in (1, 3, 8, 16) for d in (2048, 3072)]
+    faster += [(8, 2, 2048, 640), (16, 3, 2048, 640), (1, 32, 4096, 20480), (4, 32, 4096, 11000), (8, 32, 4096, 5696), (16, 32, 4096, 4096)]
+    slower = [(b, l, 1024, 640) for b in (1, 3, 8) for l in (8, 32)] + [(b, 1, 512, 64) for b in (1, 8)] + [(3, 8, 1536, 640)]
+    slower += [(1, 1, 2048, 640), (3, 2, 2048, 640), (3, 3, 2048, 640), (8, 1, 2048, 640), (16, 1, 4096, 640), (1, 4, 2048, 20480), (4, 4, 2048, 20480)]
+    pays = lambda b, l, d, s: glue.decode_chain_pays(b, l, d, d // 128, s)
+    assert all(pays(*c) for c in faster) and not any(pays(*c) for c in slower)
+
+    cfg = D.LlamaConfig(n_layer=1, d_model=512, n_head=4, n_kv_head=1, d_ff=256, vocab=64, max_seq=16, fused_projections=True, hip_glue=True,
+                        gate_up_interleaved=True)
+    model = D.build_llama(cfg, device="cpu")
+    monkeypatch.setattr(glue, "decode_chain_served", lambda *a: True)
+    monkeypatch.setattr(D, "_planned_nf4", lambda lin: pytest.fail("a weight was looked at"))
+    assert model._decode_step_chain(torch.zeros(1, 512, dtype=torch.bfloat16), torch.zeros(1, dtype=torch.long), *D.new_caches(cfg, 1, "cpu")) is None

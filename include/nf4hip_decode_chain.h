@@ -28,14 +28,22 @@ extern "C" {
  * `layers` and `head` are host arrays and not referred to after the call.  `workspace`: at least
  * nf4hip_decode_chain_workspace_bytes() bytes (0: this shape or device is not served), 16-byte aligned, any contents, this
  * call's alone until it has run.  The workgroups wait for each other, and only for workgroups that are already running: the step ends
- * however few of them the device holds at a time.  max_workgroups > 0: at most so many (a workgroup takes a whole CU; the
- * answer is the same bit for bit). */
+ * however few of them the device holds at a time, and those that find a CU later join at the next linear.  max_workgroups > 0: at
+ * most so many (a workgroup takes a whole CU; the answer is the same bit for bit).
+ *
+ * nf4hip_decode_chain_joined: the same with workgroups held back, as other work on the device holds them back by itself:
+ * first_members (0: all) of them at most share the first linear, more_members more each one after it. */
 size_t nf4hip_decode_chain_workspace_bytes(int64_t batch, int64_t n_layer, int64_t d_model, int n_head, int n_kv_head, int64_t d_ff,
                                            int64_t vocab, int64_t max_seq);
 int nf4hip_decode_chain(const void* x, const void* const* layers, const void* const* head, const void* norm_first, float eps,
                         const int64_t* pos, const float* cos, const float* sin, void* kcache, void* vcache, int64_t batch,
                         int64_t n_layer, int64_t d_model, int n_head, int n_kv_head, int64_t d_ff, int64_t vocab, int64_t max_seq,
                         int max_workgroups, void* out, void* workspace, size_t workspace_bytes, void* stream);
+int nf4hip_decode_chain_joined(const void* x, const void* const* layers, const void* const* head, const void* norm_first, float eps,
+                               const int64_t* pos, const float* cos, const float* sin, void* kcache, void* vcache, int64_t batch,
+                               int64_t n_layer, int64_t d_model, int n_head, int n_kv_head, int64_t d_ff, int64_t vocab,
+                               int64_t max_seq, int max_workgroups, int first_members, int more_members, void* out,
+                               void* workspace, size_t workspace_bytes, void* stream);
 
 #ifdef __cplusplus
 }

@@ -14,7 +14,10 @@ constexpr int CHAIN_MAX_KSPLITS = 4;  // K ranges of the down projection: sixtee
 constexpr int CHAIN_MAX_SPLITS = 8;   // ranges of cached keys
 constexpr int CHAIN_ATTN_SLOT = 4 * 128 + 8;  // tagged values one range of keys leaves: output, (maximum, sum) of four heads
 constexpr int CHAIN_MAX_POLLS = 1 << 21;      // seconds: what is waited for comes from workgroups that are running
-constexpr uint64_t CHAIN_MUSTER_TICKS = 20000;  // of the 100 MHz clock
+constexpr uint64_t CHAIN_MUSTER_TICKS = 5000;  // of the 100 MHz clock
+constexpr int CHAIN_CTL_BYTES = 1024;           // control words of a launch: arrivals, then members of each phase
+constexpr int CHAIN_CTL_MEMBERS = 32;           // first of those
+static_assert((CHAIN_CTL_MEMBERS + 4 * CHAIN_LAYERS + 1) * 4 <= CHAIN_CTL_BYTES, "a word per phase");
 
 struct ChainLinear {
     const uint8_t* codes;
@@ -46,6 +49,8 @@ struct ChainArgs {
     uint16_t* out;
     uint8_t* ws;
     ChainShape shape[CHAIN_KINDS];
+    int workgroups;                  // of the launch
+    int first_members, more_members;  // at most first_members + phase * more_members of them take part in a phase
     int batch, n_layer, layer0, model_layers, with_head, n_head, n_kv, max_seq, d_model, max_splits;
     float eps;
     // byte offsets in the workspace; *_off of sets: inside the set of a layer

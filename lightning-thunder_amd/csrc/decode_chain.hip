@@ -13,10 +13,15 @@
 //   load: 1.2 us from store to use, six or seven exchanges per layer.  Every such access is an agent-scope one (see nf4_common.h).  Scratch
 //   of tagged words is used again by the next layer: a workgroup writes it only when all that read the last layer's have
 //   left something that it has read since.
-// * Nobody waits for a workgroup that does not run: each counts itself in, and when all of the grid are there -- or 200 us
-//   have passed -- those that are, share the work; the others leave.  Every phase is dealt in tasks by the shape alone, a
-//   workgroup takes task me, me + members, .., and leaves the results of all its tasks of a phase ahead of its first wait in
-//   the next, so any number of members ends with the same bits.  (A wait that lasts seconds all the same gives NaN.)
+// * Nobody waits for a workgroup that does not run: each counts itself in, and when all of the grid are there -- or 50 us
+//   have passed -- those that are, share the work.  Every phase (a linear; the attention goes with the output projection) is dealt in
+//   tasks by the shape alone, a workgroup takes task me, me + members, .., and leaves the results of all its tasks of a phase
+//   ahead of its first wait in the next, so any number of members ends with the same bits.  (A wait that lasts seconds all the
+//   same gives NaN.)
+//   While some are missing, the first that comes to the next layer (the next phase, where few are there) settles how many share it, and the
+//   late ones join there: a workgroup needs a CU to itself, and kernels of other streams may hold most of them when a step
+//   begins.  One sequence, 64 / 192 / 240 / 255 CUs held for another 0.42 ms: 1.6 / 1.6 / 1.6 / 2.1 ms (late ones gone for good 2.3 / 3.6 / 13.5 / 205;
+//   by launches 1.75 / 1.9 / 2.05 / 2.05); with none held it costs 0..0.5 %.
 // * Every sum is taken in the order of the kernel that the launch-by-launch step runs at Llama-3-8B's shapes (1, 5..16 sequences: the two
 //   steps give the same bits; other batches and widths: the same roundings of stored tensors, sums in another order).
 //   Through 32 layers any other order would move the logits by 0.05 of their norm, as two correct bf16 evaluations differ.
@@ -219,22 +224,57 @@ __global__ __launch_bounds__(THREADS, 1) void chain_kernel(ChainArgs) {
     if (pos64 < 0 || pos64 >= a.max_seq) return;  // uniform: a position outside the cache touches nothing
     const int p = (int)pos64;
 
+    const int head_phase = 4 * a.n_layer, last_phase = head_phase - (a.with_head ? 0 : 1);
     // ---- who takes part
-    if (tid == 0) {
-        uint32_t* ctl = reinterpret_cast<uint32_t*>(a.ws + a.ctl_off);
-        const uint32_t rank = __hip_atomic_fetch_add(&ctl[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        auto decide = [&](uint32_t count) {
-            uint32_t none = 0;
-            __hip_atomic_compare_exchange_strong(&ctl[16], &none, count, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        };
-        if (rank == gridDim.x - 1) decide(gridDim.x);
-        const uint64_t t0 = wall_clock64();
-        uint32_t members;
-        while ((members = __hip_atomic_load(&ctl[16], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == 0)
-            if (wall_clock64() - t0 > CHAIN_MUSTER_TICKS)
-                decide(__hip_atomic_load(&ctl[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-        lds_write<uint32_t>(CTL_OFF, rank);
-        lds_write<uint32_t>(CTL_OFF + 4, members);
+    if (wave == 0) {
+        uint32_t* const ctl = reinterpret_cast<uint32_t*>(a.ws + a.ctl_off);
+        uint32_t r = 0, members = 0;
+        if (tid == 0) {
+            r = __hip_atomic_fetch_add(&ctl[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            auto decide = [&](uint32_t count) {
+                uint32_t none = 0;
+                __hip_atomic_compare_exchange_strong(&ctl[CHAIN_CTL_MEMBERS], &none, count, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            };
+            const uint32_t most = (uint32_t)min(a.workgroups, a.first_members);
+            if (r == most - 1) decide(most);
+            const uint64_t t0 = wall_clock64();
+            while ((members = __hip_atomic_load(&ctl[CHAIN_CTL_MEMBERS], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == 0)
+                if (wall_clock64() - t0 > CHAIN_MUSTER_TICKS)
+                    decide(min(__hip_atomic_load(&ctl[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), most));
+        }
+        r = (uint32_t)uniform((int)r);
+        members = (uint32_t)uniform((int)members);
+        // Late: it joins at the first phase that is dealt to more than its number, once that is settled.  (Phases are settled in order, and each
+        // by who has seen the one before and counts afterwards: never for fewer.)
+        int first = 0;
+        for (int tries = 0; members <= r; ++tries) {
+            first = last_phase + 1;
+            members = 0;
+#pragma unroll
+            for (int i = 2; i >= 0; --i) {
+                const int phase = tid + 64 * i;
+                uint32_t v = ~0u;
+                if (phase <= last_phase) v = __hip_atomic_load(&ctl[CHAIN_CTL_MEMBERS + phase], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const uint64_t mine = __ballot(phase <= last_phase && (v == 0 || v > r));
+                if (mine) {
+                    first = 64 * i + __ffsll((unsigned long long)mine) - 1;
+                    members = (uint32_t)__builtin_amdgcn_readlane((int)v, first - 64 * i);
+                }
+            }
+            if (first > last_phase) break;  // all of the step is dealt to others
+            if (members == 0) {
+                if (tries > CHAIN_MAX_POLLS) {
+                    first = last_phase + 1;
+                    break;
+                }
+                __builtin_amdgcn_s_sleep(64);  // 2 us
+            }
+        }
+        if (tid == 0) {
+            lds_write<uint32_t>(CTL_OFF, r);
+            lds_write<uint32_t>(CTL_OFF + 4, members);
+            lds_write<uint32_t>(CTL_OFF + 8, (uint32_t)first);
+        }
     }
     // pointers of the stream and the rotary tables' row, while the others arrive
     if (tid < 4 * a.n_layer + 1) {
@@ -247,30 +287,42 @@ __global__ __launch_bounds__(THREADS, 1) void chain_kernel(ChainArgs) {
         lds_write<float>(ROPE_OFF + HD * 4 + (tid - 768) * 4, a.sin_t[(int64_t)p * HD + tid - 768]);
     }
     barrier();
-    const int rank = uniform((int)lds_read<uint32_t>(CTL_OFF));
-    const int G = uniform((int)lds_read<uint32_t>(CTL_OFF + 4));
-    if (rank >= G) return;
-    const int me = G == (int)gridDim.x ? (int)blockIdx.x : rank;
+    int phase = uniform((int)lds_read<uint32_t>(CTL_OFF + 8));
+    if (phase > last_phase) return;
+    // Those who share the phases up to `stop`, and this workgroup's number among them: of its arrival, while some are missing.
+    int G = uniform((int)lds_read<uint32_t>(CTL_OFF + 4)), me = 0, stop = 0;
+    auto settled = [&]() {
+        ARGS;
+        const int last = 4 * a.n_layer - (a.with_head ? 0 : 1);  // (again: see above)
+        const bool all = G == a.workgroups;
+        me = all ? (int)blockIdx.x : uniform((int)lds_read<uint32_t>(CTL_OFF));
+        // It stops the stream of weights, 4 us: once a layer, or with less than a quarter of the workgroups, which take longer for a phase, once
+        // a phase.  The late ones read it from the words of all the phases that it covers.
+        stop = all ? last : 4 * G < a.workgroups ? phase : min(phase | 3, last);
+        uint32_t* const members = reinterpret_cast<uint32_t*>(a.ws + a.ctl_off) + CHAIN_CTL_MEMBERS;
+        if (!all && wave == 0 && thread_id() < stop - phase)
+            __hip_atomic_store(&members[phase + 1 + thread_id()], (uint32_t)G, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    settled();
 
     // ---- the stream of weights
-    const int head_phase = 4 * a.n_layer, last_phase = head_phase - (a.with_head ? 0 : 1);
     // where it stands: a tile of one task of one linear
     const uint8_t *st_codes = nullptr, *st_absmax = nullptr;
     uint32_t st_left = 0;   // bytes of the task's codes from here on
     uint32_t st_tile = 0;   // codes of a tile
-    int st_task = me, st_phase = 0, st_mode = CHAIN_SLICES;
+    int st_task = me, st_phase = phase, st_mode = CHAIN_SLICES;
     uint32_t st_even = 0, st_odd = 0, st_scales = 0;  // lane constants of the requests
     auto enter = [&]() {
         ARGS;
         // (called with nothing left of the last task)
         int kind = 0;
-        while (st_phase <= last_phase) {
+        while (st_phase <= stop) {
             kind = st_phase == head_phase ? CHAIN_HEAD : st_phase & 3;
             if (st_task < a.shape[kind].row_tasks * a.shape[kind].ksplits) break;
             ++st_phase;
             st_task = me;
         }
-        if (st_phase > last_phase) return;
+        if (st_phase > stop) return;
         const auto& s = a.shape[kind];
         const u32x4 ptr = lds_read<u32x4>(PTR_OFF + st_phase * 16);
         const int q = s.ksplits == 1 ? 0 : st_task % s.ksplits, r0 = (s.ksplits == 1 ? st_task : st_task / s.ksplits) * s.rows_per_task;
@@ -329,12 +381,16 @@ __global__ __launch_bounds__(THREADS, 1) void chain_kernel(ChainArgs) {
         __builtin_amdgcn_raw_ptr_buffer_load_lds(cr, (lds_void_ptr)(uintptr_t)ring, 16, st_even, 0, 0, 2);
         __builtin_amdgcn_raw_ptr_buffer_load_lds(cr, (lds_void_ptr)(uintptr_t)(ring + SLOT_BYTES), 16, st_odd, 0, 0, 2);
     };
-    enter();
-    request(0, 0);
-    advance();
-    request(2 * SLOT_BYTES, ABS_BYTES);
-    advance();
     uint32_t slots = 0, abs_now = 0;  // where the current tile's codes and absmax are
+    auto prime = [&]() {  // the first two tiles
+        enter();
+#pragma unroll 1
+        for (int i = 0; i < 2; ++i) {
+            request(slots ^ (i ? 2 * SLOT_BYTES : 0), i == 0 ? abs_now : abs_now == 2 * ABS_BYTES ? 0 : abs_now + ABS_BYTES);
+            advance();
+        }
+    };
+    prime();
     uint32_t parity = 0;              // which reduction buffer the next tile writes
     bool dead = false;  // a wait ran out: nothing is waited for any more, the step's answer is NaN
 
@@ -344,7 +400,7 @@ __global__ __launch_bounds__(THREADS, 1) void chain_kernel(ChainArgs) {
         lut_hi = lut[tid >> 6];
         lut_lo = lut[(tid >> 2) & 15];
     };
-    request_lut(a.layers[0].lin[0].lut, tid);
+    request_lut(phase == head_phase ? a.head.lut : a.layers[phase >> 2].lin[phase & 3].lut, tid);
 
     auto spin = [&](auto&& attempt) {  // attempt(): does this lane still miss something?
         int tries = 0;
@@ -1256,32 +1312,71 @@ __global__ __launch_bounds__(THREADS, 1) void chain_kernel(ChainArgs) {
     using Rows = std::integral_constant<int, CHAIN_ROWS>;
     using Quads = std::integral_constant<int, CHAIN_QUADS>;
     asm volatile("" ::"v"(lut_hi), "v"(lut_lo));
-    const int n_layer = a.n_layer, qkv_mode = a.shape[CHAIN_QKV].mode;
-    for (int l = 0; l < n_layer; ++l) {
+    // Some were missing: the first that comes here settles how many share the next phases, and the stream goes on.  (Its requests past
+    // the stop, of no bytes, name the same LDS.)
+    auto settle = [&]() {
         ARGS;
-        const float* const lut1 = a.layers[l].lin[1].lut;
-        if (qkv_mode == CHAIN_ROWS)
-            linear(Qkv{}, Rows{}, l, lut1);
-        else if (qkv_mode == CHAIN_QUADS)
-            linear(Qkv{}, Quads{}, l, lut1);
-        else
-            linear(Qkv{}, Slices{}, l, lut1);
-        barrier();  // the attention's scratch is where the last sums were
-        attention(l);
-        barrier();  // ... and the other way round
-        const float* const lut2 = a.layers[l].lin[2].lut;
-        if (qkv_mode == CHAIN_ROWS)
-            linear(Out{}, Rows{}, l, lut2);
-        else
-            linear(Out{}, Slices{}, l, lut2);
-        linear(GateUp{}, Slices{}, l, a.layers[l].lin[3].lut);
+        uint32_t v = 0;
+        if ((thread_id() & 63) == 0) {
+            uint32_t* const ctl = reinterpret_cast<uint32_t*>(a.ws + a.ctl_off);
+            v = __hip_atomic_load(&ctl[CHAIN_CTL_MEMBERS + phase], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (v == 0) {
+                const uint32_t here = __hip_atomic_load(&ctl[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const uint32_t count = min(here, (uint32_t)min(a.workgroups, a.first_members + phase * a.more_members));
+                if (__hip_atomic_compare_exchange_strong(&ctl[CHAIN_CTL_MEMBERS + phase], &v, count, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+                    v = count;
+            }
+        }
+        G = uniform((int)v);
+        settled();
+        wait_vm<0>();
+        st_phase = phase;
+        st_task = me;
+        prime();
+    };
+    const int n_layer = a.n_layer, qkv_mode = a.shape[CHAIN_QKV].mode;
+    const int from = phase;
+    auto takes_part = [&](int this_phase) {
+        if (this_phase < from) return false;  // (a late workgroup may begin in the middle of a layer)
+        if (this_phase > stop) {
+            phase = uniform(this_phase);
+            settle();
+        }
+        return true;
+    };
+    for (int l = phase >> 2; l < n_layer; ++l) {
+        ARGS;
+        if (takes_part(4 * l)) {
+            const float* const lut1 = a.layers[l].lin[1].lut;
+            if (qkv_mode == CHAIN_ROWS)
+                linear(Qkv{}, Rows{}, l, lut1);
+            else if (qkv_mode == CHAIN_QUADS)
+                linear(Qkv{}, Quads{}, l, lut1);
+            else
+                linear(Qkv{}, Slices{}, l, lut1);
+            barrier();  // the attention's scratch is where the last sums were
+        }
+        if (takes_part(4 * l + 1)) {
+            attention(l);
+            barrier();  // ... and the other way round
+            const float* const lut2 = a.layers[l].lin[2].lut;
+            if (qkv_mode == CHAIN_ROWS)
+                linear(Out{}, Rows{}, l, lut2);
+            else
+                linear(Out{}, Slices{}, l, lut2);
+        }
+        if (takes_part(4 * l + 2)) linear(GateUp{}, Slices{}, l, a.layers[l].lin[3].lut);
+        takes_part(4 * l + 3);
         const float* const next = l + 1 < a.n_layer ? a.layers[l + 1].lin[0].lut : a.with_head ? a.head.lut : nullptr;
         if (qkv_mode == CHAIN_ROWS)
             linear(Down{}, Rows{}, l, next);
         else
             linear(Down{}, Slices{}, l, next);
     }
-    if (a.with_head) linear(Head{}, Slices{}, a.n_layer, nullptr);
+    if (a.with_head) {
+        takes_part(head_phase);
+        linear(Head{}, Slices{}, n_layer, nullptr);
+    }
     wait_vm<0>();  // requests past the end of the stream still name this workgroup's LDS
 #endif
 }
@@ -1405,7 +1500,7 @@ bool plan(ChainArgs& a, size_t& bytes, int64_t batch, int64_t n_layer, int64_t d
         at += (n + 255) & ~(int64_t)255;
         return r;
     };
-    a.ctl_off = (int)take(4096);
+    a.ctl_off = (int)take((n_layer + CHAIN_LAYERS - 1) / CHAIN_LAYERS * CHAIN_CTL_BYTES);
     a.apart_off = (int)take(groups * a.max_splits * CHAIN_ATTN_SLOT * 8);
     a.dpart_off = (int)take(a.shape[CHAIN_DOWN].ksplits * M * d_model * 8);
     a.layer_off = at;
@@ -1441,11 +1536,12 @@ __attribute__((visibility("default"))) size_t nf4hip_decode_chain_workspace_byte
     return plan(a, bytes, batch, n_layer, d_model, n_head, n_kv_head, d_ff, vocab, max_seq, chip_cus()) ? bytes : 0;
 }
 
-__attribute__((visibility("default"))) int nf4hip_decode_chain(const void* x, const void* const* layers, const void* const* head, const void* norm_first,
+__attribute__((visibility("default"))) int nf4hip_decode_chain_joined(const void* x, const void* const* layers, const void* const* head, const void* norm_first,
                                                               float eps, const int64_t* pos, const float* cos_t, const float* sin_t, void* kcache,
                                                               void* vcache, int64_t batch, int64_t n_layer, int64_t d_model, int n_head, int n_kv_head,
-                                                              int64_t d_ff, int64_t vocab, int64_t max_seq, int max_workgroups, void* out,
-                                                              void* workspace, size_t workspace_bytes, void* stream) {
+                                                              int64_t d_ff, int64_t vocab, int64_t max_seq, int max_workgroups, int first_members,
+                                                              int more_members, void* out, void* workspace, size_t workspace_bytes, void* stream) {
+    if (first_members < 0 || more_members < 0 || more_members > (1 << 16)) return nf4hip_decode_fail("nf4hip_decode_chain: a negative or too large number of workgroups");
     if (!x || !layers || !head || !norm_first || !pos || !cos_t || !sin_t || !kcache || !vcache || !out) return nf4hip_decode_fail("nf4hip_decode_chain: null pointer");
     ChainArgs a;
     size_t need = 0;
@@ -1478,6 +1574,9 @@ __attribute__((visibility("default"))) int nf4hip_decode_chain(const void* x, co
         return ChainLinear{static_cast<const uint8_t*>(p[0]), static_cast<const float*>(p[1]), static_cast<const float*>(p[2])};
     };
     a.head = linear(head);
+    a.workgroups = max_workgroups > 0 && max_workgroups < workgroups ? max_workgroups : workgroups;
+    a.first_members = first_members > 0 && first_members < a.workgroups ? first_members : a.workgroups;
+    a.more_members = more_members;
     const hipStream_t s = static_cast<hipStream_t>(stream);
     const int64_t zero_bytes = a.layer_off, unset_bytes = (int64_t)need - a.in_stride - zero_bytes;
     const int64_t fill_wgs = (zero_bytes + unset_bytes + BEGIN_THREADS * 64 - 1) / (BEGIN_THREADS * 64);
@@ -1487,7 +1586,7 @@ __attribute__((visibility("default"))) int nf4hip_decode_chain(const void* x, co
         a.layer0 = (int)l0;
         a.n_layer = (int)(n_layer - l0 < CHAIN_LAYERS ? n_layer - l0 : CHAIN_LAYERS);
         a.with_head = l0 + a.n_layer == n_layer;
-        a.ctl_off = (int)(l0 / CHAIN_LAYERS * 128);
+        a.ctl_off = (int)(l0 / CHAIN_LAYERS * CHAIN_CTL_BYTES);
         a.kcache = static_cast<uint16_t*>(kcache) + l0 * a.cache_stride;
         a.vcache = static_cast<uint16_t*>(vcache) + l0 * a.cache_stride;
         for (int i = 0; i < a.n_layer; ++i) {
@@ -1496,9 +1595,18 @@ __attribute__((visibility("default"))) int nf4hip_decode_chain(const void* x, co
             a.layers[i].norm_mid = static_cast<const uint16_t*>(p[12]);
             a.layers[i].norm_next = static_cast<const uint16_t*>(p[13]);
         }
-        hipLaunchKernelGGL(chain_kernel, dim3((unsigned)(max_workgroups > 0 && max_workgroups < workgroups ? max_workgroups : workgroups)), dim3(THREADS), SMEM_BYTES, s, a);
+        hipLaunchKernelGGL(chain_kernel, dim3((unsigned)a.workgroups), dim3(THREADS), SMEM_BYTES, s, a);
     }
     return hipGetLastError() == hipSuccess ? 0 : nf4hip_decode_fail("nf4hip_decode_chain: launch failed");
+}
+
+__attribute__((visibility("default"))) int nf4hip_decode_chain(const void* x, const void* const* layers, const void* const* head, const void* norm_first,
+                                                              float eps, const int64_t* pos, const float* cos_t, const float* sin_t, void* kcache,
+                                                              void* vcache, int64_t batch, int64_t n_layer, int64_t d_model, int n_head, int n_kv_head,
+                                                              int64_t d_ff, int64_t vocab, int64_t max_seq, int max_workgroups, void* out,
+                                                              void* workspace, size_t workspace_bytes, void* stream) {
+    return nf4hip_decode_chain_joined(x, layers, head, norm_first, eps, pos, cos_t, sin_t, kcache, vcache, batch, n_layer, d_model, n_head, n_kv_head, d_ff,
+                                      vocab, max_seq, max_workgroups, 0, 0, out, workspace, workspace_bytes, stream);
 }
 
 }  // extern "C"

@@ -37,6 +37,8 @@ CHAIN_SYMBOLS = {
     "nf4hip_decode_chain_workspace_bytes": (ctypes.c_size_t, [_i64, _i64, _i64, _i32, _i32, _i64, _i64, _i64]),
     "nf4hip_decode_chain": (_i32, [_vp, _vp, _vp, _vp, _f32, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _i32, _i64, _i64, _i64, _i32, _vp, _vp,
                                    ctypes.c_size_t, _vp]),
+    "nf4hip_decode_chain_joined": (_i32, [_vp, _vp, _vp, _vp, _f32, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _i32, _i64, _i64, _i64, _i32, _i32, _i32,
+                                          _vp, _vp, ctypes.c_size_t, _vp]),
 }
 
 _lib = None
@@ -220,13 +222,15 @@ def decode_chain_takes(x, linears, norms, pos, cos, sin, kcache, vcache, n_head:
 
 
 def decode_chain(x: torch.Tensor, linears, norms, eps: float, pos: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, kcache: torch.Tensor,
-                 vcache: torch.Tensor, n_head: int, n_kv_head: int, d_ff: int, vocab: int, max_workgroups: int = 0, checked: bool = False) -> torch.Tensor:
+                 vcache: torch.Tensor, n_head: int, n_kv_head: int, d_ff: int, vocab: int, max_workgroups: int = 0, checked: bool = False, first_members: int = 0,
+                 more_members: int = 0) -> torch.Tensor:
     """A whole decode step from the embedded tokens ``x`` [B, d] to the logits [B, vocab] (``nf4hip_decode_chain``).
 
     ``linears``: (qweight, absmax, quant_map) of every layer's QKV, output, gate-up and down projection in that order, then of the
     output head; ``norms``: the two norm weights of every layer in order, then the final one.  ``kcache`` / ``vcache``
     [n_layer, B, n_kv_head, max_seq, 128].  Two launches on the current stream; the scratch is this call's own (under
-    capture it belongs to the graph).  ``checked``: ``decode_chain_takes`` has just said yes to these operands."""
+    capture it belongs to the graph).  ``checked``: ``decode_chain_takes`` has just said yes to these operands.
+    ``max_workgroups``, ``first_members``, ``more_members``: fewer workgroups, or some of them late; the answer is the same."""
     lib = load()
     if not checked:
         _bf16_cuda(x, kcache, vcache, *norms)
@@ -244,9 +248,9 @@ def decode_chain(x: torch.Tensor, linears, norms, eps: float, pos: torch.Tensor,
     with torch.cuda.device(x.device):
         need = lib.nf4hip_decode_chain_workspace_bytes(B, n_layer, d, n_head, n_kv_head, d_ff, vocab, max_seq)
         ws = torch.empty(max(need, 1), dtype=torch.uint8, device=x.device)
-        _check(lib, lib.nf4hip_decode_chain(x.data_ptr(), layer_ptrs, head_ptrs, norms[0].data_ptr(), float(eps), pos.data_ptr(), cos.data_ptr(),
-                                            sin.data_ptr(), kcache.data_ptr(), vcache.data_ptr(), B, n_layer, d, n_head, n_kv_head, d_ff, vocab, max_seq,
-                                            max_workgroups, out.data_ptr(), ws.data_ptr(), ws.numel(), _stream(x)))
+        _check(lib, lib.nf4hip_decode_chain_joined(x.data_ptr(), layer_ptrs, head_ptrs, norms[0].data_ptr(), float(eps), pos.data_ptr(), cos.data_ptr(),
+                                                   sin.data_ptr(), kcache.data_ptr(), vcache.data_ptr(), B, n_layer, d, n_head, n_kv_head, d_ff, vocab,
+                                                   max_seq, max_workgroups, first_members, more_members, out.data_ptr(), ws.data_ptr(), ws.numel(), _stream(x)))
     return out
 
 

@@ -46,6 +46,9 @@ def test_symbols_and_argument_errors(glue):
         return lib.nf4hip_decode_chain(x, (ctypes.c_void_p * 14)(*layers), (ctypes.c_void_p * 3)(*head), A, 1e-5, A, A, A, A, A, batch, 1, 4096, 32, 8,
                                        14336, 32000, 640, 0, A, A, ws_bytes, None)
 
+    for first, more in ((-1, 0), (1, -1), (1, 1 << 17)):
+        assert lib.nf4hip_decode_chain_joined(A, (ctypes.c_void_p * 14)(*(A,) * 14), (ctypes.c_void_p * 3)(A, A, A), A, 1e-5, A, A, A, A, A, 1, 1, 4096, 32, 8,
+                                              14336, 32000, 640, 0, first, more, A, A, 1 << 40, None) == -1 and "number of workgroups" in err()
     assert call(x=None) == -1 and "null" in err()
     assert call(batch=17) == -1 and "not served" in err()
     assert call(ws_bytes=4096) == -1 and "workspace" in err()
@@ -68,14 +71,14 @@ def _model(D, ta, batch, layers, d, d_ff, vocab, max_seq, seed=1):
 
 @pytest.fixture
 def chain_calls(glue, monkeypatch):
-    """Counts the calls of glue.decode_chain and caps their workgroups; every step that the kernel serves is one, also where launches
+    """Counts the calls of glue.decode_chain, caps their workgroups and makes some late; every step that the kernel serves is one, also where launches
     are faster."""
-    calls = {"n": 0, "workgroups": 0}
+    calls = {"n": 0, "workgroups": 0, "late": {}}
     real = glue.decode_chain
 
     def counted(*args, **kw):
         calls["n"] += 1
-        return real(*args, max_workgroups=calls["workgroups"], **kw)
+        return real(*args, max_workgroups=calls["workgroups"], **calls["late"], **kw)
 
     monkeypatch.setattr(glue, "decode_chain", counted)
     monkeypatch.setattr(glue, "decode_chain_pays", lambda *a: True)
@@ -175,6 +178,54 @@ def test_fewer_workgroups_same_bits(D, ta, chain_calls, batch, layers, d, d_ff, 
             assert not ref[0].isnan().any()
         assert all(torch.equal(a, b) for a, b in zip(got, ref)), workgroups
     assert chain_calls["n"] == 5
+
+
+CTL_BYTES, CTL_MEMBERS = 1024, 32  # decode_chain.h: per launch, the arrivals and then how many shared each phase
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,layers,d,d_ff", [(1, 3, 4096, 14336), (1, 2, 1024, 2304), (6, 2, 2048, 5632), (2, 2, 4096, 14336), (16, 2, 4096, 8448), (3, 35, 1024, 2048)])
+def test_late_workgroups_join_same_bits(D, ta, glue, chain_calls, monkeypatch, batch, layers, d, d_ff):
+    """Workgroups that are late take part from the next phase or layer on; those that never get a turn leave.  (35 layers are two launches.)"""
+    print(f"chain late {batch=} {layers=} {d=} {d_ff=}", flush=True)
+    cfg, model, kc, vc, tok = _model(D, ta, batch, layers, d, d_ff, 1000, 640)
+    pos = torch.full((1,), 300, device=DEV, dtype=torch.long)
+    step = lambda k, v: model(tok, pos, k, v)
+    with torch.no_grad():
+        ref = [kc.clone(), vc.clone()]
+        ref.insert(0, step(*ref))
+        real, scratch = torch.empty, []
+
+        def empty(*args, **kw):
+            t = real(*args, **kw)
+            if kw.get("dtype") is torch.uint8:
+                scratch.append(t)
+            return t
+
+        # first, more: one, then one more per phase; few, never more; all but one late; one late; odd steps, past all of them; most, never more
+        for first, more in ((1, 1), (3, 0), (1, 1 << 16), (255, 1), (37, 50), (100, 0)):
+            chain_calls["late"] = {"first_members": first, "more_members": more}
+            got = [kc.clone(), vc.clone()]
+            scratch.clear()
+            with monkeypatch.context() as m:
+                m.setattr(torch, "empty", empty)
+                got.insert(0, step(*got))
+            assert all(torch.equal(a, b) for a, b in zip(got, ref)), (first, more)
+            ws = max(scratch, key=lambda t: t.numel())
+            cus = torch.cuda.get_device_properties(0).multi_processor_count
+            for launch in range(-(-layers // 32)):
+                ctl = ws[launch * CTL_BYTES:(launch + 1) * CTL_BYTES].view(torch.int32).tolist()
+                phases = 4 * min(32, layers - 32 * launch) + (1 if 32 * (launch + 1) >= layers else 0)
+                members = ctl[CTL_MEMBERS:CTL_MEMBERS + phases]
+                # what was settled: phase by phase for less than a quarter, then layer by layer, until all are there (the device is idle:
+                # all have arrived when the second phase is settled)
+                want, i = [0] * phases, 0
+                while i < phases:
+                    m = min(cus, first + i * more)
+                    stop = i if m == cus or 4 * m < cus else min(i | 3, phases - 1)
+                    want[i:stop + 1] = [m] * (stop + 1 - i)
+                    i = phases if m == cus else stop + 1
+                assert ctl[0] == cus and members == want, (first, more, ctl[0], members)
 
 
 @pytest.mark.gpu

@@ -55,14 +55,14 @@ struct Raw8 {
     uint32_t d[DTYPE == F32 ? 8 : 4];
 };
 
-template <int DTYPE, bool STREAM>
+template <int DTYPE>
 __device__ __forceinline__ Raw8<DTYPE> load8(const void* w, int64_t e0) {
     Raw8<DTYPE> r;
     const uint4* p = reinterpret_cast<const uint4*>(static_cast<const char*>(w) + e0 * (DTYPE == F32 ? 4 : 2));
-    const uint4 a = STREAM ? load16_stream(p) : *p;
+    const uint4 a = load16_stream(p);
     r.d[0] = a.x; r.d[1] = a.y; r.d[2] = a.z; r.d[3] = a.w;
     if (DTYPE == F32) {
-        const uint4 b = STREAM ? load16_stream(p + 1) : p[1];
+        const uint4 b = load16_stream(p + 1);
         r.d[4] = b.x; r.d[5] = b.y; r.d[6] = b.z; r.d[7] = b.w;
     }
     return r;
@@ -71,7 +71,7 @@ __device__ __forceinline__ Raw8<DTYPE> load8(const void* w, int64_t e0) {
 // the same where the array may end inside: elements at or beyond n read as 0
 template <int DTYPE>
 __device__ __forceinline__ Raw8<DTYPE> load8_edge(const void* w, int64_t e0, int64_t n) {
-    if (e0 + 8 <= n) return load8<DTYPE, false>(w, e0);
+    if (e0 + 8 <= n) return load8<DTYPE>(w, e0);
     Raw8<DTYPE> r = {};
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -116,12 +116,16 @@ __device__ __forceinline__ float group_max(float m, int lanes) {
 // two ds_bpermute each span's arithmetic came on top: [28672, 8192] bf16 took
 // 126 us, now 92-96 (602 MB: 6.3-6.5 TB/s).
 // Spans per workgroup (same shape): 1 / 2 / 4 / 8 took 110 / 97 / 92-96 / 101 us.
+// The weight is read past the last-level cache, whatever its size: it is read once, and where kernels have left the cache full of
+// lines to be written back, taking it in waits for those.  Past the cache / through it, us a weight, quantising 1 GB of weights one after
+// the other: [4096, 4096] bf16 13.2 / 14.8, [14336, 4096] 29.2 / 34.1, [28672, 4096] 49.7 / 55.7, just written by a copy 13.9 / 13.8, 28.1 / 28.5,
+// 49.5 / 63.5; behind 512 MB of writes to another buffer 14.1 / 18.6, 30.6 / 48, 54.7 / 83.  Only the same weight over and over gains by the
+// cache (12.5 / 12.6, 29.3 / 26.9, 50.2 / 47.3).
 constexpr int Q_SLOTS = 4;
 
 template <int THREADS, int DTYPE>
 __global__ __launch_bounds__(THREADS) void quantize_kernel(const void* __restrict__ w, int64_t n, int block_log2,
-                                                           uint8_t* __restrict__ packed, float* __restrict__ absmax,
-                                                           bool stream_in) {
+                                                           uint8_t* __restrict__ packed, float* __restrict__ absmax) {
     __shared__ float wave_max[Q_SLOTS][THREADS / 64];
     __shared__ uint2 cells[CODE_CELLS];
     const int tid = threadIdx.x;
@@ -129,12 +133,9 @@ __global__ __launch_bounds__(THREADS) void quantize_kernel(const void* __restric
     const int64_t first = (int64_t)blockIdx.x * (Q_SLOTS * THREADS * 8) + tid * 8;
     const bool whole = ((int64_t)blockIdx.x + 1) * (Q_SLOTS * THREADS * 8) <= n;
     Raw8<DTYPE> raw[Q_SLOTS];
-    if (whole && stream_in) {
+    if (whole) {
 #pragma unroll
-        for (int c = 0; c < Q_SLOTS; ++c) raw[c] = load8<DTYPE, true>(w, first + c * (THREADS * 8));
-    } else if (whole) {
-#pragma unroll
-        for (int c = 0; c < Q_SLOTS; ++c) raw[c] = load8<DTYPE, false>(w, first + c * (THREADS * 8));
+        for (int c = 0; c < Q_SLOTS; ++c) raw[c] = load8<DTYPE>(w, first + c * (THREADS * 8));
     } else {
 #pragma unroll
         for (int c = 0; c < Q_SLOTS; ++c) raw[c] = load8_edge<DTYPE>(w, first + c * (THREADS * 8), n);
@@ -560,14 +561,10 @@ void enqueue_quantize(const void* w, int64_t n, int block_log2, uint8_t* packed,
     const int threads = block_log2 == 12 ? 512 : 256;  // a span holds a whole block
     const int64_t per = (int64_t)threads * 8 * Q_SLOTS;
     const dim3 grid((unsigned)((n + per - 1) / per));
-    // A weight that does not fit the 256 MB last-level cache is read past it; of a smaller one that was just written, or is read
-    // again, much is still there
-    // (us back to back, past the cache / through it: [14336, 4096] bf16 29.1 / 25.7, fp32 53.0 / 42.3; [28672, 8192] bf16 96 / 109).
-    const bool stream_in = n * (DTYPE == F32 ? 4 : 2) > ((int64_t)256 << 20);
     if (threads == 512)
-        hipLaunchKernelGGL((quantize_kernel<512, DTYPE>), grid, dim3(512), 0, stream, w, n, block_log2, packed, absmax, stream_in);
+        hipLaunchKernelGGL((quantize_kernel<512, DTYPE>), grid, dim3(512), 0, stream, w, n, block_log2, packed, absmax);
     else
-        hipLaunchKernelGGL((quantize_kernel<256, DTYPE>), grid, dim3(256), 0, stream, w, n, block_log2, packed, absmax, stream_in);
+        hipLaunchKernelGGL((quantize_kernel<256, DTYPE>), grid, dim3(256), 0, stream, w, n, block_log2, packed, absmax);
 }
 
 hipError_t enqueue_compress(const float* absmax, int64_t nblocks, int nested_log2, const float* map256, const DqOffset& o,

@@ -196,7 +196,6 @@ __device__ __forceinline__ float sum8_down(float v) {
     v += __uint_as_float(dpp<QUAD_X2>(__float_as_uint(v)));
     return v + __uint_as_float(dpp<QUAD_X1>(__float_as_uint(v)));
 }
-__device__ __forceinline__ float exp_below(float v, float top) { return v == -INFINITY ? 0.0f : __expf(v - top); }
 __device__ __forceinline__ uint32_t max4(const u32x4& v) { return max(max(v.x, v.y), max(v.z, v.w)); }
 
 #endif
@@ -477,7 +476,6 @@ __global__ __launch_bounds__(THREADS, 1) void chain_kernel(ChainArgs) {
             return rsqrtf(t / (float)K + a.eps);
         };
 
-        
         // byte -> two code-book values: every wave is past the barrier behind the last use of the table
         {
             const uint32_t vb = F16 ? (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)lut_hi) | ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)lut_lo) << 16)
@@ -854,8 +852,6 @@ __global__ __launch_bounds__(THREADS, 1) void chain_kernel(ChainArgs) {
                 if (reducer && scaled) rstd = rstd_of_sums();
             }
             barrier();  // the table; the reduction buffers are free
-            
-
 
             float resid_ss = 0.0f;
             auto finish_tile = [&](int t, const float (&pt)[4]) {
@@ -973,14 +969,14 @@ __global__ __launch_bounds__(THREADS, 1) void chain_kernel(ChainArgs) {
                 if (t + 1 < tiles) wait_vm<5>();
                 barrier();
             }
-            
+
             if (reducer) {
                 float pt[4];
                 read_sums(pt);
                 finish_tile(tiles - 1, pt);
                 leave();
             }
-            
+
             if constexpr (KIND == CHAIN_OUT) {
                 if (reducer) {
                     resid_ss = row16_down(lane < 16 ? resid_ss : 0.0f);
@@ -1610,4 +1606,3 @@ __attribute__((visibility("default"))) int nf4hip_decode_chain(const void* x, co
 }
 
 }  // extern "C"
-

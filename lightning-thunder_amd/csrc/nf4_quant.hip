@@ -243,12 +243,13 @@ __device__ __forceinline__ void dequant8_store(uint32_t word, float s, const flo
 // elements of each span, so every load and store of a wave is contiguous.  Bound by HBM, mostly by the writes.
 //
 // The loads of all spans are in flight before the first is used: codes first (they come from the farthest), then the
-// statistics, with one branch for the whole workgroup instead of one around each load.  An output that does not fit the
-// last-level cache (STREAM) has its codes read past the cache too; behind a smaller one they may stay there.
+// statistics, with one branch for the whole workgroup instead of one around each load.  Codes are read past the last-level
+// cache whatever the size of the output: past the cache / through it, us a weight to bf16, 0.5 to 1 GB of weights one after the other:
+// [4096, 4096] 10.0 / 10.8, [14336, 4096] 28.2 / 29.8, [22528, 4096] 41.7 / 43.9; behind 512 MB of writes 13.3 / 14.7, 32.6 / 35.6,
+// 46.9 / 53.9.  Only the same weight over and over into the same output gains by the cache (10.0 / 8.9, 25.1 / 23.1, 37.0 / 34.6).
 // 16-bit outputs are packed by one conversion per two values.
 // A streamed output's first store waits for the last load (lm_head 213 -> 210 us; nested 215 -> 209).
-// us, with a check around every load and the codes always read past the cache -> now: [14336, 4096] bf16 39.5 -> 34.9 (of
-// which about 12 is the call), fp32 107 -> 102; nested [28672, 8192] bf16 99 -> 95 back to back.  Statistics first: 106 for the last.
+// us, with a check around every load -> now: nested [28672, 8192] bf16 99 -> 95 back to back.  Statistics first: 106.
 // Spans per workgroup 1 / 2 / 4 / 8: 132 / 134 / 115 / 120.
 // Nested absmax: the map is copied into LDS meanwhile, so that no load waits for another.  With the map looked up in
 // global memory (code -> map entry -> value, two dependent loads per span) the kernel took 175 us for that weight.
@@ -270,7 +271,7 @@ __global__ __launch_bounds__(256) void dequantize_kernel(const uint8_t* __restri
     if (whole) {
 #pragma unroll
         for (int c = 0; c < DQ_SLOTS; ++c)
-            word[c] = STREAM ? __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(packed) + ((first + c * 2048) >> 3)) : reinterpret_cast<const uint32_t*>(packed)[(first + c * 2048) >> 3];
+            word[c] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(packed) + ((first + c * 2048) >> 3));
     } else {
         const int64_t nbytes = (n + 1) / 2;
 #pragma unroll

@@ -207,7 +207,7 @@ class Llama(nn.Module):
         # one query of the library and the first linear that does not fit are all that an eager step of another model pays
         if not glue.decode_chain_served(x.device, B, cfg.n_layer, d, cfg.n_head, cfg.n_kv_head, cfg.d_ff, cfg.vocab, cfg.max_seq):
             return None
-        if not glue.decode_chain_pays(B, cfg.n_layer, d, cfg.n_head, cfg.max_seq):
+        if not glue.decode_chain_pays(B, cfg.n_layer, d, cfg.n_head, cfg.max_seq, cfg.vocab):
             return None
         shapes = ((cfg.n_head + 2 * cfg.n_kv_head) * hd, d), (cfg.n_head * hd, d), (2 * cfg.d_ff, d), (d, cfg.d_ff)
         linears = []

@@ -159,25 +159,33 @@ def decode_chain_served(device: torch.device, batch: int, n_layer: int, d_model:
         return load().nf4hip_decode_chain_workspace_bytes(batch, n_layer, d_model, n_head, n_kv_head, d_ff, vocab, max_seq) > 0
 
 
-def decode_chain_pays(batch: int, n_layer: int, d_model: int, n_head: int, max_seq: int) -> bool:
+def decode_chain_pays(batch: int, n_layer: int, d_model: int, n_head: int, max_seq: int, vocab: int) -> bool:
     """Is a step as one kernel faster than one launch per linear, over the positions of a cache of this length?
 
     Modelled from graph replays of both on one MI355X (us, launches / one kernel; four query heads per kv head).  A layer gains by its
     width, as six exchanges between workgroups take about as long as five launches of small kernels: eight layers, 512 positions, 1 / 3 / 8 / 16
     sequences, d 1024 (d_ff 4096) 213 / 245, 236 / 286, 274 / 320, 308 / 359; d 1536 (4096) 229 / 235, 261 / 274, 314 / 307, 366 / 351; d 2048
     (8192) 254 / 231, 302 / 284, 365 / 308, 432 / 376; d 3072 (8192) 316 / 269, 363 / 320, 430 / 373, 524 / 443; d 4096 (14336) 448 / 355,
-    476 / 395, 531 / 453, 619 / 543.  It loses about 6.5 ns per key of a range of keys, of which a workgroup has one (four layers, d 4096: one
-    sequence at 4000 / 12000 / 20000 positions 235 / 207, 278 / 271, 356 / 379; eight at 4000 / 8000 / 10900 352 / 338, 442 / 455, 504 / 544;
-    sixteen at 2048 / 4000 / 5600 388 / 374, 473 / 490, 543 / 588; d 2048, one at 8000 / 20000 181 / 198, 245 / 296): the position is not known
-    where a step is recorded, so the middle of the cache stands for it.  The launch that fills the scratch and the wait for all workgroups cost
-    7..12 us a step (one layer of d 2048, 1 / 3 / 8 sequences 50 / 55, 56 / 66, 67 / 70; two 79 / 80, 90 / 96, 108 / 104; four 139 / 130, 159 / 158,
-    197 / 172; one layer of d 4096 75 / 70, 81 / 82, 90 / 90)."""
-    per_layer = 4.0 * d_model / 1024 - 4.7
-    if batch > 4 and d_model >= 2048:
-        per_layer = max(per_layer, 8.0)
-    ranges = max(1, min(8, 1024 // (batch * n_head)))
-    per_layer -= 0.0065 * (max_seq / 2 / ranges)
-    return n_layer * per_layer >= (7.0 if batch == 1 else 11.5)
+    476 / 395, 531 / 453, 619 / 543.  Two sequences gain more than one or three (d 2048, six layers, 100 positions 229 / 210), and with up to four a
+    large output head gains too (d 2048, two layers, two sequences, 500 positions, vocabulary 43000 / 99000: 91 / 91, 110 / 106).  A layer loses 4 to 7 ns
+    per key of a range of keys, of which a workgroup has one (four layers, d 4096: one sequence at 4000 / 12000 / 20000 positions 235 / 207, 278 / 271,
+    356 / 379; eight at 4000 / 8000 / 10900 352 / 338, 442 / 455, 504 / 544; sixteen at 2048 / 4000 / 5600 388 / 374, 473 / 490, 543 / 588; d 2048, one at
+    8000 / 20000 181 / 198, 245 / 296): the position is not known where a step is recorded, so the middle of the cache stands for it.  The launch
+    that fills the scratch and the wait for all workgroups cost 7..14 us a step (one layer of d 2048, 1 / 3 / 8 sequences 50 / 55, 56 / 66, 67 / 70; two
+    79 / 80, 90 / 96, 108 / 104; four 139 / 130, 159 / 158, 197 / 172; one layer of d 4096 75 / 70, 81 / 82, 90 / 90).  Over 407 drawn models (d 512..4096,
+    1..24 layers, 1..16 sequences, up to 20000 positions) the side that this picks is 0.1 % slower than the faster one on average, 6 % at most."""
+    width = d_model / 1024
+    keys = max_seq / 2 / max(1, min(8, 1024 // (batch * n_head))) / 1000
+    head = width * vocab / 1e5
+    if batch <= 2:
+        layer, gain = (3.6 * width - 3.9 - 6.7 * keys, 2.8 * head - 10) if batch == 1 else (3.0 * width - 1.2 - 4.5 * keys, 2.8 * head - 11.5)
+    elif batch <= 4:
+        layer, gain = 4.0 * width - 5.0 - 4.5 * keys, 1.6 * head - 14
+    else:
+        layer, gain = 4.0 * width - 4.7 - 5.5 * keys, -11.5
+        if d_model >= 2048 or (batch > 8 and d_model >= 1536):
+            layer = max(4.0 * width - 4.7, 8.0) - 5.5 * keys
+    return n_layer * layer + gain >= 0
 
 
 def _chain_misfit(x, linears, norms, pos, cos, sin, kcache, vcache, n_head: int, n_kv_head: int, d_ff: int, vocab: int) -> str | None:

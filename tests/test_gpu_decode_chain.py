@@ -338,12 +338,15 @@ def test_a_model_that_is_refused_is_asked_about_once(D, glue, monkeypatch):
 
 def test_rule_of_use(D, glue, monkeypatch):
     """Where both steps were timed, the rule names the faster one (cases within 2 % left out)."""
-    # batch, layers, d_model, max_seq
+    # batch, layers, d_model, max_seq, vocabulary (32000)
     faster = [(b, l, 4096, 640) for b in (1, 3, 8, 16) for l in (2, 8, 32)] + [(b, 8, d, 640) for b in (1, 3, 8, 16) for d in (2048, 3072)]
     faster += [(8, 2, 2048, 640), (16, 3, 2048, 640), (1, 32, 4096, 20480), (4, 32, 4096, 11000), (8, 32, 4096, 5696), (16, 32, 4096, 4096)]
     slower = [(b, l, 1024, 640) for b in (1, 3, 8) for l in (8, 32)] + [(b, 1, 512, 64) for b in (1, 8)] + [(3, 8, 1536, 640)]
     slower += [(1, 1, 2048, 640), (3, 2, 2048, 640), (3, 3, 2048, 640), (8, 1, 2048, 640), (16, 1, 4096, 640), (1, 4, 2048, 20480), (4, 4, 2048, 20480)]
-    pays = lambda b, l, d, s: glue.decode_chain_pays(b, l, d, d // 128, s)
+    faster += [(2, 6, 2048, 192), (2, 7, 1536, 192, 59152), (2, 6, 2048, 3968, 37328), (2, 3, 2048, 3136, 62520), (2, 4, 2048, 1856, 115400), (9, 5, 1536, 2624), (11, 7, 1536, 1664)]
+    faster += [(1, 2, 2048, 768, 96376), (2, 2, 2048, 448, 99304)]
+    slower += [(4, 2, 2048, 2816), (3, 2, 2048, 256), (3, 3, 2048, 1472, 45712), (13, 3, 1024, 5568), (1, 2, 2048, 640, 44248)]
+    pays = lambda b, l, d, s, vocab=32000: glue.decode_chain_pays(b, l, d, d // 128, s, vocab)
     assert all(pays(*c) for c in faster) and not any(pays(*c) for c in slower)
 
     cfg = D.LlamaConfig(n_layer=1, d_model=512, n_head=4, n_kv_head=1, d_ff=256, vocab=64, max_seq=16, fused_projections=True, hip_glue=True,

@@ -21,7 +21,7 @@
 //   While some are missing, the first that comes to the next layer (the next phase, where few are there) settles how many share it, and the
 //   late ones join there: a workgroup needs a CU to itself, and kernels of other streams may hold most of them when a step
 //   begins.  One sequence, 64 / 192 / 240 / 255 CUs held for another 0.42 ms: 1.6 / 1.6 / 1.6 / 2.1 ms (late ones gone for good 2.3 / 3.6 / 13.5 / 205;
-//   by launches 1.75 / 1.9 / 2.05 / 2.05); with none held it costs 0..0.5 %.
+//   by launches 1.75 / 1.9 / 2.05 / 2.05); with none held it costs 0..1 % (the code that takes the stream up again is there at five places).
 // * Every sum is taken in the order of the kernel that the launch-by-launch step runs at Llama-3-8B's shapes (1, 5..16 sequences: the two
 //   steps give the same bits; other batches and widths: the same roundings of stored tensors, sums in another order).
 //   Through 32 layers any other order would move the logits by 0.05 of their norm, as two correct bf16 evaluations differ.
@@ -35,7 +35,7 @@
 // * Attention: a (sequence, kv head, range of cached keys) per workgroup, sums as in decode_glue.hip; the first keys and values are
 //   under way before the queries are known.
 //
-// Measured (graph replay, Llama-3-8B, 512 / 576 positions, one MI355X): 1 sequence 1584 -> 1214 us, 8 sequences 2025 -> 1652.
+// Measured (graph replay, Llama-3-8B, 512 / 576 positions, MI355X, from box to box): 1 sequence 1584..1612 -> 1209..1230 us, 8 sequences 2025 -> 1650..1698.
 // What bounds it now, per layer and for one sequence (38 us; stamps of the 100 MHz clock): tiles 22 us (1.1 us each in the gate-up
 // projection while their data is there, 1.3 where HBM sets the pace, 1.6 in the others, whose 4x4x4 MFMAs fill the matrix
 // pipe), six exchanges 9, attention's own work 4, the rest waits for the slowest workgroup.  Tried and not kept: a third tile
@@ -381,11 +381,12 @@ __global__ __launch_bounds__(THREADS, 1) void chain_kernel(ChainArgs) {
         __builtin_amdgcn_raw_ptr_buffer_load_lds(cr, (lds_void_ptr)(uintptr_t)(ring + SLOT_BYTES), 16, st_odd, 0, 0, 2);
     };
     uint32_t slots = 0, abs_now = 0;  // where the current tile's codes and absmax are
-    auto prime = [&]() {  // the first two tiles
-        enter();
+    auto prime = [&]() {  // the first two tiles of what begins at st_task (and nothing is left of what was before)
+        st_left = 0;
+        st_task -= G;
 #pragma unroll 1
-        for (int i = 0; i < 2; ++i) {
-            request(slots ^ (i ? 2 * SLOT_BYTES : 0), i == 0 ? abs_now : abs_now == 2 * ABS_BYTES ? 0 : abs_now + ABS_BYTES);
+        for (int i = 0; i < 3; ++i) {
+            if (i) request(slots ^ (i == 2 ? 2 * SLOT_BYTES : 0), i == 1 ? abs_now : abs_now == 2 * ABS_BYTES ? 0 : abs_now + ABS_BYTES);
             advance();
         }
     };

@@ -120,7 +120,7 @@ __device__ __forceinline__ float group_max(float m, int lanes) {
 // lines to be written back, taking it in waits for those.  Past the cache / through it, us a weight, quantising 1 GB of weights one after
 // the other: [4096, 4096] bf16 13.2 / 14.8, [14336, 4096] 29.2 / 34.1, [28672, 4096] 49.7 / 55.7, just written by a copy 13.9 / 13.8, 28.1 / 28.5,
 // 49.5 / 63.5; behind 512 MB of writes to another buffer 14.1 / 18.6, 30.6 / 48, 54.7 / 83.  Only the same weight over and over gains by the
-// cache (12.5 / 12.6, 29.3 / 26.9, 50.2 / 47.3).
+// cache (12.5 / 12.6, 29.3 / 26.9, 50.2 / 47.3; [8192, 4096] 18.1 / 16.8), and a weight is quantised once.
 constexpr int Q_SLOTS = 4;
 
 template <int THREADS, int DTYPE>
@@ -243,25 +243,26 @@ __device__ __forceinline__ void dequant8_store(uint32_t word, float s, const flo
 // elements of each span, so every load and store of a wave is contiguous.  Bound by HBM, mostly by the writes.
 //
 // The loads of all spans are in flight before the first is used: codes first (they come from the farthest), then the
-// statistics, with one branch for the whole workgroup instead of one around each load.  Codes are read past the last-level
-// cache whatever the size of the output: past the cache / through it, us a weight to bf16, 0.5 to 1 GB of weights one after the other:
-// [4096, 4096] 10.0 / 10.8, [14336, 4096] 28.2 / 29.8, [22528, 4096] 41.7 / 43.9; behind 512 MB of writes 13.3 / 14.7, 32.6 / 35.6,
-// 46.9 / 53.9.  Only the same weight over and over into the same output gains by the cache (10.0 / 8.9, 25.1 / 23.1, 37.0 / 34.6).
+// statistics, with one branch for the whole workgroup instead of one around each load.
 // 16-bit outputs are packed by one conversion per two values.
-// A streamed output's first store waits for the last load (lm_head 213 -> 210 us; nested 215 -> 209).
+// A streamed output's (DQ_STREAM) first store waits for the last load (lm_head 213 -> 210 us; nested 215 -> 209).
 // us, with a check around every load -> now: nested [28672, 8192] bf16 99 -> 95 back to back.  Statistics first: 106.
 // Spans per workgroup 1 / 2 / 4 / 8: 132 / 134 / 115 / 120.
 // Nested absmax: the map is copied into LDS meanwhile, so that no load waits for another.  With the map looked up in
 // global memory (code -> map entry -> value, two dependent loads per span) the kernel took 175 us for that weight.
 constexpr int DQ_SLOTS = 4;
 
-template <bool NESTED, bool STREAM, int OUT>
+// How a weight's codes are read and its output written: both through the last-level cache; codes past it; output streamed as well.
+enum : int { DQ_NEAR = 0, DQ_FAR = 1, DQ_STREAM = 2 };
+
+template <bool NESTED, int WAY, int OUT>
 __global__ __launch_bounds__(256) void dequantize_kernel(const uint8_t* __restrict__ packed,
                                                          const float* __restrict__ absmax, NestedAbsmax nq,
                                                          const float* __restrict__ lut16, int64_t n, int block_log2,
                                                          void* __restrict__ out) {
     __shared__ float lut[16];
     __shared__ float map[NESTED ? 256 : 1];
+    constexpr bool STREAM = WAY == DQ_STREAM;
     const int tid = threadIdx.x;
     const int64_t first = (int64_t)blockIdx.x * (DQ_SLOTS * 2048) + tid * 8;
     const bool whole = ((int64_t)blockIdx.x + 1) * (DQ_SLOTS * 2048) <= n;
@@ -270,8 +271,10 @@ __global__ __launch_bounds__(256) void dequantize_kernel(const uint8_t* __restri
     float s[DQ_SLOTS];  // absmax, or with nested absmax the second-level value
     if (whole) {
 #pragma unroll
-        for (int c = 0; c < DQ_SLOTS; ++c)
-            word[c] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(packed) + ((first + c * 2048) >> 3));
+        for (int c = 0; c < DQ_SLOTS; ++c) {
+            const uint32_t* const at = reinterpret_cast<const uint32_t*>(packed) + ((first + c * 2048) >> 3);
+            word[c] = WAY == DQ_NEAR ? *at : __builtin_nontemporal_load(at);
+        }
     } else {
         const int64_t nbytes = (n + 1) / 2;
 #pragma unroll
@@ -615,14 +618,14 @@ hipError_t launch_dq_statistics(const float* absmax, int64_t nblocks, int nested
 
 namespace {
 
-template <bool STREAM, int OUT>
+template <int WAY, int OUT>
 void enqueue_dequantize(const uint8_t* packed, const float* absmax, const NestedAbsmax& nested, const float* lut16,
                         int64_t n, int block_log2, void* out, hipStream_t stream) {
     const dim3 grid((unsigned)((n + 2048 * DQ_SLOTS - 1) / (2048 * DQ_SLOTS))), threads(256);
     if (nested.q)
-        hipLaunchKernelGGL((dequantize_kernel<true, STREAM, OUT>), grid, threads, 0, stream, packed, absmax, nested, lut16, n, block_log2, out);
+        hipLaunchKernelGGL((dequantize_kernel<true, WAY, OUT>), grid, threads, 0, stream, packed, absmax, nested, lut16, n, block_log2, out);
     else
-        hipLaunchKernelGGL((dequantize_kernel<false, STREAM, OUT>), grid, threads, 0, stream, packed, absmax, nested, lut16, n, block_log2, out);
+        hipLaunchKernelGGL((dequantize_kernel<false, WAY, OUT>), grid, threads, 0, stream, packed, absmax, nested, lut16, n, block_log2, out);
 }
 
 }  // namespace
@@ -634,11 +637,17 @@ hipError_t launch_dequantize(const uint8_t* packed, const float* absmax, const N
     // An output that fits in the 256 MB last-level cache is written with ordinary stores, so that the
     // GEMM that usually follows finds it there; a larger one cannot stay anyway and is streamed
     // (non-temporal stores: 20 % faster on their own, 5 % slower for that GEMM).
+    // Codes are read through that cache where two or three such weights fit it with their outputs, and may be found there again.  Through it /
+    // past it, us a weight to bf16, the same one over and over; 0.4 to 0.5 GB of weights in turn; behind 512 MB of writes: [4096, 4096] 8.7 / 10.1,
+    // 10.9 / 10.0, 14.2 / 14.0; [8192, 4096], 64 MB, 13.5 / 16.1, 18.4 / 17.5, 23.2 / 21.1; [10240, 4096] 16.7 / 18.7, 21.9 / 20.7, 27.6 / 25.2;
+    // [14336, 4096] 22.8 / 25.0, 29.4 / 28.0, 35.6 / 32.0; [22528, 4096] 34.6 / 36.7, 43.5 / 41.6, 52.2 / 46.6: 3 us against 1 up to 64 MB, 2 against
+    // 1 to 6 beyond.  (Three in turn: [8192, 4096] 14.0 / 16.8, [14336, 4096] 26.6 / 25.5.)
     const int64_t out_bytes = n * (out_dtype == F32 ? 4 : 2);
-    const bool stream_out = out_bytes > ((int64_t)192 << 20);
-    const auto enqueue = out_dtype == F32    ? (stream_out ? enqueue_dequantize<true, F32> : enqueue_dequantize<false, F32>)
-                         : out_dtype == BF16 ? (stream_out ? enqueue_dequantize<true, BF16> : enqueue_dequantize<false, BF16>)
-                                             : (stream_out ? enqueue_dequantize<true, F16> : enqueue_dequantize<false, F16>);
+    const int way = out_bytes > ((int64_t)192 << 20) ? DQ_STREAM : out_bytes > ((int64_t)64 << 20) ? DQ_FAR : DQ_NEAR;
+    const auto pick = [way](auto near, auto far, auto stream_out) { return way == DQ_NEAR ? near : way == DQ_FAR ? far : stream_out; };
+    const auto enqueue = out_dtype == F32    ? pick(enqueue_dequantize<DQ_NEAR, F32>, enqueue_dequantize<DQ_FAR, F32>, enqueue_dequantize<DQ_STREAM, F32>)
+                         : out_dtype == BF16 ? pick(enqueue_dequantize<DQ_NEAR, BF16>, enqueue_dequantize<DQ_FAR, BF16>, enqueue_dequantize<DQ_STREAM, BF16>)
+                                             : pick(enqueue_dequantize<DQ_NEAR, F16>, enqueue_dequantize<DQ_FAR, F16>, enqueue_dequantize<DQ_STREAM, F16>);
     enqueue(packed, absmax, nested, lut16, n, block_log2, out, stream);
     return hipGetLastError();
 }

@@ -132,6 +132,23 @@ def test_dequantize_shapes(ta, oracle, shape, blocksize):
     assert (err <= bound).all()
 
 
+# 16-bit outputs of 64 and 192 MiB and one element more (rule of how codes are read and the output is written), the last span of a workgroup
+# cut off; fp32 outputs reach the same sizes with half the elements
+@pytest.mark.parametrize("n", [2**24, 2**24 + 1, 2**25, 2**25 + 1, 3 * 2**24 + 7, 3 * 2**25, 3 * 2**25 + 1])
+def test_dequantize_large_outputs(ta, n):
+    _sync_print(f"dequantize large {n}")
+    g = torch.Generator(device=DEV).manual_seed(n)
+    packed = torch.randint(0, 256, ((n + 1) // 2, 1), dtype=torch.uint8, device=DEV, generator=g)
+    absmax = torch.rand((n + 63) // 64, device=DEV, generator=g) * 0.1 + 1e-3
+    lut = ta.nf4_code(DEV)
+    codes = torch.stack([packed.view(-1) >> 4, packed.view(-1) & 15], dim=1).view(-1)[:n]
+    nq = ta.compress_absmax(absmax)
+    for stats, values in ((absmax, absmax), (nq, ta.functional.reconstruct_absmax(nq))):
+        want = lut[codes.int()] * values.repeat_interleave(64)[:n]  # one product, rounded once to fp32 and once to the output's type
+        for dtype in (torch.bfloat16, torch.float16, torch.float32) if n <= 3 * 2**24 + 7 else (torch.bfloat16,):
+            assert torch.equal(ta.dequantize_nf4(packed, stats, lut, 64, dtype, (n,)), want.to(dtype)), (dtype, stats is nq)
+
+
 def test_nested_absmax(ta, oracle):
     _sync_print("nested absmax")
     w = _weights((1024, 1024), seed=11)

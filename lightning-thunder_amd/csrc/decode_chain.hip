@@ -21,7 +21,7 @@
 //   While some are missing, the first that comes to the next layer (the next phase, where few are there) settles how many share it, and the
 //   late ones join there: a workgroup needs a CU to itself, and kernels of other streams may hold most of them when a step
 //   begins.  One sequence, 64 / 192 / 240 / 255 CUs held for another 0.42 ms: 1.6 / 1.6 / 1.6 / 2.1 ms (late ones gone for good 2.3 / 3.6 / 13.5 / 205;
-//   by launches 1.75 / 1.9 / 2.05 / 2.05); with none held it costs 0..1 % (the code that takes the stream up again is there at five places).
+//   by launches 1.75 / 1.9 / 2.05 / 2.05); with none held it costs 0..1 %.
 // * Every sum is taken in the order of the kernel that the launch-by-launch step runs at Llama-3-8B's shapes (1, 5..16 sequences: the two
 //   steps give the same bits; other batches and widths: the same roundings of stored tensors, sums in another order).
 //   Through 32 layers any other order would move the logits by 0.05 of their norm, as two correct bf16 evaluations differ.
@@ -35,7 +35,7 @@
 // * Attention: a (sequence, kv head, range of cached keys) per workgroup, sums as in decode_glue.hip; the first keys and values are
 //   under way before the queries are known.
 //
-// Measured (graph replay, Llama-3-8B, 512 / 576 positions, MI355X, from box to box): 1 sequence 1584..1612 -> 1209..1230 us, 8 sequences 2025 -> 1650..1698.
+// Measured (graph replay, Llama-3-8B, 512 / 576 positions, MI355X, from box to box): 1 sequence 1584..1612 -> 1190..1215 us, 8 sequences 2025 -> 1620..1670.
 // What bounds it now, per layer and for one sequence (38 us; stamps of the 100 MHz clock): tiles 22 us (1.1 us each in the gate-up
 // projection while their data is there, 1.3 where HBM sets the pace, 1.6 in the others, whose 4x4x4 MFMAs fill the matrix
 // pipe), six exchanges 9, attention's own work 4, the rest waits for the slowest workgroup.  Tried and not kept: a third tile
@@ -200,6 +200,10 @@ __device__ __forceinline__ uint32_t max4(const u32x4& v) { return max(max(v.x, v
 
 #endif
 
+// One kernel per way of multiplying QKV (CHAIN_ROWS: one sequence; CHAIN_QUADS: five to eight; CHAIN_SLICES): with all three in one, 137
+// scalar registers were spilled instead of 61..67, 32 layers of the 8B shapes took 1214 us with one sequence and 1657 with eight (now 1198,
+// 1629), four layers of d 2048 with six 167 (163).
+template <int QKV_MODE>
 __global__ __launch_bounds__(THREADS, 1) void chain_kernel(ChainArgs) {
 #if defined(__HIP_DEVICE_COMPILE__)
     // What a part of the step derives from the thread's number and the arguments it derives again: kept across parts they
@@ -1331,7 +1335,7 @@ __global__ __launch_bounds__(THREADS, 1) void chain_kernel(ChainArgs) {
         st_task = me;
         prime();
     };
-    const int n_layer = a.n_layer, qkv_mode = a.shape[CHAIN_QKV].mode;
+    const int n_layer = a.n_layer;
     const int from = phase;
     auto takes_part = [&](int this_phase) {
         if (this_phase < from) return false;  // (a late workgroup may begin in the middle of a layer)
@@ -1345,9 +1349,9 @@ __global__ __launch_bounds__(THREADS, 1) void chain_kernel(ChainArgs) {
         ARGS;
         if (takes_part(4 * l)) {
             const float* const lut1 = a.layers[l].lin[1].lut;
-            if (qkv_mode == CHAIN_ROWS)
+            if constexpr (QKV_MODE == CHAIN_ROWS)
                 linear(Qkv{}, Rows{}, l, lut1);
-            else if (qkv_mode == CHAIN_QUADS)
+            else if constexpr (QKV_MODE == CHAIN_QUADS)
                 linear(Qkv{}, Quads{}, l, lut1);
             else
                 linear(Qkv{}, Slices{}, l, lut1);
@@ -1357,7 +1361,7 @@ __global__ __launch_bounds__(THREADS, 1) void chain_kernel(ChainArgs) {
             attention(l);
             barrier();  // ... and the other way round
             const float* const lut2 = a.layers[l].lin[2].lut;
-            if (qkv_mode == CHAIN_ROWS)
+            if constexpr (QKV_MODE == CHAIN_ROWS)
                 linear(Out{}, Rows{}, l, lut2);
             else
                 linear(Out{}, Slices{}, l, lut2);
@@ -1365,7 +1369,7 @@ __global__ __launch_bounds__(THREADS, 1) void chain_kernel(ChainArgs) {
         if (takes_part(4 * l + 2)) linear(GateUp{}, Slices{}, l, a.layers[l].lin[3].lut);
         takes_part(4 * l + 3);
         const float* const next = l + 1 < a.n_layer ? a.layers[l + 1].lin[0].lut : a.with_head ? a.head.lut : nullptr;
-        if (qkv_mode == CHAIN_ROWS)
+        if constexpr (QKV_MODE == CHAIN_ROWS)
             linear(Down{}, Rows{}, l, next);
         else
             linear(Down{}, Slices{}, l, next);
@@ -1556,10 +1560,13 @@ __attribute__((visibility("default"))) int nf4hip_decode_chain_joined(const void
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return nf4hip_decode_fail("nf4hip_decode_chain: no current device");
     if (!ready[dev]) {
-        if (hipFuncSetAttribute(reinterpret_cast<const void*>(chain_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, SMEM_BYTES) != hipSuccess)
-            return nf4hip_decode_fail("nf4hip_decode_chain: LDS size");
+        for (const auto kernel : {chain_kernel<CHAIN_SLICES>, chain_kernel<CHAIN_ROWS>, chain_kernel<CHAIN_QUADS>})
+            if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, SMEM_BYTES) != hipSuccess)
+                return nf4hip_decode_fail("nf4hip_decode_chain: LDS size");
         ready[dev] = true;
     }
+    const int mode = a.shape[CHAIN_QKV].mode;
+    const auto kernel = mode == CHAIN_ROWS ? chain_kernel<CHAIN_ROWS> : mode == CHAIN_QUADS ? chain_kernel<CHAIN_QUADS> : chain_kernel<CHAIN_SLICES>;
     a.eps = eps;
     a.pos = pos;
     a.cos_t = cos_t;
@@ -1592,7 +1599,7 @@ __attribute__((visibility("default"))) int nf4hip_decode_chain_joined(const void
             a.layers[i].norm_mid = static_cast<const uint16_t*>(p[12]);
             a.layers[i].norm_next = static_cast<const uint16_t*>(p[13]);
         }
-        hipLaunchKernelGGL(chain_kernel, dim3((unsigned)a.workgroups), dim3(THREADS), SMEM_BYTES, s, a);
+        hipLaunchKernelGGL(kernel, dim3((unsigned)a.workgroups), dim3(THREADS), SMEM_BYTES, s, a);
     }
     return hipGetLastError() == hipSuccess ? 0 : nf4hip_decode_fail("nf4hip_decode_chain: launch failed");
 }

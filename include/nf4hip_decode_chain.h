@@ -28,7 +28,7 @@ extern "C" {
  * `layers` and `head` are host arrays and not referred to after the call.  `workspace`: at least
  * nf4hip_decode_chain_workspace_bytes() bytes (0: this shape or device is not served), 16-byte aligned, any contents, this
  * call's alone until it has run.  The workgroups wait for each other, and only for workgroups that are already running: the step ends
- * however few of them the device holds at a time, and those that find a CU later join at the next linear.  max_workgroups > 0: at
+ * however few of them the device holds at a time, and those that find a CU later join at the next linear or layer.  max_workgroups > 0: at
  * most so many (a workgroup takes a whole CU; the answer is the same bit for bit).
  *
  * nf4hip_decode_chain_joined: the same with workgroups held back, as other work on the device holds them back by itself:
